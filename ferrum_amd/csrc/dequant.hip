@@ -46,8 +46,8 @@ __device__ __forceinline__ void emit4(const uint8_t* w, size_t src_row, size_t d
             lo = f32_to_f16_bits(v0) | (f32_to_f16_bits(v1) << 16);
             hi = f32_to_f16_bits(v2) | (f32_to_f16_bits(v3) << 16);
         } else {
-            lo = f32_to_bf16_bits(v0) | (f32_to_bf16_bits(v1) << 16);
-            hi = f32_to_bf16_bits(v2) | (f32_to_bf16_bits(v3) << 16);
+            lo = f32_pair_to_bf16_bits(v0, v1);
+            hi = f32_pair_to_bf16_bits(v2, v3);
         }
         *reinterpret_cast<uint2*>(static_cast<uint16_t*>(out) + base) = make_uint2(lo, hi);
     }

@@ -30,7 +30,7 @@ __device__ __forceinline__ uint32_t pack2(float a, float b) {
     if constexpr (DT == 1) {
         return f32_to_f16_bits(a) | (f32_to_f16_bits(b) << 16);
     } else {
-        return f32_to_bf16_bits(a) | (f32_to_bf16_bits(b) << 16);
+        return f32_pair_to_bf16_bits(a, b);
     }
 }
 

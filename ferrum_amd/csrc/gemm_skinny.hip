@@ -617,8 +617,8 @@ __global__ __launch_bounds__(kResThreads) void expert_resident_kernel(const uint
                                 packed.x = f32_to_f16_bits(acc[t][0]) | (f32_to_f16_bits(acc[t][1]) << 16);
                                 packed.y = f32_to_f16_bits(acc[t][2]) | (f32_to_f16_bits(acc[t][3]) << 16);
                             } else {
-                                packed.x = f32_to_bf16_bits(acc[t][0]) | (f32_to_bf16_bits(acc[t][1]) << 16);
-                                packed.y = f32_to_bf16_bits(acc[t][2]) | (f32_to_bf16_bits(acc[t][3]) << 16);
+                                packed.x = f32_pair_to_bf16_bits(acc[t][0], acc[t][1]);
+                                packed.y = f32_pair_to_bf16_bits(acc[t][2], acc[t][3]);
                             }
                             *reinterpret_cast<uint2*>(static_cast<uint16_t*>(ydst) + base) = packed;
                         } else {
@@ -815,8 +815,8 @@ __global__ __launch_bounds__(kResThreads) void expert_ring_kernel(const uint8_t*
                             packed.x = f32_to_f16_bits(acc[t][0]) | (f32_to_f16_bits(acc[t][1]) << 16);
                             packed.y = f32_to_f16_bits(acc[t][2]) | (f32_to_f16_bits(acc[t][3]) << 16);
                         } else {
-                            packed.x = f32_to_bf16_bits(acc[t][0]) | (f32_to_bf16_bits(acc[t][1]) << 16);
-                            packed.y = f32_to_bf16_bits(acc[t][2]) | (f32_to_bf16_bits(acc[t][3]) << 16);
+                            packed.x = f32_pair_to_bf16_bits(acc[t][0], acc[t][1]);
+                            packed.y = f32_pair_to_bf16_bits(acc[t][2], acc[t][3]);
                         }
                         *reinterpret_cast<uint2*>(static_cast<uint16_t*>(ydst) + base) = packed;
                     }

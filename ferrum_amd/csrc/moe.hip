@@ -106,7 +106,7 @@ __device__ __forceinline__ void store8(void* p, size_t i, uint32_t dtype, const 
 #pragma unroll
         for (int j = 0; j < 4; ++j)
             w[j] = dtype == FH_F16 ? (f32_to_f16_bits(v[2 * j]) | (f32_to_f16_bits(v[2 * j + 1]) << 16))
-                                   : (f32_to_bf16_bits(v[2 * j]) | (f32_to_bf16_bits(v[2 * j + 1]) << 16));
+                                   : (f32_pair_to_bf16_bits(v[2 * j], v[2 * j + 1]));
         *reinterpret_cast<uint4*>(static_cast<uint16_t*>(p) + i) = make_uint4(w[0], w[1], w[2], w[3]);
     }
 }

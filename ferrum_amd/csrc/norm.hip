@@ -56,8 +56,8 @@ __device__ __forceinline__ void store4(void* p, size_t group, float4 v) {
         static_cast<uint2*>(p)[group] = make_uint2(f32_to_f16_bits(v.x) | (f32_to_f16_bits(v.y) << 16),
                                                    f32_to_f16_bits(v.z) | (f32_to_f16_bits(v.w) << 16));
     } else {
-        static_cast<uint2*>(p)[group] = make_uint2(f32_to_bf16_bits(v.x) | (f32_to_bf16_bits(v.y) << 16),
-                                                   f32_to_bf16_bits(v.z) | (f32_to_bf16_bits(v.w) << 16));
+        static_cast<uint2*>(p)[group] = make_uint2(f32_pair_to_bf16_bits(v.x, v.y),
+                                                   f32_pair_to_bf16_bits(v.z, v.w));
     }
 }
 

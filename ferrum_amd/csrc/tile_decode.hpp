@@ -41,7 +41,7 @@ __device__ __forceinline__ uint32_t fma_pair(float qa, float qb, float scale, fl
         r.y = (_Float16)fmaf(qb, scale, offset);
         return __builtin_bit_cast(uint32_t, r);
     } else {
-        return f32_to_bf16_bits(fmaf(qa, scale, offset)) | (f32_to_bf16_bits(fmaf(qb, scale, offset)) << 16);
+        return f32_pair_to_bf16_bits(fmaf(qa, scale, offset), fmaf(qb, scale, offset));
     }
 }
 
