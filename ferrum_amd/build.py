@@ -19,7 +19,9 @@ OBJ_DIR = os.path.join(HERE, "build")
 LIB_DIR = os.path.join(HERE, "lib")
 LIB_PATH = os.path.join(LIB_DIR, "libferrum_hip.so")
 
-SOURCES = ["capi.hip", "dequant.hip", "gemv.hip", "gemv_stream.hip", "probe.hip", "gemm.hip", "gemm_skinny.hip", "moe.hip", "norm.hip"]
+SOURCES = ["capi.hip", "dequant.hip", "gemv.hip", "gemv_stream.hip", "probe.hip", "gemm.hip", "gemm_rows.hip",
+           "gemm_rows_q4_k.hip", "gemm_rows_q5_k.hip", "gemm_rows_q6_k.hip", "gemm_rows_iq4_xs.hip", "gemm_rows_q8_0.hip",
+           "gemm_skinny.hip", "moe.hip", "norm.hip"]
 
 FLAGS = [
     "--offload-arch=gfx950",
@@ -84,8 +86,10 @@ def build(extra_flags: list[str] | None = None, jobs: int = 8, output: str | Non
         # the sources with hand-scheduled loads are also compiled to assembly text, which is checked
         # for what the compiler must not have done around those loads
         texts = {s: pool.submit(_assembly, s, extra) for s in isa_check.CHECKED_SOURCES}
+        counted = {s: pool.submit(_assembly, s, extra) for s in isa_check.COUNTED_SOURCES}
         objs = list(pool.map(lambda s: _compile(s, extra), SOURCES))
         broken = [v for s, t in texts.items() for v in isa_check.violations(t.result(), s)]
+        broken += [v for s, t in counted.items() for v in isa_check.counted_violations(t.result(), s)]
     if broken:
         raise RuntimeError("the generated code breaks an invariant of the hand-scheduled loads:\n" + "\n".join(broken[:40]))
     target = output or LIB_PATH

@@ -342,7 +342,7 @@ fh_status fh_device_create(int32_t ordinal, fh_device** out) {
     d->tuning["gemm_skinny_max_rows"] = 64; // largest M that takes the register-dequant MFMA kernel (0 = never)
     d->tuning["expert_grouped_min_assignments"] = 32;  // fewest assignments grouped by expert (0 = never)
     d->tuning["moe_fold_route"] = 1;        // fh_moe_ffn, one token: the gate|up launch routes the token itself (0 = a moe_route launch first)
-    d->tuning["gemm_few_tiles_split"] = 1;  // up to 16 rows and few weight tiles per workgroup: super-blocks dealt over the waves (0 = whole tiles per wave)
+    d->tuning["gemm_few_tiles_split"] = 1;  // few rows: a tile's super-blocks dealt over the waves, any K (0 = whole tiles per wave, the kernels for rows that fit LDS or not)
     d->tuning["moe_fold_combine"] = 1;      // fh_moe_ffn with few tokens: down projection and weighted sum in one launch (0 = two)
     d->tuning["gemm_resident"] = 1;         // rows that fit LDS whole take the rows-resident kernel (0 = square tiles)
     d->tuning["gemv_stream_own_loads"] = 1; // the streamed Q4_K GEMV's waves load the super-blocks they multiply (tiles of up to 14 rows); 0: the tile row by row
@@ -734,6 +734,46 @@ fh_status fh_embedding_gather_quantized(fh_device* device, const fh_qmatrix* wei
 
 namespace {
 
+// A dense product's shape and the device's kernel switches; the caller sets w, x and y.
+GemmArgs gemm_args(const fh_device* device, uint32_t ggml_type, uint64_t n, uint64_t k, uint32_t m, uint32_t x_dtype,
+                   uint32_t y_dtype) {
+    GemmArgs g{};
+    g.ggml_type = ggml_type;
+    g.n = (uint32_t)n;
+    g.k = (uint32_t)k;
+    g.m = m;
+    g.x_dtype = x_dtype;
+    g.y_dtype = y_dtype;
+    g.cu_count = device->props.multiProcessorCount;
+    g.wide_min_rows = (int)tuning(device, "gemm_wide_min_rows");
+    g.wide_shape = (int)tuning(device, "gemm_wide_shape");
+    g.wide32_tile = (int)tuning(device, "gemm_wide32_tile");
+    g.skinny_max_rows = (int)tuning(device, "gemm_skinny_max_rows");
+    g.resident_switch = tuning(device, "gemm_resident") != 0;
+    g.rows_resident = g.resident_switch && expert_rows_fit_lds((uint32_t)k, 1, 1);
+    g.few_rows = tuning(device, "gemm_few_tiles_split") != 0;
+    return g;
+}
+
+// Brings the scratch to what the product needs behind `used` bytes of the caller's at its head.
+fh_status prepare_gemm(fh_device* device, GemmArgs& g, size_t used) {
+    const size_t at = align256(used);
+    fh_status st = ensure_scratch(device, at + g.rows_plan.partial_bytes);
+    if (st != FH_OK) return st;
+    g.counters = scratch_counters(device);
+    g.partials = reinterpret_cast<float*>(scratch_data(device) + at);
+    return FH_OK;
+}
+
+// the exact product of several rows, by whichever kernel
+const char* batch_name(uint32_t ggml_type) {
+    return ggml_type == kQ4K    ? "q4_k_gemm"
+           : ggml_type == kQ5K  ? "q5_k_gemm"
+           : ggml_type == kQ6K  ? "q6_k_gemm"
+           : ggml_type == kQ8_0 ? "q8_0_gemm"
+                                : "iq4_xs_gemm";
+}
+
 // `f32_tile_from`: row count from which f32 activations take the f16 tiles; negative = the
 // device's gemm_f32_min_rows setting
 fh_status project(fh_device* device, const fh_qmatrix* weight, const fh_view* x, uint32_t m,
@@ -773,34 +813,34 @@ fh_status project(fh_device* device, const fh_qmatrix* weight, const fh_view* x,
     const int64_t f32_tile_rows = f32_tile_from >= 0 ? f32_tile_from : tuning(device, "gemm_f32_min_rows");
     const bool f32_tile = !silu_mul && x->dtype == FH_F32 && f32_tile_rows > 0 && m >= (uint64_t)f32_tile_rows &&
                           ((uintptr_t)xr.begin & 15u) == 0;
-    const void* tile_x = xr.begin;
-    if (f32_tile) {
-        st = ensure_scratch(device, (size_t)m * k * sizeof(uint16_t));
-        if (st != FH_OK) return st;
-        launch_round_to_f16(device->stream, reinterpret_cast<const float*>(xr.begin),
-                            reinterpret_cast<uint16_t*>(scratch_data(device)), (size_t)m * k);
-        tile_x = scratch_data(device);
-    }
     const bool tile = f32_tile || (!silu_mul && m >= (uint32_t)tuning(device, "gemm_min_rows") && x->dtype != FH_F32);
-    if (tile) {
-        GemmArgs a{};
-        a.ggml_type = weight->ggml_type;
-        a.w = weight->ptr;
-        a.x = tile_x;
-        a.y = const_cast<uint8_t*>(yr.begin);
-        a.n = (uint32_t)n;
-        a.k = (uint32_t)k;
-        a.m = m;
-        a.x_dtype = f32_tile ? FH_F16 : x->dtype;
-        a.y_dtype = y->dtype;
-        a.cu_count = device->props.multiProcessorCount;
-        a.wide_min_rows = (int)tuning(device, "gemm_wide_min_rows");
-        a.wide_shape = (int)tuning(device, "gemm_wide_shape");
-        a.wide32_tile = (int)tuning(device, "gemm_wide32_tile");
-        a.skinny_max_rows = (int)tuning(device, "gemm_skinny_max_rows");
-        a.rows_resident = tuning(device, "gemm_resident") != 0 && expert_rows_fit_lds((uint32_t)k, 1, 1);
-        a.few_tiles_split = tuning(device, "gemm_few_tiles_split") != 0;
-        device->last_operation = launch_gemm(device->stream, a);
+    // A batch of exact f32 rows: the GEMV kernels read every weight once per row, the few-rows kernel
+    // once per sixteen.  Four rows of 17408 x 5120 take it 36 us, the GEMV 36 for Q4_K (20 and 27 for two
+    // and three) and 43 - 58 for the other formats; sixteen rows 38 against 121 - 230.  Where a GEMV
+    // kernel or its K segments are asked for by name, those run.
+    const bool f32_batch = !tile && !silu_mul && x->dtype == FH_F32 && m >= (weight->ggml_type == kQ4K ? 5u : 4u) &&
+                           m >= (uint32_t)tuning(device, "gemm_min_rows") && tuning(device, "gemv_stream") == 1 &&
+                           tuning(device, "k_quant_gemv_ksplit") == 0;
+    GemmArgs g{};
+    if (tile || f32_batch) g = gemm_args(device, weight->ggml_type, n, k, m, f32_tile ? FH_F16 : x->dtype, y->dtype);
+    if (f32_batch && g.few_rows) {
+        g.rows_plan = gemm_rows_plan(g.ggml_type, g.n, g.k, g.m, g.x_dtype, g.cu_count);
+        if (g.rows_plan.counters > fh_device::kCounterWords) g.rows_plan = RowsPlan{};
+    }
+    if (tile || g.rows_plan.rows != 0) {
+        g.w = weight->ptr;
+        g.x = xr.begin;
+        g.y = const_cast<uint8_t*>(yr.begin);
+        if (tile) gemm_takes_rows(g);
+        st = prepare_gemm(device, g, f32_tile ? (size_t)m * k * sizeof(uint16_t) : 0);
+        if (st != FH_OK) return st;
+        if (f32_tile) {
+            launch_round_to_f16(device->stream, reinterpret_cast<const float*>(xr.begin),
+                                reinterpret_cast<uint16_t*>(scratch_data(device)), (size_t)m * k);
+            g.x = scratch_data(device);
+        }
+        const char* const name = launch_gemm(device->stream, g);
+        device->last_operation = tile ? name : batch_name(weight->ggml_type);
     } else {
         GemvArgs a{};
         a.ggml_type = weight->ggml_type;
@@ -823,13 +863,7 @@ fh_status project(fh_device* device, const fh_qmatrix* weight, const fh_view* x,
         const char* name = "";
         st = run_gemv(device, a, &name);
         if (st != FH_OK) return st;
-        if (m > 1)
-            name = weight->ggml_type == kQ4K   ? "q4_k_gemm"
-                   : weight->ggml_type == kQ5K ? "q5_k_gemm"
-                   : weight->ggml_type == kQ6K ? "q6_k_gemm"
-                   : weight->ggml_type == kQ8_0 ? "q8_0_gemm"
-                                                : "iq4_xs_gemm";
-        device->last_operation = name;
+        device->last_operation = m > 1 ? batch_name(weight->ggml_type) : name;
     }
     FH_HIP(hipGetLastError());
     return FH_OK;
@@ -1604,27 +1638,15 @@ fh_status expert_project(fh_device* device, const fh_qmatrix* weight, const fh_v
         if (form == FH_INPUT_GATHER) return project(device, shared->weight, x, shared->tokens, shared->y, false);
         if (shared->tokens < (uint64_t)tuning(device, "gemm_min_rows") || ((uintptr_t)sxr.begin & 15u) != 0)
             return project(device, shared->weight, shared->x, shared->tokens, shared->y, true);
-        st = ensure_scratch(device, (size_t)shared->tokens * k * sizeof(uint16_t));
+        GemmArgs g = gemm_args(device, weight->ggml_type, rows, k, shared->tokens, x->dtype, y->dtype);
+        gemm_takes_rows(g);
+        st = prepare_gemm(device, g, (size_t)shared->tokens * k * sizeof(uint16_t));
         if (st != FH_OK) return st;
         launch_expert_silu_mul(device->stream, sxr.begin, scratch_data(device), shared->tokens, (uint32_t)k, x->dtype,
                                x->dtype);
-        GemmArgs g{};
-        g.ggml_type = weight->ggml_type;
         g.w = shared->weight->ptr;
         g.x = scratch_data(device);
         g.y = const_cast<uint8_t*>(syr.begin);
-        g.n = (uint32_t)rows;
-        g.k = (uint32_t)k;
-        g.m = shared->tokens;
-        g.x_dtype = x->dtype;
-        g.y_dtype = y->dtype;
-        g.cu_count = device->props.multiProcessorCount;
-        g.wide_min_rows = (int)tuning(device, "gemm_wide_min_rows");
-        g.wide_shape = (int)tuning(device, "gemm_wide_shape");
-        g.wide32_tile = (int)tuning(device, "gemm_wide32_tile");
-        g.skinny_max_rows = (int)tuning(device, "gemm_skinny_max_rows");
-        g.rows_resident = tuning(device, "gemm_resident") != 0 && expert_rows_fit_lds((uint32_t)k, 1, 1);
-        g.few_tiles_split = tuning(device, "gemm_few_tiles_split") != 0;
         device->last_operation = launch_gemm(device->stream, g);
         FH_HIP(hipGetLastError());
         return FH_OK;

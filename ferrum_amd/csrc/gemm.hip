@@ -11,6 +11,7 @@
 // Tile: 128 (M) x 128 (N) x 64 (K) per 256-thread workgroup; four waves in a
 // 2 x 2 arrangement, each owning 64 x 64 outputs as 2 x 2 MFMA 32x32x16 tiles.
 // LDS rows are padded to 72 halfs so 128-bit fragment reads are conflict free.
+#include <algorithm>
 #include <type_traits>
 
 #include "device_utils.hpp"
@@ -1181,14 +1182,22 @@ double wide16_estimate(uint32_t m, uint32_t n, uint32_t k, int cus) {
     return (rounds < 1.0 ? 1.0 : rounds) * 105.0 * wide_row_length_factor(k);
 }
 
-// The rows-resident kernel: a start that grows with the matrix, then a cost per group of rows that
-// LDS holds at once (32 rows of up to 2560, 16 of up to 5120), since every weight is decoded once
-// per group.  Measured at 48 - 512 rows on the shapes above and 151936 x 2048; within a sixth of each.
-double resident_estimate(uint32_t m, uint32_t n, uint32_t k) {
-    const double weights = (double)n * (double)k;
-    if ((size_t)32 * k * 2 <= 160u * 1024) return 12.0 + weights * 0.68e-7 + weights * 1.25e-7 * ((m + 31) / 32);
-    const double start = weights * 1.5e-7;
-    return 12.0 + (start < 14.0 ? start : 14.0) + weights * 8.3e-8 * ((m + 15) / 16);
+// The rows-resident kernel: a start, the stream of the matrix, and a decode of every weight per group
+// of rows that LDS holds at once (32 rows of up to 2560, 16 of up to 5120; us per million weights).
+// Measured at 4 - 64 rows on 20480 .. 151936 x 2048 / 5120; within a tenth of most of those.
+double resident_estimate(uint32_t ggml_type, uint32_t m, uint32_t n, uint32_t k) {
+    const double weights = (double)n * (double)k * 1e-6;
+    const bool groups_of_32 = (size_t)32 * k * 2 <= 160u * 1024;
+    const double groups = groups_of_32 ? (m + 31) / 32 : (m + 15) / 16;
+    if (ggml_type == kQ6K) return 13.0 + weights * (groups_of_32 ? 0.01 + 0.2 * groups : 0.033 + 0.195 * groups);
+    const double heavier = ggml_type == kQ4K ? 1.0 : ggml_type == kQ5K ? 1.5 : ggml_type == kIQ4XS ? 1.45 : 1.35;
+    return 8.0 + heavier * weights * (groups_of_32 ? 0.02 + 0.135 * groups : 0.047 + 0.09 * groups);
+}
+
+// What the heavier decodes add to the tiles' estimates, which were measured on Q4_K (at 512 rows of
+// 17408 x 5120 112 us, Q5_K 117, IQ4_XS 115, Q6_K and Q8_0 141).
+double wide_format_factor(uint32_t ggml_type) {
+    return ggml_type == kQ6K || ggml_type == kQ8_0 ? 1.22 : ggml_type == kQ4K ? 1.0 : 1.04;
 }
 
 template <uint32_t TYPE, int DT, int NT, int RT>
@@ -1246,38 +1255,87 @@ void launch_wide_nt(hipStream_t s, const GemmArgs& a, const WidePlan& plan, cons
 
 }  // namespace
 
-const char* launch_gemm(hipStream_t s, const GemmArgs& a) {
-    // the 256-row tile pays off only when its workgroups cover at least half the chip
+namespace {
+
+// Which of the tile forms would take a product of at least wide_min_rows rows, and the estimates.
+struct TileChoice {
+    bool wide_pays;      // the 16x16x32 form's workgroups cover at least half the chip
+    WidePlan p32;        // the 32x32x16 form's tile, nt = 0 when it does not compete
+    double us32, us16;
+};
+TileChoice tile_choice(const GemmArgs& a) {
+    TileChoice c{};
     const uint64_t wide_wgs = (uint64_t)((a.m + kWM - 1) / kWM) * ((a.n + 127) / 128);
-    const bool wide_pays = a.m >= (uint32_t)a.wide_min_rows && wide_wgs * 2 >= (uint64_t)a.cu_count;
+    c.wide_pays = a.m >= (uint32_t)a.wide_min_rows && wide_wgs * 2 >= (uint64_t)a.cu_count;
+    c.us32 = 1e300;
+    if (a.wide_shape != 0 && a.m >= (uint32_t)a.wide_min_rows) {
+        if (a.wide32_tile != 0) {
+            c.p32 = wide32_make(a.m, a.n, a.wide32_tile / 10, a.wide32_tile % 10, a.cu_count);
+            if (c.p32.tiles_n == 0) c.p32 = wide32_make(a.m, a.n, 1, 4);   // no width of the 96-column tile fits this shape
+            c.us32 = 0.0;
+        } else {
+            c.p32 = wide32_plan(a.m, a.n, a.k, a.cu_count, &c.us32);
+            if (c.p32.nt == 0 && a.wide_shape == 2 && c.wide_pays) {
+                c.p32 = wide32_make(a.m, a.n, 2, 5);
+                c.us32 = 0.0;
+            }
+        }
+    }
+    c.us16 = c.wide_pays && a.wide_shape != 2 ? wide16_estimate(a.m, a.n, a.k, a.cu_count) : 1e300;
+    c.us32 *= wide_format_factor(a.ggml_type);
+    c.us16 *= wide_format_factor(a.ggml_type);
+    return c;
+}
+
+}  // namespace
+
+// Up to 128 rows the few-rows kernel competes: the smallest estimate among it, the kernel that keeps
+// rows in LDS (where they fit) and the tiles takes the call.  It wins wherever a round or two of its
+// workgroups cover the matrix (Q4_K, f16, us, against the kernel that had these rows: 16 / 32 / 64 x
+// 17408 x 5120 17.7 / 21.2 / 37.8 against 19.7 / 31.9 / 45.9, 16 x 4096 x 2048 4.4 / 5.4), and for rows
+// too long for LDS there is nothing else (8 / 64 / 128 x 5120 x 17408 20.9 / 40.7 / 77 against 43.6 /
+// 106 / 189 on a slab and a square-tile kernel).  Over many rounds its starts add up and the resident
+// kernel's waves, which stream from tile to tile, are ahead (16 x 151936 x 5120 133 against 116).
+bool gemm_takes_rows(GemmArgs& a) {
+    if (!a.few_rows || a.m < 2 || a.m > 128) return false;
+    if (a.wide32_tile != 0 && a.wide_shape != 0 && a.m >= (uint32_t)a.wide_min_rows) return false;   // a tile is asked for
+    const RowsPlan plan = gemm_rows_plan(a.ggml_type, a.n, a.k, a.m, a.x_dtype, a.cu_count);
+    if (plan.counters > fh_device::kCounterWords) return false;
+    if (a.resident_switch) {
+        const TileChoice c = tile_choice(a);
+        double other = std::min(c.us32, c.us16);
+        if (a.rows_resident) other = std::min(other, resident_estimate(a.ggml_type, a.m, a.n, a.k));
+        if (plan.estimate_us >= other) return false;
+    } else if (a.m > (uint32_t)a.skinny_max_rows) {
+        return false;
+    }
+    a.rows_plan = plan;
+    return true;
+}
+
+const char* launch_gemm(hipStream_t s, const GemmArgs& a) {
+    if (a.rows_plan.rows != 0) {
+        static const char* const names[2][5] = {
+            {"q4_k_gemm_mfma_resident", "q5_k_gemm_mfma_resident", "q6_k_gemm_mfma_resident", "iq4_xs_gemm_mfma_resident",
+             "q8_0_gemm_mfma_resident"},
+            {"q4_k_gemm_mfma_skinny", "q5_k_gemm_mfma_skinny", "q6_k_gemm_mfma_skinny", "iq4_xs_gemm_mfma_skinny",
+             "q8_0_gemm_mfma_skinny"}};
+        launch_gemm_rows(s, a);
+        const int f = a.ggml_type == kQ4K ? 0 : a.ggml_type == kQ5K ? 1 : a.ggml_type == kQ6K ? 2 : a.ggml_type == kIQ4XS ? 3 : 4;
+        return names[a.rows_resident || a.m > (uint32_t)a.skinny_max_rows ? 0 : 1][f];
+    }
+    const TileChoice choice = tile_choice(a);
+    const bool wide_pays = choice.wide_pays;
+    WidePlan p32 = choice.p32;
+    const double us32 = choice.us32, us16 = choice.us16;
     // Rows that fit LDS for their whole length take the kernel that keeps them there and streams
-    // the weights past them through registers.  Against the register-dequant kernel that stages
-    // the rows slab by slab (up to 64 rows) it is 15% faster at 2 - 16 rows and up to twice at 64
-    // (64 x 4096 x 4096: 14.1 against 29.7 us; 64 x 17408 x 5120: 52.8 against 74.0 us, the same
-    // bits), except for 512-long rows in 16-row batches or
-    // less, where a launch is 4 us either way; against the square tiles 1.4 - 2.2 times
+    // the weights past them through registers: against the square tiles 1.4 - 2.2 times
     // (512 x 1024 x 2048: 11.5 against 22.8 us).
     // Rows longer than 2560 fit only 16 at a time, and every weight is then decoded M / 16 times:
     // that still wins up to 256 rows (256 x 5120 x 5120: 51 against 86 us) and loses at 512 (95
     // against 84 us).
     // From wide_min_rows rows on, the tiles of the 32x32x16 form compete: the smallest estimate
     // among them, the 16x16x32 form and the rows-resident kernel takes the call.
-    WidePlan p32{};
-    double us32 = 1e300;
-    if (a.wide_shape != 0 && a.m >= (uint32_t)a.wide_min_rows) {
-        if (a.wide32_tile != 0) {
-            p32 = wide32_make(a.m, a.n, a.wide32_tile / 10, a.wide32_tile % 10, a.cu_count);
-            if (p32.tiles_n == 0) p32 = wide32_make(a.m, a.n, 1, 4);   // no width of the 96-column tile fits this shape
-            us32 = 0.0;
-        } else {
-            p32 = wide32_plan(a.m, a.n, a.k, a.cu_count, &us32);
-            if (p32.nt == 0 && a.wide_shape == 2 && wide_pays) {
-                p32 = wide32_make(a.m, a.n, 2, 5);
-                us32 = 0.0;
-            }
-        }
-    }
-    const double us16 = wide_pays && a.wide_shape != 2 ? wide16_estimate(a.m, a.n, a.k, a.cu_count) : 1e300;
     if (a.rows_resident) {
         const bool few = a.m <= (uint32_t)a.skinny_max_rows;
         const bool groups_of_32 = (size_t)32 * a.k * 2 <= 160u * 1024;
@@ -1285,16 +1343,15 @@ const char* launch_gemm(hipStream_t s, const GemmArgs& a) {
         // cost grows with the row count: 65 x 17408 x 5120 takes 67 against 82 us and 128 rows
         // 87 against 87; with groups of 32 (K = 2048) 128 rows take 30 against 41 us and 256
         // rows 49 against 49.
-        bool take = few          ? !(a.k <= 512 && a.m <= 16)
+        bool take = few          ? true
                     : wide_pays ? a.m <= (groups_of_32 ? 192u : 96u)
                                 : groups_of_32 || a.m <= 256;
         // (the estimates were measured on rows of 2048 and more; shorter ones keep the rule above)
         if (p32.nt != 0 && (a.k >= 1024 || a.wide32_tile != 0))
-            take = resident_estimate(a.m, a.n, a.k) < (us32 < us16 ? us32 : us16);
+            take = resident_estimate(a.ggml_type, a.m, a.n, a.k) < (us32 < us16 ? us32 : us16);
         if (take) return launch_gemm_resident(s, a);
     }
     if (p32.nt != 0 && us16 < us32) p32.nt = 0;
-    if (p32.nt == 0 && a.m <= (uint32_t)a.skinny_max_rows) return launch_gemm_skinny(s, a);
     if (wide_pays || p32.nt != 0) {
         const WidePlan plan = wide_plan(a.m, a.n, a.cu_count);
         if (a.ggml_type == kQ4K) {

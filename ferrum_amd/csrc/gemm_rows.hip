@@ -1,0 +1,94 @@
+// Plan and launch of the few-rows projection (gemm_rows.hpp).
+#include "gemm_rows.hpp"
+
+namespace fh {
+
+namespace {
+
+// What one super-block of one weight tile costs a wave, in us, with two waves on the SIMD: the decode,
+// the matrix instructions of 16 or 32 rows and their share of the stream.  From 17408 x 5120 and
+// 5120 x 17408 (f16: 17.7 / 21.2 us at 16 / 32 rows for Q4_K, 30.8 / 40.5 for Q6_K; f32: 38).
+double unit_us(uint32_t ggml_type, uint32_t x_dtype, uint32_t rows) {
+    if (x_dtype == FH_F32) return 2.3;
+    switch (ggml_type) {
+        case kQ4K: return rows == 16 ? 0.90 : 1.15;
+        case kQ6K: return rows == 16 ? 1.80 : 2.40;
+        default: return rows == 16 ? 1.30 : 1.70;
+    }
+}
+
+constexpr double kStartUs = 4.0;      // launch, first loads, exchange of the waves' sums
+constexpr double kExchangeUs = 4.0;   // partial sums of K segments through device memory
+
+}  // namespace
+
+RowsPlan gemm_rows_plan(uint32_t ggml_type, uint32_t n, uint32_t k, uint32_t m, uint32_t x_dtype, int cu_count) {
+    RowsPlan plan{};
+    const uint32_t nb = k / 256, tiles = (n + 15) / 16, cus = cu_count > 0 ? (uint32_t)cu_count : 256u;
+    plan.rows = x_dtype != FH_F32 && m > 16 ? 32 : 16;
+    plan.groups = (m + plan.rows - 1) / plan.rows;
+    plan.k_waves = nb >= 8 ? 8 : nb >= 4 ? 4 : nb >= 2 ? 2 : 1;
+    const uint32_t tile_waves = 8 / plan.k_waves;
+    const double unit = unit_us(ggml_type, x_dtype, 16);
+    // Tiles per wave and K segments, from the matrix alone: the sums of a row then do not depend on how
+    // many rows come with it.  Rounds of one workgroup per compute unit, each as long as the
+    // super-blocks of its longest wave.  8 x 17408 x 5120: 17.2 us with five tiles in one round of 218
+    // workgroups, 21 - 26 with fewer tiles in more rounds, 25 - 31 with K cut in two; 8 x 5120 x 17408:
+    // 20.8 with four tiles and three segments, 22 - 41 without segments.
+    double best = 1e300;
+    for (uint32_t segments = 1; segments <= 8; ++segments) {
+        const uint32_t seg_blocks = (nb + segments - 1) / segments;
+        if ((nb + seg_blocks - 1) / seg_blocks != segments || (segments > 1 && seg_blocks < plan.k_waves)) continue;
+        const uint32_t per_wave = (seg_blocks + plan.k_waves - 1) / plan.k_waves;
+        for (uint32_t t = 1; t <= 5; ++t) {
+            const uint32_t tile_groups = (tiles + t * tile_waves - 1) / (t * tile_waves);
+            const uint64_t wgs = (uint64_t)tile_groups * segments;
+            const double us = (double)((wgs + cus - 1) / cus) * (kStartUs + per_wave * t * unit) +
+                              (segments > 1 ? kExchangeUs : 0.0);
+            if (us < best) {
+                best = us;
+                plan.tiles = t;
+                plan.segments = segments;
+                plan.seg_blocks = seg_blocks;
+                plan.tile_groups = tile_groups;
+            }
+        }
+    }
+    const uint32_t per_wave = (plan.seg_blocks + plan.k_waves - 1) / plan.k_waves;
+    // (from two rounds on a compute unit's next workgroup starts as soon as one ends: rounds need not be whole)
+    const double rounds = (double)((uint64_t)plan.tile_groups * plan.segments * plan.groups) / (double)cus;
+    plan.estimate_us = (rounds <= 1.0 ? 1.0 : rounds <= 2.0 ? 2.0 : rounds + 0.2) *
+                           (kStartUs + per_wave * plan.tiles * unit_us(ggml_type, x_dtype, plan.rows)) +
+                       (plan.segments > 1 ? kExchangeUs : 0.0);
+    plan.counters = plan.segments > 1 ? (size_t)plan.tile_groups * plan.groups : 0;
+    plan.partial_bytes = plan.segments > 1 ? (size_t)plan.segments * m * n * sizeof(float) : 0;
+    return plan;
+}
+
+void launch_gemm_rows(hipStream_t s, const GemmArgs& a) {
+    const RowsPlan& plan = a.rows_plan;
+    RowsParams p{};
+    p.w = static_cast<const uint8_t*>(a.w);
+    p.x = static_cast<const uint8_t*>(a.x);
+    p.y = a.y;
+    p.m = a.m;
+    p.n = a.n;
+    p.nb = a.k / 256;
+    p.y_dtype = a.y_dtype;
+    p.k_waves = plan.k_waves;
+    p.groups = plan.groups;
+    p.tile_groups = plan.tile_groups;
+    p.segments = plan.segments;
+    p.seg_blocks = plan.seg_blocks;
+    p.partials = a.partials;
+    p.counters = a.counters;
+    switch (a.ggml_type) {
+        case kQ4K: return launch_rows_q4_k(s, a.x_dtype, plan, p);
+        case kQ5K: return launch_rows_q5_k(s, a.x_dtype, plan, p);
+        case kQ6K: return launch_rows_q6_k(s, a.x_dtype, plan, p);
+        case kIQ4XS: return launch_rows_iq4_xs(s, a.x_dtype, plan, p);
+        default: return launch_rows_q8_0(s, a.x_dtype, plan, p);
+    }
+}
+
+}  // namespace fh

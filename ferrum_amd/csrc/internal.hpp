@@ -243,6 +243,19 @@ struct GemvScratch {
 };
 GemvScratch gemv_scratch(const GemvArgs& a);
 
+// gemm_rows.hip: a few rows, f16 / bf16 on weights rounded to their type or f32 on exact f32 weights
+struct RowsPlan {
+    uint32_t rows;            // rows a workgroup multiplies: 16 or 32
+    uint32_t groups;          // groups of that many rows
+    uint32_t k_waves;         // waves that share a tile's super-blocks
+    uint32_t tiles;           // weight tiles of 16 rows per wave
+    uint32_t tile_groups, segments, seg_blocks;
+    size_t counters;          // scratch counter words (0: K is not cut)
+    size_t partial_bytes;     // scratch for partial sums
+    double estimate_us;
+};
+RowsPlan gemm_rows_plan(uint32_t ggml_type, uint32_t n, uint32_t k, uint32_t m, uint32_t x_dtype, int cu_count);
+
 // gemm.hip
 struct GemmArgs {
     uint32_t ggml_type;
@@ -255,7 +268,7 @@ struct GemmArgs {
     int wide_min_rows;   // smallest M that takes the 256-row tile
     int wide_shape;      // matrix instruction of the 256-row tile: 0 = 16x16x32, 1 = 32x32x16 where it wins, 2 = always
     int wide32_tile;     // 0 = chosen by shape; else 10 x (row tiles per wave) + column tiles of the 32x32x16 form
-    int skinny_max_rows; // largest M that takes the register-dequant kernel
+    int skinny_max_rows; // largest M that takes the register-dequant kernel where the rows-resident one is switched off
     // routed-expert form of the register-dequant kernel: w is [experts, n, k],
     // x and y rows are assignments, m is their count; tokens of expert e are
     // expert_order[expert_offsets[e] .. expert_offsets[e + 1])
@@ -278,10 +291,19 @@ struct GemmArgs {
     // then weighs launch_gemm_resident against the other kernels)
     bool rows_resident;
     bool use_resident;    // set by launch_gemm_resident only
-    bool few_tiles_split; // up to 16 rows, few weight tiles per workgroup: the tiles' super-blocks are dealt over the waves
+    bool resident_switch; // rows_resident before the rows' length is looked at
+    bool few_rows;        // the few-rows kernel may take the product (gemm_takes_rows)
+    RowsPlan rows_plan;   // set by gemm_takes_rows; its K segments meet in these:
+    float* partials;
+    uint32_t* counters;
     bool weight_ring;     // routed form, rows resident: Q4_K and Q6_K weights through LDS rings where they fit beside the rows
 };
 const char* launch_gemm(hipStream_t s, const GemmArgs& a);
+// whether launch_gemm hands this product to the few-rows kernel: fills a.rows_plan, whose partial sums and
+// counters the caller then provides
+bool gemm_takes_rows(GemmArgs& a);
+
+void launch_gemm_rows(hipStream_t s, const GemmArgs& a);   // gemm_rows.hip, by a.rows_plan
 
 // gemm_skinny.hip
 const char* launch_gemm_skinny(hipStream_t s, const GemmArgs& a);

@@ -19,6 +19,13 @@ cannot see the timing of:
   a hand-issued load and the hand-placed wait that covers it; there must be none, except
   stores behind LDS-direct loads, which can only lengthen the wait.
 
+A second kind of kernel (``COUNTED_SOURCES``) leaves its LDS-direct loads and its register
+loads to the compiler, which orders and counts both, and only says when the former have
+landed: ``s_waitcnt vmcnt(n)``, n being the register loads the source issues behind them.
+The invariant is that the generated code has at least n of them there
+(``counted_violations``): with fewer, n outstanding loads could include one that the wait
+is for.
+
 The check reads the assembly hipcc writes with ``-S`` for this library's own sources
 (text, before it becomes a code object) and returns every violation it finds.  It is a
 linear scan in program-text order, which is the order these straight-line stretches are
@@ -34,6 +41,8 @@ import re
 VALIDATED_HIPCC = "7.2.26015"
 
 CHECKED_SOURCES = ("gemm.hip", "gemv_stream.hip", "gemm_skinny.hip", "probe.hip")
+COUNTED_SOURCES = ("gemm_rows_q4_k.hip", "gemm_rows_q5_k.hip", "gemm_rows_q6_k.hip", "gemm_rows_iq4_xs.hip",
+                   "gemm_rows_q8_0.hip")
 
 _KERNEL_LABEL = re.compile(r"^(_Z\w+|\w+):\s*(;.*)?$")
 _VREG_RANGE = re.compile(r"\bv\[(\d+):(\d+)\]")
@@ -115,6 +124,36 @@ def violations(asm: str, source: str = "") -> list[str]:
                 found.extend(_scan_to_wait(body, at, _vregs(match.group(1)), name, where))
         if hand_loads and scratch.get(name, 0) != 0:
             found.append(f"{where}{name}: a kernel with hand-scheduled loads uses {scratch[name]} bytes of scratch")
+    return found
+
+
+def counted_violations(asm: str, source: str = "") -> list[str]:
+    """Kernels whose LDS-direct loads the compiler issues: behind every run of them, up to the next
+    hand-placed wait in the text or the function's end, there must be at least as many loads into
+    registers as the hand-placed ``s_waitcnt vmcnt(n)`` of the kernel leaves outstanding."""
+    found: list[str] = []
+    where = (source + ":") if source else ""
+    for name, body in _functions(asm):
+        waits = [int(m.group(1)) for _, text, in_asm in body
+                 if in_asm and (m := re.match(r"s_waitcnt vmcnt\((\d+)\)", text))]
+        runs, current = [], None    # (line of the run's last LDS-direct load, loads behind it)
+        for number, text, in_asm in body:
+            if text.startswith("global_load_lds_"):
+                current = [number, 0]
+                if runs and runs[-1][1] == 0:
+                    runs[-1] = current
+                else:
+                    runs.append(current)
+            elif current is not None and in_asm and text.startswith("s_waitcnt vmcnt"):
+                current = None
+            elif current is not None and text.startswith("global_load_"):
+                current[1] += 1
+        if runs and not waits:
+            found.append(f"{where}{runs[0][0]}: {name}: LDS-direct loads without a hand-placed wait")
+        for number, behind in runs:
+            if waits and behind < max(waits):
+                found.append(f"{where}{number}: {name}: {behind} register loads follow this LDS-direct load, "
+                             f"the wait for it allows {max(waits)} outstanding")
     return found
 
 

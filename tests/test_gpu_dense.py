@@ -730,6 +730,35 @@ def test_few_rows_deal_a_tiles_super_blocks_over_the_waves(api, d, ggml, m, n, k
     assert np.array_equal(half.tensor.to_f32(), oracle.round_storage(got, code).reshape(m, n))
 
 
+# Edges of the few-rows kernel: rows of 1, 2, 4, 9 and 17 super-blocks (1, 2, 4 or 8 waves along K, a
+# wave without a block, an odd block out), rows whose K is cut into segments, ragged last tiles and row
+# groups of 16 and 32, exact f32 rows.  16-bit rows against the tile-rounded oracle, f32 rows against
+# the exact one, both at the matmul bar; the same bits on a second call (the sums have one order).
+@pytest.mark.parametrize("ggml", [12, 13, 14, 23, 8], ids=["q4_k", "q5_k", "q6_k", "iq4_xs", "q8_0"])
+@pytest.mark.parametrize("m,n,k,dtype", [
+    (2, 70, 256, "F16"), (17, 100, 512, "BF16"), (32, 301, 1024, "F16"), (5, 1003, 2304, "BF16"), (33, 533, 4352, "F16"),
+    (64, 48, 2048, "BF16"), (16, 1030, 17408, "F16"), (100, 96, 17408, "BF16"), (3, 20, 9216, "F16"),
+    (6, 61, 256, "F32"), (17, 333, 1280, "F32"), (40, 19, 4352, "F32"), (7, 1030, 17408, "F32")])
+def test_few_rows_on_the_edges_of_the_kernel(api, d, ggml, m, n, k, dtype):
+    packed = synth.matrix(ggml, n, k, seed=251 + n)
+    w = qm(api, d, ggml, n, k, packed)
+    code = {"F32": oracle.F32, "F16": oracle.F16, "BF16": oracle.BF16}[dtype]
+    x = oracle.round_storage(synth.activations(m, k, seed=252 + m), code).reshape(m, k)
+    xt = api.Tensor.from_f32(d, (m, k), getattr(api.DType, dtype), x)
+    out = d.project_quantized(xt, w, out_dtype=api.DType.F32)
+    assert out.operation.endswith("_gemm" if dtype == "F32" else "_skinny" if k > 5120 and m <= 64 else "_resident")
+    got = out.tensor.to_f32()
+    want = oracle.project(ggml, packed, n, k, x, accumulate="f64", weight_round=code, threads=8)
+    assert_matmul_parity(got, want, f"few rows {m}x{n}x{k} {dtype}")
+    again = d.project_quantized(xt, w, out_dtype=api.DType.F32).tensor.to_f32()
+    assert np.array_equal(bits(again), bits(got))
+    if dtype == "F32" and m > 5:    # a row's sums do not depend on the rows beside it
+        part = d.project_quantized(api.Tensor.from_f32(d, (m - 1, k), api.DType.F32, x[:-1]), w).tensor.to_f32()
+        assert np.array_equal(bits(part), bits(got[:-1]))
+    stored = d.project_quantized(xt, w).tensor.to_f32()      # 16-bit results: the packed stores
+    assert np.array_equal(bits(stored), bits(oracle.round_storage(got, code).reshape(m, n)))
+
+
 @pytest.mark.parametrize("ggml,m,dtype", [(12, 130, "F16"), (12, 300, "BF16"), (14, 200, "F16"), (8, 130, "F16")],
                          ids=["q4_k-130", "q4_k-300-bf16", "q6_k-200", "q8_0-130"])
 def test_rows_too_long_for_lds_take_the_128_row_tiles(api, d, ggml, m, dtype):

@@ -83,6 +83,31 @@ def test_a_store_may_stand_behind_a_request_into_lds_but_not_behind_a_register_l
     assert any("hand-counted wait" in v for v in isa_check.violations(load, "x.hip"))
 
 
+COUNTED = """
+_Z4rowsv:
+	global_load_lds_dwordx4 v[2:3], off
+	global_load_lds_dwordx4 v[4:5], off
+	global_load_dwordx4 v[8:11], v[6:7], off
+	global_load_dwordx4 v[12:15], v[6:7], off offset:16
+	;;#ASMSTART
+	s_waitcnt vmcnt(2)
+	;;#ASMEND
+	ds_read_b128 v[20:23], v1
+	s_endpgm
+.Lfunc_end0:
+"""
+
+
+def test_the_compilers_loads_behind_a_counted_lds_load_are_counted():
+    assert isa_check.counted_violations(COUNTED) == []
+    # one of them moved ahead of the LDS-direct loads: two outstanding loads could include the awaited one
+    load = "\tglobal_load_dwordx4 v[12:15], v[6:7], off offset:16\n"
+    moved = COUNTED.replace(load, "", 1).replace("_Z4rowsv:\n", "_Z4rowsv:\n" + load, 1)
+    assert any("1 register loads follow" in v for v in isa_check.counted_violations(moved, "x.hip"))
+    unwaited = COUNTED.replace("s_waitcnt vmcnt(2)", "s_nop 0", 1)
+    assert any("without a hand-placed wait" in v for v in isa_check.counted_violations(unwaited, "x.hip"))
+
+
 def test_the_release_is_read_from_hipcc_version_text():
     assert isa_check.hipcc_release("HIP version: 7.2.26015-fc0010cf6a\nAMD clang version 22") == "7.2.26015"
     assert isa_check.hipcc_release("nothing") == ""
@@ -98,4 +123,9 @@ def test_the_built_library_came_through_the_check():
         with open(path) as f:
             asm = f.read()
         assert isa_check.violations(asm, os.path.basename(path)) == []
+        assert "global_load_lds_dwordx4" in asm
+    for source in isa_check.COUNTED_SOURCES:
+        with open(os.path.join(build.OBJ_DIR, os.path.splitext(source)[0] + ".s")) as f:
+            asm = f.read()
+        assert isa_check.counted_violations(asm, source) == []
         assert "global_load_lds_dwordx4" in asm
