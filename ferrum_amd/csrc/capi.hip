@@ -1540,6 +1540,20 @@ fh_status fh_expert_assign(fh_device* device, const fh_view* hidden, uint32_t to
 
 namespace {
 
+// Whether streaming every hit expert once for all of its rows beats streaming it once per row.  The
+// per-assignment launch reads an expert's matrix for each of its assignments at the chip's rate (5.6
+// MB/us: 2.85 us per token of the 256-expert top-8 FFN); the grouped one waits for the workgroup that
+// streams one share of one expert (18.6 KB/us) behind a grouping and a staging launch.  256 experts top-8
+// of 2048 x 512 plus a shared one, us, per assignment against grouped: 4 tokens 30 / 117, 16 64 / 118,
+// 24 87 / 120, 32 110 / 122; 128 experts of 2048 x 768, 16 tokens 88 / 130, 24 124 / 135, 32 164 / 140;
+// 32 experts top-4 of 1024 x 256, 32 tokens 23 / 37.  From five assignments per expert on they are grouped.
+bool grouping_pays(const fh_qmatrix& weight, uint32_t assignments, int cu_count) {
+    if (assignments >= 5 * weight.experts) return true;
+    const double bytes = (double)weight.rows * (double)(weight.stored_cols / 256) * block_bytes(weight.ggml_type);
+    const double shares = std::max(1.0, (double)cu_count / (double)weight.experts);
+    return assignments * bytes / 5.6e6 > 7.0 + bytes / (shares * 18.6e3);
+}
+
 fh_status expert_project(fh_device* device, const fh_qmatrix* weight, const fh_view* x, uint32_t x_rows,
                          uint32_t form, uint32_t assignments, const fh_view* metadata, const fh_view* y,
                          const SharedExpert* shared = nullptr, const RouteTokenArgs* route = nullptr,
@@ -1626,7 +1640,9 @@ fh_status expert_project(fh_device* device, const fh_qmatrix* weight, const fh_v
     const bool f32_grouped = form == FH_INPUT_ROWS && x->dtype == FH_F32 && f32_rows > 0 &&
                              assignments >= (uint64_t)f32_rows && ((uintptr_t)xr.begin & 15u) == 0;
     const bool grouped = (x->dtype != FH_F32 || f32_grouped) && grouped_min > 0 &&
-                         assignments >= (uint64_t)grouped_min && weight->experts <= 1024 &&
+                         assignments >= (uint64_t)grouped_min &&
+                         (f32_grouped || grouping_pays(*weight, assignments, device->props.multiProcessorCount)) &&
+                         weight->experts <= 1024 &&
                          (rows * dtype_bytes(y->dtype)) % 4 == 0;
     if (grouped && route != nullptr) return fail(FH_ERR_DISPATCH, "only the per-assignment launch routes its token");
     if (grouped && shared != nullptr &&
@@ -1990,8 +2006,10 @@ fh_status fh_moe_ffn(fh_device* device, const fh_view* hidden, const fh_view* ro
         // own after the grouping, and that call may put partial sums where the lists lie: both then group for themselves.)
         const bool shared_stays_inside = !shared || (rides && expert_rows_fit_lds((uint32_t)h, a, (uint32_t)e) &&
                                                      expert_rows_fit_lds((uint32_t)inter, a, (uint32_t)e));
+        const int cus = device->props.multiProcessorCount;
         const bool regroup_once = fused && dt != FH_F32 && group_from > 0 && a >= (uint64_t)group_from && e <= 1024 &&
-                                  shared_stays_inside && !stored_padded;
+                                  shared_stays_inside && !stored_padded && grouping_pays(*input_experts, a, cus) &&
+                                  grouping_pays(*output_experts, a, cus);
         if (regroup_once) {
             const size_t words = ((size_t)e + 1 + a + 3) & ~(size_t)3;
             const size_t widest = std::max<size_t>(h, inter);

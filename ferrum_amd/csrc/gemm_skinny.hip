@@ -22,6 +22,9 @@
 // farther.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <cmath>
+
 #include "device_utils.hpp"
 #include "lds_direct.hpp"
 #include "quarter.hpp"
@@ -614,6 +617,14 @@ __global__ __launch_bounds__(kResThreads) void expert_ring_kernel(const uint8_t*
     }
 }
 
+// Tokens an expert's workgroup takes in one pass over its weights: 32 with more than 6 per expert on
+// average (8 where 32 rows do not fit LDS), else 16.  At 8 on average one of 256 experts is likely to
+// have more than 16, and its second pass doubles the launch: 256 experts top-8, 256 tokens 209 us in
+// passes of 16, 158 in passes of 32; 128 tokens 144 against 150.
+bool passes_of_32(uint32_t k, uint32_t m, uint32_t experts) {
+    return m > 8 * experts || (m > 6 * experts && (size_t)32 * k * 2 <= kResLdsBytes);
+}
+
 template <uint32_t TYPE, int DT>
 void launch_tt(hipStream_t s, const GemmArgs& a) {
     const uint8_t* w = static_cast<const uint8_t*>(a.w);
@@ -654,16 +665,19 @@ void launch_tt(hipStream_t s, const GemmArgs& a) {
         }
         return;
     }
-    const bool wide = a.m > 8 * a.experts;   // mean tokens per expert > 8: 32 tokens a pass
+    const bool wide = passes_of_32(a.k, a.m, a.experts);
     const size_t lds = (size_t)(wide ? 32 : 16) * a.k * 2;
     if (expert_rows_fit_lds(a.k, a.m, a.experts)) {
-        // the expert's rows are cut into shares so that about one workgroup per compute unit
-        // exists: every share gathers the expert's tokens again, and at 256 experts one share
-        // each (236 us for the 512-token routed FFN) beats four (264 us)
+        // An expert's rows are cut into shares so that about one workgroup per compute unit has work.
+        // Every share gathers the expert's tokens again: with all of 256 experts hit one share each
+        // (236 us for the 512-token routed FFN) beats four (264).  With fewer assignments than experts
+        // the compute units of those that nobody chose would idle: the hit ones, were the ids drawn
+        // evenly, share the chip (256 experts top-8, 4 / 8 / 16 tokens: 116 / 117 / 118 us with one
+        // share, 62 / 80 / 102 with four).
         const uint32_t tiles = (a.n + 15) / 16;
         const uint32_t target = a.cu_count > 0 ? (uint32_t)a.cu_count : 256u;
-        uint32_t shares = (target + a.experts - 1) / a.experts;
-        shares = shares < 1 ? 1 : shares;
+        const double hit = (double)a.experts * (1.0 - std::pow(1.0 - 1.0 / (double)a.experts, (double)a.m));
+        const uint32_t shares = std::max((target + a.experts - 1) / a.experts, (uint32_t)(target / std::max(hit, 1.0)));
         uint32_t tiles_per_wg = (tiles + shares - 1) / shares;
         tiles_per_wg = (tiles_per_wg + kResWaves - 1) / kResWaves * kResWaves;
         const dim3 rgrid((tiles + tiles_per_wg - 1) / tiles_per_wg, a.experts);
@@ -735,8 +749,7 @@ void launch_tt(hipStream_t s, const GemmArgs& a) {
 }  // namespace
 
 bool expert_rows_fit_lds(uint32_t k, uint32_t m, uint32_t experts) {
-    // more than 8 tokens per expert on average: 32 tokens a pass, else 16
-    return (size_t)(m > 8 * experts ? 32 : 16) * k * 2 <= kResLdsBytes;
+    return (size_t)(passes_of_32(k, m, experts) ? 32 : 16) * k * 2 <= kResLdsBytes;
 }
 
 const char* launch_gemm_resident(hipStream_t s, const GemmArgs& dense) {

@@ -248,6 +248,28 @@ def test_grouped_expert_projection_matches_the_oracle_and_the_direct_form(api, d
 
 
 @pytest.mark.parametrize("dtype", ["F16", "BF16"])
+@pytest.mark.parametrize("assignments,grouped", [(31, False), (32, False), (319, False), (320, True)])
+def test_few_assignments_per_expert_are_projected_one_by_one(api, d, assignments, grouped, dtype):
+    # 64 experts: up to five assignments each on average the per-assignment launch (exact weights),
+    # from there the grouped tiles (weights rounded to the row's type), each against its oracle
+    experts, rows, cols = 64, 40, 512
+    code = oracle.F16 if dtype == "F16" else oracle.BF16
+    packed = synth.matrix(Q4_K, experts * rows, cols, seed=261)
+    w = api.QuantizedExpertMatrix.new(d, packed, api.QuantizationFormat.Q4_K, experts, rows, cols)
+    meta = np.zeros((assignments, 3), dtype=np.uint32)
+    meta[:, 0] = np.sort(synth.rng(262).integers(0, experts, assignments))
+    meta[:, 1] = np.arange(assignments)
+    meta[:, 2] = np.float32(1.0).view(np.uint32)
+    x = oracle.round_storage(synth.activations(assignments, cols, seed=263) * 0.25, code).reshape(assignments, cols)
+    got = d.expert_project_quantized(api.Tensor.from_f32(d, x.shape, getattr(api.DType, dtype), x),
+                                     api.Tensor.from_bits(d, meta.shape, meta), w, cols, experts, out_dtype=api.DType.F32)
+    assert d.last_operation() == ("expert_project_q4_k_grouped_mfma" if grouped else "expert_project_q4_k_factored")
+    want = oracle.expert_project(Q4_K, packed, experts, rows, cols, x, meta.view(np.float32), accumulate="f64",
+                                 weight_round=code if grouped else 0)
+    assert_matmul_parity(got.to_f32(), want, f"{assignments} assignments of 64 experts, {dtype}")
+
+
+@pytest.mark.parametrize("dtype", ["F16", "BF16"])
 @pytest.mark.parametrize("cols,crowd", [(256, 37), (512, 37), (512, 11), (768, 37), (1024, 11), (1024, 37)])
 @pytest.mark.parametrize("ggml", [Q4_K, Q6_K])
 def test_grouped_projection_with_short_rows_streams_weights_through_lds(api, d, ggml, cols, crowd, dtype):
