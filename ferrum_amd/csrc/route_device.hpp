@@ -207,8 +207,21 @@ __device__ __forceinline__ void route_token(const RouteTokenArgs& a, uint32_t to
     if (shared_gate != nullptr && publish) {
         float dot = 0.f;
         if (gate_w != nullptr) {
-            for (uint32_t i = lane; i < hidden; i += 64)
-                dot += load_as_f32(gate_x, (size_t)token * hidden + i, gate_x_dtype) * gate_w[i];
+            // sixteen elements a lane in flight (one by one the row is a chain of hidden / 64 round trips: 16
+            // of the launch's 23 us at 2048), added in the order of the plain loop
+            const size_t row = (size_t)token * hidden;
+            for (uint32_t i0 = lane; i0 < hidden; i0 += 16 * 64) {
+                float xv[16], wv[16];
+#pragma unroll
+                for (int j = 0; j < 16; ++j) {
+                    const uint32_t i = i0 + 64u * j;
+                    xv[j] = i < hidden ? load_as_f32(gate_x, row + i, gate_x_dtype) : 0.f;
+                    wv[j] = i < hidden ? gate_w[i] : 0.f;
+                }
+#pragma unroll
+                for (int j = 0; j < 16; ++j)
+                    if (i0 + 64u * j < hidden) dot += xv[j] * wv[j];
+            }
             dot = wave_sum(dot);
         }
         if (lane == 0) shared_gate[token] = gate_w != nullptr ? 1.f / (1.f + expf(-dot)) : 1.f;
