@@ -193,11 +193,11 @@ namespace {
 // schedule, so rows that hold NaN report the same (flagged) index: 1024
 // threads per row scan columns tid, tid + 1024, ...; groups of 32 lanes merge
 // by a shuffle-down tree; thread 0 folds the 32 group results in order.
-__global__ __launch_bounds__(1024) void argmax_rows_kernel(const void* __restrict__ logits, uint32_t dtype,
-                                                           uint32_t width, uint32_t* __restrict__ out) {
+__device__ __forceinline__ void argmax_one_row(const void* __restrict__ logits, uint32_t dtype, uint32_t width,
+                                               uint32_t row, uint32_t* __restrict__ out) {
     __shared__ float best_value[32];
     __shared__ uint32_t best_index[32], bad_any[32];
-    const uint32_t tid = threadIdx.x, row = blockIdx.x;
+    const uint32_t tid = threadIdx.x;
     const size_t base = (size_t)row * width;
     float best = -INFINITY;
     uint32_t index = 0xffffffffu, bad = 0;
@@ -237,11 +237,118 @@ __global__ __launch_bounds__(1024) void argmax_rows_kernel(const void* __restric
     }
 }
 
+__global__ __launch_bounds__(1024) void argmax_rows_kernel(const void* __restrict__ logits, uint32_t dtype,
+                                                           uint32_t width, uint32_t* __restrict__ out) {
+    argmax_one_row(logits, dtype, width, blockIdx.x, out);
+}
+
+// Rows of a vocabulary: one workgroup needs a round trip per 1024 columns (151936 f32 logits: 66 us), so
+// a row is cut into pieces of 8192 columns, one workgroup each, whose maxima meet in device memory; the
+// last to arrive folds them (151936: 5 us).  The first maximal index of a row without NaN
+// does not depend on the order in which it is searched; a row that holds one is searched again by the
+// last workgroup in the schedule above.
+constexpr uint32_t kArgmaxPiece = 8192;
+
+__global__ __launch_bounds__(1024) void argmax_pieces_kernel(const void* __restrict__ logits, uint32_t dtype,
+                                                             uint32_t width, unsigned long long* __restrict__ partial,
+                                                             uint32_t* __restrict__ counters, uint32_t* __restrict__ out) {
+    typedef unsigned long long u64;
+    __shared__ float best_value[16];
+    __shared__ uint32_t best_index[16], flags_any[16], last_flag;
+    const uint32_t tid = threadIdx.x, row = blockIdx.y, pieces = gridDim.x;
+    const size_t base = (size_t)row * width;
+    float value[8];
+    const uint32_t first = blockIdx.x * kArgmaxPiece + tid;
+#pragma unroll
+    for (uint32_t i = 0; i < 8; ++i) {
+        const uint32_t j = first + i * 1024;
+        value[i] = j < width ? load_as_f32(logits, base + j, dtype) : -INFINITY;
+    }
+    float best = -INFINITY;
+    uint32_t index = 0xffffffffu, flags = 0;   // bit 0: a non-finite value, bit 1: a NaN
+#pragma unroll
+    for (uint32_t i = 0; i < 8; ++i) {
+        const uint32_t j = first + i * 1024;
+        if (j >= width) continue;
+        if (!isfinite(value[i])) flags |= isnan(value[i]) ? 3u : 1u;
+        if (value[i] > best || index == 0xffffffffu) {
+            best = value[i];
+            index = j;
+        }
+    }
+    auto merge = [&](float other, uint32_t other_index) {
+        if (other_index != 0xffffffffu &&
+            (index == 0xffffffffu || other > best || (other == best && other_index < index))) {
+            best = other;
+            index = other_index;
+        }
+    };
+    auto fold_wave = [&]() {
+#pragma unroll
+        for (uint32_t offset = 32; offset > 0; offset /= 2) {
+            merge(__shfl_xor(best, offset, 64), __shfl_xor(index, offset, 64));
+            flags |= __shfl_xor(flags, offset, 64);
+        }
+    };
+    fold_wave();
+    if ((tid & 63u) == 0) {
+        best_value[tid >> 6] = best;
+        best_index[tid >> 6] = index;
+        flags_any[tid >> 6] = flags;
+    }
+    __syncthreads();
+    if (tid == 0) {
+        for (uint32_t w = 1; w < 16; ++w) {
+            merge(best_value[w], best_index[w]);
+            flags |= flags_any[w];
+        }
+        // device-scope accesses, coherent across the chip's L2 slices; the ticket follows the piece
+        u64* const mine = partial + 2 * ((size_t)row * pieces + blockIdx.x);
+        __hip_atomic_store(mine, (u64)__float_as_uint(best) | ((u64)index << 32), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(mine + 1, (u64)flags, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): the stores above have completed
+        const uint32_t ticket = __hip_atomic_fetch_add(counters + row, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        last_flag = ticket == pieces - 1 ? 1u : 0u;
+        if (last_flag) __hip_atomic_store(counters + row, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __syncthreads();
+    if (last_flag == 0) return;
+    if (tid < 64) {
+        best = -INFINITY;
+        index = 0xffffffffu;
+        flags = 0;
+        for (uint32_t i = tid; i < pieces; i += 64) {
+            u64* const other = partial + 2 * ((size_t)row * pieces + i);
+            const u64 found = __hip_atomic_load(other, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            flags |= (uint32_t)__hip_atomic_load(other + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            merge(__uint_as_float((uint32_t)found), (uint32_t)(found >> 32));
+        }
+        fold_wave();
+        if (tid == 0) {
+            out[2 * (size_t)row] = index;
+            out[2 * (size_t)row + 1] = flags & 1u;
+            flags_any[0] = flags;
+        }
+    }
+    __syncthreads();
+    if ((flags_any[0] & 2u) != 0) argmax_one_row(logits, dtype, width, row, out);
+}
+
 }  // namespace
 
+size_t argmax_partial_bytes(uint32_t rows, uint32_t width) {
+    // a row of one piece, and more rows than counter words or grid rows, keep one workgroup a row
+    if (width <= kArgmaxPiece || rows > 65535u) return 0;
+    return (size_t)rows * ((width + kArgmaxPiece - 1) / kArgmaxPiece) * 2 * sizeof(unsigned long long);
+}
+
 const char* launch_argmax_rows(hipStream_t s, const void* logits, uint32_t dtype, uint32_t rows, uint32_t width,
-                               uint32_t* out) {
-    hipLaunchKernelGGL(argmax_rows_kernel, dim3(rows), dim3(1024), 0, s, logits, dtype, width, out);
+                               void* partial, uint32_t* counters, uint32_t* out) {
+    if (argmax_partial_bytes(rows, width) != 0)
+        hipLaunchKernelGGL(argmax_pieces_kernel, dim3((width + kArgmaxPiece - 1) / kArgmaxPiece, rows), dim3(1024), 0, s,
+                           logits, dtype, width, static_cast<unsigned long long*>(partial), counters, out);
+    else
+        hipLaunchKernelGGL(argmax_rows_kernel, dim3(rows), dim3(1024), 0, s, logits, dtype, width, out);
     return "argmax_rows";
 }
 

@@ -859,6 +859,41 @@ def test_argmax_rows_matches_the_oracle(api, d, dtype_name):
         d.argmax_rows(api.Tensor.zeros(d, (4,), dtype))
 
 
+@pytest.mark.parametrize("width", [8192, 8193, 16385, 30000])
+def test_argmax_of_rows_cut_into_pieces(api, d, width):
+    # rows of more than 8192 columns are searched piece by piece: ties across pieces, the maximum in a last
+    # piece of one column, rows of -inf, signed zeros, and NaN where the reference's schedule starts a
+    # thread's scan (columns below 1024) and where it does not
+    x = synth.rng(137).standard_normal((8, width)).astype(np.float32)
+    x[0, 7] = x[0, width - 1] = 9.0
+    x[1, width - 1] = 9.0
+    x[2, :] = -np.inf
+    x[3, :] = -1.0
+    x[3, 5000] = -0.0
+    x[3, width - 2] = 0.0
+    x[4, 9] = np.nan
+    x[5, 4000] = np.nan
+    x[5, 4001] = np.inf
+    x[6, :1024] = np.nan
+    x[7, width - 1] = np.nan
+    for _ in range(2):     # the counters are left at zero
+        got = d.argmax_rows(api.Tensor.from_f32(d, x.shape, api.DType.F32, x))
+        assert np.array_equal(got.raw().view(np.uint32).reshape(8, 2), oracle.argmax_rows(x))
+
+
+@pytest.mark.parametrize("ggml,n,k,dtype", [(Q6_K, 700, 17408, "F32"), (Q6_K, 700, 17408, "BF16"), (Q4_K, 4200, 1024, "F16"),
+                                            (Q4_K, 1100, 17408, "F32"), (Q4_K, 300, 512, "F16")])
+def test_one_activated_row_has_the_bits_of_the_separate_calls(api, d, ggml, n, k, dtype):
+    # large matrices: the activated row is written out for the streamed kernel; small ones activate it in place
+    w = qm(api, d, ggml, n, k, synth.matrix(ggml, n, k, seed=138))
+    dt = getattr(api.DType, dtype)
+    packed = api.Tensor.from_f32(d, (1, 2 * k), dt, synth.activations(1, 2 * k, seed=139))
+    fused = d.project_quantized(packed, w, silu_mul=True)
+    separate = d.project_quantized(d.expert_silu_mul(packed, k), w)
+    assert np.array_equal(fused.tensor.raw(), separate.tensor.raw())
+    assert np.abs(fused.tensor.to_f32()).max() > 1e-3
+
+
 def test_lm_head_projection_then_argmax_picks_the_oracle_token(api, d):
     n, k = 4096, 1024
     packed = synth.matrix(Q6_K, n, k, seed=141)
