@@ -97,6 +97,7 @@ SYMBOLS = {
     "fh_set_tuning": (_I32, [_P, ctypes.c_char_p, _I64]),
     "fh_get_tuning": (_I32, [_P, ctypes.c_char_p, ctypes.POINTER(_I64)]),
     "fh_buffer_alloc": (_I32, [_P, _SZ, ctypes.POINTER(_P)]),
+    "fh_buffer_alloc_uninitialized": (_I32, [_P, _SZ, ctypes.POINTER(_P)]),
     "fh_buffer_free": (None, [_P]),
     "fh_buffer_size": (_SZ, [_P]),
     "fh_buffer_device_ptr": (_P, [_P]),
@@ -235,10 +236,11 @@ def decode(raw: np.ndarray, dtype: DType) -> np.ndarray:
 
 
 class Buffer:
-    def __init__(self, device: "Device", nbytes: int):
+    def __init__(self, device: "Device", nbytes: int, zeroed: bool = True):
         self.device = device
         handle = ctypes.c_void_p()
-        _check(_lib.fh_buffer_alloc(device._handle, nbytes, ctypes.byref(handle)))
+        allocate = _lib.fh_buffer_alloc if zeroed else _lib.fh_buffer_alloc_uninitialized
+        _check(allocate(device._handle, nbytes, ctypes.byref(handle)))
         self._handle = handle
         self.nbytes = nbytes
 
@@ -268,18 +270,24 @@ class Tensor:
     def __init__(self, buffer: Buffer, offset: int, shape, dtype: DType):
         self.buffer, self.offset, self.dtype = buffer, offset, DType(dtype)
         self._shape = tuple(int(d) for d in shape)
+        self._numel = math.prod(self._shape)
 
     @staticmethod
     def zeros(device: "Device", shape, dtype: DType) -> "Tensor":
         shape = tuple(int(d) for d in shape)
-        n = int(np.prod(shape, dtype=np.int64)) if shape else 1
-        return Tensor(Buffer(device, max(n, 1) * DType(dtype).size_bytes()), 0, shape, dtype)
+        return Tensor(Buffer(device, max(math.prod(shape), 1) * DType(dtype).size_bytes()), 0, shape, dtype)
+
+    @staticmethod
+    def _output(device: "Device", shape, dtype: DType) -> "Tensor":
+        """A tensor an operator is about to write whole: its contents are undefined until then."""
+        shape = tuple(int(d) for d in shape)
+        return Tensor(Buffer(device, max(math.prod(shape), 1) * DType(dtype).size_bytes(), zeroed=False), 0, shape, dtype)
 
     @staticmethod
     def from_f32(device: "Device", shape, dtype: DType, values) -> "Tensor":
         shape = tuple(int(d) for d in shape)
         a = np.ascontiguousarray(values, dtype=np.float32).reshape(-1)
-        if a.size != int(np.prod(shape, dtype=np.int64)):
+        if a.size != math.prod(shape):
             raise ShapeError("value count does not match shape")
         t = Tensor.zeros(device, shape, dtype)
         if a.size:
@@ -298,14 +306,14 @@ class Tensor:
         return self._shape
 
     def numel(self) -> int:
-        return int(np.prod(self._shape, dtype=np.int64)) if self._shape else 1
+        return self._numel
 
     def byte_size(self) -> int:
         return self.numel() * self.dtype.size_bytes()
 
     def view(self, element_offset: int, shape) -> "Tensor":
         shape = tuple(int(d) for d in shape)
-        n = int(np.prod(shape, dtype=np.int64))
+        n = math.prod(shape)
         if element_offset < 0 or element_offset + n > self.numel():
             raise RangeError("view exceeds tensor")
         return Tensor(self.buffer, self.offset + element_offset * self.dtype.size_bytes(), shape,
@@ -601,14 +609,14 @@ class Device:
 
     def dequantize(self, weight, dtype: DType = DType.F32) -> Tensor:
         rows = weight.rows() if isinstance(weight, QuantizedMatrix) else weight.experts() * weight.rows_per_expert()
-        out = Tensor.zeros(self, (rows, weight.columns()), dtype)
+        out = Tensor._output(self, (rows, weight.columns()), dtype)
         v = out._view()
         _check(_lib.fh_dequantize(self._handle, _handle_of(weight), ctypes.byref(v)))
         return out
 
     def embedding_gather_quantized(self, weight: QuantizedMatrix, tokens, output_dtype: DType) -> Output:
         ids = np.ascontiguousarray(tokens, dtype=np.uint32)
-        out = Tensor.zeros(self, (ids.size, weight.columns()), output_dtype)
+        out = Tensor._output(self, (ids.size, weight.columns()), output_dtype)
         v = out._view()
         _check(_lib.fh_embedding_gather_quantized(
             self._handle, _handle_of(weight), ids.ctypes.data_as(ctypes.POINTER(ctypes.c_uint32)),
@@ -628,7 +636,7 @@ class Device:
         m, n = dims[0], weight.rows()
         dtype = a.dtype if out_dtype is None else DType(out_dtype)
         if out is None:
-            out = Tensor.zeros(self, (m, n), dtype)
+            out = Tensor._output(self, (m, n), dtype)
         if m == 0:
             return Output(out, "")
         xv, yv = a._view(), out._view()
@@ -672,7 +680,7 @@ class Device:
             raise ShapeError("argmax requires nonempty [rows,width]")
         if logits.buffer.device is not self:
             raise DeviceMismatch("tensor belongs to another device")
-        out = Tensor.zeros(self, (dims[0], 2), DType.F32)
+        out = Tensor._output(self, (dims[0], 2), DType.F32)
         lv, ov = logits._view(), out._view()
         _check(_lib.fh_argmax_rows(self._handle, ctypes.byref(lv), dims[0], dims[1], ctypes.byref(ov)))
         return out
@@ -694,8 +702,8 @@ class Device:
             raise ParameterError("epsilon must be finite and positive")
         if any(t.buffer.device is not self for t in (a, b, weight)):
             raise DeviceMismatch("tensor belongs to another device")
-        residual = residual if residual is not None else Tensor.zeros(self, dims, a.dtype)
-        normed = normed if normed is not None else Tensor.zeros(self, dims, a.dtype)
+        residual = residual if residual is not None else Tensor._output(self, dims, a.dtype)
+        normed = normed if normed is not None else Tensor._output(self, dims, a.dtype)
         views = [t._view() for t in (a, b, weight, residual, normed)]
         _check(_lib.fh_add_rmsnorm(self._handle, ctypes.byref(views[0]), ctypes.byref(views[1]),
                                    ctypes.byref(views[2]), a.numel() // width, width, epsilon,
@@ -711,7 +719,7 @@ class Device:
                                            or selection_bias.dtype != DType.F32):
             raise ShapeError("invalid sparse routing geometry")
         if out is None:
-            out = Tensor.zeros(self, (dims[0] * max(policy.top_k, 1), 3), DType.F32)
+            out = Tensor._output(self, (dims[0] * max(policy.top_k, 1), 3), DType.F32)
         lv, ov, pc = logits._view(), out._view(), policy._c()
         bv = selection_bias._view() if selection_bias is not None else None
         _check(_lib.fh_moe_route(self._handle, ctypes.byref(lv), dims[0],
@@ -731,8 +739,8 @@ class Device:
         if gate_vector is not None and (x is None or x.shape() != (dims[0], gate_vector.shape()[0])
                                         or gate_vector.dtype != DType.F32):
             raise ShapeError("the shared-expert gate needs x [tokens, hidden] and an f32 vector [hidden]")
-        meta = Tensor.zeros(self, (dims[0] * policy.top_k, 3), DType.F32)
-        gate = Tensor.zeros(self, (dims[0],), DType.F32) if (want_gate or gate_vector is not None) else None
+        meta = Tensor._output(self, (dims[0] * policy.top_k, 3), DType.F32)
+        gate = Tensor._output(self, (dims[0],), DType.F32) if (want_gate or gate_vector is not None) else None
         lv, mv, pc = logits._view(), meta._view(), policy._c()
         xv = x._view() if gate_vector is not None else None
         wv = gate_vector._view() if gate_vector is not None else None
@@ -755,9 +763,9 @@ class Device:
         if gate_vector is not None and (x is None or x.shape() != (dims[0], gate_vector.shape()[0])
                                         or gate_vector.dtype != DType.F32):
             raise ShapeError("the shared-expert gate needs x [tokens, hidden] and an f32 vector [hidden]")
-        ids = Tensor.zeros(self, (dims[0] * policy.top_k,), DType.F32)
-        weights = Tensor.zeros(self, (dims[0] * policy.top_k,), DType.F32)
-        gate = Tensor.zeros(self, (dims[0],), DType.F32)
+        ids = Tensor._output(self, (dims[0] * policy.top_k,), DType.F32)
+        weights = Tensor._output(self, (dims[0] * policy.top_k,), DType.F32)
+        gate = Tensor._output(self, (dims[0],), DType.F32)
         lv, iv, wtv, gv, pc = logits._view(), ids._view(), weights._view(), gate._view(), policy._c()
         xv = x._view() if gate_vector is not None else None
         wv = gate_vector._view() if gate_vector is not None else None
@@ -774,7 +782,7 @@ class Device:
         dims = x.shape()
         if len(dims) != 2 or dims[0] == 0 or dims[1] != weight.columns():
             raise ShapeError("quantized projection requires [M,K] matching [N,K]")
-        y = Tensor.zeros(self, (dims[0], weight.rows()), out_dtype or x.dtype)
+        y = Tensor._output(self, (dims[0], weight.rows()), out_dtype or x.dtype)
         xv, yv = x._view(), y._view()
         _check(_lib.fh_hybrid_project(self._handle, _handle_of(weight), ctypes.byref(xv), dims[0], ctypes.byref(yv),
                                       1 if exact else 0))
@@ -809,7 +817,7 @@ class Device:
                 or shared_weight.format().ggml_type() != weight.format().ggml_type()):
             raise ShapeError("expert projection geometry")
         y = Tensor.zeros(self, (routes, weight.rows_per_expert()), x.dtype)
-        ys = Tensor.zeros(self, (tokens, weight.rows_per_expert()), x.dtype)
+        ys = Tensor._output(self, (tokens, weight.rows_per_expert()), x.dtype)
         xv, iv, yv, ysv = x._view(), ids._view(), y._view(), ys._view()
         sxv = shared_x._view() if shared_x is not None else None
         _check(_lib.fh_hybrid_project_id_with_shared(
@@ -823,7 +831,7 @@ class Device:
         routes = ids.numel()
         if routes == 0 or ids.dtype != DType.F32:
             raise ShapeError("route map needs routes")
-        offsets = Tensor.zeros(self, (experts + 1,), DType.F32)
+        offsets = Tensor._output(self, (experts + 1,), DType.F32)
         order = Tensor.zeros(self, (routes,), DType.F32)
         position = Tensor.zeros(self, (routes,), DType.F32)
         iv, ov, sv, pv = ids._view(), offsets._view(), order._view(), position._view()
@@ -836,7 +844,7 @@ class Device:
         dims, routes = x.shape(), order.numel()
         if len(dims) != 2 or used == 0 or routes != dims[0] * used:
             raise ShapeError("route gather needs [tokens, hidden] and tokens * used routes")
-        out = Tensor.zeros(self, (routes, dims[1]), x.dtype)
+        out = Tensor._output(self, (routes, dims[1]), x.dtype)
         xv, sv, ov = x._view(), order._view(), out._view()
         _check(_lib.fh_hybrid_moe_gather(self._handle, ctypes.byref(xv), ctypes.byref(sv), dims[1], used, routes,
                                          ctypes.byref(ov)))
@@ -866,7 +874,7 @@ class Device:
                 or shared_weight.format().ggml_type() != weight.format().ggml_type()):
             raise ShapeError("expert projection geometry")
         y = Tensor.zeros(self, (dims[0], weight.rows_per_expert()), x.dtype)
-        ys = Tensor.zeros(self, (sd[0], weight.rows_per_expert()), x.dtype)
+        ys = Tensor._output(self, (sd[0], weight.rows_per_expert()), x.dtype)
         xv, fv, sxv, yv, ysv = x._view(), offsets._view(), shared_x._view(), y._view(), ys._view()
         _check(_lib.fh_hybrid_project_mm_id_with_shared(
             self._handle, _handle_of(weight), _handle_of(shared_weight), ctypes.byref(xv), ctypes.byref(fv), dims[0],
@@ -881,7 +889,7 @@ class Device:
         if (down.shape() != (tokens * used, hidden) or weights.numel() != tokens * used
                 or shared_gate.shape() != (tokens,) or (position is not None and position.numel() != tokens * used)):
             raise ShapeError("expert combine geometry mismatch")
-        out = Tensor.zeros(self, (tokens, hidden), DType.F32)
+        out = Tensor._output(self, (tokens, hidden), DType.F32)
         views = [t._view() if t is not None else None for t in (down, weights, position, shared, shared_gate, out)]
         ref = lambda v: ctypes.byref(v) if v is not None else None
         _check(_lib.fh_hybrid_moe_combine(self._handle, ref(views[0]), ref(views[1]), ref(views[2]), ref(views[3]),
@@ -898,7 +906,7 @@ class Device:
                 or (shared_gate is not None and shared_gate.shape() != (tokens,))):
             raise ShapeError("expert combine geometry mismatch")
         if out is None:
-            out = Tensor.zeros(self, (tokens, hidden), input.dtype)
+            out = Tensor._output(self, (tokens, hidden), input.dtype)
         iv, mv, sv, ov = input._view(), metadata._view(), shared._view(), out._view()
         gv = shared_gate._view() if shared_gate is not None else None
         _check(_lib.fh_expert_combine_shared(self._handle, ctypes.byref(iv), ctypes.byref(mv), tokens, hidden,
@@ -913,7 +921,7 @@ class Device:
                 or x[0] * top_k != meta[0] or metadata.dtype != DType.F32):
             raise ShapeError("expert assignments require [S,H] and [S*top_k,3]")
         if out is None:
-            out = Tensor.zeros(self, (meta[0], x[1]), hidden.dtype)
+            out = Tensor._output(self, (meta[0], x[1]), hidden.dtype)
         hv, mv, ov = hidden._view(), metadata._view(), out._view()
         _check(_lib.fh_expert_assign(self._handle, ctypes.byref(hv), x[0], x[1], ctypes.byref(mv),
                                      top_k, ctypes.byref(ov)))
@@ -974,7 +982,7 @@ class Device:
         if out is None:
             out = Tensor.zeros(self, (meta[0], n), input.dtype)
         if shared_out is None:
-            shared_out = Tensor.zeros(self, (tokens, n), input.dtype)
+            shared_out = Tensor._output(self, (tokens, n), input.dtype)
         xv, mv, ov, sov = input._view(), metadata._view(), out._view(), shared_out._view()
         sxv = shared_input._view() if shared_input is not None else None
         _check(_lib.fh_expert_project_with_shared(
@@ -988,7 +996,7 @@ class Device:
         if len(x) != 2 or intermediate == 0 or intermediate * 2 != x[1]:
             raise ShapeError("packed expert activation geometry mismatch")
         if out is None:
-            out = Tensor.zeros(self, (x[0], intermediate), input.dtype)
+            out = Tensor._output(self, (x[0], intermediate), input.dtype)
         iv, ov = input._view(), out._view()
         _check(_lib.fh_expert_silu_mul(self._handle, ctypes.byref(iv), x[0], intermediate,
                                        ctypes.byref(ov)))
@@ -1001,7 +1009,7 @@ class Device:
                 or metadata.shape() != (x[0], 3) or metadata.dtype != DType.F32):
             raise ShapeError("expert combine geometry mismatch")
         if out is None:
-            out = Tensor.zeros(self, (tokens, hidden), input.dtype)
+            out = Tensor._output(self, (tokens, hidden), input.dtype)
         iv, mv, ov = input._view(), metadata._view(), out._view()
         _check(_lib.fh_expert_combine(self._handle, ctypes.byref(iv), ctypes.byref(mv), tokens,
                                       hidden, top_k, ctypes.byref(ov)))
@@ -1090,7 +1098,7 @@ class SparseMoe:
         if shared_gate is not None and shared_gate.numel() != dims[0]:
             raise ShapeError("shared gate requires one value per token")
         if out is None:
-            out = Tensor.zeros(self.device, dims, hidden.dtype)
+            out = Tensor._output(self.device, dims, hidden.dtype)
         hv, lv, ov, pc = hidden._view(), router_logits._view(), out._view(), self.routing._c()
         bv = self.selection_bias._view() if self.selection_bias is not None else None
         gv = shared_gate._view() if shared_gate is not None else None

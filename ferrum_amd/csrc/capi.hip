@@ -73,6 +73,25 @@ fh_status resolve(const fh_device* device, const fh_view* view, uint64_t element
 
 bool fits_u32(uint64_t v) { return v <= 0xffffffffull; }
 
+void drain_pool(fh_device* d) {
+    if (d->pool.empty()) return;
+    (void)hipStreamSynchronize(d->stream);
+    for (auto& block : d->pool) (void)hipFree(block.second);
+    d->pool.clear();
+    d->pool_bytes = 0;
+}
+
+// Memory from the system; what the pool holds is given back when there is none.
+hipError_t allocate(fh_device* d, void** out, size_t bytes) {
+    hipError_t e = hipMalloc(out, bytes);
+    if (e == hipErrorOutOfMemory && !d->pool.empty()) {
+        (void)hipGetLastError();
+        drain_pool(d);
+        e = hipMalloc(out, bytes);
+    }
+    return e;
+}
+
 // Device scratch: kCounterWords zeroed counter words followed by a data area
 // of at least `data_bytes`.  Growing it waits for the stream first.  Recorded executions
 // carry the scratch address in their kernel arguments, so a block that is outgrown while
@@ -96,7 +115,7 @@ fh_status ensure_scratch(fh_device* d, size_t data_bytes) {
     d->scratch = nullptr;
     d->scratch_bytes = 0;
     size_t cap = counter_bytes + (data_bytes < (16u << 20) ? (16u << 20) : data_bytes);
-    hipError_t e = hipMalloc(&d->scratch, cap);
+    hipError_t e = allocate(d, &d->scratch, cap);
     if (e != hipSuccess) return fail(FH_ERR_ALLOCATION, "hipMalloc(%zu): %s", cap, hipGetErrorString(e));
     d->scratch_bytes = cap;
     FH_HIP(hipMemsetAsync(d->scratch, 0, counter_bytes, d->stream));
@@ -122,7 +141,7 @@ fh_status ensure_block(fh_device* d, fh_buffer*& slot, size_t bytes, const char*
     }
     slot->ptr = nullptr;
     slot->bytes = 0;
-    hipError_t e = hipMalloc(&slot->ptr, bytes);
+    hipError_t e = allocate(d, &slot->ptr, bytes);
     if (e != hipSuccess) return fail(FH_ERR_ALLOCATION, "hipMalloc(%zu): %s", bytes, hipGetErrorString(e));
     slot->bytes = bytes;
     return FH_OK;
@@ -281,9 +300,60 @@ void drain_deferred(fh_device* d) {
     d->deferred_graphs.clear();
 }
 
-int64_t tuning(const fh_device* d, const char* key) {
-    auto it = d->tuning.find(key);
-    return it == d->tuning.end() ? 0 : it->second;
+constexpr struct {
+    const char* name;
+    int64_t fh_tuning::*value;
+} kTuningKeys[] = {
+    {"k_quant_gemv_ksplit", &fh_tuning::k_quant_gemv_ksplit},
+    {"gemm_min_rows", &fh_tuning::gemm_min_rows},
+    {"gemm_wide_shape", &fh_tuning::gemm_wide_shape},
+    {"gemm_wide32_tile", &fh_tuning::gemm_wide32_tile},
+    {"gemm_wide_min_rows", &fh_tuning::gemm_wide_min_rows},
+    {"gemm_skinny_max_rows", &fh_tuning::gemm_skinny_max_rows},
+    {"expert_grouped_min_assignments", &fh_tuning::expert_grouped_min_assignments},
+    {"moe_fold_route", &fh_tuning::moe_fold_route},
+    {"gemm_few_tiles_split", &fh_tuning::gemm_few_tiles_split},
+    {"moe_fold_combine", &fh_tuning::moe_fold_combine},
+    {"gemm_resident", &fh_tuning::gemm_resident},
+    {"gemv_stream_own_loads", &fh_tuning::gemv_stream_own_loads},
+    {"expert_weight_ring", &fh_tuning::expert_weight_ring},
+    {"gemv_stream", &fh_tuning::gemv_stream},
+    {"moe_routing_temporary_limit", &fh_tuning::moe_routing_temporary_limit},
+    {"gemm_f32_min_rows", &fh_tuning::gemm_f32_min_rows},
+    {"probe_read_form", &fh_tuning::probe_read_form},
+};
+
+// the switch of that name, or null
+template <class Device>
+auto tuning_of(Device* d, const char* key) -> decltype(&(d->tuning.gemm_min_rows)) {
+    for (const auto& k : kTuningKeys)
+        if (std::strcmp(k.name, key) == 0) return &(d->tuning.*k.value);
+    return nullptr;
+}
+
+// ---- freed blocks kept for the next buffers ----------------------------------------------
+
+constexpr size_t kPoolBytes = 256u << 20;       // most memory kept
+constexpr size_t kPoolBlockBytes = 64u << 20;   // largest block kept
+
+// Blocks come in sizes a quarter of a power of two apart (4 KiB at least), so that a batch a little larger
+// or smaller finds them.
+size_t block_capacity(size_t bytes) {
+    if (bytes > kPoolBlockBytes) return bytes;
+    size_t step = 4096;
+    while (step * 8 < bytes) step *= 2;
+    return (bytes + step - 1) / step * step;
+}
+
+hipError_t take_block(fh_device* d, size_t capacity, void** out) {
+    const auto found = d->pool.find(capacity);
+    if (found != d->pool.end()) {
+        *out = found->second;
+        d->pool_bytes -= capacity;
+        d->pool.erase(found);
+        return hipSuccess;
+    }
+    return allocate(d, out, capacity);
 }
 
 }  // namespace
@@ -334,23 +404,6 @@ fh_status fh_device_create(int32_t ordinal, fh_device** out) {
         delete d;
         return hip_fail(e, "hipStreamCreateWithFlags");
     }
-    d->tuning["k_quant_gemv_ksplit"] = 0;   // 0 = automatic
-    d->tuning["gemm_min_rows"] = 2;         // smallest M that takes the MFMA tile path
-    d->tuning["gemm_wide_shape"] = 1;       // matrix instruction of the 128- and 256-row tiles: 0 = 16x16x32, 1 = whichever is estimated faster, 2 = 32x32x16
-    d->tuning["gemm_wide32_tile"] = 0;      // 0 = by shape; 12, 14, 15 (128-row tile x 64, 128, 160 columns), 24, 25 (256-row tile)
-    d->tuning["gemm_wide_min_rows"] = 33;   // smallest M that takes the 256-row tile (it wins from there up)
-    d->tuning["gemm_skinny_max_rows"] = 64; // largest M that takes the register-dequant MFMA kernel (0 = never)
-    d->tuning["expert_grouped_min_assignments"] = 32;  // fewest assignments grouped by expert (0 = never)
-    d->tuning["moe_fold_route"] = 1;        // fh_moe_ffn, one token: the gate|up launch routes the token itself (0 = a moe_route launch first)
-    d->tuning["gemm_few_tiles_split"] = 1;  // few rows: a tile's super-blocks dealt over the waves, any K (0 = whole tiles per wave, the kernels for rows that fit LDS or not)
-    d->tuning["moe_fold_combine"] = 1;      // fh_moe_ffn with few tokens: down projection and weighted sum in one launch (0 = two)
-    d->tuning["gemm_resident"] = 1;         // rows that fit LDS whole take the rows-resident kernel (0 = square tiles)
-    d->tuning["gemv_stream_own_loads"] = 1; // the streamed Q4_K GEMV's waves load the super-blocks they multiply (tiles of up to 14 rows); 0: the tile row by row
-    d->tuning["expert_weight_ring"] = 1;    // grouped Q4_K / Q6_K expert projection with short rows: weights through LDS rings (0 = straight into registers)
-    d->tuning["gemv_stream"] = 1;           // dense Q4_K / Q6_K GEMV on the streamed matrix-core kernel: 0 never, 1 where it wins, 2 wherever it runs
-    d->tuning["moe_routing_temporary_limit"] = 128ll << 20;  // bytes of routing temporaries per SparseMoe chunk (src/metal/legacy.rs:95)
-    d->tuning["gemm_f32_min_rows"] = 0;     // f32 activations take the f16 tile kernels from this many rows (0 = never)
-    d->tuning["probe_read_form"] = 0;       // fh_probe_read: 100 x threads per workgroup + loads per lane (+ 1000000: LDS-direct loads); 0 = 256 x 8
     fh_status st = ensure_scratch(d, 0);
     if (st == FH_OK) {
         // This device's address of the fixed scratch (the device is current).  Its counters are set to zero
@@ -393,6 +446,7 @@ void fh_device_destroy(fh_device* device) {
         device->capturing = false;
     }
     drain_deferred(device);
+    drain_pool(device);
     if (device->stream) {
         (void)hipStreamSynchronize(device->stream);
         (void)hipStreamDestroy(device->stream);
@@ -452,8 +506,8 @@ void* fh_device_stream(fh_device* device) { return device ? device->stream : nul
 
 fh_status fh_set_tuning(fh_device* device, const char* key, int64_t value) {
     if (device == nullptr || key == nullptr) return fail(FH_ERR_PARAMETER, "null argument");
-    auto it = device->tuning.find(key);
-    if (it == device->tuning.end()) return fail(FH_ERR_PARAMETER, "unknown tuning key %s", key);
+    int64_t* const setting = tuning_of(device, key);
+    if (setting == nullptr) return fail(FH_ERR_PARAMETER, "unknown tuning key %s", key);
     std::string k(key);
     bool ok = true;
     if (k == "k_quant_gemv_ksplit") {
@@ -487,35 +541,31 @@ fh_status fh_set_tuning(fh_device* device, const char* key, int64_t value) {
         ok = value > 0 && !device->capturing;
     }
     if (!ok) return fail(FH_ERR_PARAMETER, "value %lld is out of range for %s", (long long)value, key);
-    it->second = value;
+    *setting = value;
     return FH_OK;
 }
 
 fh_status fh_get_tuning(const fh_device* device, const char* key, int64_t* value) {
     if (device == nullptr || key == nullptr || value == nullptr)
         return fail(FH_ERR_PARAMETER, "null argument");
-    auto it = device->tuning.find(key);
-    if (it == device->tuning.end()) return fail(FH_ERR_PARAMETER, "unknown tuning key %s", key);
-    *value = it->second;
+    const int64_t* const setting = tuning_of(device, key);
+    if (setting == nullptr) return fail(FH_ERR_PARAMETER, "unknown tuning key %s", key);
+    *value = *setting;
     return FH_OK;
 }
 
 // ---- buffers -------------------------------------------------------------------
 
-fh_status fh_buffer_alloc(fh_device* device, size_t bytes, fh_buffer** out) {
+fh_status fh_buffer_alloc_uninitialized(fh_device* device, size_t bytes, fh_buffer** out) {
     if (device && device->capturing) return fail(FH_ERR_SYNCHRONIZATION, "not available while an execution is being recorded");
     if (device == nullptr || out == nullptr) return fail(FH_ERR_PARAMETER, "null argument");
     *out = nullptr;
     if (bytes == 0) return fail(FH_ERR_ALLOCATION, "zero-length buffer");
     FH_HIP(hipSetDevice(device->ordinal));
     void* p = nullptr;
-    hipError_t e = hipMalloc(&p, bytes);
-    if (e != hipSuccess) return fail(FH_ERR_ALLOCATION, "hipMalloc(%zu): %s", bytes, hipGetErrorString(e));
-    e = hipMemsetAsync(p, 0, bytes, device->stream);
-    if (e != hipSuccess) {
-        (void)hipFree(p);
-        return hip_fail(e, "hipMemsetAsync");
-    }
+    const size_t capacity = block_capacity(bytes);
+    hipError_t e = take_block(device, capacity, &p);
+    if (e != hipSuccess) return fail(FH_ERR_ALLOCATION, "hipMalloc(%zu): %s", capacity, hipGetErrorString(e));
     fh_buffer* b = new (std::nothrow) fh_buffer();
     if (b == nullptr) {
         (void)hipFree(p);
@@ -525,19 +575,46 @@ fh_status fh_buffer_alloc(fh_device* device, size_t bytes, fh_buffer** out) {
     ++device->handles;
     b->ptr = p;
     b->bytes = bytes;
+    b->capacity = capacity;
     *out = b;
+    return FH_OK;
+}
+
+fh_status fh_buffer_alloc(fh_device* device, size_t bytes, fh_buffer** out) {
+    fh_status st = fh_buffer_alloc_uninitialized(device, bytes, out);
+    if (st != FH_OK) return st;
+    const hipError_t e = hipMemsetAsync((*out)->ptr, 0, bytes, device->stream);
+    if (e != hipSuccess) {
+        fh_buffer_free(*out);
+        *out = nullptr;
+        return hip_fail(e, "hipMemsetAsync");
+    }
     return FH_OK;
 }
 
 void fh_buffer_free(fh_buffer* buffer) {
     if (buffer == nullptr) return;
-    release_memory(buffer->device, buffer->ptr);
-    drop_device_handle(buffer->device);
+    fh_device* const d = buffer->device;
+    // Nothing waits: whatever the library still has to do with the block comes before the next buffer's
+    // work on the stream.  A block whose address the caller has been given may be in use elsewhere and
+    // goes back to the system.  A full pool holds sizes that are no longer asked for and is emptied.
+    if (!d->closed && !d->capturing && !buffer->exposed && buffer->capacity <= kPoolBlockBytes) {
+        if (d->pool_bytes + buffer->capacity > kPoolBytes) drain_pool(d);
+        d->pool.emplace(buffer->capacity, buffer->ptr);
+        d->pool_bytes += buffer->capacity;
+    } else {
+        release_memory(d, buffer->ptr);
+    }
+    drop_device_handle(d);
     delete buffer;
 }
 
 size_t fh_buffer_size(const fh_buffer* buffer) { return buffer ? buffer->bytes : 0; }
-void* fh_buffer_device_ptr(fh_buffer* buffer) { return buffer ? buffer->ptr : nullptr; }
+void* fh_buffer_device_ptr(fh_buffer* buffer) {
+    if (buffer == nullptr) return nullptr;
+    buffer->exposed = true;
+    return buffer->ptr;
+}
 
 fh_status fh_buffer_upload(fh_buffer* buffer, size_t offset, const void* src, size_t bytes) {
     if (buffer && buffer->device->capturing) return fail(FH_ERR_SYNCHRONIZATION, "not available while an execution is being recorded");
@@ -645,7 +722,7 @@ fh_status fh_qmatrix_create(fh_device* device, uint32_t ggml_type, uint64_t rows
     FH_HIP(hipSetDevice(device->ordinal));
     void* dptr = nullptr;
     // 16 spare bytes keep vector loads of the last block inside the allocation
-    hipError_t e = hipMalloc(&dptr, upload_len + 16);
+    hipError_t e = allocate(device, &dptr, upload_len + 16);
     if (e != hipSuccess)
         return fail(FH_ERR_ALLOCATION, "hipMalloc(%zu): %s", upload_len, hipGetErrorString(e));
     e = hipMemcpyAsync(dptr, p, upload_len, hipMemcpyHostToDevice, device->stream);
@@ -745,13 +822,13 @@ GemmArgs gemm_args(const fh_device* device, uint32_t ggml_type, uint64_t n, uint
     g.x_dtype = x_dtype;
     g.y_dtype = y_dtype;
     g.cu_count = device->props.multiProcessorCount;
-    g.wide_min_rows = (int)tuning(device, "gemm_wide_min_rows");
-    g.wide_shape = (int)tuning(device, "gemm_wide_shape");
-    g.wide32_tile = (int)tuning(device, "gemm_wide32_tile");
-    g.skinny_max_rows = (int)tuning(device, "gemm_skinny_max_rows");
-    g.resident_switch = tuning(device, "gemm_resident") != 0;
+    g.wide_min_rows = (int)device->tuning.gemm_wide_min_rows;
+    g.wide_shape = (int)device->tuning.gemm_wide_shape;
+    g.wide32_tile = (int)device->tuning.gemm_wide32_tile;
+    g.skinny_max_rows = (int)device->tuning.gemm_skinny_max_rows;
+    g.resident_switch = device->tuning.gemm_resident != 0;
     g.rows_resident = g.resident_switch && expert_rows_fit_lds((uint32_t)k, 1, 1);
-    g.few_rows = tuning(device, "gemm_few_tiles_split") != 0;
+    g.few_rows = device->tuning.gemm_few_tiles_split != 0;
     return g;
 }
 
@@ -810,17 +887,17 @@ fh_status project(fh_device* device, const fh_qmatrix* weight, const fh_view* x,
     // caller asks for the tile kernels from some row count on, as the reference's hybrid
     // engine does from 5 rows (HybridModel::project, src/hybrid/engine.rs:3407-3500): the
     // activations are then rounded to f16 into the device scratch first.
-    const int64_t f32_tile_rows = f32_tile_from >= 0 ? f32_tile_from : tuning(device, "gemm_f32_min_rows");
+    const int64_t f32_tile_rows = f32_tile_from >= 0 ? f32_tile_from : device->tuning.gemm_f32_min_rows;
     const bool f32_tile = !silu_mul && x->dtype == FH_F32 && f32_tile_rows > 0 && m >= (uint64_t)f32_tile_rows &&
                           ((uintptr_t)xr.begin & 15u) == 0;
-    const bool tile = f32_tile || (!silu_mul && m >= (uint32_t)tuning(device, "gemm_min_rows") && x->dtype != FH_F32);
+    const bool tile = f32_tile || (!silu_mul && m >= (uint32_t)device->tuning.gemm_min_rows && x->dtype != FH_F32);
     // A batch of exact f32 rows: the GEMV kernels read every weight once per row, the few-rows kernel
     // once per sixteen.  Four rows of 17408 x 5120 take it 36 us, the GEMV 36 for Q4_K (20 and 27 for two
     // and three) and 43 - 58 for the other formats; sixteen rows 38 against 121 - 230.  Where a GEMV
     // kernel or its K segments are asked for by name, those run.
     const bool f32_batch = !tile && !silu_mul && x->dtype == FH_F32 && m >= (weight->ggml_type == kQ4K ? 5u : 4u) &&
-                           m >= (uint32_t)tuning(device, "gemm_min_rows") && tuning(device, "gemv_stream") == 1 &&
-                           tuning(device, "k_quant_gemv_ksplit") == 0;
+                           m >= (uint32_t)device->tuning.gemm_min_rows && device->tuning.gemv_stream == 1 &&
+                           device->tuning.k_quant_gemv_ksplit == 0;
     GemmArgs g{};
     if (tile || f32_batch) g = gemm_args(device, weight->ggml_type, n, k, m, f32_tile ? FH_F16 : x->dtype, y->dtype);
     if (f32_batch && g.few_rows) {
@@ -854,9 +931,9 @@ fh_status project(fh_device* device, const fh_qmatrix* weight, const fh_view* x,
         a.y_dtype = y->dtype;
         a.metadata = nullptr;
         a.experts = 1;
-        a.ksplit = (int)tuning(device, "k_quant_gemv_ksplit");
-        a.stream = (int)tuning(device, "gemv_stream");
-        a.stream_own = tuning(device, "gemv_stream_own_loads") != 0;
+        a.ksplit = (int)device->tuning.k_quant_gemv_ksplit;
+        a.stream = (int)device->tuning.gemv_stream;
+        a.stream_own = device->tuning.gemv_stream_own_loads != 0;
         a.cu_count = device->props.multiProcessorCount;
         a.x_mode = silu_mul ? kXSiluMul : kXPlain;
         a.x_rows = m;
@@ -931,9 +1008,9 @@ fh_status fh_project_quantized_no_alloc(fh_device* device, const fh_qmatrix* wei
     a.x_dtype = x->dtype;
     a.y_dtype = y->dtype;
     a.experts = 1;
-    a.ksplit = (int)tuning(device, "k_quant_gemv_ksplit");
-    a.stream = (int)tuning(device, "gemv_stream");
-    a.stream_own = tuning(device, "gemv_stream_own_loads") != 0;
+    a.ksplit = (int)device->tuning.k_quant_gemv_ksplit;
+    a.stream = (int)device->tuning.gemv_stream;
+    a.stream_own = device->tuning.gemv_stream_own_loads != 0;
     a.cu_count = device->props.multiProcessorCount;
     a.x_mode = kXPlain;
     a.x_rows = m;
@@ -963,7 +1040,7 @@ fh_status fh_probe_read(fh_device* device, const fh_qmatrix* weight) {
     fh_status st = ensure_scratch(device, 0);
     if (st != FH_OK) return st;
     device->last_operation = launch_read_probe(device->stream, weight->ptr, weight->bytes,
-                                               reinterpret_cast<uint32_t*>(scratch_data(device)), tuning(device, "probe_read_form"));
+                                               reinterpret_cast<uint32_t*>(scratch_data(device)), device->tuning.probe_read_form);
     FH_HIP(hipGetLastError());
     return FH_OK;
 }
@@ -1467,7 +1544,7 @@ fh_status hybrid_project_mm_id(fh_device* device, const fh_qmatrix* weight, cons
     g.experts = (uint32_t)weight->experts;
     g.expert_offsets = reinterpret_cast<const uint32_t*>(fr.begin);
     g.expert_order = nullptr;   // rows are already expert-sorted
-    g.weight_ring = tuning(device, "expert_weight_ring") != 0;
+    g.weight_ring = device->tuning.expert_weight_ring != 0;
     if (shared != nullptr) {
         g.shared_w = shared->weight->ptr;
         g.shared_rows = shared->tokens;
@@ -1653,11 +1730,11 @@ fh_status expert_project(fh_device* device, const fh_qmatrix* weight, const fh_v
         if (overlaps(xr, syr) || overlaps(mr, syr) || overlaps(yr, syr))
             return fail(FH_ERR_RANGE, "shared expert output aliases another tensor");
     }
-    const int64_t grouped_min = tuning(device, "expert_grouped_min_assignments");
+    const int64_t grouped_min = device->tuning.expert_grouped_min_assignments;
     // f32 rows join the grouped form when the caller has opted f32 activations into the f16
     // tiles (gemm_f32_min_rows, the hybrid engine's prompt path project_mm_id_in,
     // src/hybrid/engine.rs:3164): they are rounded to f16 into the scratch first
-    const int64_t f32_rows = tuning(device, "gemm_f32_min_rows");
+    const int64_t f32_rows = device->tuning.gemm_f32_min_rows;
     const bool f32_grouped = form == FH_INPUT_ROWS && x->dtype == FH_F32 && f32_rows > 0 &&
                              assignments >= (uint64_t)f32_rows && ((uintptr_t)xr.begin & 15u) == 0;
     const bool grouped = (x->dtype != FH_F32 || f32_grouped) && grouped_min > 0 &&
@@ -1673,7 +1750,7 @@ fh_status expert_project(fh_device* device, const fh_qmatrix* weight, const fh_v
         st = expert_project(device, weight, x, x_rows, form, assignments, metadata, y, nullptr);
         if (st != FH_OK) return st;
         if (form == FH_INPUT_GATHER) return project(device, shared->weight, x, shared->tokens, shared->y, false);
-        if (shared->tokens < (uint64_t)tuning(device, "gemm_min_rows") || ((uintptr_t)sxr.begin & 15u) != 0)
+        if (shared->tokens < (uint64_t)device->tuning.gemm_min_rows || ((uintptr_t)sxr.begin & 15u) != 0)
             return project(device, shared->weight, shared->x, shared->tokens, shared->y, true);
         GemmArgs g = gemm_args(device, weight->ggml_type, rows, k, shared->tokens, x->dtype, y->dtype);
         gemm_takes_rows(g);
@@ -1744,7 +1821,7 @@ fh_status expert_project(fh_device* device, const fh_qmatrix* weight, const fh_v
         g.expert_order = order;
         g.gather_metadata = gathers ? reinterpret_cast<const float*>(mr.begin) : nullptr;
         g.x_rows = x_rows;
-        g.weight_ring = tuning(device, "expert_weight_ring") != 0;
+        g.weight_ring = device->tuning.expert_weight_ring != 0;
         if (shared != nullptr) {
             g.shared_w = shared->weight->ptr;
             g.shared_rows = shared->tokens;
@@ -1924,7 +2001,7 @@ fh_status fh_moe_ffn(fh_device* device, const fh_view* hidden, const fh_view* ro
     // tokens are taken in chunks whose routing temporaries stay under the limit (src/nn/moe.rs:232-256)
     const size_t per_assignment = (2 * (size_t)h + 3 * inter) * es + 3 * sizeof(float);
     const size_t per_token = per_assignment * k + ((size_t)e + (size_t)h) * es;
-    const size_t limit = (size_t)tuning(device, "moe_routing_temporary_limit");
+    const size_t limit = (size_t)device->tuning.moe_routing_temporary_limit;
     const uint32_t chunk = (uint32_t)std::min<size_t>(tokens, std::max<size_t>(1, limit / per_token));
 
     // workspace layout for one chunk
@@ -1970,14 +2047,14 @@ fh_status fh_moe_ffn(fh_device* device, const fh_view* hidden, const fh_view* ro
         // 23.2 us): the projection's launch stages an entry's activations once for 32 rows, this one
         // once for 8.
         const bool folded = count == 1 && a <= 31 && (!shared || rides) && !stored_padded &&
-                            tuning(device, "moe_fold_combine") != 0 &&
+                            device->tuning.moe_fold_combine != 0 &&
                             (!shared_gate || shared_gate->dtype == FH_F32) &&
                             expert_down_combine_fits(output_experts->ggml_type, (uint32_t)h, (uint32_t)inter, k, shared);
         // ... and so does the routing: every workgroup of the gate|up launch routes the token
         // itself before it asks for its expert's rows, which takes a launch and the wait for its
         // records out of the chain
-        const int64_t grouped_from = tuning(device, "expert_grouped_min_assignments");
-        const bool routes_inside = folded && tuning(device, "moe_fold_route") != 0 &&
+        const int64_t grouped_from = device->tuning.expert_grouped_min_assignments;
+        const bool routes_inside = folded && device->tuning.moe_fold_route != 0 &&
                                    (grouped_from <= 0 || a < (uint64_t)grouped_from) &&   // the per-assignment launch
                                    gemv_routes((uint32_t)two_i, (uint32_t)h, (uint32_t)e, k);
         RouteTokenArgs inside{};
@@ -2022,7 +2099,7 @@ fh_status fh_moe_ffn(fh_device* device, const fh_view* hidden, const fh_view* ro
         // Both projections of a chunk group the same records by expert: the second finds the first's
         // offsets and order at the head of the scratch (the router's ids are all valid, and the scratch
         // is brought to the larger call's size before the first, so it does not move in between).
-        const int64_t group_from = tuning(device, "expert_grouped_min_assignments");
+        const int64_t group_from = device->tuning.expert_grouped_min_assignments;
         // (With a shared expert whose rows do not fit LDS a projection runs the shared matrix as a dense call of its
         // own after the grouping, and that call may put partial sums where the lists lie: both then group for themselves.)
         const bool shared_stays_inside = !shared || (rides && expert_rows_fit_lds((uint32_t)h, a, (uint32_t)e) &&

@@ -14,6 +14,27 @@
 #include "../../include/ferrum_hip.h"
 #include "../../include/ferrum_hip_probe.h"
 
+// Kernel-selection switches, set by name through fh_set_tuning (kTuningKeys in capi.hip).
+struct fh_tuning {
+    int64_t k_quant_gemv_ksplit = 0;   // 0 = automatic
+    int64_t gemm_min_rows = 2;         // smallest M that takes the MFMA tile path
+    int64_t gemm_wide_shape = 1;       // matrix instruction of the 128- and 256-row tiles: 0 = 16x16x32, 1 = whichever is estimated faster, 2 = 32x32x16
+    int64_t gemm_wide32_tile = 0;      // 0 = by shape; 12, 14, 15 (128-row tile x 64, 128, 160 columns), 24, 25 (256-row tile)
+    int64_t gemm_wide_min_rows = 33;   // smallest M that takes the 256-row tile (it wins from there up)
+    int64_t gemm_skinny_max_rows = 64; // with gemm_resident 0: largest M that takes the few-rows kernel (0 = never)
+    int64_t expert_grouped_min_assignments = 32;  // fewest assignments grouped by expert (0 = never)
+    int64_t moe_fold_route = 1;        // fh_moe_ffn, one token: the gate|up launch routes the token itself (0 = a moe_route launch first)
+    int64_t gemm_few_tiles_split = 1;  // few rows: a tile's super-blocks dealt over the waves, any K (0 = whole tiles per wave, the kernels for rows that fit LDS or not)
+    int64_t moe_fold_combine = 1;      // fh_moe_ffn with few tokens: down projection and weighted sum in one launch (0 = two)
+    int64_t gemm_resident = 1;         // rows that fit LDS whole take the rows-resident kernel (0 = square tiles)
+    int64_t gemv_stream_own_loads = 1; // the streamed Q4_K GEMV's waves load the super-blocks they multiply (tiles of up to 14 rows); 0: the tile row by row
+    int64_t expert_weight_ring = 1;    // grouped Q4_K / Q6_K expert projection with short rows: weights through LDS rings (0 = straight into registers)
+    int64_t gemv_stream = 1;           // dense Q4_K / Q6_K GEMV on the streamed matrix-core kernel: 0 never, 1 where it wins, 2 wherever it runs
+    int64_t moe_routing_temporary_limit = 128ll << 20;  // bytes of routing temporaries per SparseMoe chunk (src/metal/legacy.rs:95)
+    int64_t gemm_f32_min_rows = 0;     // f32 activations take the f16 tile kernels from this many rows (0 = never)
+    int64_t probe_read_form = 0;       // fh_probe_read: 100 x threads per workgroup + loads per lane (+ 1000000: LDS-direct loads); 0 = 256 x 8
+};
+
 struct fh_device {
     // The device object lives until fh_device_destroy has been called and the last buffer,
     // matrix, graph or event created on it is gone: their release functions read it.
@@ -24,7 +45,13 @@ struct fh_device {
     hipDeviceProp_t props{};
     const char* last_operation = "";
     bool capturing = false;
-    std::map<std::string, int64_t> tuning;
+    fh_tuning tuning;
+    // Blocks of freed buffers, by size, for the buffers to come (fh_buffer_alloc): hipMalloc and hipFree
+    // take 10 - 20 us each and the latter waits for the GPU (a routed FFN of 200 f32 tokens whose operators
+    // return new tensors: 453 us without the pool, 286 with it).  All work of the library on a buffer is on
+    // `stream`, so a block can be handed on at once; buffers whose address has left the library are freed.
+    std::multimap<size_t, void*> pool;
+    size_t pool_bytes = 0;
     // scratch owned by the device: [counter words | floats / ids]
     void* scratch = nullptr;
     size_t scratch_bytes = 0;
@@ -49,6 +76,8 @@ struct fh_buffer {
     fh_device* device = nullptr;
     void* ptr = nullptr;
     size_t bytes = 0;
+    size_t capacity = 0;    // bytes of the block behind ptr
+    bool exposed = false;   // fh_buffer_device_ptr has handed out the address
 };
 
 struct fh_qmatrix {

@@ -129,8 +129,14 @@ fh_status fh_get_tuning(const fh_device* device, const char* key, int64_t* value
 
 /* ---- buffers ----------------------------------------------------------------
  * MetalDevice::allocate (zero-initialised, src/metal/mod.rs:727-734) and the
- * host copies behind Tensor::from_f32 / to_f32 (src/tensor/mod.rs). */
+ * host copies behind Tensor::from_f32 / to_f32 (src/tensor/mod.rs).
+ * fh_buffer_alloc_uninitialized leaves the contents undefined, for outputs an
+ * operator writes whole.  A device keeps up to 256 MiB of freed buffers (of up to
+ * 64 MiB each) for the next ones and returns them to the system when it is
+ * destroyed or memory runs out; freeing does not wait for the stream then.
+ * Buffers whose address fh_buffer_device_ptr has given out are not kept. */
 fh_status fh_buffer_alloc(fh_device* device, size_t bytes, fh_buffer** out);
+fh_status fh_buffer_alloc_uninitialized(fh_device* device, size_t bytes, fh_buffer** out);
 void fh_buffer_free(fh_buffer* buffer);
 size_t fh_buffer_size(const fh_buffer* buffer);
 void* fh_buffer_device_ptr(fh_buffer* buffer);

@@ -835,6 +835,30 @@ def test_releases_asked_for_while_recording_wait_for_its_end(api, d):
     assert np.array_equal(d.project_quantized(x, w).tensor.raw(), want)
 
 
+@pytest.mark.parametrize("nbytes", [4, 4096, 40_000, 1_000_000, 64 << 20, (64 << 20) + 4])
+def test_a_buffer_is_zero_whatever_held_its_memory_before(api, d, nbytes):
+    # the block of a freed buffer serves the next one of its size class behind the work already enqueued
+    for size in (nbytes, nbytes, max(nbytes - 4, 4)):
+        t = api.Tensor.zeros(d, (size // 4,), api.DType.F32)
+        assert not t.raw().any()
+        t.buffer.upload(0, np.full(size // 4, 7, np.uint32))
+        del t
+
+
+def test_a_full_pool_makes_room_and_an_exposed_address_is_not_handed_on(api):
+    dev = api.Device.new()
+    for step in range(12):
+        held = [api.Buffer(dev, (40 << 20) + step * (1 << 20), zeroed=False) for _ in range(4)]
+        del held
+    b = api.Buffer(dev, 3 << 20)
+    address = b.device_ptr()
+    del b
+    kept = [api.Buffer(dev, 3 << 20) for _ in range(4)]
+    assert address and all(k.nbytes == 3 << 20 for k in kept)
+    x = api.Tensor.zeros(dev, (8, 1024), api.DType.F16)
+    assert not x.raw().any()
+
+
 # ------------------------------------------------------------- greedy selection
 
 @pytest.mark.parametrize("dtype_name", ["F32", "F16", "BF16"])
