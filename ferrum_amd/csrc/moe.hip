@@ -10,13 +10,20 @@
 namespace fh {
 namespace {
 
-// One wave per token: route_token of route_device.hpp.
+// One wave per token: route_token of route_device.hpp.  A token's row times the gate vector is a second
+// wave's work (blockDim.x 128): the selection is one dependent chain of some 8 us, and the dot product
+// stood behind it (200 tokens of 2048 f32, 256 experts: the launch takes 12.4 us, 25.2 with one wave
+// for both).
 template <int kPerLane>   // experts <= 64 * kPerLane
-__global__ __launch_bounds__(64) void moe_route_kernel(const RouteTokenArgs a, uint32_t tokens) {
+__global__ __launch_bounds__(128) void moe_route_kernel(const RouteTokenArgs a, uint32_t tokens) {
     extern __shared__ float scores_lds[];  // experts floats
     const uint32_t token = blockIdx.x;
     if (token >= tokens) return;
-    route_token<kPerLane>(a, token, threadIdx.x, scores_lds);
+    if (threadIdx.x >= 64u) {
+        route_gate(a, token, threadIdx.x - 64u);
+        return;
+    }
+    route_token<kPerLane>(a, token, threadIdx.x, scores_lds, nullptr, true, blockDim.x == 64);
 }
 
 // out[a, :] = hidden[token(a), :]; rows are copied in pieces of sizeof(V).
@@ -444,7 +451,8 @@ const char* launch_moe_route(hipStream_t s, const void* logits, uint32_t logits_
     args.shared_gate = x.shared_gate;
     args.ids_out = x.ids_out;
     args.weights_out = x.weights_out;
-#define FH_ROUTE(PL) hipLaunchKernelGGL(moe_route_kernel<PL>, dim3(tokens), dim3(64), lds, s, args, tokens)
+    const uint32_t threads = args.shared_gate != nullptr && args.gate_w != nullptr ? 128u : 64u;
+#define FH_ROUTE(PL) hipLaunchKernelGGL(moe_route_kernel<PL>, dim3(tokens), dim3(threads), lds, s, args, tokens)
     if (p.experts <= 64) FH_ROUTE(1);
     else if (p.experts <= 128) FH_ROUTE(2);
     else if (p.experts <= 256) FH_ROUTE(4);

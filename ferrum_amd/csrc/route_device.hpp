@@ -3,6 +3,8 @@
 // kernel and by the projection that routes its one token itself.
 #pragma once
 
+#include <type_traits>
+
 #include "device_utils.hpp"
 #include "internal.hpp"
 
@@ -34,6 +36,45 @@ __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
     return a > b ? a : b;
 }
 
+// Shared-expert gate of h_moe_route (src/metal/shaders/hybrid.metal:2259-2319) for one token by one wave:
+// sigmoid(dot(x[token], gate_w)), or 1 without a gate vector.
+// Sixteen elements a lane are in flight (one by one the row is a chain of hidden / 64 round trips),
+// added in the order of the plain loop.  The element type is resolved outside the loop: a test of it
+// at every load keeps the compiler from issuing the sixteen together.
+template <int DT>
+__device__ __forceinline__ float route_gate_dot(const RouteTokenArgs& a, uint32_t token, uint32_t lane) {
+    const uint32_t hidden = a.hidden;
+    const size_t row = (size_t)token * hidden;
+    float dot = 0.f;
+    for (uint32_t i0 = lane; i0 < hidden; i0 += 16 * 64) {
+        float xv[16], wv[16];
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+            // (past the row: its last element once more, not added)
+            const uint32_t i = min(i0 + 64u * j, hidden - 1);
+            xv[j] = load_as_f32<DT>(a.gate_x, row + i);
+            wv[j] = a.gate_w[i];
+        }
+#pragma unroll
+        for (int j = 0; j < 16; ++j)
+            if (i0 + 64u * j < hidden) dot += xv[j] * wv[j];
+    }
+    return dot;
+}
+
+__device__ __forceinline__ void route_gate(const RouteTokenArgs& a, uint32_t token, uint32_t lane) {
+    if (a.shared_gate == nullptr) return;
+    float gate = 1.f;
+    if (a.gate_w != nullptr) {
+        float dot = a.gate_x_dtype == 0   ? route_gate_dot<0>(a, token, lane)
+                    : a.gate_x_dtype == 1 ? route_gate_dot<1>(a, token, lane)
+                                          : route_gate_dot<2>(a, token, lane);
+        dot = wave_sum(dot);
+        gate = 1.f / (1.f + expf(-dot));
+    }
+    if (lane == 0) a.shared_gate[token] = gate;
+}
+
 // One wave per token.  Scores are computed by all lanes in parallel; the
 // softmax normaliser is then summed by one lane in expert order so it carries
 // the same f32 rounding as a sequential host loop.  Selection runs top_k
@@ -41,22 +82,17 @@ __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
 // token the kernel is one wave's dependent instruction stream, so its length is
 // its duration: reductions are DPP, owners are found by ballot.
 // `local`: when set, the token's top_k records {id, token, weight} are also written there (LDS of
-// the calling workgroup); `publish`: whether this wave writes the outputs in device memory.
+// the calling workgroup); `publish`: whether this wave writes the outputs in device memory; `gate`:
+// whether it computes the shared expert's gate as well.
 template <int kPerLane>   // experts <= 64 * kPerLane
 __device__ __forceinline__ void route_token(const RouteTokenArgs& a, uint32_t token, uint32_t lane, float* scores_lds,
-                                            float* local = nullptr, bool publish = true) {
+                                            float* local = nullptr, bool publish = true, bool gate = true) {
     const void* logits = a.logits;
-    const uint32_t logits_dtype = a.logits_dtype;
     const float* bias = a.bias;
     float* metadata = a.metadata;
     const uint32_t experts = a.experts, top_k = a.top_k, sigmoid = a.sigmoid, normalize = a.normalize;
     const float eps = a.eps, scaling = a.scaling;
     const uint32_t rank_order = a.rank_order;
-    const void* gate_x = a.gate_x;
-    const uint32_t gate_x_dtype = a.gate_x_dtype;
-    const float* gate_w = a.gate_w;
-    const uint32_t hidden = a.hidden;
-    float* shared_gate = a.shared_gate;
     float* ids_out = a.ids_out;
     float* weights_out = a.weights_out;
     const size_t base = (size_t)token * experts;
@@ -64,12 +100,20 @@ __device__ __forceinline__ void route_token(const RouteTokenArgs& a, uint32_t to
     float score[kPerLane];
     float logit[kPerLane];
     float maximum = -INFINITY;
+    // (the type is resolved outside: a test of it at every load chains the loads)
+    auto load_logits = [&](auto kind) {
 #pragma unroll
-    for (int i = 0; i < kPerLane; ++i) {
-        uint32_t e = lane + 64u * i;
-        logit[i] = e < experts ? load_as_f32(logits, base + e, logits_dtype) : -INFINITY;
-        maximum = fmaxf(maximum, logit[i]);
-    }
+        for (int i = 0; i < kPerLane; ++i) {
+            const uint32_t e = lane + 64u * i;
+            const float v = load_as_f32<decltype(kind)::value>(logits, base + min(e, experts - 1));
+            logit[i] = e < experts ? v : -INFINITY;
+        }
+    };
+    if (a.logits_dtype == 0) load_logits(std::integral_constant<int, 0>{});
+    else if (a.logits_dtype == 1) load_logits(std::integral_constant<int, 1>{});
+    else load_logits(std::integral_constant<int, 2>{});
+#pragma unroll
+    for (int i = 0; i < kPerLane; ++i) maximum = fmaxf(maximum, logit[i]);
     if (sigmoid) {
 #pragma unroll
         for (int i = 0; i < kPerLane; ++i) score[i] = 1.f / (1.f + expf(-logit[i]));
@@ -202,30 +246,7 @@ __device__ __forceinline__ void route_token(const RouteTokenArgs& a, uint32_t to
         if (weights_out != nullptr && publish) weights_out[slot] = weight;
     }
 
-    // Shared-expert gate of h_moe_route (src/metal/shaders/hybrid.metal:2259-2319):
-    // sigmoid(dot(x[token], gate_w)), or 1 without a gate vector.
-    if (shared_gate != nullptr && publish) {
-        float dot = 0.f;
-        if (gate_w != nullptr) {
-            // sixteen elements a lane in flight (one by one the row is a chain of hidden / 64 round trips: 16
-            // of the launch's 23 us at 2048), added in the order of the plain loop
-            const size_t row = (size_t)token * hidden;
-            for (uint32_t i0 = lane; i0 < hidden; i0 += 16 * 64) {
-                float xv[16], wv[16];
-#pragma unroll
-                for (int j = 0; j < 16; ++j) {
-                    const uint32_t i = i0 + 64u * j;
-                    xv[j] = i < hidden ? load_as_f32(gate_x, row + i, gate_x_dtype) : 0.f;
-                    wv[j] = i < hidden ? gate_w[i] : 0.f;
-                }
-#pragma unroll
-                for (int j = 0; j < 16; ++j)
-                    if (i0 + 64u * j < hidden) dot += xv[j] * wv[j];
-            }
-            dot = wave_sum(dot);
-        }
-        if (lane == 0) shared_gate[token] = gate_w != nullptr ? 1.f / (1.f + expf(-dot)) : 1.f;
-    }
+    if (gate && publish) route_gate(a, token, lane);
 }
 
 }  // namespace fh
