@@ -1514,21 +1514,16 @@ fh_status hybrid_project_mm_id(fh_device* device, const fh_qmatrix* weight, cons
             return project(device, shared->weight, shared->x, shared->tokens, shared->y, false, 5);
         }
     }
-    // the tiles are f16 / bf16, as the reference's h_mm_id kernels make theirs; f32 rows are rounded to f16 first
+    // The tiles are f16 / bf16, as the reference's h_mm_id kernels make theirs.  f32 rows are rounded to f16
+    // by the kernel that gathers them into LDS, or first where they are too wide for that one.
+    const bool rounds_inside = x->dtype == FH_F32 && expert_rows_fit_lds((uint32_t)k, routes, (uint32_t)weight->experts);
     const void* tile_x = xr.begin;
-    const void* shared_tile_x = sxr.begin;
-    if (x->dtype == FH_F32) {
-        const size_t shared_elements = shared != nullptr ? (size_t)shared->tokens * k : 0;
-        st = ensure_scratch(device, ((size_t)routes * k + shared_elements) * sizeof(uint16_t));
+    if (x->dtype == FH_F32 && !rounds_inside) {   // (a shared expert has left for its own call above)
+        st = ensure_scratch(device, (size_t)routes * k * sizeof(uint16_t));
         if (st != FH_OK) return st;
         uint16_t* x16 = reinterpret_cast<uint16_t*>(scratch_data(device));
         launch_round_to_f16(device->stream, reinterpret_cast<const float*>(xr.begin), x16, (size_t)routes * k);
         tile_x = x16;
-        if (shared != nullptr) {
-            launch_round_to_f16(device->stream, reinterpret_cast<const float*>(sxr.begin), x16 + (size_t)routes * k,
-                                shared_elements);
-            shared_tile_x = x16 + (size_t)routes * k;
-        }
     }
     GemmArgs g{};
     g.ggml_type = weight->ggml_type;
@@ -1544,11 +1539,12 @@ fh_status hybrid_project_mm_id(fh_device* device, const fh_qmatrix* weight, cons
     g.experts = (uint32_t)weight->experts;
     g.expert_offsets = reinterpret_cast<const uint32_t*>(fr.begin);
     g.expert_order = nullptr;   // rows are already expert-sorted
+    g.x_rounds = rounds_inside;
     g.weight_ring = device->tuning.expert_weight_ring != 0;
     if (shared != nullptr) {
         g.shared_w = shared->weight->ptr;
         g.shared_rows = shared->tokens;
-        g.shared_x = shared_tile_x;
+        g.shared_x = sxr.begin;
         g.shared_y = const_cast<uint8_t*>(syr.begin);
     }
     launch_gemm_skinny(device->stream, g);

@@ -24,6 +24,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 #include "device_utils.hpp"
 #include "lds_direct.hpp"
@@ -241,7 +242,11 @@ struct ResidentShared {
 // in flight at a time.  The row behind a slot is found through up to two tables (the expert-sorted
 // order, then the assignment's token).  All eight pieces look their rows up together, table by
 // table, before any row is read: a round trip per table and one for the rows, where piece after
-// piece would chain up to twenty-four.
+// piece would chain up to twenty-four.  F32: the rows are f32 and rounded to f16 on the way, as
+// launch_round_to_f16 rounds them: a launch for the routed rows, one for the shared expert's and a
+// trip through memory less per projection (1600 routes of 200 tokens, 256 IQ4_XS experts: 116 us for
+// the three launches of a 1024 x 2048 projection, 70 of a 2048 x 512 one; 114 and 62 for one).
+template <bool F32>
 __device__ __forceinline__ void gather_rows(uint16_t* xs, const uint16_t* __restrict__ xsrc, uint32_t mt,
                                             uint32_t pieces, uint32_t k, uint32_t ld, uint32_t first_token,
                                             const uint32_t* __restrict__ order, const float* __restrict__ metadata,
@@ -269,14 +274,32 @@ __device__ __forceinline__ void gather_rows(uint16_t* xs, const uint16_t* __rest
                 row[j] = token < x_rows ? token : x_rows - 1;
             }
         }
+        if constexpr (F32) {
+            const float* const source = reinterpret_cast<const float*>(xsrc);
+            float4 lo[8], hi[8];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] = *reinterpret_cast<const u32x4*>(xsrc + (size_t)row[j] * k + 8 * (size_t)pc[j]);
+            for (int j = 0; j < 8; ++j) {
+                const float4* const at = reinterpret_cast<const float4*>(source + (size_t)row[j] * k + 8 * (size_t)pc[j]);
+                lo[j] = at[0];
+                hi[j] = at[1];
+            }
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                v[j] = u32x4{f32_to_f16_bits(lo[j].x) | (f32_to_f16_bits(lo[j].y) << 16),
+                             f32_to_f16_bits(lo[j].z) | (f32_to_f16_bits(lo[j].w) << 16),
+                             f32_to_f16_bits(hi[j].x) | (f32_to_f16_bits(hi[j].y) << 16),
+                             f32_to_f16_bits(hi[j].z) | (f32_to_f16_bits(hi[j].w) << 16)};
+        } else {
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                v[j] = *reinterpret_cast<const u32x4*>(xsrc + (size_t)row[j] * k + 8 * (size_t)pc[j]);
+        }
 #pragma unroll
         for (int j = 0; j < 8; ++j) *reinterpret_cast<u32x4*>(xs + dst[j]) = v[j];
     }
 }
 
-template <uint32_t TYPE, int DT, int TT>
+template <uint32_t TYPE, int DT, int TT, bool F32 = false>
 __global__ __launch_bounds__(kResThreads) void expert_resident_kernel(const uint8_t* __restrict__ w,
                                                                      const uint16_t* __restrict__ x,
                                                                      void* __restrict__ y, uint32_t n,
@@ -331,7 +354,7 @@ __global__ __launch_bounds__(kResThreads) void expert_resident_kernel(const uint
         const uint16_t* xsrc = shared && sh.x != nullptr ? sh.x : x;
         void* ydst = shared ? sh.y : y;
         if (item != 0) __syncthreads();  // the previous item is done with the rows
-        gather_rows(xs, xsrc, mt, pieces, k, ld, first_token, shared ? nullptr : order, shared ? nullptr : metadata,
+        gather_rows<F32>(xs, xsrc, mt, pieces, k, ld, first_token, shared ? nullptr : order, shared ? nullptr : metadata,
                     x_rows, tid);
         __syncthreads();
         if (tile_begin >= tile_end) continue;  // uniform per wave; no barrier follows in this item
@@ -443,7 +466,7 @@ __global__ __launch_bounds__(kResThreads) void expert_resident_kernel(const uint
 // chunk's quants out of LDS.  It needs room for the rings beside the token rows (rows of up to
 // ~1024 weights for 32 tokens), and n a multiple of 16 (a tile is read whole).  Q4_K and Q6_K (a
 // tile of either is a whole number of 16-byte pieces at a 16-byte aligned address).
-template <uint32_t TYPE, int DT, int TT, int NB>
+template <uint32_t TYPE, int DT, int TT, int NB, bool F32>
 __global__ __launch_bounds__(kResThreads) void expert_ring_kernel(const uint8_t* __restrict__ w,
                                                                  const uint16_t* __restrict__ x,
                                                                  void* __restrict__ y, uint32_t n,
@@ -509,7 +532,7 @@ __global__ __launch_bounds__(kResThreads) void expert_ring_kernel(const uint8_t*
             }
             ++requested;
         };
-        gather_rows(xs, xsrc, mt, pieces, k, ld, first_token, shared ? nullptr : order, shared ? nullptr : metadata,
+        gather_rows<F32>(xs, xsrc, mt, pieces, k, ld, first_token, shared ? nullptr : order, shared ? nullptr : metadata,
                     x_rows, tid);
         __syncthreads();
         if (my_tiles == 0) continue;  // uniform per wave; no barrier follows in this item
@@ -697,42 +720,39 @@ void launch_tt(hipStream_t s, const GemmArgs& a) {
         // weights through rings in LDS where those fit beside the rows (short rows: the down projections)
         // (Q4_K 49 against 55 us and Q6_K 74 against 77 for 256 experts x 2048 x 512 over 4096 rows; IQ4_XS,
         // whose rows' operands do not fit the registers beside its decode, 62 either way: it stays)
-        if constexpr (TYPE == kQ4K || TYPE == kQ6K) {
-            const size_t tile_bytes = (size_t)16 * nb * Quarter<TYPE>::kBlockBytes;
-            const size_t room = kResLdsBytes > lds ? (kResLdsBytes - lds) / (kResWaves * tile_bytes) : 0;
-            const uint32_t ring_tiles = room >= 3 ? 3u : (uint32_t)room;
-            if (a.weight_ring && a.n % 16 == 0 && nb <= 4 && ring_tiles >= 2) {
-                const size_t ring_lds = lds + kResWaves * ring_tiles * tile_bytes;
-                typedef void (*Ring)(const uint8_t*, const uint16_t*, void*, uint32_t, uint32_t, uint32_t, const uint32_t*,
-                                     const uint32_t*, uint32_t, const float*, uint32_t, uint32_t, const ResidentShared,
-                                     uint32_t);
-                static const Ring rings[2][4] = {
-                    {expert_ring_kernel<TYPE, DT, 1, 1>, expert_ring_kernel<TYPE, DT, 1, 2>, expert_ring_kernel<TYPE, DT, 1, 3>,
-                     expert_ring_kernel<TYPE, DT, 1, 4>},
-                    {expert_ring_kernel<TYPE, DT, 2, 1>, expert_ring_kernel<TYPE, DT, 2, 2>, expert_ring_kernel<TYPE, DT, 2, 3>,
-                     expert_ring_kernel<TYPE, DT, 2, 4>}};
-                const Ring kernel = rings[wide ? 1 : 0][nb - 1];
-                (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
-                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)ring_lds);
-                hipLaunchKernelGGL(kernel, rgrid, dim3(kResThreads), ring_lds, s, w, x, a.y, a.n, nb, a.y_dtype,
-                                   a.expert_offsets, a.expert_order, tiles_per_wg, a.gather_metadata, a.x_rows, a.m, sh,
-                                   ring_tiles);
-                return;
+        auto launch = [&](auto rounds) {
+            constexpr bool kF32 = DT == 1 && decltype(rounds)::value;
+            if constexpr (TYPE == kQ4K || TYPE == kQ6K) {
+                const size_t tile_bytes = (size_t)16 * nb * Quarter<TYPE>::kBlockBytes;
+                const size_t room = kResLdsBytes > lds ? (kResLdsBytes - lds) / (kResWaves * tile_bytes) : 0;
+                const uint32_t ring_tiles = room >= 3 ? 3u : (uint32_t)room;
+                if (a.weight_ring && a.n % 16 == 0 && nb <= 4 && ring_tiles >= 2) {
+                    const size_t ring_lds = lds + kResWaves * ring_tiles * tile_bytes;
+                    typedef void (*Ring)(const uint8_t*, const uint16_t*, void*, uint32_t, uint32_t, uint32_t,
+                                         const uint32_t*, const uint32_t*, uint32_t, const float*, uint32_t, uint32_t,
+                                         const ResidentShared, uint32_t);
+                    static const Ring rings[2][4] = {
+                        {expert_ring_kernel<TYPE, DT, 1, 1, kF32>, expert_ring_kernel<TYPE, DT, 1, 2, kF32>,
+                         expert_ring_kernel<TYPE, DT, 1, 3, kF32>, expert_ring_kernel<TYPE, DT, 1, 4, kF32>},
+                        {expert_ring_kernel<TYPE, DT, 2, 1, kF32>, expert_ring_kernel<TYPE, DT, 2, 2, kF32>,
+                         expert_ring_kernel<TYPE, DT, 2, 3, kF32>, expert_ring_kernel<TYPE, DT, 2, 4, kF32>}};
+                    const Ring kernel = rings[wide ? 1 : 0][nb - 1];
+                    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)ring_lds);
+                    hipLaunchKernelGGL(kernel, rgrid, dim3(kResThreads), ring_lds, s, w, x, a.y, a.n, nb, a.y_dtype,
+                                       a.expert_offsets, a.expert_order, tiles_per_wg, a.gather_metadata, a.x_rows, a.m,
+                                       sh, ring_tiles);
+                    return;
+                }
             }
-        }
-        if (wide) {
-            auto kernel = expert_resident_kernel<TYPE, DT, 2>;
-            (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+            auto kernel = wide ? expert_resident_kernel<TYPE, DT, 2, kF32> : expert_resident_kernel<TYPE, DT, 1, kF32>;
+            (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                      (int)lds);
             hipLaunchKernelGGL(kernel, rgrid, dim3(kResThreads), lds, s, w, x, a.y, a.n, nb, a.y_dtype,
                                a.expert_offsets, a.expert_order, tiles_per_wg, a.gather_metadata, a.x_rows, a.m, sh);
-        } else {
-            auto kernel = expert_resident_kernel<TYPE, DT, 1>;
-            (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-            hipLaunchKernelGGL(kernel, rgrid, dim3(kResThreads), lds, s, w, x, a.y, a.n, nb, a.y_dtype,
-                               a.expert_offsets, a.expert_order, tiles_per_wg, a.gather_metadata, a.x_rows, a.m, sh);
-        }
+        };
+        if (DT == 1 && a.x_rounds) launch(std::true_type{});
+        else launch(std::false_type{});
         return;
     }
     const dim3 grid((a.n + kSkRows - 1) / kSkRows, a.experts);

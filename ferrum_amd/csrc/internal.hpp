@@ -318,6 +318,7 @@ struct GemmArgs {
     uint32_t shared_rows;
     const void* shared_x;
     void* shared_y;
+    bool x_rounds;   // routed form, rows resident, x_dtype f16: x and shared_x are f32 rows that the kernel rounds to f16
     // dense product: the rows are short enough to stay in LDS for the whole K (launch_gemm
     // then weighs launch_gemm_resident against the other kernels)
     bool rows_resident;

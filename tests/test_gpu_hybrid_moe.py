@@ -192,6 +192,24 @@ def test_project_mm_id_keeps_inside_its_rows_whatever_the_offsets_say(api, d, co
     assert np.isfinite(d.hybrid_project_mm_id(w, x, carrier(api, d, table)).to_f32()).all()
 
 
+@pytest.mark.parametrize("ggml,cols,routes", [
+    (Q4_K, 512, 40), (Q4_K, 512, 200),     # weights through LDS rings, passes of 16 and of 32 tokens
+    (Q4_K, 2048, 200), (IQ4_XS, 512, 40),  # weights straight into registers
+    (Q4_K, 5120, 40), (Q4_K, 5376, 40),    # the widest rows of that kernel, and wider ones
+])
+def test_project_mm_id_rounds_f32_rows_as_a_separate_rounding_would(api, d, ggml, cols, routes):
+    experts, rows = 8, 80
+    fmt = api.QuantizationFormat(ggml)
+    w = api.QuantizedExpertMatrix.new(d, synth.matrix(ggml, experts * rows, cols, seed=451), fmt, experts, rows, cols)
+    offsets, _, _ = d.hybrid_moe_map(carrier(api, d, synth.rng(452).integers(0, experts, routes).astype(np.uint32)), experts)
+    x = synth.activations(routes, cols, seed=453)
+    x[0, :4] = [65519.0, 1e-7, -2.0 ** -25, 2049.0]   # the largest f16, subnormals, a tie
+    wide = d.hybrid_project_mm_id(w, api.Tensor.from_f32(d, x.shape, api.DType.F32, x), offsets)
+    half = api.Tensor.from_f32(d, x.shape, api.DType.F16, oracle.round_storage(x, oracle.F16))
+    narrow = d.hybrid_project_mm_id(w, half, offsets, out_dtype=api.DType.F32)
+    assert np.array_equal(bits(wide.to_f32()), bits(narrow.to_f32()))
+
+
 def test_prompt_chain_map_gather_mm_id_combine_matches_the_decode_chain_and_the_oracle(api, d):
     # HybridModel::moe_ffn's two branches (src/hybrid/engine.rs:3030-3075): per-route GEMVs with
     # `identity` rows, or map -> gather -> expert GEMM over sorted rows -> combine through position
