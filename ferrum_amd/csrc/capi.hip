@@ -73,21 +73,26 @@ fh_status resolve(const fh_device* device, const fh_view* view, uint64_t element
 
 bool fits_u32(uint64_t v) { return v <= 0xffffffffull; }
 
-void drain_pool(fh_device* d) {
-    if (d->pool.empty()) return;
+// Gives back what the pool holds; whether it held anything.
+bool drain_pool(fh_device* d) {
+    std::multimap<size_t, void*> blocks;
+    {
+        std::lock_guard<std::mutex> hold(d->pool_lock);
+        blocks.swap(d->pool);
+        d->pool_bytes = 0;
+    }
+    if (blocks.empty()) return false;
     (void)hipStreamSynchronize(d->stream);
-    for (auto& block : d->pool) (void)hipFree(block.second);
-    d->pool.clear();
-    d->pool_bytes = 0;
+    for (auto& block : blocks) (void)hipFree(block.second);
+    return true;
 }
 
 // Memory from the system; what the pool holds is given back when there is none.
 hipError_t allocate(fh_device* d, void** out, size_t bytes) {
     hipError_t e = hipMalloc(out, bytes);
-    if (e == hipErrorOutOfMemory && !d->pool.empty()) {
+    if (e == hipErrorOutOfMemory) {
         (void)hipGetLastError();
-        drain_pool(d);
-        e = hipMalloc(out, bytes);
+        if (drain_pool(d)) e = hipMalloc(out, bytes);
     }
     return e;
 }
@@ -346,14 +351,38 @@ size_t block_capacity(size_t bytes) {
 }
 
 hipError_t take_block(fh_device* d, size_t capacity, void** out) {
-    const auto found = d->pool.find(capacity);
-    if (found != d->pool.end()) {
-        *out = found->second;
-        d->pool_bytes -= capacity;
-        d->pool.erase(found);
-        return hipSuccess;
+    {
+        std::lock_guard<std::mutex> hold(d->pool_lock);
+        const auto found = d->pool.find(capacity);
+        if (found != d->pool.end()) {
+            *out = found->second;
+            d->pool_bytes -= capacity;
+            d->pool.erase(found);
+            return hipSuccess;
+        }
     }
     return allocate(d, out, capacity);
+}
+
+// Takes a freed buffer's block into the pool; false: the caller frees it.  Nothing waits: whatever the
+// library still has to do with the block comes before the next buffer's work on the stream.  A block whose
+// address the caller has been given may be in use elsewhere and goes back to the system.
+bool keep_block(fh_device* d, const fh_buffer& buffer) {
+    if (d->closed || d->capturing || buffer.exposed || buffer.capacity > kPoolBlockBytes) return false;
+    bool full;
+    {
+        std::lock_guard<std::mutex> hold(d->pool_lock);
+        full = d->pool_bytes + buffer.capacity > kPoolBytes;
+    }
+    if (full) drain_pool(d);   // it holds sizes that are no longer asked for
+    try {
+        std::lock_guard<std::mutex> hold(d->pool_lock);
+        d->pool.emplace(buffer.capacity, buffer.ptr);
+        d->pool_bytes += buffer.capacity;
+    } catch (...) {   // no memory for the entry
+        return false;
+    }
+    return true;
 }
 
 }  // namespace
@@ -595,16 +624,7 @@ fh_status fh_buffer_alloc(fh_device* device, size_t bytes, fh_buffer** out) {
 void fh_buffer_free(fh_buffer* buffer) {
     if (buffer == nullptr) return;
     fh_device* const d = buffer->device;
-    // Nothing waits: whatever the library still has to do with the block comes before the next buffer's
-    // work on the stream.  A block whose address the caller has been given may be in use elsewhere and
-    // goes back to the system.  A full pool holds sizes that are no longer asked for and is emptied.
-    if (!d->closed && !d->capturing && !buffer->exposed && buffer->capacity <= kPoolBlockBytes) {
-        if (d->pool_bytes + buffer->capacity > kPoolBytes) drain_pool(d);
-        d->pool.emplace(buffer->capacity, buffer->ptr);
-        d->pool_bytes += buffer->capacity;
-    } else {
-        release_memory(d, buffer->ptr);
-    }
+    if (!keep_block(d, *buffer)) release_memory(d, buffer->ptr);
     drop_device_handle(d);
     delete buffer;
 }

@@ -4,9 +4,11 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstdint>
 #include <cstdio>
 #include <map>
+#include <mutex>
 #include <utility>
 #include <vector>
 #include <string>
@@ -38,7 +40,7 @@ struct fh_tuning {
 struct fh_device {
     // The device object lives until fh_device_destroy has been called and the last buffer,
     // matrix, graph or event created on it is gone: their release functions read it.
-    int handles = 1;       // the caller's own handle, plus one per live object
+    std::atomic<int> handles{1};   // the caller's own handle, plus one per live object
     bool closed = false;   // fh_device_destroy has run: the stream is gone, memory is freed directly
     int ordinal = 0;
     hipStream_t stream = nullptr;
@@ -50,6 +52,8 @@ struct fh_device {
     // take 10 - 20 us each and the latter waits for the GPU (a routed FFN of 200 f32 tokens whose operators
     // return new tensors: 453 us without the pool, 286 with it).  All work of the library on a buffer is on
     // `stream`, so a block can be handed on at once; buffers whose address has left the library are freed.
+    // Python may drop a buffer on any thread: the pool has a lock.
+    std::mutex pool_lock;
     std::multimap<size_t, void*> pool;
     size_t pool_bytes = 0;
     // scratch owned by the device: [counter words | floats / ids]
