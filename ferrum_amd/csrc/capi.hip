@@ -126,6 +126,14 @@ fh_status ensure_scratch(fh_device* d, size_t data_bytes) {
     FH_HIP(hipMemsetAsync(d->scratch, 0, counter_bytes, d->stream));
     return FH_OK;
 }
+
+// Whether the scratch can be brought to `data_bytes` now: it does not grow while an execution is being
+// recorded.  Kernels that only save time by using it leave such a call to those that need none.
+bool scratch_available(const fh_device* d, size_t data_bytes) {
+    return !d->capturing ||
+           (d->scratch != nullptr && d->scratch_bytes >= fh_device::kCounterWords * sizeof(uint32_t) + data_bytes);
+}
+
 // A block the library owns for its own temporaries (it holds no count on the device), grown like
 // the scratch: outside recordings only, by at least 2x, old blocks kept for the recorded executions
 // that carry their address.
@@ -855,7 +863,8 @@ GemmArgs gemm_args(const fh_device* device, uint32_t ggml_type, uint64_t n, uint
 // Brings the scratch to what the product needs behind `used` bytes of the caller's at its head.
 fh_status prepare_gemm(fh_device* device, GemmArgs& g, size_t used) {
     const size_t at = align256(used);
-    fh_status st = ensure_scratch(device, at + g.rows_plan.partial_bytes);
+    if (!scratch_available(device, at + g.rows_plan.partial_bytes)) g.rows_plan = RowsPlan{};
+    fh_status st = ensure_scratch(device, g.rows_plan.partial_bytes != 0 ? at + g.rows_plan.partial_bytes : used);
     if (st != FH_OK) return st;
     g.counters = scratch_counters(device);
     g.partials = reinterpret_cast<float*>(scratch_data(device) + at);
@@ -922,7 +931,8 @@ fh_status project(fh_device* device, const fh_qmatrix* weight, const fh_view* x,
     if (tile || f32_batch) g = gemm_args(device, weight->ggml_type, n, k, m, f32_tile ? FH_F16 : x->dtype, y->dtype);
     if (f32_batch && g.few_rows) {
         g.rows_plan = gemm_rows_plan(g.ggml_type, g.n, g.k, g.m, g.x_dtype, g.cu_count);
-        if (g.rows_plan.counters > fh_device::kCounterWords) g.rows_plan = RowsPlan{};
+        if (g.rows_plan.counters > fh_device::kCounterWords || !scratch_available(device, g.rows_plan.partial_bytes))
+            g.rows_plan = RowsPlan{};
     }
     if (tile || g.rows_plan.rows != 0) {
         g.w = weight->ptr;
@@ -967,12 +977,15 @@ fh_status project(fh_device* device, const fh_qmatrix* weight, const fh_view* x,
             if (gemv_takes_stream(plain, &stream)) {
                 const GemvScratch need = gemv_scratch(plain);
                 const size_t partial_bytes = align256((size_t)need.segments * n * sizeof(float));
-                st = ensure_scratch(device, partial_bytes + (size_t)k * dtype_bytes(x->dtype));
-                if (st != FH_OK) return st;
-                uint8_t* const row = scratch_data(device) + partial_bytes;   // behind the partial sums
-                launch_expert_silu_mul(device->stream, xr.begin, row, 1, (uint32_t)k, x->dtype, x->dtype);
-                plain.x = row;
-                a = plain;
+                const size_t bytes = partial_bytes + (size_t)k * dtype_bytes(x->dtype);
+                if (scratch_available(device, bytes)) {
+                    st = ensure_scratch(device, bytes);
+                    if (st != FH_OK) return st;
+                    uint8_t* const row = scratch_data(device) + partial_bytes;   // behind the partial sums
+                    launch_expert_silu_mul(device->stream, xr.begin, row, 1, (uint32_t)k, x->dtype, x->dtype);
+                    plain.x = row;
+                    a = plain;
+                }
             }
         }
         const char* name = "";
@@ -1104,7 +1117,7 @@ fh_status fh_argmax_rows(fh_device* device, const fh_view* logits, uint32_t rows
     st = resolve(device, out, (uint64_t)rows * 2, "argmax output", &orr, 4);
     if (st != FH_OK) return st;
     if (overlaps(lr, orr)) return fail(FH_ERR_RANGE, "argmax output aliases its input");
-    st = ensure_scratch(device, argmax_partial_bytes(rows, width));
+    st = ensure_scratch(device, argmax_partial_bytes(rows, width));   // 9 MiB at most, which it always holds
     if (st != FH_OK) return st;
     device->last_operation = launch_argmax_rows(device->stream, lr.begin, logits->dtype, rows, width,
                                                 scratch_data(device), scratch_counters(device),

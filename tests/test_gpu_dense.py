@@ -1076,3 +1076,24 @@ def test_rows_resident_gemm_matches_the_rounded_weight_oracle(api, d, ggml, m, n
         d.set_tuning("gemm_resident", 1)
     assert not tiles.operation.endswith("_resident")
     assert rel_l2(got, tiles.tensor.to_f32()) <= 1e-5
+
+
+@pytest.mark.parametrize("m,n,k,dtype_name", [(320, 5120, 17408, "F32")])
+def test_a_batch_whose_partial_sums_outgrow_the_scratch_can_be_recorded_first(api, m, n, k, dtype_name):
+    """Partial sums of K segments save time only: a device whose scratch cannot hold them while it records
+    takes a kernel that needs none, and replays are that kernel's results."""
+    dev = api.Device.new()
+    dtype = api.DType[dtype_name]
+    w = qm(api, dev, Q4_K, n, k, synth.matrix(Q4_K, n, k, seed=711))
+    x = api.Tensor.from_f32(dev, (m, k), dtype, synth.activations(m, k, seed=712))
+    recorded = api.Tensor.zeros(dev, (m, n), api.DType.F32)
+    dev.synchronize()
+    with dev.execution() as ex:
+        dev.project_quantized(x, w, out=recorded)
+    ex.graph.launch()
+    dev.synchronize()
+    direct = dev.project_quantized(x, w, out_dtype=api.DType.F32).tensor.to_f32()   # the scratch may grow here
+    for _ in range(2):
+        ex.graph.launch()
+        dev.synchronize()
+        assert rel_l2(recorded.to_f32(), direct) <= 1e-5
