@@ -60,6 +60,25 @@ constexpr uint32_t kXRowBytes = DT == 0 ? 1024u : 512u;   // a row's share of a 
 template <int DT, int ROWS>
 constexpr uint32_t kWaveLds = (uint32_t)ROWS * kXRowBytes<DT>;
 
+// Steps FROM .. FROM + COUNT of a super-block of exact f32 operands.  Four steps are chained in the
+// accumulator (16 roundings one after the other), the rest is added in pairs: with all 64 steps in one
+// chain the product was up to four times as far from 64 bits as the GEMV kernels are (rel-L2 of 64 x 777 x
+// 5120 Q5_K 4.5e-7, now 1.12e-7, the GEMV 1.11e-7; 16 x 1024 x 1024 Q4_K 2.8e-7, 1.00e-7, 1.02e-7).  It costs
+// a tenth: a block of projections over 24 rows 213 us, 195 in one chain, 585 on the GEMV.
+template <int FROM, int COUNT>
+__device__ __forceinline__ float4v pairwise(const FloatOperands& a, const u32x4 (&x)[16]) {
+    if constexpr (COUNT > 4) {
+        const float4v lo = pairwise<FROM, COUNT / 2>(a, x);
+        return lo + pairwise<FROM + COUNT / 2, COUNT / 2>(a, x);
+    } else {
+        float4v sum{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = FROM; s < FROM + COUNT; ++s)
+            sum = __builtin_amdgcn_mfma_f32_16x16x4f32(a.v[s], __uint_as_float(x[s >> 2][s & 3]), sum, 0, 0, 0);
+        return sum;
+    }
+}
+
 // ROWS: activation rows of a workgroup, 16 or 32 (a slab of 8 for up to 8 rows measured 17.0 against
 // 17.3 us at 8 x 17408 x 5120: not worth a third more kernels); T: weight tiles per wave.
 // A workgroup has one item of work and a compute unit one workgroup (the operands of a super-block,
@@ -159,11 +178,7 @@ __global__ __launch_bounds__(kRowsThreads) void gemm_rows_kernel(const RowsParam
                     raw[t].decode_into(g, a);
                     if constexpr (kMore) raw[t].load(wrow[t] + (size_t)(b + p.k_waves) * kBB, g);
 #pragma unroll
-                    for (int s = 0; s < 64; ++s)
-#pragma unroll
-                        for (int i = 0; i < TT; ++i)
-                            acc[t][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(
-                                a.v[s], __uint_as_float(frag[i][s >> 2][s & 3]), acc[t][i], 0, 0, 0);
+                    for (int i = 0; i < TT; ++i) acc[t][i] += pairwise<0, 64>(a, frag[i]);
                 } else {
                     PackedOperands<DT> a;
                     raw[t].decode_into(g, a);
