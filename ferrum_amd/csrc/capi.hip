@@ -1667,6 +1667,14 @@ fh_status fh_expert_assign(fh_device* device, const fh_view* hidden, uint32_t to
 
 namespace {
 
+// Whether one per-assignment launch takes this many entries.  Such a launch is not cut into runs while a shared
+// expert rides in it, so it ends with the grid's z extent and, where a long row's K is cut into segments, with
+// the counter words (one per row tile and entry: 4096 x 7168 matrices reach that at 128 entries).
+bool rider_fits(uint32_t n, uint32_t k, uint64_t entries) {
+    const GemvPlan plan = gemv_plan(n, k, 1, 0);
+    return entries <= 65535u && (plan.segments <= 1 || plan.tiles * entries <= fh_device::kCounterWords);
+}
+
 // Whether streaming every hit expert once for all of its rows beats streaming it once per row.  The
 // per-assignment launch reads an expert's matrix for each of its assignments at the chip's rate (5.6
 // MB/us: 2.85 us per token of the 256-expert top-8 FFN); the grouped one waits for the workgroup that
@@ -1772,14 +1780,17 @@ fh_status expert_project(fh_device* device, const fh_qmatrix* weight, const fh_v
                          weight->experts <= 1024 &&
                          (rows * dtype_bytes(y->dtype)) % 4 == 0;
     if (grouped && route != nullptr) return fail(FH_ERR_DISPATCH, "only the per-assignment launch routes its token");
-    if (grouped && shared != nullptr &&
-        !expert_rows_fit_lds((uint32_t)k, assignments, (uint32_t)weight->experts)) {
-        // a shared expert rides in the grouped form only in the kernel that keeps rows in LDS;
-        // with rows too wide for it the two run apart, as the separate calls would
-        st = expert_project(device, weight, x, x_rows, form, assignments, metadata, y, nullptr);
+    if (shared != nullptr &&
+        (grouped ? !expert_rows_fit_lds((uint32_t)k, assignments, (uint32_t)weight->experts)
+                 : !rider_fits((uint32_t)rows, (uint32_t)k, (uint64_t)assignments + shared->tokens))) {
+        // A shared expert rides in the grouped form only in the kernel that keeps rows in LDS, and in the
+        // per-assignment form only where the launch need not be cut into runs: otherwise the two run apart, as
+        // the separate calls would.
+        st = expert_project(device, weight, x, x_rows, form, assignments, metadata, y, nullptr, route);
         if (st != FH_OK) return st;
         if (form == FH_INPUT_GATHER) return project(device, shared->weight, x, shared->tokens, shared->y, false);
-        if (shared->tokens < (uint64_t)device->tuning.gemm_min_rows || ((uintptr_t)sxr.begin & 15u) != 0)
+        if (shared->tokens < (uint64_t)device->tuning.gemm_min_rows || x->dtype == FH_F32 ||
+            ((uintptr_t)sxr.begin & 15u) != 0)
             return project(device, shared->weight, shared->x, shared->tokens, shared->y, true);
         GemmArgs g = gemm_args(device, weight->ggml_type, rows, k, shared->tokens, x->dtype, y->dtype);
         gemm_takes_rows(g);

@@ -269,6 +269,45 @@ def test_few_assignments_per_expert_are_projected_one_by_one(api, d, assignments
     assert_matmul_parity(got.to_f32(), want, f"{assignments} assignments of 64 experts, {dtype}")
 
 
+# Rows of 6400 weights are cut into two K segments, so a per-assignment launch needs a counter word per row tile
+# (8 rows) and entry, and one that carries a shared expert cannot be cut into runs: 2048 entries of 32 tiles are
+# the most it takes, with one more the shared matrix is a call of its own (16-bit weights there).
+@pytest.mark.parametrize("tokens", [2016, 2017])
+@pytest.mark.parametrize("dtype", ["F16", "BF16"])
+def test_a_shared_expert_beside_more_entries_than_one_launch_takes(api, d, tokens, dtype):
+    experts, rows, cols, assignments = 8, 256, 6400, 32
+    code, dt = (oracle.F16, api.DType.F16) if dtype == "F16" else (oracle.BF16, api.DType.BF16)
+    fmt = api.QuantizationFormat.Q4_K
+    packed, packed_shared = synth.matrix(Q4_K, experts * rows, cols, seed=271), synth.matrix(Q4_K, rows, cols, seed=272)
+    w = api.QuantizedExpertMatrix.new(d, packed, fmt, experts, rows, cols)
+    ws = api.QuantizedMatrix.from_bytes(d, rows, cols, fmt, packed_shared)
+    meta = np.zeros((assignments, 3), dtype=np.uint32)
+    meta[:, 0] = synth.rng(273).integers(0, experts, assignments)
+    meta[:, 1] = synth.rng(274).integers(0, tokens, assignments)
+    meta[:, 2] = np.float32(1.0).view(np.uint32)
+    mt = api.Tensor.from_bits(d, meta.shape, meta)
+    rounded = code if tokens > 2016 else 0
+    y, ys = api.Tensor.zeros(d, (assignments, rows), api.DType.F32), api.Tensor.zeros(d, (tokens, rows), api.DType.F32)
+
+    x = oracle.round_storage(synth.activations(tokens, cols, seed=275) * 0.25, code).reshape(tokens, cols)
+    d.expert_project_with_shared(api.Tensor.from_f32(d, x.shape, dt, x), mt, w, ws, tokens, "gather", out=y, shared_out=ys)
+    m = meta.view(np.float32)
+    want = oracle.expert_project(Q4_K, packed, experts, rows, cols, oracle.expert_assign(x, m), m, accumulate="f64")
+    assert_matmul_parity(y.to_f32(), want, f"routed rows beside {tokens} tokens")
+    want = oracle.project(Q4_K, packed_shared, rows, cols, x, accumulate="f64", weight_round=rounded, threads=8)
+    assert_matmul_parity(ys.to_f32(), want, f"shared rows of {tokens} tokens")
+
+    gate_up = oracle.round_storage(synth.activations(tokens, 2 * cols, seed=276), code).reshape(tokens, 2 * cols)
+    routed = gate_up[:assignments]
+    d.expert_project_with_shared(api.Tensor.from_f32(d, routed.shape, dt, routed), mt, w, ws, tokens, "silu_mul",
+                                 shared_input=api.Tensor.from_f32(d, gate_up.shape, dt, gate_up), out=y, shared_out=ys)
+    act = oracle.expert_silu_mul(gate_up, cols, code)
+    want = oracle.expert_project(Q4_K, packed, experts, rows, cols, act[:assignments], m, accumulate="f64")
+    assert_matmul_parity(y.to_f32(), want, f"activated routed rows beside {tokens} tokens")
+    want = oracle.project(Q4_K, packed_shared, rows, cols, act, accumulate="f64", weight_round=rounded, threads=8)
+    assert_matmul_parity(ys.to_f32(), want, f"activated shared rows of {tokens} tokens")
+
+
 @pytest.mark.parametrize("dtype", ["F16", "BF16"])
 @pytest.mark.parametrize("cols,crowd", [(256, 37), (512, 37), (512, 11), (768, 37), (1024, 11), (1024, 37)])
 @pytest.mark.parametrize("ggml", [Q4_K, Q6_K])
