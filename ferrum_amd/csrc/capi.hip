@@ -967,25 +967,27 @@ fh_status project(fh_device* device, const fh_qmatrix* weight, const fh_view* x,
         a.cu_count = device->props.multiProcessorCount;
         a.x_mode = silu_mul ? kXSiluMul : kXPlain;
         a.x_rows = m;
-        if (silu_mul && m == 1) {
-            // The kernels that take plain rows only are the faster ones for large matrices: the activated row
-            // is then written out first, as the separate expert_silu_mul would (5120 x 17408 Q6_K: 27 us in two
-            // launches against 39 where every workgroup activates the whole row again).
+        // One activated row stays on the FMA kernel: the streamed one's operands are f16 pairs and the matrix core
+        // keeps few bits of a subnormal weight (rel-L2 to 64 bits 1e-6 for Q6_K and 2e-6 to 1.4e-5 for Q4_K on
+        // rows of mean weights, against 1.0e-7 to 2.0e-7).  In it every workgroup activates the whole row again;
+        // for large matrices the row is written out first, as the separate expert_silu_mul would, with the same
+        // bits.  us, in place against written first: 5120 x 17408 26.5 / 20.6 (Q6_K 36.2 / 28.2), 5120 x 5120
+        // 10.8 / 10.0 (15.3 / 13.1), 2048 x 12800 12.3 / 11.8 (16.1 / 14.7); 4096 x 4096, where the second launch
+        // costs more, 8.3 / 9.4 (9.3 / 9.6).
+        if (silu_mul && m == 1 && (weight->ggml_type == kQ4K || weight->ggml_type == kQ6K) && n * (k / 256) >= 81920u) {
             GemvArgs plain = a;
             plain.x_mode = kXPlain;
-            StreamPlan stream;
-            if (gemv_takes_stream(plain, &stream)) {
-                const GemvScratch need = gemv_scratch(plain);
-                const size_t partial_bytes = align256((size_t)need.segments * n * sizeof(float));
-                const size_t bytes = partial_bytes + (size_t)k * dtype_bytes(x->dtype);
-                if (scratch_available(device, bytes)) {
-                    st = ensure_scratch(device, bytes);
-                    if (st != FH_OK) return st;
-                    uint8_t* const row = scratch_data(device) + partial_bytes;   // behind the partial sums
-                    launch_expert_silu_mul(device->stream, xr.begin, row, 1, (uint32_t)k, x->dtype, x->dtype);
-                    plain.x = row;
-                    a = plain;
-                }
+            plain.stream = 0;
+            const GemvScratch need = gemv_scratch(plain);
+            const size_t partial_bytes = align256((size_t)need.segments * n * sizeof(float));
+            const size_t bytes = partial_bytes + (size_t)k * dtype_bytes(x->dtype);
+            if (scratch_available(device, bytes)) {
+                st = ensure_scratch(device, bytes);
+                if (st != FH_OK) return st;
+                uint8_t* const row = scratch_data(device) + partial_bytes;   // behind the partial sums
+                launch_expert_silu_mul(device->stream, xr.begin, row, 1, (uint32_t)k, x->dtype, x->dtype);
+                plain.x = row;
+                a = plain;
             }
         }
         const char* name = "";

@@ -905,17 +905,28 @@ def test_argmax_of_rows_cut_into_pieces(api, d, width):
         assert np.array_equal(got.raw().view(np.uint32).reshape(8, 2), oracle.argmax_rows(x))
 
 
-@pytest.mark.parametrize("ggml,n,k,dtype", [(Q6_K, 700, 17408, "F32"), (Q6_K, 700, 17408, "BF16"), (Q4_K, 4200, 1024, "F16"),
-                                            (Q4_K, 1100, 17408, "F32"), (Q4_K, 300, 512, "F16")])
+@pytest.mark.parametrize("ggml,n,k,dtype", [
+    (Q6_K, 700, 17408, "F32"), (Q6_K, 700, 17408, "BF16"), (Q4_K, 4200, 1024, "F16"), (Q4_K, 1100, 17408, "F32"),
+    (Q4_K, 300, 512, "F16"), (Q6_K, 1300, 17408, "F32"), (Q4_K, 1300, 17408, "BF16"), (Q4_K, 20500, 1024, "F16"),
+    (Q4_K, 20480, 1024, "F32"), (Q4_K, 20479, 1024, "F32")])
 def test_one_activated_row_has_the_bits_of_the_separate_calls(api, d, ggml, n, k, dtype):
-    # large matrices: the activated row is written out for the streamed kernel; small ones activate it in place
-    w = qm(api, d, ggml, n, k, synth.matrix(ggml, n, k, seed=138))
+    # Large matrices (81920 super-blocks) have the activated row written out first, small ones activate it in place;
+    # both multiply on the FMA kernel.  A lane of it chains up to 3 x 64 products: roundings of at most 2^-24, uniform,
+    # make 2^-24 / sqrt(3) * sqrt(192 / 2) = 3.4e-7 in the mean square, the tree over the lanes and segments some
+    # 1e-7 more.
+    packed_w = synth.matrix(ggml, n, k, seed=138)
+    w = qm(api, d, ggml, n, k, packed_w)
     dt = getattr(api.DType, dtype)
     packed = api.Tensor.from_f32(d, (1, 2 * k), dt, synth.activations(1, 2 * k, seed=139))
     fused = d.project_quantized(packed, w, silu_mul=True)
-    separate = d.project_quantized(d.expert_silu_mul(packed, k), w)
+    activated = d.expert_silu_mul(packed, k)
+    with fma_gemv(d):
+        separate = d.project_quantized(activated, w)
     assert np.array_equal(fused.tensor.raw(), separate.tensor.raw())
     assert np.abs(fused.tensor.to_f32()).max() > 1e-3
+    exact = d.project_quantized(packed, w, out_dtype=api.DType.F32, silu_mul=True).tensor.to_f32()
+    weights = oracle.dequantize(ggml, packed_w, n, k).reshape(n, k).astype(np.float64)
+    assert rel_l2(exact, activated.to_f32().astype(np.float64) @ weights.T) <= 4e-7
 
 
 def test_lm_head_projection_then_argmax_picks_the_oracle_token(api, d):
