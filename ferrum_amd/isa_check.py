@@ -139,10 +139,10 @@ def counted_violations(asm: str, source: str = "") -> list[str]:
         runs, current = [], None    # (line of the run's last LDS-direct load, loads behind it)
         for number, text, in_asm in body:
             if text.startswith("global_load_lds_"):
-                current = [number, 0]
-                if runs and runs[-1][1] == 0:
-                    runs[-1] = current
+                if current is not None and current[1] == 0:    # the run goes on
+                    current[0] = number
                 else:
+                    current = [number, 0]
                     runs.append(current)
             elif current is not None and in_asm and text.startswith("s_waitcnt vmcnt"):
                 current = None

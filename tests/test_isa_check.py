@@ -104,6 +104,14 @@ def test_the_compilers_loads_behind_a_counted_lds_load_are_counted():
     load = "\tglobal_load_dwordx4 v[12:15], v[6:7], off offset:16\n"
     moved = COUNTED.replace(load, "", 1).replace("_Z4rowsv:\n", "_Z4rowsv:\n" + load, 1)
     assert any("1 register loads follow" in v for v in isa_check.counted_violations(moved, "x.hip"))
+    # both of them, in a kernel whose second run of LDS-direct loads is in order: the wait has closed the first run
+    first = COUNTED[COUNTED.index("\tglobal_load_lds"):COUNTED.index("\ts_endpgm")]
+    loads = "".join(line + "\n" for line in first.splitlines() if "global_load_dwordx4" in line)
+    two_runs = COUNTED.replace(first, first + first, 1)
+    assert isa_check.counted_violations(two_runs) == []
+    ahead = COUNTED.replace(first, loads + first.replace(loads, "", 1) + first, 1)
+    found = isa_check.counted_violations(ahead, "x.hip")
+    assert len(found) == 1 and "0 register loads follow" in found[0], found
     unwaited = COUNTED.replace("s_waitcnt vmcnt(2)", "s_nop 0", 1)
     assert any("without a hand-placed wait" in v for v in isa_check.counted_violations(unwaited, "x.hip"))
 
