@@ -3,6 +3,7 @@
 // methods (src/ops/transformer.rs:96-297, src/ops/mod.rs:23-609) and its
 // binding checks (src/metal/mod.rs:840-897): shapes, ownership, bounds,
 // alignment and input/output aliasing are rejected before anything launches.
+#include <algorithm>
 #include <cmath>
 #include <cstdarg>
 #include <mutex>
@@ -119,7 +120,7 @@ fh_status ensure_scratch(fh_device* d, size_t data_bytes) {
     }
     d->scratch = nullptr;
     d->scratch_bytes = 0;
-    size_t cap = counter_bytes + (data_bytes < (16u << 20) ? (16u << 20) : data_bytes);
+    size_t cap = counter_bytes + std::max(data_bytes, fh_device::kScratchFloor);
     hipError_t e = allocate(d, &d->scratch, cap);
     if (e != hipSuccess) return fail(FH_ERR_ALLOCATION, "hipMalloc(%zu): %s", cap, hipGetErrorString(e));
     d->scratch_bytes = cap;
@@ -585,6 +586,10 @@ fh_status fh_set_tuning(fh_device* device, const char* key, int64_t value) {
 fh_status fh_get_tuning(const fh_device* device, const char* key, int64_t* value) {
     if (device == nullptr || key == nullptr || value == nullptr)
         return fail(FH_ERR_PARAMETER, "null argument");
+    if (std::strcmp(key, "held_scratch_bytes") == 0) {
+        *value = (int64_t)device->scratch_bytes;
+        return FH_OK;
+    }
     const int64_t* const setting = tuning_of(device, key);
     if (setting == nullptr) return fail(FH_ERR_PARAMETER, "unknown tuning key %s", key);
     *value = *setting;
@@ -860,11 +865,16 @@ GemmArgs gemm_args(const fh_device* device, uint32_t ggml_type, uint64_t n, uint
     return g;
 }
 
-// Brings the scratch to what the product needs behind `used` bytes of the caller's at its head.
+// Brings the scratch to what the product needs behind `used` bytes of the caller's at its head.  Partial sums
+// only save time: where there is no room for them the few-rows plan is dropped.
 fh_status prepare_gemm(fh_device* device, GemmArgs& g, size_t used) {
     const size_t at = align256(used);
     if (!scratch_available(device, at + g.rows_plan.partial_bytes)) g.rows_plan = RowsPlan{};
     fh_status st = ensure_scratch(device, g.rows_plan.partial_bytes != 0 ? at + g.rows_plan.partial_bytes : used);
+    if (st == FH_ERR_ALLOCATION && g.rows_plan.partial_bytes != 0) {
+        g.rows_plan = RowsPlan{};
+        st = ensure_scratch(device, used);
+    }
     if (st != FH_OK) return st;
     g.counters = scratch_counters(device);
     g.partials = reinterpret_cast<float*>(scratch_data(device) + at);
@@ -931,16 +941,17 @@ fh_status project(fh_device* device, const fh_qmatrix* weight, const fh_view* x,
     if (tile || f32_batch) g = gemm_args(device, weight->ggml_type, n, k, m, f32_tile ? FH_F16 : x->dtype, y->dtype);
     if (f32_batch && g.few_rows) {
         g.rows_plan = gemm_rows_plan(g.ggml_type, g.n, g.k, g.m, g.x_dtype, g.cu_count);
-        if (g.rows_plan.counters > fh_device::kCounterWords || !scratch_available(device, g.rows_plan.partial_bytes))
-            g.rows_plan = RowsPlan{};
+        if (g.rows_plan.counters > fh_device::kCounterWords) g.rows_plan = RowsPlan{};
+    }
+    if (tile) gemm_takes_rows(g);
+    if (tile || g.rows_plan.rows != 0) {
+        st = prepare_gemm(device, g, f32_tile ? (size_t)m * k * sizeof(uint16_t) : 0);
+        if (st != FH_OK) return st;
     }
     if (tile || g.rows_plan.rows != 0) {
         g.w = weight->ptr;
         g.x = xr.begin;
         g.y = const_cast<uint8_t*>(yr.begin);
-        if (tile) gemm_takes_rows(g);
-        st = prepare_gemm(device, g, f32_tile ? (size_t)m * k * sizeof(uint16_t) : 0);
-        if (st != FH_OK) return st;
         if (f32_tile) {
             launch_round_to_f16(device->stream, reinterpret_cast<const float*>(xr.begin),
                                 reinterpret_cast<uint16_t*>(scratch_data(device)), (size_t)m * k);

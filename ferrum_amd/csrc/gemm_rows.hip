@@ -1,4 +1,6 @@
 // Plan and launch of the few-rows projection (gemm_rows.hpp).
+#include <algorithm>
+
 #include "gemm_rows.hpp"
 
 namespace fh {
@@ -20,13 +22,14 @@ double unit_us(uint32_t ggml_type, uint32_t x_dtype, uint32_t rows) {
 constexpr double kStartUs = 4.0;      // launch, first loads, exchange of the waves' sums
 constexpr double kExchangeUs = 4.0;   // partial sums of K segments through device memory
 
+constexpr uint32_t kMostWorkgroups = 1u << 22;   // of a launch, and half of what a grid of 512 threads each may have
+
 }  // namespace
 
 RowsPlan gemm_rows_plan(uint32_t ggml_type, uint32_t n, uint32_t k, uint32_t m, uint32_t x_dtype, int cu_count) {
     RowsPlan plan{};
     const uint32_t nb = k / 256, tiles = (n + 15) / 16, cus = cu_count > 0 ? (uint32_t)cu_count : 256u;
     plan.rows = x_dtype != FH_F32 && m > 16 ? 32 : 16;
-    plan.groups = (m + plan.rows - 1) / plan.rows;
     plan.k_waves = nb >= 8 ? 8 : nb >= 4 ? 4 : nb >= 2 ? 2 : 1;
     const uint32_t tile_waves = 8 / plan.k_waves;
     const double unit = unit_us(ggml_type, x_dtype, 16);
@@ -55,13 +58,24 @@ RowsPlan gemm_rows_plan(uint32_t ggml_type, uint32_t n, uint32_t k, uint32_t m, 
         }
     }
     const uint32_t per_wave = (plan.seg_blocks + plan.k_waves - 1) / plan.k_waves;
+    // A batch whose partial sums exceed the scratch a device has at all times, or whose tiles the counters or
+    // the grid, runs in several launches: no batch makes the scratch grow (8192 rows of 5120 x 17408 would ask for
+    // 480 MiB), and one launch's rows, 272 there, are sixteen rounds of the chip.
+    uint64_t most = kMostWorkgroups / ((plan.tile_groups + 7) / 8 * 8);   // row groups
+    if (plan.segments > 1) {
+        most = std::min<uint64_t>(most, fh_device::kScratchFloor / ((uint64_t)plan.segments * n * sizeof(float) * plan.rows));
+        most = std::min<uint64_t>(most, fh_device::kCounterWords / plan.tile_groups);
+    }
+    plan.run_rows = (uint32_t)std::min<uint64_t>(m, std::max<uint64_t>(most, 1) * plan.rows);
     // (from two rounds on a compute unit's next workgroup starts as soon as one ends: rounds need not be whole)
-    const double rounds = (double)((uint64_t)plan.tile_groups * plan.segments * plan.groups) / (double)cus;
+    const uint64_t groups = ((uint64_t)m + plan.rows - 1) / plan.rows;
+    const double rounds = (double)(plan.tile_groups * plan.segments * groups) / (double)cus;
     plan.estimate_us = (rounds <= 1.0 ? 1.0 : rounds <= 2.0 ? 2.0 : rounds + 0.2) *
                            (kStartUs + per_wave * plan.tiles * unit_us(ggml_type, x_dtype, plan.rows)) +
                        (plan.segments > 1 ? kExchangeUs : 0.0);
+    plan.groups = (plan.run_rows + plan.rows - 1) / plan.rows;
     plan.counters = plan.segments > 1 ? (size_t)plan.tile_groups * plan.groups : 0;
-    plan.partial_bytes = plan.segments > 1 ? (size_t)plan.segments * m * n * sizeof(float) : 0;
+    plan.partial_bytes = plan.segments > 1 ? (size_t)plan.segments * plan.run_rows * n * sizeof(float) : 0;
     return plan;
 }
 
@@ -69,25 +83,28 @@ void launch_gemm_rows(hipStream_t s, const GemmArgs& a) {
     const RowsPlan& plan = a.rows_plan;
     RowsParams p{};
     p.w = static_cast<const uint8_t*>(a.w);
-    p.x = static_cast<const uint8_t*>(a.x);
-    p.y = a.y;
-    p.m = a.m;
     p.n = a.n;
     p.nb = a.k / 256;
     p.y_dtype = a.y_dtype;
     p.k_waves = plan.k_waves;
-    p.groups = plan.groups;
     p.tile_groups = plan.tile_groups;
     p.segments = plan.segments;
     p.seg_blocks = plan.seg_blocks;
     p.partials = a.partials;
     p.counters = a.counters;
-    switch (a.ggml_type) {
-        case kQ4K: return launch_rows_q4_k(s, a.x_dtype, plan, p);
-        case kQ5K: return launch_rows_q5_k(s, a.x_dtype, plan, p);
-        case kQ6K: return launch_rows_q6_k(s, a.x_dtype, plan, p);
-        case kIQ4XS: return launch_rows_iq4_xs(s, a.x_dtype, plan, p);
-        default: return launch_rows_q8_0(s, a.x_dtype, plan, p);
+    const size_t x_row = (size_t)a.k * dtype_bytes(a.x_dtype), y_row = (size_t)a.n * dtype_bytes(a.y_dtype);
+    for (uint32_t first = 0; first < a.m; first += plan.run_rows) {
+        p.x = static_cast<const uint8_t*>(a.x) + first * x_row;
+        p.y = static_cast<uint8_t*>(a.y) + first * y_row;
+        p.m = std::min(plan.run_rows, a.m - first);
+        p.groups = (p.m + plan.rows - 1) / plan.rows;
+        switch (a.ggml_type) {
+            case kQ4K: launch_rows_q4_k(s, a.x_dtype, plan, p); break;
+            case kQ5K: launch_rows_q5_k(s, a.x_dtype, plan, p); break;
+            case kQ6K: launch_rows_q6_k(s, a.x_dtype, plan, p); break;
+            case kIQ4XS: launch_rows_iq4_xs(s, a.x_dtype, plan, p); break;
+            default: launch_rows_q8_0(s, a.x_dtype, plan, p); break;
+        }
     }
 }
 

@@ -62,6 +62,7 @@ struct fh_device {
     // this device's copy of the library's fixed scratch array (fh_project_quantized_no_alloc)
     void* fixed_scratch = nullptr;
     static constexpr size_t kCounterWords = 1u << 16;
+    static constexpr size_t kScratchFloor = 16u << 20;   // the data area is never smaller
     // Releases asked for while an execution is being recorded wait for its end:
     // freeing or synchronizing inside a stream capture would invalidate it.
     // scratch blocks that were outgrown while recorded executions (which carry their address)
@@ -281,12 +282,13 @@ GemvScratch gemv_scratch(const GemvArgs& a);
 // gemm_rows.hip: a few rows, f16 / bf16 on weights rounded to their type or f32 on exact f32 weights
 struct RowsPlan {
     uint32_t rows;            // rows a workgroup multiplies: 16 or 32
-    uint32_t groups;          // groups of that many rows
+    uint32_t run_rows;        // rows of one launch; a larger batch is several, one after the other
+    uint32_t groups;          // groups of `rows` rows of such a launch
     uint32_t k_waves;         // waves that share a tile's super-blocks
     uint32_t tiles;           // weight tiles of 16 rows per wave
     uint32_t tile_groups, segments, seg_blocks;
-    size_t counters;          // scratch counter words (0: K is not cut)
-    size_t partial_bytes;     // scratch for partial sums
+    size_t counters;          // scratch counter words of a launch (0: K is not cut)
+    size_t partial_bytes;     // scratch for its partial sums
     double estimate_us;
 };
 RowsPlan gemm_rows_plan(uint32_t ggml_type, uint32_t n, uint32_t k, uint32_t m, uint32_t x_dtype, int cu_count);

@@ -123,7 +123,9 @@ void* fh_device_stream(fh_device* device);
 /* Kernel-selection switches: the legacy::Tuning setters
  * (src/metal/legacy.rs:8-111), e.g. "k_quant_gemv_ksplit" with the same value
  * rule as set_k_quant_gemv_ksplit (0 or a power of two up to 8).  Unknown
- * keys or out-of-range values give FH_ERR_PARAMETER. */
+ * keys or out-of-range values give FH_ERR_PARAMETER.
+ * fh_get_tuning alone also answers for what the library does by itself:
+ *   held_scratch_bytes  the operators' common scratch */
 fh_status fh_set_tuning(fh_device* device, const char* key, int64_t value);
 fh_status fh_get_tuning(const fh_device* device, const char* key, int64_t* value);
 

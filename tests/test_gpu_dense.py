@@ -1110,6 +1110,26 @@ def test_a_batch_whose_partial_sums_outgrow_the_scratch_can_be_recorded_first(ap
         assert rel_l2(recorded.to_f32(), direct) <= 1e-5
 
 
+@pytest.mark.parametrize("ggml,m,n,k", [(Q4_K, 1000, 5120, 17408), (Q6_K, 1800, 1030, 17408)])
+def test_an_f32_batch_of_any_size_leaves_the_scratch_as_it_is(api, ggml, m, n, k):
+    """Rows this long are cut into three K segments, whose partial sums for all of the batch would be 58 and 21 MiB;
+    the batch runs in launches whose sums fit the 16 MiB a device always has, so it needs no memory of its own.
+    A row's bits do not depend on the launch it is in."""
+    dev = api.Device.new()
+    packed = synth.matrix(ggml, n, k, seed=731)
+    w = qm(api, dev, ggml, n, k, packed)
+    x = np.resize(synth.activations(97, k, seed=732), (m, k)).astype(np.float32)    # 97: no row at the same place in two launches
+    held = dev.get_tuning("held_scratch_bytes")
+    got = dev.project_quantized(api.Tensor.from_f32(dev, (m, k), api.DType.F32, x), w).tensor.to_f32()
+    assert dev.get_tuning("held_scratch_bytes") == held
+    assert np.array_equal(bits(got), bits(np.resize(got[:97], (m, n))))
+    rows = np.unique(np.concatenate([np.arange(0, 40), np.arange(n - 40, n)]))
+    want = oracle_columns(ggml, packed, n, k, rows, x[:97], accumulate="f64")
+    assert_matmul_parity(got[:97][:, rows], want, "f32 batch in several launches")
+    part = dev.project_quantized(api.Tensor.from_f32(dev, (7, k), api.DType.F32, x[m - 7:]), w).tensor.to_f32()
+    assert np.array_equal(bits(part), bits(got[m - 7:]))
+
+
 @pytest.mark.parametrize("ggml,m,n,k", [(Q4_K, 5, 200, 256), (Q4_K, 16, 1024, 1024), (Q6_K, 24, 530, 2048), (Q5_K, 64, 777, 5120)])
 def test_a_batch_of_f32_rows_is_as_close_to_64_bits_as_its_chains_are_short(api, d, ggml, m, n, k):
     """Sixteen products follow each other in one accumulator, the rest is added in pairs and over eight waves.
