@@ -555,9 +555,9 @@ fh_status fh_set_tuning(fh_device* device, const char* key, int64_t value) {
         ok = value >= 2;
     } else if (k == "gemm_resident" || k == "moe_fold_combine" || k == "moe_fold_route") {
         ok = value == 0 || value == 1;
-    } else if (k == "gemm_few_tiles_split" || k == "gemv_stream_own_loads" || k == "expert_weight_ring") {
+    } else if (k == "gemv_stream_own_loads" || k == "expert_weight_ring") {
         ok = value == 0 || value == 1;
-    } else if (k == "gemv_stream") {
+    } else if (k == "gemv_stream" || k == "gemm_few_tiles_split") {
         ok = value >= 0 && value <= 2;
     } else if (k == "gemm_wide_shape") {
         ok = value >= 0 && value <= 2;
@@ -588,6 +588,10 @@ fh_status fh_get_tuning(const fh_device* device, const char* key, int64_t* value
         return fail(FH_ERR_PARAMETER, "null argument");
     if (std::strcmp(key, "held_scratch_bytes") == 0) {
         *value = (int64_t)device->scratch_bytes;
+        return FH_OK;
+    }
+    if (std::strcmp(key, "last_rows_plan") == 0) {
+        *value = device->last_rows_plan;
         return FH_OK;
     }
     const int64_t* const setting = tuning_of(device, key);
@@ -862,6 +866,7 @@ GemmArgs gemm_args(const fh_device* device, uint32_t ggml_type, uint64_t n, uint
     g.resident_switch = device->tuning.gemm_resident != 0;
     g.rows_resident = g.resident_switch && expert_rows_fit_lds((uint32_t)k, 1, 1);
     g.few_rows = device->tuning.gemm_few_tiles_split != 0;
+    g.few_rows_always = device->tuning.gemm_few_tiles_split == 2;
     return g;
 }
 
@@ -881,6 +886,12 @@ fh_status prepare_gemm(fh_device* device, GemmArgs& g, size_t used) {
     return FH_OK;
 }
 
+const char* run_gemm(fh_device* device, const GemmArgs& g) {
+    const RowsPlan& plan = g.rows_plan;
+    device->last_rows_plan = plan.rows * 1000 + plan.tiles * 100 + plan.segments;
+    return launch_gemm(device->stream, g);
+}
+
 // the exact product of several rows, by whichever kernel
 const char* batch_name(uint32_t ggml_type) {
     return ggml_type == kQ4K    ? "q4_k_gemm"
@@ -888,6 +899,21 @@ const char* batch_name(uint32_t ggml_type) {
            : ggml_type == kQ6K  ? "q6_k_gemm"
            : ggml_type == kQ8_0 ? "q8_0_gemm"
                                 : "iq4_xs_gemm";
+}
+
+// whether a dense GEMV of m plain rows runs on the streamed kernel
+bool gemv_streams(const fh_device* device, uint32_t ggml_type, uint64_t n, uint64_t k, uint32_t m) {
+    GemvArgs a{};
+    a.ggml_type = ggml_type;
+    a.n = (uint32_t)n;
+    a.k = (uint32_t)k;
+    a.m = m;
+    a.cu_count = device->props.multiProcessorCount;
+    a.stream = (int)device->tuning.gemv_stream;
+    a.ksplit = (int)device->tuning.k_quant_gemv_ksplit;
+    a.x_mode = kXPlain;
+    StreamPlan plan;
+    return gemv_takes_stream(a, &plan);
 }
 
 // `f32_tile_from`: row count from which f32 activations take the f16 tiles; negative = the
@@ -931,17 +957,23 @@ fh_status project(fh_device* device, const fh_qmatrix* weight, const fh_view* x,
                           ((uintptr_t)xr.begin & 15u) == 0;
     const bool tile = f32_tile || (!silu_mul && m >= (uint32_t)device->tuning.gemm_min_rows && x->dtype != FH_F32);
     // A batch of exact f32 rows: the GEMV kernels read every weight once per row, the few-rows kernel
-    // once per sixteen.  Four rows of 17408 x 5120 take it 36 us, the GEMV 36 for Q4_K (20 and 27 for two
-    // and three) and 43 - 58 for the other formats; sixteen rows 38 against 121 - 230.  Where a GEMV
+    // once per sixteen.  Against the FMA GEMV f32_rows_pay decides.  Where the streamed GEMV would run, the few-rows
+    // kernel takes over from five Q4_K rows and four Q6_K rows on: it is the faster one from six (5 / 6 / 16 x 17408
+    // x 5120 Q4_K 47.8 / 47.0 / 46.0 against 43.8 / 51.7 / 121 us, 5 / 6 x 4096 x 4096 11.8 / 11.7 against 11.1 / 12.4)
+    // and at five the closer one to 64 bits (1e-7; the streamed kernel's operands are f16 pairs).  Where a GEMV
     // kernel or its K segments are asked for by name, those run.
     const bool f32_batch = !tile && !silu_mul && x->dtype == FH_F32 && m >= (weight->ggml_type == kQ4K ? 5u : 4u) &&
                            m >= (uint32_t)device->tuning.gemm_min_rows && device->tuning.gemv_stream == 1 &&
                            device->tuning.k_quant_gemv_ksplit == 0;
+    device->last_rows_plan = 0;
     GemmArgs g{};
     if (tile || f32_batch) g = gemm_args(device, weight->ggml_type, n, k, m, f32_tile ? FH_F16 : x->dtype, y->dtype);
     if (f32_batch && g.few_rows) {
         g.rows_plan = gemm_rows_plan(g.ggml_type, g.n, g.k, g.m, g.x_dtype, g.cu_count);
-        if (g.rows_plan.counters > fh_device::kCounterWords) g.rows_plan = RowsPlan{};
+        if (g.rows_plan.counters > fh_device::kCounterWords ||
+            (!g.few_rows_always && !gemv_streams(device, weight->ggml_type, n, k, m) &&
+             !f32_rows_pay(g.rows_plan, g.ggml_type, g.n, g.k, m, g.cu_count)))
+            g.rows_plan = RowsPlan{};
     }
     if (tile) gemm_takes_rows(g);
     if (tile || g.rows_plan.rows != 0) {
@@ -957,7 +989,7 @@ fh_status project(fh_device* device, const fh_qmatrix* weight, const fh_view* x,
                                 reinterpret_cast<uint16_t*>(scratch_data(device)), (size_t)m * k);
             g.x = scratch_data(device);
         }
-        const char* const name = launch_gemm(device->stream, g);
+        const char* const name = run_gemm(device, g);
         device->last_operation = tile ? name : batch_name(weight->ggml_type);
     } else {
         GemvArgs a{};
@@ -1814,7 +1846,7 @@ fh_status expert_project(fh_device* device, const fh_qmatrix* weight, const fh_v
         g.w = shared->weight->ptr;
         g.x = scratch_data(device);
         g.y = const_cast<uint8_t*>(syr.begin);
-        device->last_operation = launch_gemm(device->stream, g);
+        device->last_operation = run_gemm(device, g);
         FH_HIP(hipGetLastError());
         return FH_OK;
     }

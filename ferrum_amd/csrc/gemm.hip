@@ -1301,12 +1301,12 @@ bool gemm_takes_rows(GemmArgs& a) {
     if (a.wide32_tile != 0 && a.wide_shape != 0 && a.m >= (uint32_t)a.wide_min_rows) return false;   // a tile is asked for
     const RowsPlan plan = gemm_rows_plan(a.ggml_type, a.n, a.k, a.m, a.x_dtype, a.cu_count);
     if (plan.counters > fh_device::kCounterWords) return false;
-    if (a.resident_switch) {
+    if (!a.few_rows_always && a.resident_switch) {
         const TileChoice c = tile_choice(a);
         double other = std::min(c.us32, c.us16);
         if (a.rows_resident) other = std::min(other, resident_estimate(a.ggml_type, a.m, a.n, a.k));
         if (plan.estimate_us >= other) return false;
-    } else if (a.m > (uint32_t)a.skinny_max_rows) {
+    } else if (!a.few_rows_always && a.m > (uint32_t)a.skinny_max_rows) {
         return false;
     }
     a.rows_plan = plan;

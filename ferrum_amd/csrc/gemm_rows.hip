@@ -79,6 +79,29 @@ RowsPlan gemm_rows_plan(uint32_t ggml_type, uint32_t n, uint32_t k, uint32_t m, 
     return plan;
 }
 
+// A batch of exact f32 rows.  The GEMV reads every weight once per row, but with few rows and small matrices its
+// workgroups fill a chip that one launch of this kernel leaves idle.  Q4_K and Q5_K take the faster of the two by
+// estimate, fitted to 4 - 48 rows of fifteen shapes from 256 x 256 to 151936 x 2048 and within 5% of the faster one
+// in all but three of 196 measurements, the worst 14% (four Q5_K rows of 151936 x 2048; us, GEMV against this kernel: 16 x 256 x 256 Q5_K 3.7 / 6.8,
+// 8 x 1024 x 4096 7.4 / 11.6 and 16 rows 10.6 / 11.7, 4 / 8 / 16 x 5120 x 5120 17.8 / 29.7 / 54.0 against 21.0).  Both
+// are 1.0e-7 (rel-L2) from 64 bits there.  For the other formats the GEMV is at 1.8e-7 to 2.2e-7 and this kernel at
+// 0.9e-7 to 1.2e-7, so they keep it also where the GEMV is faster (16 x 256 x 256 Q6_K 3.9 / 7.6, 8 x 1024 x 4096
+// 8.1 / 12.3, even from 16 rows there and from four at 4096 x 4096).
+bool f32_rows_pay(const RowsPlan& plan, uint32_t ggml_type, uint32_t n, uint32_t k, uint32_t m, int cu_count) {
+    if (ggml_type != kQ4K && ggml_type != kQ5K) return true;
+    if (m >= 6 && (uint64_t)n * (k / 256) >= 65536u) return true;   // (from 4096 x 4096 on without exception)
+    // us per super-block: of a weight tile and wave here, per million of the matrix and per row there (rows of more
+    // than 24 are cut into K segments, which meet in memory)
+    const double unit = ggml_type == kQ4K ? 2.6 : 3.0;
+    const double gemv_unit = (ggml_type == kQ4K ? 21.0 : 35.0) * (k > 24 * 256 ? 1.4 : 1.0);
+    const uint32_t per_wave = (plan.seg_blocks + plan.k_waves - 1) / plan.k_waves;
+    const uint64_t groups = ((uint64_t)m + plan.rows - 1) / plan.rows;
+    const double rounds = (double)(plan.tile_groups * plan.segments * groups) / (double)(cu_count > 0 ? cu_count : 256);
+    const double here = (rounds <= 1.0 ? 1.0 : rounds <= 2.0 ? 2.0 : rounds + 0.2) * (3.7 + per_wave * (0.9 + plan.tiles * unit));
+    const double blocks = (double)m * (double)n * (double)(k / 256) * 1e-6;
+    return here < 4.0 + std::max(0.0, blocks - 0.08) * gemv_unit;   // (80000 super-blocks run side by side)
+}
+
 void launch_gemm_rows(hipStream_t s, const GemmArgs& a) {
     const RowsPlan& plan = a.rows_plan;
     RowsParams p{};

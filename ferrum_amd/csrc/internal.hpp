@@ -26,7 +26,7 @@ struct fh_tuning {
     int64_t gemm_skinny_max_rows = 64; // with gemm_resident 0: largest M that takes the few-rows kernel (0 = never)
     int64_t expert_grouped_min_assignments = 32;  // fewest assignments grouped by expert (0 = never)
     int64_t moe_fold_route = 1;        // fh_moe_ffn, one token: the gate|up launch routes the token itself (0 = a moe_route launch first)
-    int64_t gemm_few_tiles_split = 1;  // few rows: a tile's super-blocks dealt over the waves, any K (0 = whole tiles per wave, the kernels for rows that fit LDS or not)
+    int64_t gemm_few_tiles_split = 1;  // few rows: a tile's super-blocks dealt over the waves, any K: 0 never (whole tiles per wave, the kernels for rows that fit LDS or not), 1 where it wins, 2 wherever it runs
     int64_t moe_fold_combine = 1;      // fh_moe_ffn with few tokens: down projection and weighted sum in one launch (0 = two)
     int64_t gemm_resident = 1;         // rows that fit LDS whole take the rows-resident kernel (0 = square tiles)
     int64_t gemv_stream_own_loads = 1; // the streamed Q4_K GEMV's waves load the super-blocks they multiply (tiles of up to 14 rows); 0: the tile row by row
@@ -46,6 +46,7 @@ struct fh_device {
     hipStream_t stream = nullptr;
     hipDeviceProp_t props{};
     const char* last_operation = "";
+    int64_t last_rows_plan = 0;   // of the last dense product: 0, or the few-rows kernel's rows, tiles and K segments
     bool capturing = false;
     fh_tuning tuning;
     // Blocks of freed buffers, by size, for the buffers to come (fh_buffer_alloc): hipMalloc and hipFree
@@ -292,6 +293,8 @@ struct RowsPlan {
     double estimate_us;
 };
 RowsPlan gemm_rows_plan(uint32_t ggml_type, uint32_t n, uint32_t k, uint32_t m, uint32_t x_dtype, int cu_count);
+// whether that plan's kernel, and not the FMA GEMV once per row, takes m exact f32 rows
+bool f32_rows_pay(const RowsPlan& plan, uint32_t ggml_type, uint32_t n, uint32_t k, uint32_t m, int cu_count);
 
 // gemm.hip
 struct GemmArgs {
@@ -331,6 +334,7 @@ struct GemmArgs {
     bool use_resident;    // set by launch_gemm_resident only
     bool resident_switch; // rows_resident before the rows' length is looked at
     bool few_rows;        // the few-rows kernel may take the product (gemm_takes_rows)
+    bool few_rows_always; // ... and does, whatever the estimates say
     RowsPlan rows_plan;   // set by gemm_takes_rows; its K segments meet in these:
     float* partials;
     uint32_t* counters;

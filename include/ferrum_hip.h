@@ -125,7 +125,9 @@ void* fh_device_stream(fh_device* device);
  * rule as set_k_quant_gemv_ksplit (0 or a power of two up to 8).  Unknown
  * keys or out-of-range values give FH_ERR_PARAMETER.
  * fh_get_tuning alone also answers for what the library does by itself:
- *   held_scratch_bytes  the operators' common scratch */
+ *   held_scratch_bytes  the operators' common scratch
+ *   last_rows_plan      how the last dense product ran on the few-rows kernel: 1000 x activation
+ *                       rows (16 or 32) + 100 x weight tiles per wave + K segments; 0 on others */
 fh_status fh_set_tuning(fh_device* device, const char* key, int64_t value);
 fh_status fh_get_tuning(const fh_device* device, const char* key, int64_t* value);
 

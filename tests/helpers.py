@@ -44,6 +44,17 @@ def oracle_columns(ggml_type, packed, n, k, rows, x, **kw):
 
 
 @contextlib.contextmanager
+def few_rows(d, switch):
+    """Batches inside the block: 0 none, 1 those it wins, 2 all that can run on the few-rows kernel."""
+    before = d.get_tuning("gemm_few_tiles_split")
+    d.set_tuning("gemm_few_tiles_split", switch)
+    try:
+        yield
+    finally:
+        d.set_tuning("gemm_few_tiles_split", before)
+
+
+@contextlib.contextmanager
 def fma_gemv(d):
     """Dense Q4_K and Q6_K GEMVs inside the block take the FMA kernel, the one the fused and
     per-assignment launches run on, so results can be compared with them bit for bit (the

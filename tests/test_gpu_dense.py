@@ -12,7 +12,7 @@ import pytest
 
 import ferrum_fixtures as fx
 import oracle
-from helpers import assert_matmul_parity, bits, fma_gemv, oracle_columns, rel_l2
+from helpers import assert_matmul_parity, bits, few_rows, fma_gemv, oracle_columns, rel_l2
 from ferrum_amd import synth
 
 pytestmark = pytest.mark.gpu
@@ -745,18 +745,41 @@ def test_few_rows_on_the_edges_of_the_kernel(api, d, ggml, m, n, k, dtype):
     code = {"F32": oracle.F32, "F16": oracle.F16, "BF16": oracle.BF16}[dtype]
     x = oracle.round_storage(synth.activations(m, k, seed=252 + m), code).reshape(m, k)
     xt = api.Tensor.from_f32(d, (m, k), getattr(api.DType, dtype), x)
-    out = d.project_quantized(xt, w, out_dtype=api.DType.F32)
-    assert out.operation.endswith("_gemm" if dtype == "F32" else "_skinny" if k > 5120 and m <= 64 else "_resident")
-    got = out.tensor.to_f32()
-    want = oracle.project(ggml, packed, n, k, x, accumulate="f64", weight_round=code, threads=8)
-    assert_matmul_parity(got, want, f"few rows {m}x{n}x{k} {dtype}")
-    again = d.project_quantized(xt, w, out_dtype=api.DType.F32).tensor.to_f32()
-    assert np.array_equal(bits(again), bits(got))
-    if dtype == "F32" and m > 5:    # a row's sums do not depend on the rows beside it
-        part = d.project_quantized(api.Tensor.from_f32(d, (m - 1, k), api.DType.F32, x[:-1]), w).tensor.to_f32()
-        assert np.array_equal(bits(part), bits(got[:-1]))
-    stored = d.project_quantized(xt, w).tensor.to_f32()      # 16-bit results: the packed stores
-    assert np.array_equal(bits(stored), bits(oracle.round_storage(got, code).reshape(m, n)))
+    with few_rows(d, 2):
+        out = d.project_quantized(xt, w, out_dtype=api.DType.F32)
+        assert out.operation.endswith("_gemm" if dtype == "F32" else "_skinny" if k > 5120 and m <= 64 else "_resident")
+        assert d.get_tuning("last_rows_plan") // 1000 == (32 if dtype != "F32" and m > 16 else 16)
+        got = out.tensor.to_f32()
+        want = oracle.project(ggml, packed, n, k, x, accumulate="f64", weight_round=code, threads=8)
+        assert_matmul_parity(got, want, f"few rows {m}x{n}x{k} {dtype}")
+        again = d.project_quantized(xt, w, out_dtype=api.DType.F32).tensor.to_f32()
+        assert np.array_equal(bits(again), bits(got))
+        if dtype == "F32" and m > 5:    # a row's sums do not depend on the rows beside it
+            part = d.project_quantized(api.Tensor.from_f32(d, (m - 1, k), api.DType.F32, x[:-1]), w).tensor.to_f32()
+            assert np.array_equal(bits(part), bits(got[:-1]))
+        stored = d.project_quantized(xt, w).tensor.to_f32()      # 16-bit results: the packed stores
+        assert np.array_equal(bits(stored), bits(oracle.round_storage(got, code).reshape(m, n)))
+
+
+@pytest.mark.parametrize("ggml", [12, 13, 14, 23, 8], ids=["q4_k", "q5_k", "q6_k", "iq4_xs", "q8_0"])
+@pytest.mark.parametrize("m,n,k", [(16, 256, 256), (48, 100, 512), (8, 1024, 1024), (6, 4096, 4096), (40, 4100, 1024)])
+def test_small_f32_batches_stay_on_the_gemv(api, d, ggml, m, n, k):
+    """Q4_K and Q5_K batches take the few-rows kernel where it is the faster one, the other formats, whose GEMV is
+    farther from 64 bits, always; both multiply exact weights by exact rows.  The GEMV's chains are up to 64 products
+    (2.0e-7 in the mean square, 2^-24 / sqrt(3) * sqrt(64 / 2)), the other kernel's 16 and 24 adds (1.6e-7)."""
+    w = qm(api, d, ggml, n, k, synth.matrix(ggml, n, k, seed=261))
+    x = api.Tensor.from_f32(d, (m, k), api.DType.F32, synth.activations(m, k, seed=262))
+    got = d.project_quantized(x, w).tensor.to_f32()
+    small = m * n * (k // 256) < 80000 and ggml in (12, 13)
+    assert (d.get_tuning("last_rows_plan") == 0) == small
+    with few_rows(d, 0), fma_gemv(d):
+        gemv = d.project_quantized(x, w).tensor.to_f32()
+        assert d.get_tuning("last_rows_plan") == 0
+    with few_rows(d, 2):
+        rows = d.project_quantized(x, w).tensor.to_f32()
+        assert d.get_tuning("last_rows_plan") != 0
+    assert np.array_equal(got, gemv if small else rows)
+    assert rel_l2(rows, gemv) <= 2.6e-7     # the two in the mean square
 
 
 @pytest.mark.parametrize("ggml,m,dtype", [(12, 130, "F16"), (12, 300, "BF16"), (14, 200, "F16"), (8, 130, "F16")],
