@@ -1721,17 +1721,27 @@ bool rider_fits(uint32_t n, uint32_t k, uint64_t entries) {
 }
 
 // Whether streaming every hit expert once for all of its rows beats streaming it once per row.  The
-// per-assignment launch reads an expert's matrix for each of its assignments at the chip's rate (5.6
-// MB/us: 2.85 us per token of the 256-expert top-8 FFN); the grouped one waits for the workgroup that
-// streams one share of one expert (18.6 KB/us) behind a grouping and a staging launch.  256 experts top-8
-// of 2048 x 512 plus a shared one, us, per assignment against grouped: 4 tokens 30 / 117, 16 64 / 118,
-// 24 87 / 120, 32 110 / 122; 128 experts of 2048 x 768, 16 tokens 88 / 130, 24 124 / 135, 32 164 / 140;
-// 32 experts top-4 of 1024 x 256, 32 tokens 23 / 37.  From five assignments per expert on they are grouped.
+// per-assignment launch reads an expert's matrix for each of its assignments at the rate of its decode (rows
+// whose super-blocks leave more than a third of the kernel's block slots idle, as five on eight do, a fifth
+// below it); the grouped one waits for the workgroup that streams one share of one expert, behind a grouping
+// and a staging launch (9 and 16.5 us before either streams).  One projection, f16, us, per assignment against grouped: 64 experts of 2048 x 1280, 64 /
+// 96 / 128 assignments Q4_K 28 / 36 / 44 against 32, IQ4_XS 37 / 50 / 62 against 38; 128 of 2048 x 768, 128 / 192 /
+// 256 Q4_K 25 / 32 / 40 against 35, IQ4_XS 35 / 47 / 60 against 44; 256 of 1024 x 2048, 256 / 384 Q6_K 81 / 124
+// against 117.  From five assignments per expert on they are grouped.
 bool grouping_pays(const fh_qmatrix& weight, uint32_t assignments, int cu_count) {
     if (assignments >= 5 * weight.experts) return true;
-    const double bytes = (double)weight.rows * (double)(weight.stored_cols / 256) * block_bytes(weight.ggml_type);
+    struct Rates { double each, share; };   // bytes per us: of the chip, and of a compute unit that multiplies groups
+    const Rates rates = weight.ggml_type == kQ4K    ? Rates{6.4e6, 21.0e3}
+                        : weight.ggml_type == kQ5K  ? Rates{5.9e6, 17.0e3}
+                        : weight.ggml_type == kQ6K  ? Rates{5.9e6, 16.5e3}
+                        : weight.ggml_type == kQ8_0 ? Rates{7.8e6, 25.0e3}
+                                                    : Rates{4.4e6, 14.5e3};
+    const uint32_t nb = (uint32_t)(weight.stored_cols / 256);
+    const GemvPlan plan = gemv_plan((uint32_t)weight.rows, nb * 256, 1, 0);
+    const bool idles = plan.segments * (uint32_t)(plan.bs * plan.it) * 2 >= nb * 3;
+    const double bytes = (double)weight.rows * nb * block_bytes(weight.ggml_type);
     const double shares = std::max(1.0, (double)cu_count / (double)weight.experts);
-    return assignments * bytes / 5.6e6 > 7.0 + bytes / (shares * 18.6e3);
+    return 9.0 + assignments * bytes / rates.each * (idles ? 1.2 : 1.0) > 16.5 + bytes / (shares * rates.share);
 }
 
 fh_status expert_project(fh_device* device, const fh_qmatrix* weight, const fh_view* x, uint32_t x_rows,

@@ -8,7 +8,7 @@ import pytest
 
 import ferrum_fixtures as fx
 import oracle
-from helpers import assert_matmul_parity, bits, fma_gemv, rel_l2
+from helpers import assert_matmul_parity, bits, fma_gemv, oracle_columns, rel_l2
 from ferrum_amd import synth
 
 pytestmark = pytest.mark.gpu
@@ -267,6 +267,28 @@ def test_few_assignments_per_expert_are_projected_one_by_one(api, d, assignments
     want = oracle.expert_project(Q4_K, packed, experts, rows, cols, x, meta.view(np.float32), accumulate="f64",
                                  weight_round=code if grouped else 0)
     assert_matmul_parity(got.to_f32(), want, f"{assignments} assignments of 64 experts, {dtype}")
+
+
+# Where the two launches take the same time depends on the format's decode and on the row length: 64 experts of
+# 2048 x 1280 (rows that leave block slots idle) are grouped at 96 assignments and not at 64, in every format.
+@pytest.mark.parametrize("ggml", [8, 12, 13, 14, 23], ids=["q8_0", "q4_k", "q5_k", "q6_k", "iq4_xs"])
+def test_the_grouping_line_follows_the_decode(api, d, ggml):
+    experts, rows, cols = 64, 2048, 1280
+    one = synth.matrix(ggml, rows, cols, seed=281)
+    w = api.QuantizedExpertMatrix.new(d, np.tile(one, experts), api.QuantizationFormat(ggml), experts, rows, cols)
+    for assignments, grouped in ((64, False), (96, True)):
+        meta = np.zeros((assignments, 3), dtype=np.uint32)
+        meta[:, 0] = synth.rng(282).integers(0, experts, assignments)
+        meta[:, 1] = np.arange(assignments)
+        meta[:, 2] = np.float32(1.0).view(np.uint32)
+        x = oracle.round_storage(synth.activations(assignments, cols, seed=283), oracle.F16).reshape(assignments, cols)
+        got = d.expert_project_quantized(api.Tensor.from_f32(d, x.shape, api.DType.F16, x),
+                                         api.Tensor.from_bits(d, meta.shape, meta), w, cols, experts, out_dtype=api.DType.F32)
+        assert d.last_operation().endswith("_grouped_mfma") == grouped
+        picked = np.unique(synth.rng(284).integers(0, rows, 40))
+        want = oracle_columns(ggml, one, rows, cols, picked, x, accumulate="f64",     # (every expert holds the same matrix)
+                              weight_round=oracle.F16 if grouped else 0)
+        assert_matmul_parity(got.to_f32()[:, picked], want, f"{assignments} assignments")
 
 
 # Rows of 6400 weights are cut into two K segments, so a per-assignment launch needs a counter word per row tile
