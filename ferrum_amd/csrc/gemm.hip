@@ -1182,16 +1182,22 @@ double wide16_estimate(uint32_t m, uint32_t n, uint32_t k, int cus) {
     return (rounds < 1.0 ? 1.0 : rounds) * 105.0 * wide_row_length_factor(k);
 }
 
-// The rows-resident kernel: a start, the stream of the matrix, and a decode of every weight per group
+// The rows-resident kernel: a start (the rows' gather, then the first weights), the stream of the matrix, and a decode of every weight per group
 // of rows that LDS holds at once (32 rows of up to 2560, 16 of up to 5120; us per million weights).
-// Measured at 4 - 64 rows on 20480 .. 151936 x 2048 / 5120; within a tenth of most of those.
+// Measured at 2 - 80 rows on 4096 x 1024 .. 151936 x 2048 and 5120 x 5120 .. 34816 x 5120.  (Q5_K's vocabulary
+// matrix sits close to the few-rows kernel's estimate: 151936 x 2048 takes 66 us here and 91 there; at 80 rows of
+// 17408 x 5120 the fifth group of 16 makes this kernel slower than the 128-row tiles, Q4_K 59 against 55, Q8_0 78 / 70.)
 double resident_estimate(uint32_t ggml_type, uint32_t m, uint32_t n, uint32_t k) {
     const double weights = (double)n * (double)k * 1e-6;
     const bool groups_of_32 = (size_t)32 * k * 2 <= 160u * 1024;
     const double groups = groups_of_32 ? (m + 31) / 32 : (m + 15) / 16;
     if (ggml_type == kQ6K) return 13.0 + weights * (groups_of_32 ? 0.01 + 0.2 * groups : 0.033 + 0.195 * groups);
+    if (groups_of_32) {
+        const double heavier = ggml_type == kQ4K ? 1.0 : ggml_type == kQ5K ? 1.2 : ggml_type == kIQ4XS ? 1.15 : 1.35;
+        return 5.0 + 2.4 * (k / 1024.0) + heavier * weights * (0.02 + 0.135 * groups);
+    }
     const double heavier = ggml_type == kQ4K ? 1.0 : ggml_type == kQ5K ? 1.5 : ggml_type == kIQ4XS ? 1.45 : 1.35;
-    return 8.0 + heavier * weights * (groups_of_32 ? 0.02 + 0.135 * groups : 0.047 + 0.09 * groups);
+    return 8.0 + heavier * weights * (0.047 + 0.09 * groups + (groups > 4 ? 0.08 : 0.0));
 }
 
 // What the heavier decodes add to the tiles' estimates, which were measured on Q4_K (at 512 rows of

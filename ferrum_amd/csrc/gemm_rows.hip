@@ -67,11 +67,17 @@ RowsPlan gemm_rows_plan(uint32_t ggml_type, uint32_t n, uint32_t k, uint32_t m, 
         most = std::min<uint64_t>(most, fh_device::kCounterWords / plan.tile_groups);
     }
     plan.run_rows = (uint32_t)std::min<uint64_t>(m, std::max<uint64_t>(most, 1) * plan.rows);
-    // (from two rounds on a compute unit's next workgroup starts as soon as one ends: rounds need not be whole)
+    // (from two rounds on a compute unit's next workgroup starts as soon as one ends: rounds need not be whole,
+    // except that up to 16 rows, whose workgroups mostly wait for weights of their own, the second costs more than
+    // the first and the third is whole: 8 x 28672 x 4096 in two rounds takes 26.5 us for Q4_K and 36 for Q5_K, the
+    // rows-resident kernel 24 and 33; 32 x 34816 x 5120 42 for Q4_K, that kernel 50)
     const uint64_t groups = ((uint64_t)m + plan.rows - 1) / plan.rows;
     const double rounds = (double)(plan.tile_groups * plan.segments * groups) / (double)cus;
-    plan.estimate_us = (rounds <= 1.0 ? 1.0 : rounds <= 2.0 ? 2.0 : rounds + 0.2) *
-                           (kStartUs + per_wave * plan.tiles * unit_us(ggml_type, x_dtype, plan.rows)) +
+    const bool waits = m <= 16 && x_dtype != FH_F32;
+    const double counted = rounds <= 1.0   ? 1.0
+                           : rounds <= 2.0 ? (waits ? 2.3 : 2.0)
+                                           : std::max(rounds + 0.2, waits ? 3.0 : 0.0);
+    plan.estimate_us = counted * (kStartUs + per_wave * plan.tiles * unit_us(ggml_type, x_dtype, plan.rows)) +
                        (plan.segments > 1 ? kExchangeUs : 0.0);
     plan.groups = (plan.run_rows + plan.rows - 1) / plan.rows;
     plan.counters = plan.segments > 1 ? (size_t)plan.tile_groups * plan.groups : 0;

@@ -761,6 +761,22 @@ def test_few_rows_on_the_edges_of_the_kernel(api, d, ggml, m, n, k, dtype):
         assert np.array_equal(bits(stored), bits(oracle.round_storage(got, code).reshape(m, n)))
 
 
+@pytest.mark.parametrize("ggml,m,n,k,few", [(13, 8, 151936, 2048, False), (12, 8, 28672, 4096, False), (13, 16, 28672, 4096, False),
+                                            (12, 8, 17408, 5120, True), (12, 32, 34816, 5120, True), (12, 80, 17408, 5120, True)])
+def test_16_bit_rows_take_the_faster_of_two_kernels(api, d, ggml, m, n, k, few):
+    """Where the few-rows kernel's rounds are many or not whole the rows-resident kernel is ahead: 66 against 91 us for
+    Q5_K's vocabulary matrix, 24 against 26.5 and 33 against 36 at 28672 x 4096; it is behind in the other three, 18
+    against 24, 42 against 50 and 50 against 59.  The two multiply the same rounded weights."""
+    tile = synth.matrix(ggml, 64, k, seed=271)
+    w = qm(api, d, ggml, n, k, np.tile(tile, n // 64))
+    x = api.Tensor.from_f32(d, (m, k), api.DType.F16, synth.activations(m, k, seed=272))
+    got = d.project_quantized(x, w, out_dtype=api.DType.F32).tensor.to_f32()
+    assert (d.get_tuning("last_rows_plan") != 0) == few
+    want = oracle.project(ggml, tile, 64, k, x.to_f32(), accumulate="f64", weight_round=oracle.F16, threads=8)
+    assert_matmul_parity(got[:, :64], want, "first rows")
+    assert np.array_equal(bits(got), bits(np.tile(got[:, :64], n // 64)))
+
+
 @pytest.mark.parametrize("ggml", [12, 13, 14, 23, 8], ids=["q4_k", "q5_k", "q6_k", "iq4_xs", "q8_0"])
 @pytest.mark.parametrize("m,n,k", [(16, 256, 256), (48, 100, 512), (8, 1024, 1024), (6, 4096, 4096), (40, 4100, 1024)])
 def test_small_f32_batches_stay_on_the_gemv(api, d, ggml, m, n, k):
