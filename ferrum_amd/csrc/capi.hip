@@ -74,26 +74,54 @@ fh_status resolve(const fh_device* device, const fh_view* view, uint64_t element
 
 bool fits_u32(uint64_t v) { return v <= 0xffffffffull; }
 
-// Gives back what the pool holds; whether it held anything.
-bool drain_pool(fh_device* d) {
-    std::multimap<size_t, void*> blocks;
-    {
-        std::lock_guard<std::mutex> hold(d->pool_lock);
-        blocks.swap(d->pool);
-        d->pool_bytes = 0;
-    }
-    if (blocks.empty()) return false;
+// Gives back what the pool holds; whether that was anything.  The caller has pool_lock.  A device that is
+// recording keeps its blocks: neither a wait on its stream nor a free may fall into a recording.
+bool drain_locked(fh_device* d) {
+    if (d->pool.empty() || d->capturing) return false;
     (void)hipStreamSynchronize(d->stream);
-    for (auto& block : blocks) (void)hipFree(block.second);
+    for (auto& block : d->pool) (void)hipFree(block.second);
+    d->pool.clear();
+    d->pool_bytes = 0;
     return true;
 }
 
-// Memory from the system; what the pool holds is given back when there is none.
+// Every device object between fh_device_create and fh_device_destroy.
+std::mutex g_live_lock;
+fh_device* g_live = nullptr;
+
+void enter_live(fh_device* d) {
+    std::lock_guard<std::mutex> hold(g_live_lock);
+    d->next_live = g_live;
+    g_live = d;
+}
+
+void leave_live(fh_device* d) {
+    std::lock_guard<std::mutex> hold(g_live_lock);
+    for (fh_device** at = &g_live; *at != nullptr; at = &(*at)->next_live)
+        if (*at == d) {
+            *at = d->next_live;
+            return;
+        }
+}
+
+// Gives back what the device objects on this GPU keep for themselves; whether that was anything.
+bool drain_pools(int ordinal) {
+    bool any = false;
+    std::lock_guard<std::mutex> hold(g_live_lock);
+    for (fh_device* d = g_live; d != nullptr; d = d->next_live) {
+        if (d->ordinal != ordinal) continue;
+        std::lock_guard<std::mutex> hold_pool(d->pool_lock);
+        any = drain_locked(d) || any;
+    }
+    return any;
+}
+
+// Memory from the system; what the pools on this GPU hold is given back when there is none.
 hipError_t allocate(fh_device* d, void** out, size_t bytes) {
     hipError_t e = hipMalloc(out, bytes);
     if (e == hipErrorOutOfMemory) {
         (void)hipGetLastError();
-        if (drain_pool(d)) e = hipMalloc(out, bytes);
+        if (drain_pools(d->ordinal)) e = hipMalloc(out, bytes);
     }
     return e;
 }
@@ -377,15 +405,10 @@ hipError_t take_block(fh_device* d, size_t capacity, void** out) {
 // library still has to do with the block comes before the next buffer's work on the stream.  A block whose
 // address the caller has been given may be in use elsewhere and goes back to the system.
 bool keep_block(fh_device* d, const fh_buffer& buffer) {
+    std::lock_guard<std::mutex> hold(d->pool_lock);
     if (d->closed || d->capturing || buffer.exposed || buffer.capacity > kPoolBlockBytes) return false;
-    bool full;
-    {
-        std::lock_guard<std::mutex> hold(d->pool_lock);
-        full = d->pool_bytes + buffer.capacity > kPoolBytes;
-    }
-    if (full) drain_pool(d);   // it holds sizes that are no longer asked for
+    if (d->pool_bytes + buffer.capacity > kPoolBytes) drain_locked(d);   // it holds sizes that are no longer asked for
     try {
-        std::lock_guard<std::mutex> hold(d->pool_lock);
         d->pool.emplace(buffer.capacity, buffer.ptr);
         d->pool_bytes += buffer.capacity;
     } catch (...) {   // no memory for the entry
@@ -468,6 +491,7 @@ fh_status fh_device_create(int32_t ordinal, fh_device** out) {
         delete d;
         return st;
     }
+    enter_live(d);
     *out = d;
     return FH_OK;
 }
@@ -484,7 +508,12 @@ void fh_device_destroy(fh_device* device) {
         device->capturing = false;
     }
     drain_deferred(device);
-    drain_pool(device);
+    leave_live(device);
+    {
+        std::lock_guard<std::mutex> hold(device->pool_lock);
+        drain_locked(device);
+        device->closed = true;   // buffers freed from here on are not kept
+    }
     if (device->stream) {
         (void)hipStreamSynchronize(device->stream);
         (void)hipStreamDestroy(device->stream);
@@ -505,7 +534,6 @@ void fh_device_destroy(fh_device* device) {
     device->retired_scratch.clear();
     device->scratch = nullptr;
     device->scratch_bytes = 0;
-    device->closed = true;
     drop_device_handle(device);
 }
 
@@ -544,6 +572,11 @@ void* fh_device_stream(fh_device* device) { return device ? device->stream : nul
 
 fh_status fh_set_tuning(fh_device* device, const char* key, int64_t value) {
     if (device == nullptr || key == nullptr) return fail(FH_ERR_PARAMETER, "null argument");
+    if (std::strcmp(key, "held_pool_bytes") == 0 && value == 0) {
+        FH_HIP(hipSetDevice(device->ordinal));
+        drain_pools(device->ordinal);
+        return FH_OK;
+    }
     int64_t* const setting = tuning_of(device, key);
     if (setting == nullptr) return fail(FH_ERR_PARAMETER, "unknown tuning key %s", key);
     std::string k(key);
@@ -588,6 +621,10 @@ fh_status fh_get_tuning(const fh_device* device, const char* key, int64_t* value
         return fail(FH_ERR_PARAMETER, "null argument");
     if (std::strcmp(key, "held_scratch_bytes") == 0) {
         *value = (int64_t)device->scratch_bytes;
+        return FH_OK;
+    }
+    if (std::strcmp(key, "held_pool_bytes") == 0) {
+        *value = (int64_t)device->pool_bytes;
         return FH_OK;
     }
     if (std::strcmp(key, "last_rows_plan") == 0) {
@@ -2266,6 +2303,7 @@ fh_status fh_moe_ffn(fh_device* device, const fh_view* hidden, const fh_view* ro
 fh_status fh_execution_begin(fh_device* device) {
     if (device == nullptr) return fail(FH_ERR_PARAMETER, "null device");
     if (device->capturing) return fail(FH_ERR_DISPATCH, "nested executions are not supported");
+    std::lock_guard<std::mutex> hold(device->pool_lock);   // no thread is waiting on the stream to empty the pool
     FH_HIP(hipStreamBeginCapture(device->stream, hipStreamCaptureModeThreadLocal));
     device->capturing = true;
     return FH_OK;

@@ -47,16 +47,18 @@ struct fh_device {
     hipDeviceProp_t props{};
     const char* last_operation = "";
     int64_t last_rows_plan = 0;   // of the last dense product: 0, or the few-rows kernel's rows, tiles and K segments
-    bool capturing = false;
+    std::atomic<bool> capturing{false};   // changes under pool_lock: what empties the pool waits on the stream
     fh_tuning tuning;
     // Blocks of freed buffers, by size, for the buffers to come (fh_buffer_alloc): hipMalloc and hipFree
     // take 10 - 20 us each and the latter waits for the GPU (a routed FFN of 200 f32 tokens whose operators
     // return new tensors: 453 us without the pool, 286 with it).  All work of the library on a buffer is on
     // `stream`, so a block can be handed on at once; buffers whose address has left the library are freed.
-    // Python may drop a buffer on any thread: the pool has a lock.
+    // Python may drop a buffer on any thread, and another device object on the same GPU that finds no memory
+    // empties this one's pool: the pool has a lock.
     std::mutex pool_lock;
     std::multimap<size_t, void*> pool;
     size_t pool_bytes = 0;
+    fh_device* next_live = nullptr;   // device objects that have not been destroyed (g_live in capi.hip)
     // scratch owned by the device: [counter words | floats / ids]
     void* scratch = nullptr;
     size_t scratch_bytes = 0;

@@ -125,6 +125,8 @@ void* fh_device_stream(fh_device* device);
  * rule as set_k_quant_gemv_ksplit (0 or a power of two up to 8).  Unknown
  * keys or out-of-range values give FH_ERR_PARAMETER.
  * fh_get_tuning alone also answers for what the library does by itself:
+ *   held_pool_bytes     freed buffers kept for the next ones (see below); fh_set_tuning with 0 gives
+ *                       back what every device object on this GPU keeps
  *   held_scratch_bytes  the operators' common scratch
  *   last_rows_plan      how the last dense product ran on the few-rows kernel: 1000 x activation
  *                       rows (16 or 32) + 100 x weight tiles per wave + K segments; 0 on others */
@@ -137,7 +139,8 @@ fh_status fh_get_tuning(const fh_device* device, const char* key, int64_t* value
  * fh_buffer_alloc_uninitialized leaves the contents undefined, for outputs an
  * operator writes whole.  A device keeps up to 256 MiB of freed buffers (of up to
  * 64 MiB each) for the next ones and returns them to the system when it is
- * destroyed or memory runs out; freeing does not wait for the stream then.
+ * destroyed or an allocation of any device object on that GPU finds no memory;
+ * freeing does not wait for the stream then.
  * Buffers whose address fh_buffer_device_ptr has given out are not kept. */
 fh_status fh_buffer_alloc(fh_device* device, size_t bytes, fh_buffer** out);
 fh_status fh_buffer_alloc_uninitialized(fh_device* device, size_t bytes, fh_buffer** out);

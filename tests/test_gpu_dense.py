@@ -886,16 +886,53 @@ def test_a_buffer_is_zero_whatever_held_its_memory_before(api, d, nbytes):
 
 def test_a_full_pool_makes_room_and_an_exposed_address_is_not_handed_on(api):
     dev = api.Device.new()
+    kept = lambda: dev.get_tuning("held_pool_bytes")
+    seen = []
     for step in range(12):
         held = [api.Buffer(dev, (40 << 20) + step * (1 << 20), zeroed=False) for _ in range(4)]
         del held
+        seen.append(kept())
+    assert 4 * 40 << 20 <= max(seen) <= 256 << 20 and sum(b < a for a, b in zip(seen, seen[1:])) > 1   # emptied more than once
+    dev.set_tuning("held_pool_bytes", 0)
+    assert kept() == 0
     b = api.Buffer(dev, 3 << 20)
-    address = b.device_ptr()
     del b
-    kept = [api.Buffer(dev, 3 << 20) for _ in range(4)]
-    assert address and all(k.nbytes == 3 << 20 for k in kept)
+    assert kept() == 3 << 20
+    b = api.Buffer(dev, (3 << 20) - 100)      # of the same size class
+    assert kept() == 0
+    assert b.device_ptr()
+    del b
+    assert kept() == 0                        # its address has left the library
+    big = api.Buffer(dev, (64 << 20) + 4)
+    del big
+    assert kept() == 0
     x = api.Tensor.zeros(dev, (8, 1024), api.DType.F16)
     assert not x.raw().any()
+    with pytest.raises(api.Error):
+        dev.set_tuning("held_pool_bytes", 1)
+
+
+def test_one_device_object_gives_back_what_another_on_the_gpu_keeps(api):
+    # what an allocation that finds no memory does before it tries once more
+    first, second = api.Device.new(), api.Device.new()
+    w = qm(api, first, Q4_K, 64, 512, synth.matrix(Q4_K, 64, 512, seed=161))
+    x = api.Tensor.from_f32(first, (1, 512), api.DType.F32, synth.activations(1, 512, seed=162))
+    y = api.Tensor.zeros(first, (1, 64), api.DType.F32)
+    want = first.project_quantized(x, w).tensor.raw()
+    assert first.get_tuning("held_pool_bytes") > 0      # that result is gone again
+    with first.execution() as recorded:
+        first.project_quantized(x, w, out=y)
+        before = first.get_tuning("held_pool_bytes")
+        second.set_tuning("held_pool_bytes", 0)         # a device that is recording is left alone
+        assert first.get_tuning("held_pool_bytes") == before > 0
+    second.set_tuning("held_pool_bytes", 0)
+    assert first.get_tuning("held_pool_bytes") == 0
+    recorded.graph.launch()
+    assert np.array_equal(y.raw(), want)
+    handle, first._handle = first._handle, None
+    api._lib.fh_device_destroy(handle)
+    second.set_tuning("held_pool_bytes", 0)             # the other one is no longer looked at
+    assert second.get_tuning("held_pool_bytes") == 0
 
 
 # ------------------------------------------------------------- greedy selection
