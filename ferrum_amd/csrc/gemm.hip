@@ -1209,12 +1209,11 @@ double wide_format_factor(uint32_t ggml_type) {
 template <uint32_t TYPE, int DT, int NT, int RT>
 void launch_wide32(hipStream_t s, const GemmArgs& a, const WidePlan& plan) {
     const size_t lds = Wide32<RT>::kWeightsAt + 2 * (size_t)(32 * NT) * kLd * sizeof(uint16_t);
-    static bool configured = false;
-    if (!configured) {
+    static std::atomic<uint64_t> raised{0};
+    once_per_device(raised, [] {
         (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_wide32_kernel<TYPE, DT, NT, RT>),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        configured = true;
-    }
+    });
     const uint32_t groups = (plan.tiles_n + 7) / 8;
     dim3 grid(groups * 8 * plan.tiles_m);
     hipLaunchKernelGGL((gemm_wide32_kernel<TYPE, DT, NT, RT>), grid, dim3(512), lds, s,
@@ -1225,12 +1224,11 @@ void launch_wide32(hipStream_t s, const GemmArgs& a, const WidePlan& plan) {
 template <uint32_t TYPE, int DT, int NT>
 void launch_wide(hipStream_t s, const GemmArgs& a, const WidePlan& plan) {
     const size_t lds = 2 * (size_t)(16 * NT) * kLd * sizeof(uint16_t);
-    static bool configured = false;
-    if (!configured) {
+    static std::atomic<uint64_t> raised{0};
+    once_per_device(raised, [] {
         (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_wide_kernel<TYPE, DT, NT>),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        configured = true;
-    }
+    });
     const uint32_t groups = (plan.tiles_n + 7) / 8;
     dim3 grid(groups * 8 * plan.tiles_m);
     hipLaunchKernelGGL((gemm_wide_kernel<TYPE, DT, NT>), grid, dim3(kWideThreads), lds, s,

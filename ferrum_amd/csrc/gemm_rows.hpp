@@ -293,12 +293,11 @@ template <uint32_t TYPE, int DT, int ROWS, int T>
 void launch_one(hipStream_t s, const RowsPlan& plan, const RowsParams& p) {
     constexpr uint32_t kSums = T * (ROWS / 16) * 1024u;   // partial sums of a wave
     constexpr size_t kLds = kRowsWaves * (kWaveLds<DT, ROWS> > kSums ? kWaveLds<DT, ROWS> : kSums);
-    static const bool configured = [] {
+    static std::atomic<uint64_t> raised{0};
+    once_per_device(raised, [] {
         (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_rows_kernel<TYPE, DT, ROWS, T>),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLds);
-        return true;
-    }();
-    (void)configured;
+    });
     hipLaunchKernelGGL((gemm_rows_kernel<TYPE, DT, ROWS, T>), dim3((p.tile_groups + 7) / 8 * 8 * p.groups, plan.segments),
                        dim3(kRowsThreads), kLds, s, p);
 }

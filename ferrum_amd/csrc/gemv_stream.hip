@@ -576,15 +576,14 @@ const char* launch_gemv_stream(hipStream_t s, const GemvArgs& a, const StreamPla
          {gemv_stream_q6k<FH_F16, 8, 2>, gemv_stream_q6k<FH_F16, 8, 3>, gemv_stream_q6k<FH_F16, 8, 6>},
          {gemv_stream_q6k<FH_BF16, 8, 2>, gemv_stream_q6k<FH_BF16, 8, 3>, gemv_stream_q6k<FH_BF16, 8, 6>}},
     };
-    static bool raised = false;
-    if (!raised) {
+    static std::atomic<uint64_t> raised{0};
+    once_per_device(raised, [] {
         for (const auto& format : kernels)
             for (const auto& row : format)
                 for (Kernel kernel : row)
                     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
                                               hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-        raised = true;
-    }
+    });
     const int shape = plan.seg_blocks <= 16u ? 0 : plan.seg_blocks <= 24u ? 1 : 2;
     const int format = a.ggml_type == kQ6K ? 1 : 0;
     // Q4_K tiles of up to 14 rows (two load instructions per super-block): every wave loads what it
@@ -600,13 +599,12 @@ const char* launch_gemv_stream(hipStream_t s, const GemvArgs& a, const StreamPla
             {gemv_stream_q4k_own<FH_BF16, 8, 2>, gemv_stream_q4k_own<FH_BF16, 8, 3>, gemv_stream_q4k_own<FH_BF16, 8, 6>},
         };
         Kernel kernel = own_kernels[a.x_dtype][shape];
-        static bool once = false;
-        if (!once) {
+        static std::atomic<uint64_t> own_raised{0};
+        once_per_device(own_raised, [] {
             for (const auto& row : own_kernels)
                 for (Kernel k : row)
                     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-            once = true;
-        }
+        });
         p.tile_bytes = own_bytes;
         const uint32_t lds = own_bytes + plan.waves * kSlotBytes + plan.waves * 64u;
         hipLaunchKernelGGL(kernel, dim3(plan.tiles, plan.segments, a.m), dim3(plan.waves * kWave), lds, s, p);

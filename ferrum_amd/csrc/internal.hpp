@@ -138,6 +138,18 @@ constexpr uint32_t block_bytes_of(uint32_t ggml_type) {
 inline size_t block_bytes(uint32_t ggml_type) {
     return block_bytes_of(ggml_type);
 }
+// Runs `raise` once for the current device (two threads may both, on ordinals from 64 on every call does): a
+// kernel's dynamic LDS limit belongs to its copy on a device.
+template <class Raise>
+void once_per_device(std::atomic<uint64_t>& done, Raise&& raise) {
+    int ordinal = 64;
+    (void)hipGetDevice(&ordinal);
+    const uint64_t bit = ordinal < 64 ? 1ull << ordinal : 0;
+    if ((done.load(std::memory_order_acquire) & bit) != 0) return;
+    raise();
+    done.fetch_or(bit, std::memory_order_release);
+}
+
 inline size_t dtype_bytes(uint32_t dtype) { return dtype == FH_F32 ? 4 : 2; }
 
 // ---- launchers (one per kernel family); each returns the kernel name ----
