@@ -7,6 +7,8 @@ with its closed-form inputs and its tolerances; the second half applies the
 benchmark's bars (dequant bit-exact; max relative error 1e-3 and relative L2
 1e-5 with f32 accumulation) at the benchmark shapes on seeded synthetic blocks.
 """
+import functools
+
 import numpy as np
 import pytest
 
@@ -593,17 +595,19 @@ def test_a_recorded_execution_survives_the_growth_of_the_scratch(api, d):
 
 
 def test_f32_batches_of_any_size_run_through_the_long_k_gemv(api, d):
-    # q4_k_gemm accepts any M (src/metal/shaders/ops.metal:1102-1121): a long-K projection of 110 f32
-    # rows needs more row-tile counters than one launch has, so the batch is cut into runs
+    # q4_k_gemm accepts any M (src/metal/shaders/ops.metal:1102-1121): on the GEMV, which has these batches where
+    # the few-rows kernel is switched off, a long-K projection of 110 f32 rows needs more row-tile counters
+    # than one launch has, so the batch is cut into runs
     n, k, m = 5120, 17408, 110
     packed = synth.matrix(Q4_K, n, k, seed=131)
     w = qm(api, d, Q4_K, n, k, packed)
     x = synth.activations(m, k, seed=132)
-    out = d.project_quantized(api.Tensor.from_f32(d, (m, k), api.DType.F32, x), w)
-    assert out.operation == "q4_k_gemm"
-    got = out.tensor.to_f32()
-    first = d.project_quantized(api.Tensor.from_f32(d, (60, k), api.DType.F32, x[:60]), w).tensor.to_f32()
-    last = d.project_quantized(api.Tensor.from_f32(d, (50, k), api.DType.F32, x[60:]), w).tensor.to_f32()
+    with few_rows(d, 0):
+        out = d.project_quantized(api.Tensor.from_f32(d, (m, k), api.DType.F32, x), w)
+        assert out.operation == "q4_k_gemm" and d.get_tuning("last_rows_plan") == 0
+        got = out.tensor.to_f32()
+        first = d.project_quantized(api.Tensor.from_f32(d, (60, k), api.DType.F32, x[:60]), w).tensor.to_f32()
+        last = d.project_quantized(api.Tensor.from_f32(d, (50, k), api.DType.F32, x[60:]), w).tensor.to_f32()
     assert np.array_equal(bits(got[:60]), bits(first)) and np.array_equal(bits(got[60:]), bits(last))
     rows = np.unique(synth.rng(133).integers(0, n, 48))
     picked = [0, 59, 60, 101, 102, 103, 109]
@@ -712,21 +716,21 @@ def test_few_rows_deal_a_tiles_super_blocks_over_the_waves(api, d, ggml, m, n, k
     code = oracle.F16 if dtype == "F16" else oracle.BF16
     x = oracle.round_storage(synth.activations(m, k, seed=182), code).reshape(m, k)
     xt = api.Tensor.from_f32(d, (m, k), getattr(api.DType, dtype), x)
-    out = d.project_quantized(xt, w, out_dtype=api.DType.F32)
-    assert out.operation.endswith("_gemm_mfma_resident")
-    d.set_tuning("gemm_few_tiles_split", 0)
-    try:
+    with few_rows(d, 2):
+        out = d.project_quantized(xt, w, out_dtype=api.DType.F32)
+    # (both kernels report the name the rows-resident one has always had)
+    assert out.operation.endswith("_gemm_mfma_resident") and d.get_tuning("last_rows_plan") // 1000 == 16
+    with few_rows(d, 0):
         whole = d.project_quantized(xt, w, out_dtype=api.DType.F32)
-    finally:
-        d.set_tuning("gemm_few_tiles_split", 1)
-    assert whole.operation == out.operation
+    assert whole.operation == out.operation and d.get_tuning("last_rows_plan") == 0
     got = out.tensor.to_f32()
     rows = np.unique(np.concatenate([np.arange(0, 40), np.arange(n - 40, n), synth.rng(183).integers(0, n, 80)]))
     want = oracle_columns(ggml, packed, n, k, rows, x, weight_round=code, accumulate="f64")
     assert_matmul_parity(got[:, rows], want, "dealt super-blocks against the tile-rounded oracle")
     assert_matmul_parity(got, whole.tensor.to_f32(), "against whole tiles per wave", l2_tol=2e-6)
     assert not np.array_equal(got, np.zeros_like(got))
-    half = d.project_quantized(xt, w, out_dtype=getattr(api.DType, dtype))      # 16-bit output: the scalar stores
+    with few_rows(d, 2):
+        half = d.project_quantized(xt, w, out_dtype=getattr(api.DType, dtype))      # 16-bit output: the scalar stores
     assert np.array_equal(half.tensor.to_f32(), oracle.round_storage(got, code).reshape(m, n))
 
 
@@ -759,6 +763,49 @@ def test_few_rows_on_the_edges_of_the_kernel(api, d, ggml, m, n, k, dtype):
             assert np.array_equal(bits(part), bits(got[:-1]))
         stored = d.project_quantized(xt, w).tensor.to_f32()      # 16-bit results: the packed stores
         assert np.array_equal(bits(stored), bits(oracle.round_storage(got, code).reshape(m, n)))
+
+
+@functools.lru_cache(maxsize=1)
+def _sixteen_thousand_rows(ggml, k):
+    return synth.matrix(ggml, 16750, k, seed=291)
+
+
+# Two to five weight tiles per wave (n picks them: one round of the chip), the ragged last tile and the packed and
+# element stores, in the 32-row, 16-row and f32 forms of every format; and four tiles with K cut in three.
+@pytest.mark.parametrize("ggml", [12, 13, 14, 23, 8], ids=["q4_k", "q5_k", "q6_k", "iq4_xs", "q8_0"])
+@pytest.mark.parametrize("tiles,n", [(2, 4150), (3, 8200), (4, 12700), (5, 16750)])
+def test_few_rows_with_several_tiles_per_wave(api, d, ggml, tiles, n):
+    k = 2048
+    packed = _sixteen_thousand_rows(ggml, k).reshape(16750, -1)[:n].reshape(-1)
+    w = qm(api, d, ggml, n, k, packed)
+    rows = np.unique(np.concatenate([np.arange(0, 24), np.arange(n - 40, n), synth.rng(292).integers(0, n, 40)]))
+    for m, dtype in ((9, "F32"), (13, "F16"), (20, "F16"), (33, "BF16")):
+        code = {"F32": oracle.F32, "F16": oracle.F16, "BF16": oracle.BF16}[dtype]
+        x = oracle.round_storage(synth.activations(m, k, seed=293 + m), code).reshape(m, k)
+        with few_rows(d, 2):
+            got = d.project_quantized(api.Tensor.from_f32(d, x.shape, getattr(api.DType, dtype), x), w,
+                                      out_dtype=api.DType.F32).tensor.to_f32()
+        assert d.get_tuning("last_rows_plan") == (32000 if m > 16 else 16000) + 100 * tiles + 1
+        want = oracle_columns(ggml, packed, n, k, rows, x, accumulate="f64", weight_round=code)
+        assert_matmul_parity(got[:, rows], want, f"{tiles} tiles, {m} {dtype} rows")
+
+
+@pytest.mark.parametrize("ggml", [12, 13, 14, 23, 8], ids=["q4_k", "q5_k", "q6_k", "iq4_xs", "q8_0"])
+def test_few_rows_with_four_tiles_and_three_segments(api, d, ggml):
+    n, k = 5120, 17408
+    tile = synth.matrix(ggml, 80, k, seed=295)      # five tiles, over and over: a wave's four are different
+    w = qm(api, d, ggml, n, k, np.tile(tile, n // 80))
+    for m, dtype in ((7, "F32"), (19, "F16")):
+        code = oracle.F32 if dtype == "F32" else oracle.F16
+        x = oracle.round_storage(synth.activations(m, k, seed=296 + m), code).reshape(m, k)
+        with few_rows(d, 2):
+            got = d.project_quantized(api.Tensor.from_f32(d, x.shape, getattr(api.DType, dtype), x), w,
+                                      out_dtype=api.DType.F32).tensor.to_f32()
+        plan = d.get_tuning("last_rows_plan")
+        assert plan == (32403 if dtype == "F16" else 16403), plan
+        want = oracle.project(ggml, tile, 80, k, x, accumulate="f64", weight_round=code, threads=8)
+        assert_matmul_parity(got[:, :80], want, f"{m} {dtype} rows")
+        assert np.array_equal(bits(got), bits(np.tile(got[:, :80], n // 80)))
 
 
 @pytest.mark.parametrize("ggml,m,n,k,few", [(13, 8, 151936, 2048, False), (12, 8, 28672, 4096, False), (13, 16, 28672, 4096, False),
@@ -1144,15 +1191,17 @@ def test_rows_resident_gemm_matches_the_rounded_weight_oracle(api, d, ggml, m, n
     w = qm(api, d, ggml, n, k, packed)
     x = oracle.round_storage(synth.activations(m, k, seed=302 + m), code).reshape(m, k)
     xt = api.Tensor.from_f32(d, x.shape, dtype, x)
-    out = d.project_quantized(xt, w, out_dtype=api.DType.F32)
-    assert out.operation.endswith("_gemm_mfma_resident")
+    with few_rows(d, 0):      # (up to 128 rows the few-rows kernel may take the call under the same name)
+        out = d.project_quantized(xt, w, out_dtype=api.DType.F32)
+    assert out.operation.endswith("_gemm_mfma_resident") and d.get_tuning("last_rows_plan") == 0
     rows = np.unique(np.concatenate([np.arange(0, min(n, 48)), np.arange(max(0, n - 40), n),
                                      synth.rng(303).integers(0, n, 32)]))
     want = oracle_columns(ggml, packed, n, k, rows, x, weight_round=code, accumulate="f64")
     got = out.tensor.to_f32()
     assert_matmul_parity(got[:, rows], want, f"rows-resident m={m} n={n} k={k}")
     # stored in the activation dtype (packed stores where rows allow, element stores on ragged ones)
-    stored = d.project_quantized(xt, w)
+    with few_rows(d, 0):
+        stored = d.project_quantized(xt, w)
     assert stored.operation == out.operation
     assert np.array_equal(bits(stored.tensor.to_f32()), bits(oracle.round_storage(got, code).reshape(m, n)))
     # every row group and tile was written: the square tiles give the same product
@@ -1206,7 +1255,9 @@ def test_an_f32_batch_of_any_size_leaves_the_scratch_as_it_is(api, ggml, m, n, k
     assert np.array_equal(bits(part), bits(got[m - 7:]))
 
 
-@pytest.mark.parametrize("ggml,m,n,k", [(Q4_K, 5, 200, 256), (Q4_K, 16, 1024, 1024), (Q6_K, 24, 530, 2048), (Q5_K, 64, 777, 5120)])
+@pytest.mark.parametrize("ggml,m,n,k", [(Q4_K, 5, 200, 256), (Q4_K, 16, 1024, 1024), (Q6_K, 24, 530, 2048), (Q5_K, 64, 777, 5120),
+                                        (IQ4_XS, 12, 300, 4096), (Q8_0, 9, 400, 4352), (Q6_K, 6, 1030, 17408), (Q8_0, 7, 1030, 17408),
+                                        (IQ4_XS, 5, 1030, 14336), (Q4_K, 6, 1030, 17408)])
 def test_a_batch_of_f32_rows_is_as_close_to_64_bits_as_its_chains_are_short(api, d, ggml, m, n, k):
     """Sixteen products follow each other in one accumulator, the rest is added in pairs and over eight waves.
     A chain of L roundings of at most 2^-24, uniform, is off by 2^-24 / sqrt(3) * sqrt(L / 2) in the mean square:
@@ -1215,6 +1266,12 @@ def test_a_batch_of_f32_rows_is_as_close_to_64_bits_as_its_chains_are_short(api,
     packed = synth.matrix(ggml, n, k, seed=721)
     w = qm(api, d, ggml, n, k, packed)
     x = np.asarray(synth.activations(m, k, seed=722), dtype=np.float32).reshape(m, k)
-    got = d.project_quantized(api.Tensor.from_f32(d, x.shape, api.DType.F32, x), w).tensor.to_f32()
+    xt = api.Tensor.from_f32(d, x.shape, api.DType.F32, x)
+    with few_rows(d, 2):
+        got = d.project_quantized(xt, w).tensor.to_f32()
+        assert d.get_tuning("last_rows_plan") != 0
     weights = oracle.dequantize(ggml, packed, n, k).reshape(n, k).astype(np.float64)
-    assert rel_l2(got, x.astype(np.float64) @ weights.T) <= 1.6e-7
+    exact = x.astype(np.float64) @ weights.T
+    assert rel_l2(got, exact) <= 1.6e-7
+    # the default is this kernel or, for Q4_K and Q5_K, a GEMV that is as close
+    assert rel_l2(d.project_quantized(xt, w).tensor.to_f32(), exact) <= 1.6e-7
