@@ -1214,25 +1214,34 @@ def test_rows_resident_gemm_matches_the_rounded_weight_oracle(api, d, ggml, m, n
     assert rel_l2(got, tiles.tensor.to_f32()) <= 1e-5
 
 
-@pytest.mark.parametrize("m,n,k,dtype_name", [(320, 5120, 17408, "F32")])
-def test_a_batch_whose_partial_sums_outgrow_the_scratch_can_be_recorded_first(api, m, n, k, dtype_name):
-    """Partial sums of K segments save time only: a device whose scratch cannot hold them while it records
-    takes a kernel that needs none, and replays are that kernel's results."""
+@pytest.mark.parametrize("m,n,k,rounded", [(320, 5120, 17408, False), (128, 2500, 31744, True)])
+def test_a_batch_whose_partial_sums_outgrow_the_scratch_can_be_recorded_first(api, m, n, k, rounded):
+    """Partial sums of K segments save time only.  Exact f32 rows run in launches whose sums fit the scratch a new
+    device has.  Rows that are rounded to f16 have 7.8 MiB of it for that, and 9.8 MiB of sums no longer fit: while
+    it records the device takes a kernel that needs none, and replays are that kernel's results."""
     dev = api.Device.new()
-    dtype = api.DType[dtype_name]
+    dev.set_tuning("gemm_few_tiles_split", 2)
+    dev.set_tuning("gemm_f32_min_rows", 2 if rounded else 0)
     w = qm(api, dev, Q4_K, n, k, synth.matrix(Q4_K, n, k, seed=711))
-    x = api.Tensor.from_f32(dev, (m, k), dtype, synth.activations(m, k, seed=712))
+    x = api.Tensor.from_f32(dev, (m, k), api.DType.F32, synth.activations(m, k, seed=712))
     recorded = api.Tensor.zeros(dev, (m, n), api.DType.F32)
     dev.synchronize()
     with dev.execution() as ex:
         dev.project_quantized(x, w, out=recorded)
+    assert (dev.get_tuning("last_rows_plan") == 0) == rounded
     ex.graph.launch()
     dev.synchronize()
+    held = dev.get_tuning("held_scratch_bytes")
     direct = dev.project_quantized(x, w, out_dtype=api.DType.F32).tensor.to_f32()   # the scratch may grow here
+    assert dev.get_tuning("last_rows_plan") != 0
+    assert (dev.get_tuning("held_scratch_bytes") > held) == rounded
     for _ in range(2):
         ex.graph.launch()
         dev.synchronize()
-        assert rel_l2(recorded.to_f32(), direct) <= 1e-5
+        if rounded:
+            assert rel_l2(recorded.to_f32(), direct) <= 1e-5
+        else:
+            assert np.array_equal(bits(recorded.to_f32()), bits(direct))
 
 
 @pytest.mark.parametrize("ggml,m,n,k", [(Q4_K, 1000, 5120, 17408), (Q6_K, 1800, 1030, 17408)])
