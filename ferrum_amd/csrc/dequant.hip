@@ -244,7 +244,7 @@ __global__ __launch_bounds__(1024) void argmax_rows_kernel(const void* __restric
 
 // Rows of a vocabulary: one workgroup needs a round trip per 1024 columns (151936 f32 logits: 66 us), so
 // a row is cut into pieces of 8192 columns, one workgroup each, whose maxima meet in device memory; the
-// last to arrive folds them (151936: 5 us).  The first maximal index of a row without NaN
+// last to arrive folds them (151936: 8 us).  The first maximal index of a row without NaN
 // does not depend on the order in which it is searched; a row that holds one is searched again by the
 // last workgroup in the schedule above.
 constexpr uint32_t kArgmaxPiece = 8192;

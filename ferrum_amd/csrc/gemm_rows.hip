@@ -9,7 +9,10 @@ namespace {
 
 // What one super-block of one weight tile costs a wave, in us, with two waves on the SIMD: the decode,
 // the matrix instructions of 16 or 32 rows and their share of the stream.  From 17408 x 5120 and
-// 5120 x 17408 (f16: 17.7 / 21.2 us at 16 / 32 rows for Q4_K, 30.8 / 40.5 for Q6_K; f32: 38).
+// 5120 x 17408 (f16: 17.7 / 21.2 us at 16 / 32 rows for Q4_K, 30.8 / 40.5 for Q6_K).  f32 rows count 2.3 in every
+// format here, as measured on Q4_K before their sums were paired: it places tiles and segments only (whether the
+// kernel takes the call is f32_rows_pay's, with the present 2.6 to 3.0; 16 rows of 17408 x 5120 take 46 us for Q4_K,
+// 60 for Q6_K), and a row's sums follow from that placement.
 double unit_us(uint32_t ggml_type, uint32_t x_dtype, uint32_t rows) {
     if (x_dtype == FH_F32) return 2.3;
     switch (ggml_type) {
