@@ -337,9 +337,14 @@ __global__ __launch_bounds__(1024) void argmax_pieces_kernel(const void* __restr
 }  // namespace
 
 size_t argmax_partial_bytes(uint32_t rows, uint32_t width) {
-    // a row of one piece, and more rows than counter words or grid rows, keep one workgroup a row
-    if (width <= kArgmaxPiece || rows > 65535u) return 0;
-    return (size_t)rows * ((width + kArgmaxPiece - 1) / kArgmaxPiece) * 2 * sizeof(unsigned long long);
+    // Rows of little more than a piece keep one workgroup each, and so do many rows, which fill the chip by themselves
+    // (us, a workgroup a row against pieces: f32 1 x 8193 8.2 / 8.7, 8 x 12000 9.1 / 8.8, 8 x 65536 18.3 / 9.3, 512 x
+    // 20000 15.4 / 24.9; bf16 1 / 64 / 512 x 151936 31 / 34 / 66 against 8.9 / 25 / 144).
+    const uint32_t pieces = (width + kArgmaxPiece - 1) / kArgmaxPiece;
+    const double width_in_pieces = (double)width / kArgmaxPiece;
+    const bool pays = 8.6 + 0.0125 * rows * pieces < 6.9 + 1.3 * width_in_pieces;
+    if (!pays || rows > 65535u) return 0;   // (a counter word and a grid row each)
+    return (size_t)rows * pieces * 2 * sizeof(unsigned long long);
 }
 
 const char* launch_argmax_rows(hipStream_t s, const void* logits, uint32_t dtype, uint32_t rows, uint32_t width,

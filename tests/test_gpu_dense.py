@@ -1028,6 +1028,20 @@ def test_argmax_of_rows_cut_into_pieces(api, d, width):
         assert np.array_equal(got.raw().view(np.uint32).reshape(8, 2), oracle.argmax_rows(x))
 
 
+def test_argmax_of_a_row_alone_and_among_many(api, d):
+    # many rows fill the chip with a workgroup each, a few are cut into pieces: the same answers
+    rows, width = 150, 16385
+    x = synth.rng(139).integers(0, 50, (rows, width)).astype(np.float32)     # ties all along every row
+    x[3, 9000] = np.nan
+    x[77, 16384] = np.inf
+    want = oracle.argmax_rows(x)
+    t = api.Tensor.from_f32(d, x.shape, api.DType.F32, x)
+    assert np.array_equal(d.argmax_rows(t).raw().view(np.uint32).reshape(rows, 2), want)
+    for at in (0, 3, 77, 149):
+        one = api.Tensor.from_f32(d, (1, width), api.DType.F32, x[at])
+        assert np.array_equal(d.argmax_rows(one).raw().view(np.uint32).reshape(2), want[at])
+
+
 @pytest.mark.parametrize("ggml,n,k,dtype", [
     (Q6_K, 700, 17408, "F32"), (Q6_K, 700, 17408, "BF16"), (Q4_K, 4200, 1024, "F16"), (Q4_K, 1100, 17408, "F32"),
     (Q4_K, 300, 512, "F16"), (Q6_K, 1300, 17408, "F32"), (Q4_K, 1300, 17408, "BF16"), (Q4_K, 20500, 1024, "F16"),
