@@ -698,13 +698,16 @@ void launch_tt(hipStream_t s, const GemmArgs& a) {
         // evenly, share the chip (256 experts top-8, 4 / 8 / 16 tokens: 116 / 117 / 118 us with one
         // share, 62 / 80 / 102 with four).  Two deviations more than the mean count as hit: a workgroup
         // over the chip's number is a round of its own (64 experts of 2816 x 2048 Q6_K, 96 assignments to 53 of
-        // them: 107 us in five shares, 92 in four).
+        // them: 107 us in five shares, 92 in four).  Below twice the shares that all experts would get it does not
+        // pay: the workgroups of the others also carry the shared expert's pieces (64 experts of 2048 x 1024 and a
+        // shared one, five tokens top-8: Q6_K 48 - 60 us in six or eight shares, 42 in four).
         const uint32_t tiles = (a.n + 15) / 16;
         const uint32_t target = a.cu_count > 0 ? (uint32_t)a.cu_count : 256u;
         const double missed = std::pow(1.0 - 1.0 / (double)a.experts, (double)a.m);
         const double hit = std::min({(double)a.experts, (double)a.m,
                                      a.experts * (1.0 - missed) + 2.0 * std::sqrt(a.experts * missed * (1.0 - missed))});
-        const uint32_t shares = std::max((target + a.experts - 1) / a.experts, (uint32_t)(target / std::max(hit, 1.0)));
+        const uint32_t all_hit = (target + a.experts - 1) / a.experts, few_hit = (uint32_t)(target / std::max(hit, 1.0));
+        const uint32_t shares = few_hit >= 2 * all_hit ? few_hit : all_hit;
         uint32_t tiles_per_wg = (tiles + shares - 1) / shares;
         tiles_per_wg = (tiles_per_wg + kResWaves - 1) / kResWaves * kResWaves;
         const dim3 rgrid((tiles + tiles_per_wg - 1) / tiles_per_wg, a.experts);
