@@ -640,12 +640,19 @@ __global__ __launch_bounds__(kResThreads) void expert_ring_kernel(const uint8_t*
     }
 }
 
-// Tokens an expert's workgroup takes in one pass over its weights: 32 with more than 6 per expert on
-// average (8 where 32 rows do not fit LDS), else 16.  At 8 on average one of 256 experts is likely to
-// have more than 16, and its second pass doubles the launch: 256 experts top-8, 256 tokens 209 us in
-// passes of 16, 158 in passes of 32; 128 tokens 144 against 150.
+// Tokens an expert's workgroup takes in one pass over its weights: 32 with more than 8 per expert on average,
+// else 16, unless 32 rows fit LDS and one expert is likely enough to have more than 16: its second pass nearly
+// doubles the launch (256 experts top-8, 256 tokens 209 us in passes of 16, 158 in passes of 32), where
+// passes of 32 cost 5 - 14% (256 experts of 1024 x 2048, 200 tokens: IQ4_XS 106 us and 121, Q8_0 133 and 150).  Ids
+// drawn evenly, the counts are close to Poisson's; the line at a chance of a fifth is 6.9 tokens per expert
+// for 256 of them, 7.3 for 128, 7.9 for 64.
 bool passes_of_32(uint32_t k, uint32_t m, uint32_t experts) {
-    return m > 8 * experts || (m > 6 * experts && (size_t)32 * k * 2 <= kResLdsBytes);
+    if (m > 8 * experts) return true;
+    if (m <= 6 * experts || (size_t)32 * k * 2 > kResLdsBytes) return false;
+    const double mean = (double)m / (double)experts;
+    double term = std::exp(-mean), up_to_16 = term;
+    for (int i = 1; i <= 16; ++i) up_to_16 += term *= mean / i;
+    return experts * (1.0 - up_to_16) > 0.2;
 }
 
 template <uint32_t TYPE, int DT>
