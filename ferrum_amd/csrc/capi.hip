@@ -1761,7 +1761,7 @@ bool rider_fits(uint32_t n, uint32_t k, uint64_t entries) {
 // per-assignment launch reads an expert's matrix for each of its assignments at the rate of its decode (rows
 // whose super-blocks leave more than a third of the kernel's block slots idle, as five on eight do, a fifth
 // below it); the grouped one waits for the workgroup that streams one share of one expert, behind a grouping
-// and a staging launch (9 and 16.5 us before either streams).  One projection, f16, us, per assignment against grouped: 64 experts of 2048 x 1280, 64 /
+// and a staging launch (9 and 15.5 us before either streams).  One projection, f16, us, per assignment against grouped: 64 experts of 2048 x 1280, 64 /
 // 96 / 128 assignments Q4_K 28 / 36 / 44 against 32, IQ4_XS 37 / 50 / 62 against 38; 128 of 2048 x 768, 128 / 192 /
 // 256 Q4_K 25 / 32 / 40 against 35, IQ4_XS 35 / 47 / 60 against 44; 256 of 1024 x 2048, 256 / 384 Q6_K 81 / 124
 // against 117.  From five assignments per expert on they are grouped.
@@ -1778,7 +1778,7 @@ bool grouping_pays(const fh_qmatrix& weight, uint32_t assignments, int cu_count)
     const bool idles = plan.segments * (uint32_t)(plan.bs * plan.it) * 2 >= nb * 3;
     const double bytes = (double)weight.rows * nb * block_bytes(weight.ggml_type);
     const double shares = std::max(1.0, (double)cu_count / (double)weight.experts);
-    return 9.0 + assignments * bytes / rates.each * (idles ? 1.2 : 1.0) > 16.5 + bytes / (shares * rates.share);
+    return 9.0 + assignments * bytes / rates.each * (idles ? 1.2 : 1.0) > 15.5 + bytes / (shares * rates.share);
 }
 
 fh_status expert_project(fh_device* device, const fh_qmatrix* weight, const fh_view* x, uint32_t x_rows,
