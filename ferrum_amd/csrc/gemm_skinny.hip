@@ -245,7 +245,7 @@ struct ResidentShared {
 // piece would chain up to twenty-four.  F32: the rows are f32 and rounded to f16 on the way, as
 // launch_round_to_f16 rounds them: a launch for the routed rows, one for the shared expert's and a
 // trip through memory less per projection (1600 routes of 200 tokens, 256 IQ4_XS experts: 116 us for
-// the three launches of a 1024 x 2048 projection, 70 of a 2048 x 512 one; 117 and 63 for one).
+// the three launches of a 1024 x 2048 projection, 70 of a 2048 x 512 one; 104 and 58 for one).
 template <bool F32>
 __device__ __forceinline__ void gather_rows(uint16_t* xs, const uint16_t* __restrict__ xsrc, uint32_t mt,
                                             uint32_t pieces, uint32_t k, uint32_t ld, uint32_t first_token,
