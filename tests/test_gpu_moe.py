@@ -248,16 +248,20 @@ def test_grouped_expert_projection_matches_the_oracle_and_the_direct_form(api, d
 
 
 @pytest.mark.parametrize("dtype", ["F16", "BF16"])
-@pytest.mark.parametrize("assignments,grouped", [(31, False), (32, False), (319, False), (320, True)])
+@pytest.mark.parametrize("assignments,grouped", [(31, False), (32, False), (319, False), (320, True), (385, True), (500, True), (508, True), (513, True)])
 def test_few_assignments_per_expert_are_projected_one_by_one(api, d, assignments, grouped, dtype):
     # 64 experts: up to five assignments each on average the per-assignment launch (exact weights),
-    # from there the grouped tiles (weights rounded to the row's type), each against its oracle
+    # from there the grouped tiles (weights rounded to the row's type), each against its oracle; in passes of 16
+    # rows at 500, of 32 at 508, with an expert of more than 16 rows on both sides
     experts, rows, cols = 64, 40, 512
     code = oracle.F16 if dtype == "F16" else oracle.BF16
     packed = synth.matrix(Q4_K, experts * rows, cols, seed=261)
     w = api.QuantizedExpertMatrix.new(d, packed, api.QuantizationFormat.Q4_K, experts, rows, cols)
     meta = np.zeros((assignments, 3), dtype=np.uint32)
-    meta[:, 0] = np.sort(synth.rng(262).integers(0, experts, assignments))
+    ids = synth.rng(262).integers(0, experts, assignments)
+    if assignments >= 500:
+        ids[:21] = 5
+    meta[:, 0] = np.sort(ids)
     meta[:, 1] = np.arange(assignments)
     meta[:, 2] = np.float32(1.0).view(np.uint32)
     x = oracle.round_storage(synth.activations(assignments, cols, seed=263) * 0.25, code).reshape(assignments, cols)
