@@ -624,6 +624,7 @@ fh_status fh_get_tuning(const fh_device* device, const char* key, int64_t* value
         return FH_OK;
     }
     if (std::strcmp(key, "held_pool_bytes") == 0) {
+        std::lock_guard<std::mutex> hold(device->pool_lock);
         *value = (int64_t)device->pool_bytes;
         return FH_OK;
     }

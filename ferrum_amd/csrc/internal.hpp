@@ -55,7 +55,7 @@ struct fh_device {
     // `stream`, so a block can be handed on at once; buffers whose address has left the library are freed.
     // Python may drop a buffer on any thread, and another device object on the same GPU that finds no memory
     // empties this one's pool: the pool has a lock.
-    std::mutex pool_lock;
+    mutable std::mutex pool_lock;
     std::multimap<size_t, void*> pool;
     size_t pool_bytes = 0;
     fh_device* next_live = nullptr;   // device objects that have not been destroyed (g_live in capi.hip)
