@@ -350,6 +350,7 @@ constexpr struct {
     {"gemm_min_rows", &fh_tuning::gemm_min_rows},
     {"gemm_wide_shape", &fh_tuning::gemm_wide_shape},
     {"gemm_wide32_tile", &fh_tuning::gemm_wide32_tile},
+    {"gemm_wide32_segments", &fh_tuning::gemm_wide32_segments},
     {"gemm_wide_min_rows", &fh_tuning::gemm_wide_min_rows},
     {"gemm_skinny_max_rows", &fh_tuning::gemm_skinny_max_rows},
     {"expert_grouped_min_assignments", &fh_tuning::expert_grouped_min_assignments},
@@ -900,6 +901,8 @@ GemmArgs gemm_args(const fh_device* device, uint32_t ggml_type, uint64_t n, uint
     g.wide_min_rows = (int)device->tuning.gemm_wide_min_rows;
     g.wide_shape = (int)device->tuning.gemm_wide_shape;
     g.wide32_tile = (int)device->tuning.gemm_wide32_tile;
+    g.wide32_segments = (int)device->tuning.gemm_wide32_segments;
+    g.cut_tiles = true;
     g.skinny_max_rows = (int)device->tuning.gemm_skinny_max_rows;
     g.resident_switch = device->tuning.gemm_resident != 0;
     g.rows_resident = g.resident_switch && expert_rows_fit_lds((uint32_t)k, 1, 1);
@@ -909,14 +912,25 @@ GemmArgs gemm_args(const fh_device* device, uint32_t ggml_type, uint64_t n, uint
 }
 
 // Brings the scratch to what the product needs behind `used` bytes of the caller's at its head.  Partial sums
-// only save time: where there is no room for them the few-rows plan is dropped.
+// only save time: where there is no room for them the product takes a kernel that needs fewer, at last one that
+// needs none.
 fh_status prepare_gemm(fh_device* device, GemmArgs& g, size_t used) {
     const size_t at = align256(used);
-    if (!scratch_available(device, at + g.rows_plan.partial_bytes)) g.rows_plan = RowsPlan{};
-    fh_status st = ensure_scratch(device, g.rows_plan.partial_bytes != 0 ? at + g.rows_plan.partial_bytes : used);
-    if (st == FH_ERR_ALLOCATION && g.rows_plan.partial_bytes != 0) {
-        g.rows_plan = RowsPlan{};
-        st = ensure_scratch(device, used);
+    fh_status st = FH_OK;
+    for (;;) {
+        const size_t partial_bytes = gemm_partial_bytes(g), need = partial_bytes != 0 ? at + partial_bytes : used;
+        if (partial_bytes == 0 || scratch_available(device, need)) {
+            st = ensure_scratch(device, need);
+            if (st != FH_ERR_ALLOCATION || partial_bytes == 0) break;
+        }
+        if (g.rows_plan.rows != 0) {
+            g.rows_plan = RowsPlan{};
+            if (g.x_dtype == FH_F32) return ensure_scratch(device, used);   // no tile takes exact f32 rows
+            if (!g.cut_tiles) g.few_rows = false;
+        } else {
+            g.cut_tiles = false;
+            gemm_takes_rows(g);
+        }
     }
     if (st != FH_OK) return st;
     g.counters = scratch_counters(device);

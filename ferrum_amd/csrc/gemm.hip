@@ -861,12 +861,16 @@ __device__ __forceinline__ void lds_direct16(const void* g, uint32_t lds_addr) {
     asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(a) : "memory");
 }
 
+// Where the tiles alone would leave part of the chip idle, K is cut into segments of `seg_blocks`
+// super-blocks each: segment s writes its f32 sums to plane s of y, which is then the scratch, and
+// add_segments_kernel adds the planes.
 template <uint32_t TYPE, int DT, int NT, int RT>
 __global__ __launch_bounds__(512) void gemm_wide32_kernel(const uint8_t* __restrict__ w,
                                                           const uint16_t* __restrict__ x,
                                                           void* __restrict__ y, uint32_t m, uint32_t n,
-                                                          uint32_t nb, uint32_t y_dtype, uint32_t cols,
-                                                          uint32_t tiles_m, uint32_t tiles_n) {
+                                                          uint32_t row_blocks, uint32_t seg_blocks, uint32_t y_dtype,
+                                                          uint32_t cols, uint32_t tiles_m, uint32_t tiles_n,
+                                                          uint32_t segments) {
     extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
     constexpr uint32_t kBlockBytes = block_bytes_of(TYPE);
     using Geo = Wide32<RT>;
@@ -875,28 +879,37 @@ __global__ __launch_bounds__(512) void gemm_wide32_kernel(const uint8_t* __restr
     constexpr bool kExtra = NT > 4;            // rows 128 .. 159 are a second decode task
 
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
-    // XCD-aware tile order: ids r, r+8, r+16, .. of a group share the XCD (id mod 8)
-    uint32_t tile_m, tile_n;
+    // XCD-aware order: workgroup ids that are equal mod 8 share an XCD, and XCD x takes the x-th eighth of the list
+    // (segment, column tile, row tile), row tiles fastest: those of a weight tile share it through that XCD's L2, and
+    // no XCD has more than one item above another (column tiles dealt over the XCDs one by one gave four of them 36
+    // of 240 items, a second round: 1024 x 2560 x 8192 in three segments 112 us, 73 dealt in eighths)
+    uint32_t tile_m, tile_n, segment;
     {
-        const uint32_t group_ids = 8 * tiles_m, id = blockIdx.x;
-        const uint32_t g = id / group_ids, r = id % group_ids;
-        tile_n = g * 8 + (r & 7u);
-        tile_m = r >> 3;
-        if (tile_n >= tiles_n) return;
+        const uint32_t items = tiles_m * tiles_n * segments, xcd = blockIdx.x & 7u, at = blockIdx.x >> 3;
+        const uint32_t begin = (uint32_t)((uint64_t)items * xcd >> 3), end = (uint32_t)((uint64_t)items * (xcd + 1) >> 3);
+        if (begin + at >= end) return;
+        const uint32_t item = begin + at, column = item / tiles_m;
+        tile_m = item - column * tiles_m;
+        segment = column / tiles_n;
+        tile_n = column - segment * tiles_n;
     }
     const uint32_t n0 = tile_n * cols, m0 = tile_m * Geo::kTileRows;
     const uint32_t ncols = n - n0 < cols ? n - n0 : cols;
-    const uint32_t k = nb << 8;
+    const uint32_t k = row_blocks << 8;
+    const uint32_t first = segment * seg_blocks, nb = min(seg_blocks, row_blocks - first);   // this segment's super-blocks
+    w += (size_t)first * kBlockBytes;
+    x += (size_t)first * 256;
+    if (segments > 1) y = static_cast<float*>(y) + (size_t)segment * m * n;
 
     if (wave >= 4) {
         // ---- producers: global -> registers -> (decode) -> LDS, blocks ahead ----
         const uint32_t pt = tid - 256, pw = wave - 4;
         const uint32_t wr = pt >> 1, wh = pt & 1u;
-        const uint8_t* wsrc = w + (size_t)(n0 + (wr < ncols ? wr : ncols - 1)) * nb * kBlockBytes;
+        const uint8_t* wsrc = w + (size_t)(n0 + (wr < ncols ? wr : ncols - 1)) * row_blocks * kBlockBytes;
         // rows 128 .. 159: every wave takes eight of them, a lane one quarter of a (row, half) task
         // of every slab, so all slabs cost the same
         const uint32_t er = 128 + 8 * pw + (lane >> 3), eh = (lane >> 2) & 1u, et = lane & 3u;
-        const uint8_t* esrc = w + (size_t)(n0 + (er < ncols ? er : ncols - 1)) * nb * kBlockBytes;
+        const uint8_t* esrc = w + (size_t)(n0 + (er < ncols ? er : ncols - 1)) * row_blocks * kBlockBytes;
         constexpr bool kDeep = !kEightDwords<TYPE>;   // Q6_K and Q8_0 sets are twice as large: one block ahead
         BlockW<TYPE> cur, n1, n2, ecur, en1, en2;
         const bool has_row = kRowsW >= 128 || wr < kRowsW;   // narrow tiles leave some decoding lanes without a row
@@ -1079,10 +1092,43 @@ __global__ __launch_bounds__(512) void gemm_wide32_kernel(const uint8_t* __restr
         }
 }
 
+// y[m, n] = the sum of `segments` planes of f32 partial sums, in segment order.  Four outputs a thread where `count`
+// is a multiple of four, which keeps 16-byte loads aligned in every plane.  A launch of its own and not the last
+// workgroup to arrive: that one would read the other segments' 40 to 160 KB tiles alone while the rest of the chip
+// has nothing left to do.
+template <int PER>
+__global__ __launch_bounds__(256) void add_segments_kernel(const float* __restrict__ partials, void* __restrict__ y,
+                                                           uint32_t segments, uint32_t count, uint32_t y_dtype) {
+    const uint32_t i = (blockIdx.x * 256 + threadIdx.x) * PER;
+    if (i >= count) return;
+    if constexpr (PER == 4) {
+        float4 sum = *reinterpret_cast<const float4*>(partials + i);
+        for (uint32_t s = 1; s < segments; ++s) {
+            const float4 v = *reinterpret_cast<const float4*>(partials + (size_t)s * count + i);
+            sum.x += v.x;
+            sum.y += v.y;
+            sum.z += v.z;
+            sum.w += v.w;
+        }
+        if (y_dtype == FH_F32) {
+            *reinterpret_cast<float4*>(static_cast<float*>(y) + i) = sum;
+        } else {
+            *reinterpret_cast<uint2*>(static_cast<uint16_t*>(y) + i) =
+                y_dtype == FH_F16 ? make_uint2(pack2<1>(sum.x, sum.y), pack2<1>(sum.z, sum.w))
+                                  : make_uint2(pack2<2>(sum.x, sum.y), pack2<2>(sum.z, sum.w));
+        }
+    } else {
+        float sum = partials[i];
+        for (uint32_t s = 1; s < segments; ++s) sum += partials[(size_t)s * count + i];
+        store_from_f32(y, i, y_dtype, sum);
+    }
+}
+
 struct WidePlan {
     int nt;
     uint32_t cols, tiles_m, tiles_n;
     int rt;   // 32x32x16 form: row tiles of 32 per multiplying wave (2: 256-row tile, 1: 128-row tile)
+    uint32_t segments, seg_blocks;   // 32x32x16 form: K segments
 };
 
 // Columns per workgroup: 128 or 136, whichever wastes the least of the chip's `cus`
@@ -1106,19 +1152,30 @@ WidePlan wide_plan(uint32_t m, uint32_t n, int cus) {
     return best;
 }
 
-// What a round of workgroups of one 32x32x16 tile takes over rows of 5120, in us: one workgroup per
-// compute unit (`alone`), or two where LDS and registers hold two, from the first pair
-// (`pair_first`) to a pair everywhere (`pair_all`; 0 = the tile runs alone).  Measured on
-// 17408 / 34816 / 8192 / 5120 columns at 48 - 2048 rows; two 128 x 128 tiles on a compute unit take
-// 88 - 108 us where one takes 64, so a pair does a fifth to a half more per microsecond.
+// What a launch of one 32x32x16 tile takes, in us: a start (launch, first loads, stores) and, per super-block of its K
+// segment, a time that depends on the format's decode and a little on how much of the chip is busy (`full`, times the
+// share of the compute units that have a workgroup); alone on their compute units, or two on some of them where LDS
+// and registers hold two.  Fitted to 4700 measurements: the five formats, twelve shapes from 1024 x 4096 to
+// 34816 x 5120, 40 - 1999 rows, one to eight segments; within 5% in the mean square, and the pick by it is on
+// average 0.4% and at most 10% slower than the fastest one.
+struct Wide32Cost {
+    double start, block[5], full;   // Q4_K, Q5_K, IQ4_XS, Q6_K, Q8_0
+};
 struct Wide32Tile {
     int rt, nt;
-    double alone, pair_first, pair_all;
+    Wide32Cost alone, pair;   // pair.start 0: one workgroup per compute unit
 };
 constexpr Wide32Tile kWide32Tiles[] = {
-    {1, 2, 49.0, 61.0, 71.0}, {1, 3, 58.6, 0.0, 0.0}, {1, 4, 64.0, 88.0, 108.0}, {1, 5, 79.0, 0.0, 0.0},
-    {2, 4, 90.0, 0.0, 0.0},   {2, 5, 108.0, 0.0, 0.0},
+    {1, 2, {5.9, {1.73, 1.96, 1.81, 2.24, 2.45}, 0.42}, {8.0, {2.59, 3.14, 2.99, 3.51, 3.57}, 0.18}},
+    {1, 3, {10.2, {2.27, 2.56, 2.36, 3.04, 3.44}, 0.0}, {}},
+    {1, 4, {10.2, {2.09, 2.46, 2.22, 2.99, 3.38}, 0.37}, {8.4, {3.98, 4.55, 4.31, 5.20, 5.78}, 0.35}},
+    {1, 5, {11.7, {2.65, 2.97, 2.75, 4.77, 5.03}, 0.40}, {}},
+    {2, 4, {13.1, {2.79, 3.06, 2.86, 3.51, 4.02}, 0.90}, {}},
+    {2, 5, {15.0, {3.33, 3.64, 3.50, 5.02, 5.28}, 1.09}, {}},
 };
+int cost_column(uint32_t ggml_type) {
+    return ggml_type == kQ4K ? 0 : ggml_type == kQ5K ? 1 : ggml_type == kIQ4XS ? 2 : ggml_type == kQ6K ? 3 : 4;
+}
 // an eighth of a tile's time is its prologue and its stores, the rest goes with the length of a row
 inline double wide_row_length_factor(uint32_t k) { return 0.125 + 0.875 * (double)k / 5120.0; }
 
@@ -1133,44 +1190,73 @@ WidePlan wide32_make(uint32_t m, uint32_t n, int rt, int nt, int cus = 256) {
     if (nt == 3) {
         const uint32_t per_row_tile = (uint32_t)cus / tiles_m;
         cols = per_row_tile == 0 ? 0 : ((n + per_row_tile - 1) / per_row_tile + 3u) & ~3u;
-        if (cols <= 64u || cols > 96u) return WidePlan{3, 96, tiles_m, 0, rt};
+        if (cols <= 64u || cols > 96u) return WidePlan{3, 96, tiles_m, 0, rt, 1, 0};
     }
-    return WidePlan{nt, cols, tiles_m, (n + cols - 1) / cols, rt};
+    return WidePlan{nt, cols, tiles_m, (n + cols - 1) / cols, rt, 1, 0};
 }
 
-double wide32_estimate(const Wide32Tile& t, uint64_t wgs, uint64_t cus) {
-    if (wgs <= cus) return t.alone;
-    if (t.pair_first == 0.0) return (double)((wgs + cus - 1) / cus) * t.alone;
+double wide32_estimate(const Wide32Tile& t, uint32_t ggml_type, uint32_t seg_blocks, uint64_t wgs, uint64_t cus) {
+    const auto round = [&](const Wide32Cost& c, double busy) {
+        return c.start + (double)seg_blocks * (c.block[cost_column(ggml_type)] + c.full * busy);
+    };
+    if (wgs <= cus) return round(t.alone, (double)wgs / (double)cus);
+    if (t.pair.start == 0.0) return (double)((wgs + cus - 1) / cus) * round(t.alone, 1.0);
     const uint64_t full = wgs / (2 * cus), rest = wgs % (2 * cus);
-    double us = (double)full * t.pair_all;
+    double us = (double)full * round(t.pair, 1.0);
     if (rest > cus) {
-        us += t.pair_first + (t.pair_all - t.pair_first) * (double)(rest - cus) / (double)cus;
+        us += round(t.pair, (double)(rest - cus) / (double)cus);
     } else if (rest > 0) {
-        us += full > 0 ? 0.66 * t.alone : t.alone;  // a last round of single workgroups starts while pairs still run
+        us += (full > 0 ? 0.66 : 1.0) * round(t.alone, 1.0);  // a last round of single workgroups starts while pairs still run
     }
     return us;
 }
 
-// The tile of the 32x32x16 form with the smallest estimate for this shape.  Tiles whose workgroups
-// would leave more than half the chip idle are left to the kernels made for few columns (nt = 0
-// when that holds for all of them).  At 17408 x 5120 that gives 128 x 64 up to 128 rows (61 us),
-// 128 x 160 up to 256 (78), 128 x 128 up to 384 (97), 256 x 160 beyond (111 at 512 rows), each
-// against the 16x16x32 form's 85 / 106 / 108 / 115 us; at 8192 x 4096 and 512 rows 128 x 128, 52
-// against 83 us.  Over 38 measured shapes the estimate picked the fastest tile every time.
-WidePlan wide32_plan(uint32_t m, uint32_t n, uint32_t k, int cus, double* estimate) {
+constexpr size_t kMostSegmentBytes = 48u << 20;   // scratch for partial sums: one round of the largest tile is 42 MB
+size_t segment_bytes(uint32_t m, uint32_t n, uint32_t segments) { return (size_t)segments * m * n * sizeof(float); }
+
+// Cuts K into exactly `segments` runs of super-blocks, none shorter than four (sixteen slabs); false: it does not go.
+bool wide32_cut(WidePlan& p, uint32_t k, uint32_t segments) {
+    const uint32_t nb = k / 256;
+    p.segments = segments;
+    p.seg_blocks = (nb + segments - 1) / segments;
+    return (nb + p.seg_blocks - 1) / p.seg_blocks == segments && (segments == 1 || nb / segments >= 4);
+}
+
+// The launch that adds the segments and what writing and reading their sums takes.
+double segments_us(uint32_t m, uint32_t n, uint32_t segments) {
+    return 2.5 + (double)segment_bytes(m, n, segments) * 0.28e-6;
+}
+
+// The tile of the 32x32x16 form, and its K segments, with the smallest estimate for this shape.  Tiles whose
+// workgroups would leave more than half the chip idle are left to the kernels made for few columns (nt = 0 when that
+// holds for all of them).  Uncut at 17408 x 5120: 128 x 128 up to 384 rows, 256 x 160 beyond (114 us at 512 rows; the
+// 16x16x32 form 115).  Cut, f16, us, against the best kernel for the whole of K:
+//   Q4_K 5120 x 17408   128 / 256 / 512 / 1024 rows  83.7 / 155 / 197 / 275 -> 49 / 72 / 116 / 203
+//   Q6_K 5120 x 17408                               133 / 184 / 229 / 396 -> 60 / 80 / 128 / 249
+//   Q4_K 2560 x 8192    128 / 256 / 512             31.9 / 91.9 / 71 -> 22.4 / 29.8 / 43
+//   Q4_K 17408 x 5120   128                         59.9 -> 50 (three segments of 128 x 128)
+WidePlan wide32_plan(uint32_t ggml_type, uint32_t m, uint32_t n, uint32_t k, int cus, uint32_t most_segments,
+                     double* estimate) {
     WidePlan best{};
     double best_us = 1e300;
     for (const Wide32Tile& t : kWide32Tiles) {
-        const WidePlan p = wide32_make(m, n, t.rt, t.nt, cus);
-        const uint64_t wgs = (uint64_t)p.tiles_m * p.tiles_n;
-        if (wgs * 2 < (uint64_t)cus) continue;
-        const double us = wide32_estimate(t, wgs, (uint64_t)cus);
-        if (us < best_us) {
-            best_us = us;
-            best = p;
+        WidePlan p = wide32_make(m, n, t.rt, t.nt, cus);
+        for (uint32_t segments = 1; segments <= most_segments; ++segments) {
+            if (!wide32_cut(p, k, segments)) continue;
+            const uint64_t wgs = (uint64_t)p.tiles_m * p.tiles_n * segments;
+            if (wgs * 2 < (uint64_t)cus) continue;
+            if (segments > 1 && (wgs > 2 * (uint64_t)cus || segment_bytes(m, n, segments) > kMostSegmentBytes)) break;
+            // (a cut has to gain a twentieth: uncut, a row's bits are the same in every tile)
+            const double us = segments == 1 ? wide32_estimate(t, ggml_type, p.seg_blocks, wgs, (uint64_t)cus)
+                                            : (wide32_estimate(t, ggml_type, p.seg_blocks, wgs, (uint64_t)cus) +
+                                               segments_us(m, n, segments)) * 1.05;
+            if (us < best_us) {
+                best_us = us;
+                best = p;
+            }
         }
     }
-    *estimate = best_us * wide_row_length_factor(k);
+    *estimate = best_us;
     return best;
 }
 
@@ -1200,7 +1286,7 @@ double resident_estimate(uint32_t ggml_type, uint32_t m, uint32_t n, uint32_t k)
     return 8.0 + heavier * weights * (0.047 + 0.09 * groups + (groups > 4 ? 0.08 : 0.0));
 }
 
-// What the heavier decodes add to the tiles' estimates, which were measured on Q4_K (at 512 rows of
+// What the heavier decodes add to the 16x16x32 form's estimate, which was measured on Q4_K (at 512 rows of
 // 17408 x 5120 112 us, Q5_K 117, IQ4_XS 115, Q6_K and Q8_0 141).
 double wide_format_factor(uint32_t ggml_type) {
     return ggml_type == kQ6K || ggml_type == kQ8_0 ? 1.22 : ggml_type == kQ4K ? 1.0 : 1.04;
@@ -1214,11 +1300,21 @@ void launch_wide32(hipStream_t s, const GemmArgs& a, const WidePlan& plan) {
         (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_wide32_kernel<TYPE, DT, NT, RT>),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     });
-    const uint32_t groups = (plan.tiles_n + 7) / 8;
-    dim3 grid(groups * 8 * plan.tiles_m);
+    const uint32_t items = plan.tiles_m * plan.tiles_n * plan.segments;
+    dim3 grid((items + 7) / 8 * 8);
+    const bool cut = plan.segments > 1;
     hipLaunchKernelGGL((gemm_wide32_kernel<TYPE, DT, NT, RT>), grid, dim3(512), lds, s,
-                       static_cast<const uint8_t*>(a.w), static_cast<const uint16_t*>(a.x), a.y, a.m, a.n,
-                       a.k / 256, a.y_dtype, plan.cols, plan.tiles_m, plan.tiles_n);
+                       static_cast<const uint8_t*>(a.w), static_cast<const uint16_t*>(a.x), cut ? a.partials : a.y, a.m, a.n,
+                       a.k / 256, plan.seg_blocks, cut ? (uint32_t)FH_F32 : a.y_dtype, plan.cols, plan.tiles_m, plan.tiles_n,
+                       plan.segments);
+    if (!cut) return;
+    const uint32_t count = a.m * a.n;
+    if (count % 4 == 0)
+        hipLaunchKernelGGL(add_segments_kernel<4>, dim3((count / 4 + 255) / 256), dim3(256), 0, s, a.partials, a.y,
+                           plan.segments, count, a.y_dtype);
+    else
+        hipLaunchKernelGGL(add_segments_kernel<1>, dim3((count + 255) / 256), dim3(256), 0, s, a.partials, a.y,
+                           plan.segments, count, a.y_dtype);
 }
 
 template <uint32_t TYPE, int DT, int NT>
@@ -1276,17 +1372,24 @@ TileChoice tile_choice(const GemmArgs& a) {
         if (a.wide32_tile != 0) {
             c.p32 = wide32_make(a.m, a.n, a.wide32_tile / 10, a.wide32_tile % 10, a.cu_count);
             if (c.p32.tiles_n == 0) c.p32 = wide32_make(a.m, a.n, 1, 4);   // no width of the 96-column tile fits this shape
+            if (!a.cut_tiles || a.wide32_segments < 2 || !wide32_cut(c.p32, a.k, (uint32_t)a.wide32_segments))
+                wide32_cut(c.p32, a.k, 1);
             c.us32 = 0.0;
         } else {
-            c.p32 = wide32_plan(a.m, a.n, a.k, a.cu_count, &c.us32);
+            // (the form asked for by name sums in one order at every row count: uncut)
+            const uint32_t most = !a.cut_tiles              ? 1u
+                                  : a.wide32_segments > 0 ? (uint32_t)a.wide32_segments
+                                  : a.wide_shape == 2     ? 1u
+                                                          : 8u;
+            c.p32 = wide32_plan(a.ggml_type, a.m, a.n, a.k, a.cu_count, most, &c.us32);
             if (c.p32.nt == 0 && a.wide_shape == 2 && c.wide_pays) {
                 c.p32 = wide32_make(a.m, a.n, 2, 5);
+                wide32_cut(c.p32, a.k, 1);
                 c.us32 = 0.0;
             }
         }
     }
     c.us16 = c.wide_pays && a.wide_shape != 2 ? wide16_estimate(a.m, a.n, a.k, a.cu_count) : 1e300;
-    c.us32 *= wide_format_factor(a.ggml_type);
     c.us16 *= wide_format_factor(a.ggml_type);
     return c;
 }
@@ -1307,7 +1410,9 @@ bool gemm_takes_rows(GemmArgs& a) {
     if (plan.counters > fh_device::kCounterWords) return false;
     if (!a.few_rows_always && a.resident_switch) {
         const TileChoice c = tile_choice(a);
-        double other = std::min(c.us32, c.us16);
+        // (a cut tile has to gain a sixth on a plan that needs no partial sums: 80 x 17408 x 5120 stays here, 55 us
+        // against 49)
+        double other = std::min(c.p32.segments > 1 && plan.segments == 1 ? c.us32 * 1.18 : c.us32, c.us16);
         if (a.rows_resident) other = std::min(other, resident_estimate(a.ggml_type, a.m, a.n, a.k));
         if (plan.estimate_us >= other) return false;
     } else if (!a.few_rows_always && a.m > (uint32_t)a.skinny_max_rows) {
@@ -1315,6 +1420,40 @@ bool gemm_takes_rows(GemmArgs& a) {
     }
     a.rows_plan = plan;
     return true;
+}
+
+namespace {
+
+// Rows that fit LDS for their whole length take the kernel that keeps them there and streams
+// the weights past them through registers: against the square tiles 1.4 - 2.2 times
+// (512 x 1024 x 2048: 11.5 against 22.8 us).
+// Rows longer than 2560 fit only 16 at a time, and every weight is then decoded M / 16 times:
+// that still wins up to 256 rows (256 x 5120 x 5120: 51 against 86 us) and loses at 512 (95
+// against 84 us).
+// From wide_min_rows rows on, the tiles of the 32x32x16 form compete: the smallest estimate
+// among them, the 16x16x32 form and the rows-resident kernel takes the call.
+bool takes_resident(const GemmArgs& a, const TileChoice& c) {
+    if (!a.rows_resident) return false;
+    const bool groups_of_32 = (size_t)32 * a.k * 2 <= 160u * 1024;
+    // (the estimates were measured on rows of 2048 and more; shorter ones keep the rule below)
+    if (c.p32.nt != 0 && (a.k >= 1024 || a.wide32_tile != 0))
+        return resident_estimate(a.ggml_type, a.m, a.n, a.k) < (c.us32 < c.us16 ? c.us32 : c.us16);
+    // Where the 256-row tile would pay, it is mostly empty below 256 rows while this kernel's
+    // cost grows with the row count: 65 x 17408 x 5120 takes 67 against 82 us and 128 rows
+    // 87 against 87; with groups of 32 (K = 2048) 128 rows take 30 against 41 us and 256
+    // rows 49 against 49.
+    return a.m <= (uint32_t)a.skinny_max_rows ? true
+           : c.wide_pays                      ? a.m <= (groups_of_32 ? 192u : 96u)
+                                              : groups_of_32 || a.m <= 256;
+}
+
+}  // namespace
+
+size_t gemm_partial_bytes(const GemmArgs& a) {
+    if (a.rows_plan.rows != 0) return a.rows_plan.partial_bytes;
+    const TileChoice c = tile_choice(a);
+    if (c.p32.nt == 0 || c.p32.segments == 1 || c.us16 < c.us32 || takes_resident(a, c)) return 0;
+    return segment_bytes(a.m, a.n, c.p32.segments);
 }
 
 const char* launch_gemm(hipStream_t s, const GemmArgs& a) {
@@ -1332,50 +1471,21 @@ const char* launch_gemm(hipStream_t s, const GemmArgs& a) {
     const bool wide_pays = choice.wide_pays;
     WidePlan p32 = choice.p32;
     const double us32 = choice.us32, us16 = choice.us16;
-    // Rows that fit LDS for their whole length take the kernel that keeps them there and streams
-    // the weights past them through registers: against the square tiles 1.4 - 2.2 times
-    // (512 x 1024 x 2048: 11.5 against 22.8 us).
-    // Rows longer than 2560 fit only 16 at a time, and every weight is then decoded M / 16 times:
-    // that still wins up to 256 rows (256 x 5120 x 5120: 51 against 86 us) and loses at 512 (95
-    // against 84 us).
-    // From wide_min_rows rows on, the tiles of the 32x32x16 form compete: the smallest estimate
-    // among them, the 16x16x32 form and the rows-resident kernel takes the call.
-    if (a.rows_resident) {
-        const bool few = a.m <= (uint32_t)a.skinny_max_rows;
-        const bool groups_of_32 = (size_t)32 * a.k * 2 <= 160u * 1024;
-        // Where the 256-row tile would pay, it is mostly empty below 256 rows while this kernel's
-        // cost grows with the row count: 65 x 17408 x 5120 takes 67 against 82 us and 128 rows
-        // 87 against 87; with groups of 32 (K = 2048) 128 rows take 30 against 41 us and 256
-        // rows 49 against 49.
-        bool take = few          ? true
-                    : wide_pays ? a.m <= (groups_of_32 ? 192u : 96u)
-                                : groups_of_32 || a.m <= 256;
-        // (the estimates were measured on rows of 2048 and more; shorter ones keep the rule above)
-        if (p32.nt != 0 && (a.k >= 1024 || a.wide32_tile != 0))
-            take = resident_estimate(a.ggml_type, a.m, a.n, a.k) < (us32 < us16 ? us32 : us16);
-        if (take) return launch_gemm_resident(s, a);
-    }
+    if (takes_resident(a, choice)) return launch_gemm_resident(s, a);
     if (p32.nt != 0 && us16 < us32) p32.nt = 0;
     if (wide_pays || p32.nt != 0) {
         const WidePlan plan = wide_plan(a.m, a.n, a.cu_count);
-        if (a.ggml_type == kQ4K) {
-            if (a.x_dtype == FH_F16) launch_wide_nt<kQ4K, 1>(s, a, plan, p32); else launch_wide_nt<kQ4K, 2>(s, a, plan, p32);
-            return "q4_k_gemm_mfma_m256";
+        const bool half = a.x_dtype == FH_F16;
+        switch (a.ggml_type) {
+            case kQ4K: half ? launch_wide_nt<kQ4K, 1>(s, a, plan, p32) : launch_wide_nt<kQ4K, 2>(s, a, plan, p32); break;
+            case kQ5K: half ? launch_wide_nt<kQ5K, 1>(s, a, plan, p32) : launch_wide_nt<kQ5K, 2>(s, a, plan, p32); break;
+            case kIQ4XS: half ? launch_wide_nt<kIQ4XS, 1>(s, a, plan, p32) : launch_wide_nt<kIQ4XS, 2>(s, a, plan, p32); break;
+            case kQ8_0: half ? launch_wide_nt<kQ8_0, 1>(s, a, plan, p32) : launch_wide_nt<kQ8_0, 2>(s, a, plan, p32); break;
+            default: half ? launch_wide_nt<kQ6K, 1>(s, a, plan, p32) : launch_wide_nt<kQ6K, 2>(s, a, plan, p32); break;
         }
-        if (a.ggml_type == kQ5K) {
-            if (a.x_dtype == FH_F16) launch_wide_nt<kQ5K, 1>(s, a, plan, p32); else launch_wide_nt<kQ5K, 2>(s, a, plan, p32);
-            return "q5_k_gemm_mfma_m256";
-        }
-        if (a.ggml_type == kIQ4XS) {
-            if (a.x_dtype == FH_F16) launch_wide_nt<kIQ4XS, 1>(s, a, plan, p32); else launch_wide_nt<kIQ4XS, 2>(s, a, plan, p32);
-            return "iq4_xs_gemm_mfma_m256";
-        }
-        if (a.ggml_type == kQ8_0) {
-            if (a.x_dtype == FH_F16) launch_wide_nt<kQ8_0, 1>(s, a, plan, p32); else launch_wide_nt<kQ8_0, 2>(s, a, plan, p32);
-            return "q8_0_gemm_mfma_m256";
-        }
-        if (a.x_dtype == FH_F16) launch_wide_nt<kQ6K, 1>(s, a, plan, p32); else launch_wide_nt<kQ6K, 2>(s, a, plan, p32);
-        return "q6_k_gemm_mfma_m256";
+        static const char* const names[5] = {"q4_k_gemm_mfma_m256", "q5_k_gemm_mfma_m256", "iq4_xs_gemm_mfma_m256",
+                                             "q6_k_gemm_mfma_m256", "q8_0_gemm_mfma_m256"};
+        return names[cost_column(a.ggml_type)];
     }
     // 128 x 128 tiles, or 64 x 64 when those would leave most of the chip idle
     const uint64_t big_wgs = (uint64_t)((a.n + kBN - 1) / kBN) * ((a.m + kBM - 1) / kBM);

@@ -22,6 +22,7 @@ struct fh_tuning {
     int64_t gemm_min_rows = 2;         // smallest M that takes the MFMA tile path
     int64_t gemm_wide_shape = 1;       // matrix instruction of the 128- and 256-row tiles: 0 = 16x16x32, 1 = whichever is estimated faster, 2 = 32x32x16
     int64_t gemm_wide32_tile = 0;      // 0 = by shape; 12, 14, 15 (128-row tile x 64, 128, 160 columns), 24, 25 (256-row tile)
+    int64_t gemm_wide32_segments = 0;  // K segments of the 32x32x16 form: 0 = by shape (a forced tile or form: uncut), else at most that many (a forced tile: exactly)
     int64_t gemm_wide_min_rows = 33;   // smallest M that takes the 256-row tile (it wins from there up)
     int64_t gemm_skinny_max_rows = 64; // with gemm_resident 0: largest M that takes the few-rows kernel (0 = never)
     int64_t expert_grouped_min_assignments = 32;  // fewest assignments grouped by expert (0 = never)
@@ -322,6 +323,8 @@ struct GemmArgs {
     int wide_min_rows;   // smallest M that takes the 256-row tile
     int wide_shape;      // matrix instruction of the 256-row tile: 0 = 16x16x32, 1 = 32x32x16 where it wins, 2 = always
     int wide32_tile;     // 0 = chosen by shape; else 10 x (row tiles per wave) + column tiles of the 32x32x16 form
+    int wide32_segments; // K segments of that form: 0 = by shape
+    bool cut_tiles;      // its partial sums have room in the scratch (`partials`)
     int skinny_max_rows; // largest M that takes the register-dequant kernel where the rows-resident one is switched off
     // routed-expert form of the register-dequant kernel: w is [experts, n, k],
     // x and y rows are assignments, m is their count; tokens of expert e are
@@ -349,7 +352,7 @@ struct GemmArgs {
     bool resident_switch; // rows_resident before the rows' length is looked at
     bool few_rows;        // the few-rows kernel may take the product (gemm_takes_rows)
     bool few_rows_always; // ... and does, whatever the estimates say
-    RowsPlan rows_plan;   // set by gemm_takes_rows; its K segments meet in these:
+    RowsPlan rows_plan;   // set by gemm_takes_rows; its K segments and the tiles' meet in these:
     float* partials;
     uint32_t* counters;
     bool weight_ring;     // routed form, rows resident: Q4_K and Q6_K weights through LDS rings where they fit beside the rows
@@ -358,6 +361,9 @@ const char* launch_gemm(hipStream_t s, const GemmArgs& a);
 // whether launch_gemm hands this product to the few-rows kernel: fills a.rows_plan, whose partial sums and
 // counters the caller then provides
 bool gemm_takes_rows(GemmArgs& a);
+
+// scratch for the partial sums of the kernel launch_gemm would run (0: its K is not cut)
+size_t gemm_partial_bytes(const GemmArgs& a);
 
 void launch_gemm_rows(hipStream_t s, const GemmArgs& a);   // gemm_rows.hip, by a.rows_plan
 

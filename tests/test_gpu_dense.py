@@ -675,6 +675,67 @@ def test_wide_gemm_on_the_32x32x16_instruction(api, d, ggml, dtype):
     assert_matmul_parity(results[25], other.tensor.to_f32(), "against the 16x16x32 tiles", l2_tol=2e-6)
 
 
+@pytest.mark.parametrize("ggml,m,n,k,segments", [
+    (12, 33, 4090, 16 * 256, 4), (14, 129, 1003, 17 * 256, 4), (13, 257, 600, 9 * 256, 2), (23, 128, 96, 32 * 256, 8),
+    (8, 300, 333, 13 * 256, 3), (12, 511, 1021, 33 * 256, 7)])
+@pytest.mark.parametrize("dtype,out", [("F16", "F32"), ("BF16", "BF16")])
+def test_tiles_whose_k_is_cut_into_segments(api, d, ggml, m, n, k, segments, dtype, out):
+    # every 32x32x16 tile with that many segments (the last one shorter), ragged rows and columns, outputs whose count
+    # is no multiple of four; against the tile-rounded oracle, and repeated with the same bits
+    packed = synth.matrix(ggml, n, k, seed=177)
+    w = qm(api, d, ggml, n, k, packed)
+    code = oracle.F16 if dtype == "F16" else oracle.BF16
+    x = oracle.round_storage(synth.activations(m, k, seed=178 + m), code).reshape(m, k)
+    xt = api.Tensor.from_f32(d, (m, k), getattr(api.DType, dtype), x)
+    rows = np.unique(np.concatenate([np.arange(0, 40), np.arange(n // 2, n // 2 + 30), np.arange(n - 40, n)]))
+    want = oracle_columns(ggml, packed, n, k, rows, x, weight_round=code, accumulate="f64")
+    try:
+        d.set_tuning("gemm_wide32_segments", segments)
+        for tile in (12, 13, 14, 15, 24, 25):
+            d.set_tuning("gemm_wide32_tile", tile)
+            got = d.project_quantized(xt, w, out_dtype=api.DType.F32)
+            assert got.operation.endswith("_gemm_mfma_m256")
+            assert_matmul_parity(got.tensor.to_f32()[:, rows], want, f"tile {tile}")
+            again = d.project_quantized(xt, w, out_dtype=getattr(api.DType, out)).tensor.to_f32()
+            stored = got.tensor.to_f32() if out == "F32" else oracle.round_storage(got.tensor.to_f32(), code).reshape(m, n)
+            assert np.array_equal(bits(again), bits(stored))
+    finally:
+        d.set_tuning("gemm_wide32_segments", 0)
+        d.set_tuning("gemm_wide32_tile", 0)
+
+
+def test_partial_sums_of_tiles_take_only_the_room_there_is(api):
+    # 512 x 5120 x 17408 in four segments: 42 MB of sums, which the scratch of a new device does not hold.  While it
+    # records the device takes another kernel; a plain call grows the scratch, and the recording stays what it was.
+    dev = api.Device.new()
+    m, n, k = 512, 5120, 17408
+    w = qm(api, dev, Q4_K, n, k, synth.matrix(Q4_K, n, k, seed=179))
+    x = api.Tensor.from_f32(dev, (m, k), api.DType.F16, synth.activations(m, k, seed=180, f16=True))
+    recorded = api.Tensor.zeros(dev, (m, n), api.DType.F32)
+    dev.synchronize()
+    held = dev.get_tuning("held_scratch_bytes")
+    with dev.execution() as ex:
+        dev.project_quantized(x, w, out=recorded)
+    ex.graph.launch()
+    dev.synchronize()
+    assert dev.get_tuning("held_scratch_bytes") == held
+    first = recorded.to_f32()
+    direct = dev.project_quantized(x, w, out_dtype=api.DType.F32).tensor.to_f32()
+    assert held < dev.get_tuning("held_scratch_bytes") <= 64 << 20
+    assert rel_l2(first, direct) <= 1e-5
+    for _ in range(2):
+        ex.graph.launch()
+        dev.synchronize()
+        assert np.array_equal(bits(recorded.to_f32()), bits(first))
+    again = api.Tensor.zeros(dev, (m, n), api.DType.F32)
+    with dev.execution() as cut:
+        dev.project_quantized(x, w, out=again)
+    for _ in range(3):
+        cut.graph.launch()
+        dev.synchronize()
+        assert np.array_equal(bits(again.to_f32()), bits(direct))
+
+
 @pytest.mark.parametrize("m", [80, 128, 200, 330, 512])
 def test_the_tile_picked_by_row_count_gives_the_bits_of_the_largest(api, d, m):
     # 17000 columns at every row count that changes the tile (128 x 68 of the 96-column tile up to
