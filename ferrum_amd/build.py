@@ -19,7 +19,7 @@ OBJ_DIR = os.path.join(HERE, "build")
 LIB_DIR = os.path.join(HERE, "lib")
 LIB_PATH = os.path.join(LIB_DIR, "libferrum_hip.so")
 
-SOURCES = ["capi.hip", "dequant.hip", "gemv.hip", "gemv_stream.hip", "probe.hip", "gemm.hip", "gemm_rows.hip",
+SOURCES = ["capi.hip", "dequant.hip", "gemv.hip", "gemv_stream.hip", "probe.hip", "gemm.hip", "gemm_pairs.hip", "gemm_rows.hip",
            "gemm_rows_q4_k.hip", "gemm_rows_q5_k.hip", "gemm_rows_q6_k.hip", "gemm_rows_iq4_xs.hip", "gemm_rows_q8_0.hip",
            "gemm_skinny.hip", "moe.hip", "norm.hip"]
 
@@ -90,6 +90,7 @@ def build(extra_flags: list[str] | None = None, jobs: int = 8, output: str | Non
         objs = list(pool.map(lambda s: _compile(s, extra), SOURCES))
         broken = [v for s, t in texts.items() for v in isa_check.violations(t.result(), s)]
         broken += [v for s, t in counted.items() for v in isa_check.counted_violations(t.result(), s)]
+        broken += [v for s in isa_check.HAND_ISSUED_SOURCES for v in isa_check.m0_violations(counted[s].result(), s)]
     if broken:
         raise RuntimeError("the generated code breaks an invariant of the hand-scheduled loads:\n" + "\n".join(broken[:40]))
     target = output or LIB_PATH

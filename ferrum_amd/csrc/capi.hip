@@ -1026,6 +1026,8 @@ fh_status project(fh_device* device, const fh_qmatrix* weight, const fh_view* x,
             (!g.few_rows_always && !gemv_streams(device, weight->ggml_type, n, k, m) &&
              !f32_rows_pay(g.rows_plan, g.ggml_type, g.n, g.k, m, g.cu_count)))
             g.rows_plan = RowsPlan{};
+        if (!g.few_rows_always && pairs_pay(g.ggml_type, g.n, g.k, m) && ((uintptr_t)xr.begin & 15u) == 0)
+            g.rows_plan = gemm_pairs_plan(g.n, g.k, g.m, g.cu_count);
     }
     if (tile) gemm_takes_rows(g);
     if (tile || g.rows_plan.rows != 0) {

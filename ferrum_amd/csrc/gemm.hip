@@ -1463,7 +1463,8 @@ const char* launch_gemm(hipStream_t s, const GemmArgs& a) {
              "q8_0_gemm_mfma_resident"},
             {"q4_k_gemm_mfma_skinny", "q5_k_gemm_mfma_skinny", "q6_k_gemm_mfma_skinny", "iq4_xs_gemm_mfma_skinny",
              "q8_0_gemm_mfma_skinny"}};
-        launch_gemm_rows(s, a);
+        if (a.rows_plan.pairs) launch_gemm_pairs(s, a);
+        else launch_gemm_rows(s, a);
         const int f = a.ggml_type == kQ4K ? 0 : a.ggml_type == kQ5K ? 1 : a.ggml_type == kQ6K ? 2 : a.ggml_type == kIQ4XS ? 3 : 4;
         return names[a.rows_resident || a.m > (uint32_t)a.skinny_max_rows ? 0 : 1][f];
     }

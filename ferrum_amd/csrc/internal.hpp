@@ -304,8 +304,10 @@ struct RowsPlan {
     uint32_t tiles;           // weight tiles of 16 rows per wave
     uint32_t tile_groups, segments, seg_blocks;
     size_t counters;          // scratch counter words of a launch (0: K is not cut)
-    size_t partial_bytes;     // scratch for its partial sums
+    size_t partial_bytes;     // scratch for its partial sums (and operands)
     double estimate_us;
+    bool pairs;               // f32 rows as pairs of f16 operands: gemm_pairs.hip
+    size_t operand_bytes;     // ... which come first in the scratch
 };
 RowsPlan gemm_rows_plan(uint32_t ggml_type, uint32_t n, uint32_t k, uint32_t m, uint32_t x_dtype, int cu_count);
 // whether that plan's kernel, and not the FMA GEMV once per row, takes m exact f32 rows
@@ -366,6 +368,12 @@ bool gemm_takes_rows(GemmArgs& a);
 size_t gemm_partial_bytes(const GemmArgs& a);
 
 void launch_gemm_rows(hipStream_t s, const GemmArgs& a);   // gemm_rows.hip, by a.rows_plan
+
+// gemm_pairs.hip: a batch of f32 rows on the f16 matrix instruction, exact integers times pairs of f16 values
+// (whether it, and not the few-rows kernel, takes m of them)
+bool pairs_pay(uint32_t ggml_type, uint32_t n, uint32_t k, uint32_t m);
+RowsPlan gemm_pairs_plan(uint32_t n, uint32_t k, uint32_t m, int cu_count);
+void launch_gemm_pairs(hipStream_t s, const GemmArgs& a);
 
 // gemm_skinny.hip
 const char* launch_gemm_skinny(hipStream_t s, const GemmArgs& a);

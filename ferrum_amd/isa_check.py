@@ -41,8 +41,9 @@ import re
 VALIDATED_HIPCC = "7.2.26015"
 
 CHECKED_SOURCES = ("gemm.hip", "gemv_stream.hip", "gemm_skinny.hip", "probe.hip")
-COUNTED_SOURCES = ("gemm_rows_q4_k.hip", "gemm_rows_q5_k.hip", "gemm_rows_q6_k.hip", "gemm_rows_iq4_xs.hip",
+COUNTED_SOURCES = ("gemm_pairs.hip", "gemm_rows_q4_k.hip", "gemm_rows_q5_k.hip", "gemm_rows_q6_k.hip", "gemm_rows_iq4_xs.hip",
                    "gemm_rows_q8_0.hip")
+HAND_ISSUED_SOURCES = ("gemm_pairs.hip",)   # counted, and their LDS-direct loads are asm statements
 
 _KERNEL_LABEL = re.compile(r"^(_Z\w+|\w+):\s*(;.*)?$")
 _VREG_RANGE = re.compile(r"\bv\[(\d+):(\d+)\]")
@@ -61,8 +62,9 @@ def _vregs(text: str) -> set[int]:
     return regs
 
 
-def _functions(asm: str):
-    """Yields (name, [(line number, instruction text, inside an asm statement)]) per function."""
+def _functions(asm: str, labels: bool = False):
+    """Yields (name, [(line number, instruction text, inside an asm statement)]) per function; with `labels`
+    the local labels are among the texts."""
     name, body, in_asm = None, [], False
     for number, raw in enumerate(asm.splitlines(), 1):
         line = raw.strip()
@@ -80,6 +82,8 @@ def _functions(asm: str):
             name, body = None, []
             continue
         if line.startswith("."):
+            if labels and name is not None and line.startswith(".LBB") and line.split(";")[0].strip().endswith(":"):
+                body.append((number, line.split(";")[0].strip(), False))
             continue
         label = _KERNEL_LABEL.match(line)
         if label and not line.startswith(".L"):
@@ -89,7 +93,7 @@ def _functions(asm: str):
             body.append((number, line.split(";")[0].strip(), in_asm))
 
 
-def violations(asm: str, source: str = "") -> list[str]:
+def violations(asm: str, source: str = "", counted: bool = False) -> list[str]:
     """Every break of the invariants in the module docstring found in `asm` (the text
     `hipcc -S --offload-device-only` writes for one source)."""
     found: list[str] = []
@@ -117,7 +121,8 @@ def violations(asm: str, source: str = "") -> list[str]:
                     found.append(f"{where}{number}: {name}: M0 is used outside an LDS-direct load statement: {text}")
             if in_asm and text.startswith("global_load_lds_"):
                 hand_loads = True
-                found.extend(_scan_to_wait(body, at, set(), name, where))
+                if not counted:
+                    found.extend(_scan_to_wait(body, at, set(), name, where))
             match = _REG_LOAD.match(text) if in_asm else None
             if match:
                 hand_loads = True
@@ -128,33 +133,53 @@ def violations(asm: str, source: str = "") -> list[str]:
 
 
 def counted_violations(asm: str, source: str = "") -> list[str]:
-    """Kernels whose LDS-direct loads the compiler issues: behind every run of them, up to the next
-    hand-placed wait in the text or the function's end, there must be at least as many loads into
-    registers as the hand-placed ``s_waitcnt vmcnt(n)`` of the kernel leaves outstanding."""
+    """Kernels that wait for LDS-direct loads by counting the register loads behind them: behind every run of the
+    former there must be at least as many of the latter as the next hand-placed ``s_waitcnt vmcnt(n)`` leaves
+    outstanding, along the text and along every branch back over the run."""
     found: list[str] = []
     where = (source + ":") if source else ""
-    for name, body in _functions(asm):
-        waits = [int(m.group(1)) for _, text, in_asm in body
-                 if in_asm and (m := re.match(r"s_waitcnt vmcnt\((\d+)\)", text))]
-        runs, current = [], None    # (line of the run's last LDS-direct load, loads behind it)
-        for number, text, in_asm in body:
-            if text.startswith("global_load_lds_"):
-                if current is not None and current[1] == 0:    # the run goes on
-                    current[0] = number
-                else:
-                    current = [number, 0]
-                    runs.append(current)
-            elif current is not None and in_asm and text.startswith("s_waitcnt vmcnt"):
-                current = None
-            elif current is not None and text.startswith("global_load_"):
-                current[1] += 1
-        if runs and not waits:
-            found.append(f"{where}{runs[0][0]}: {name}: LDS-direct loads without a hand-placed wait")
-        for number, behind in runs:
-            if waits and behind < max(waits):
-                found.append(f"{where}{number}: {name}: {behind} register loads follow this LDS-direct load, "
-                             f"the wait for it allows {max(waits)} outstanding")
+    for name, body in _functions(asm, labels=True):
+        at_label = {text[:-1]: at for at, (_, text, _) in enumerate(body) if text.endswith(":")}
+        waits = {at: int(m.group(1)) for at, (_, text, in_asm) in enumerate(body)
+                 if in_asm and (m := re.match(r"s_waitcnt vmcnt\((\d+)\)", text))}
+
+        def allowed_from(at):
+            return next((waits[w] for w in sorted(waits) if w >= at), None)
+
+        lds = [at for at, (_, text, _) in enumerate(body) if text.startswith("global_load_lds_")]
+        for at in lds:
+            number = body[at][0]
+            if not waits:
+                found.append(f"{where}{number}: {name}: LDS-direct loads without a hand-placed wait")
+                break
+            behind, needs, skip = 0, [], False
+            for here in range(at + 1, len(body)):
+                _, text, in_asm = body[here]
+                if text.startswith("global_load_lds_"):
+                    skip = behind == 0        # the run goes on: its last load counts
+                    if skip:
+                        break
+                if here in waits:
+                    needs.append((waits[here], behind))
+                    break
+                if text.startswith("global_load_") and not text.startswith("global_load_lds_"):
+                    behind += 1
+                target = text.split()[-1] if text.startswith(("s_cbranch", "s_branch")) else None
+                if target in at_label and at_label[target] < at:
+                    needs.append((allowed_from(at_label[target]), behind))
+            if skip:
+                continue
+            for allowed, behind in needs:
+                if allowed is not None and behind < allowed:
+                    found.append(f"{where}{number}: {name}: {behind} register loads follow this LDS-direct load, "
+                                 f"the wait for it allows {allowed} outstanding")
     return found
+
+
+def m0_violations(asm: str, source: str = "") -> list[str]:
+    """Of the invariants of ``violations``, those that do not depend on what else is in flight: M0 belongs to the
+    LDS-direct statements alone, and a kernel with such statements has no scratch."""
+    return violations(asm, source, counted=True)
 
 
 def _scan_to_wait(body, at, dst: set[int], name: str, where: str) -> list[str]:

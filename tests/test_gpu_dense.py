@@ -1359,3 +1359,62 @@ def test_a_batch_of_f32_rows_is_as_close_to_64_bits_as_its_chains_are_short(api,
     assert rel_l2(got, exact) <= 1.6e-7
     # the default is this kernel or, for Q4_K and Q5_K, a GEMV that is as close
     assert rel_l2(d.project_quantized(xt, w).tensor.to_f32(), exact) <= 1.6e-7
+
+
+@pytest.mark.parametrize("ggml", [12, 13, 14, 23], ids=["q4_k", "q5_k", "q6_k", "iq4_xs"])
+@pytest.mark.parametrize("m,n,k", [(17, 65601, 256), (20, 33000, 512), (32, 22003, 768), (33, 26315, 1280), (65, 2573, 6912), (49, 4099, 4352)])
+def test_f32_batches_as_pairs_of_f16(api, d, ggml, m, n, k):
+    """Rows of 1, 2, 3, 5, 17 and 27 super-blocks (a K half without one, an odd one out, K segments with a short last one),
+    ragged tiles and groups of rows, rows of very different magnitudes.  Against 64 bits: chains of at most eight matrix
+    steps and the adds behind them, which with the half unit an operand pair loses stay within the 1.6e-7 of the kernel
+    on the f32 instruction."""
+    packed = synth.matrix(ggml, n, k, seed=741)
+    w = qm(api, d, ggml, n, k, packed)
+    x = np.asarray(synth.activations(m, k, seed=742), dtype=np.float32).reshape(m, k)
+    x[1] *= 1e-25
+    x[2] *= 1e25
+    x[3, ::7] *= 1e4
+    x[4] = 0
+    x[5, : k // 2] = 0
+    xt = api.Tensor.from_f32(d, x.shape, api.DType.F32, x)
+    got = d.project_quantized(xt, w)
+    assert d.get_tuning("last_rows_plan") // 1000 == 32 or (33 <= m <= 48 and ggml == 14)
+    rows = np.unique(np.concatenate([np.arange(0, 160), np.arange(n - 160, n), synth.rng(743).integers(0, n, 200)]))
+    row_bytes = packed.size // n
+    weights = oracle.dequantize(ggml, np.ascontiguousarray(packed.reshape(n, row_bytes)[rows]).reshape(-1), len(rows), k)
+    want = x.astype(np.float64) @ weights.reshape(len(rows), k).astype(np.float64).T
+    out = got.tensor.to_f32()[:, rows]
+    assert not out[4].any()
+    for r in range(m):
+        if r != 4:
+            assert rel_l2(out[r], want[r]) <= 2.4e-7, r     # one row: the mean square over fewer outputs
+    live = [r for r in range(m) if r != 4]
+    size = np.linalg.norm(want[live], axis=1, keepdims=True)
+    assert rel_l2(out[live] / size, want[live] / size) <= 1.6e-7
+    assert np.array_equal(bits(d.project_quantized(xt, w).tensor.to_f32()), bits(got.tensor.to_f32()))
+    if d.get_tuning("last_rows_plan") // 1000 == 32 and not 33 <= m - 1 <= 48 and m > 17:    # a row's sums are its own
+        part = d.project_quantized(api.Tensor.from_f32(d, (m - 1, k), api.DType.F32, x[1:]), w).tensor.to_f32()
+        assert np.array_equal(bits(part), bits(got.tensor.to_f32()[1:]))
+    half = api.Tensor.zeros(d, (m, n), api.DType.F16)
+    d.project_quantized(xt, w, out=half)
+    assert np.array_equal(bits(half.to_f32()), bits(oracle.round_storage(got.tensor.to_f32(), oracle.F16).reshape(m, n)))
+
+
+@pytest.mark.parametrize("ggml", [12, 14], ids=["q4_k", "q6_k"])
+def test_f32_batches_with_infinities_and_nan(api, d, ggml):
+    # they reach the outputs that the products of the row as it is written give: the same ones as on the f32 instruction
+    m, n, k = 20, 2600, 6912
+    w = qm(api, d, ggml, n, k, synth.matrix(ggml, n, k, seed=751))
+    x = np.asarray(synth.activations(m, k, seed=752), dtype=np.float32).reshape(m, k)
+    x[2, 77], x[5, 900], x[7, 3], x[7, 6900], x[9, 4] = np.inf, np.nan, -np.inf, np.inf, 3e38
+    xt = api.Tensor.from_f32(d, x.shape, api.DType.F32, x)
+    got = d.project_quantized(xt, w).tensor.to_f32()
+    assert d.get_tuning("last_rows_plan") // 1000 == 32
+    with few_rows(d, 2):
+        want = d.project_quantized(xt, w).tensor.to_f32()
+        assert d.get_tuning("last_rows_plan") // 1000 == 16
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.isnan(want[5]).all()
+    inf = np.isinf(want)
+    assert np.array_equal(np.isinf(got), inf) and np.array_equal(got[inf], want[inf]) and inf[2].any()
+    fine = [r for r in range(m) if r not in (2, 5, 7, 9)]
+    assert rel_l2(got[fine], want[fine]) <= 2.6e-7
