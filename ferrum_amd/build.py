@@ -19,7 +19,8 @@ OBJ_DIR = os.path.join(HERE, "build")
 LIB_DIR = os.path.join(HERE, "lib")
 LIB_PATH = os.path.join(LIB_DIR, "libferrum_hip.so")
 
-SOURCES = ["capi.hip", "dequant.hip", "gemv.hip", "gemv_stream.hip", "probe.hip", "gemm.hip", "gemm_pairs.hip", "gemm_rows.hip",
+SOURCES = ["capi.hip", "dequant.hip", "gemv.hip", "gemv_stream.hip", "probe.hip", "gemm.hip", "gemm_pairs.hip", "gemm_decoded.hip",
+           "gemm_rows.hip",
            "gemm_rows_q4_k.hip", "gemm_rows_q5_k.hip", "gemm_rows_q6_k.hip", "gemm_rows_iq4_xs.hip", "gemm_rows_q8_0.hip",
            "gemm_skinny.hip", "moe.hip", "norm.hip"]
 

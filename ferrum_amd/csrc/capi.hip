@@ -351,6 +351,8 @@ constexpr struct {
     {"gemm_wide_shape", &fh_tuning::gemm_wide_shape},
     {"gemm_wide32_tile", &fh_tuning::gemm_wide32_tile},
     {"gemm_wide32_segments", &fh_tuning::gemm_wide32_segments},
+    {"gemm_decoded_min_rows", &fh_tuning::gemm_decoded_min_rows},
+    {"gemm_decoded_tile", &fh_tuning::gemm_decoded_tile},
     {"gemm_wide_min_rows", &fh_tuning::gemm_wide_min_rows},
     {"gemm_skinny_max_rows", &fh_tuning::gemm_skinny_max_rows},
     {"expert_grouped_min_assignments", &fh_tuning::expert_grouped_min_assignments},
@@ -902,6 +904,8 @@ GemmArgs gemm_args(const fh_device* device, uint32_t ggml_type, uint64_t n, uint
     g.wide_shape = (int)device->tuning.gemm_wide_shape;
     g.wide32_tile = (int)device->tuning.gemm_wide32_tile;
     g.wide32_segments = (int)device->tuning.gemm_wide32_segments;
+    g.decoded_min_rows = (int)device->tuning.gemm_decoded_min_rows;
+    g.decoded_tile = (int)device->tuning.gemm_decoded_tile;
     g.cut_tiles = true;
     g.skinny_max_rows = (int)device->tuning.gemm_skinny_max_rows;
     g.resident_switch = device->tuning.gemm_resident != 0;
@@ -923,7 +927,9 @@ fh_status prepare_gemm(fh_device* device, GemmArgs& g, size_t used) {
             st = ensure_scratch(device, need);
             if (st != FH_ERR_ALLOCATION || partial_bytes == 0) break;
         }
-        if (g.rows_plan.rows != 0) {
+        if (g.decoded_columns != 0) {
+            g.decoded_columns = 0;
+        } else if (g.rows_plan.rows != 0) {
             g.rows_plan = RowsPlan{};
             if (g.x_dtype == FH_F32) return ensure_scratch(device, used);   // no tile takes exact f32 rows
             if (!g.cut_tiles) g.few_rows = false;
@@ -1029,7 +1035,7 @@ fh_status project(fh_device* device, const fh_qmatrix* weight, const fh_view* x,
         if (!g.few_rows_always && pairs_pay(g.ggml_type, g.n, g.k, m) && ((uintptr_t)xr.begin & 15u) == 0)
             g.rows_plan = gemm_pairs_plan(g.n, g.k, g.m, g.cu_count);
     }
-    if (tile) gemm_takes_rows(g);
+    if (tile && !gemm_takes_rows(g)) gemm_takes_decoded(g);
     if (tile || g.rows_plan.rows != 0) {
         st = prepare_gemm(device, g, f32_tile ? (size_t)m * k * sizeof(uint16_t) : 0);
         if (st != FH_OK) return st;
@@ -1902,7 +1908,7 @@ fh_status expert_project(fh_device* device, const fh_qmatrix* weight, const fh_v
             ((uintptr_t)sxr.begin & 15u) != 0)
             return project(device, shared->weight, shared->x, shared->tokens, shared->y, true);
         GemmArgs g = gemm_args(device, weight->ggml_type, rows, k, shared->tokens, x->dtype, y->dtype);
-        gemm_takes_rows(g);
+        if (!gemm_takes_rows(g)) gemm_takes_decoded(g);
         st = prepare_gemm(device, g, (size_t)shared->tokens * k * sizeof(uint16_t));
         if (st != FH_OK) return st;
         launch_expert_silu_mul(device->stream, sxr.begin, scratch_data(device), shared->tokens, (uint32_t)k, x->dtype,

@@ -1449,7 +1449,13 @@ bool takes_resident(const GemmArgs& a, const TileChoice& c) {
 
 }  // namespace
 
+double gemm_fused_estimate(const GemmArgs& a) {
+    const TileChoice c = tile_choice(a);
+    return takes_resident(a, c) ? resident_estimate(a.ggml_type, a.m, a.n, a.k) : std::min(c.us32, c.us16);
+}
+
 size_t gemm_partial_bytes(const GemmArgs& a) {
+    if (a.decoded_columns != 0) return (size_t)(std::min(a.decoded_columns, a.n) + 31) / 32 * 32 * a.k * 2;
     if (a.rows_plan.rows != 0) return a.rows_plan.partial_bytes;
     const TileChoice c = tile_choice(a);
     if (c.p32.nt == 0 || c.p32.segments == 1 || c.us16 < c.us32 || takes_resident(a, c)) return 0;
@@ -1457,6 +1463,12 @@ size_t gemm_partial_bytes(const GemmArgs& a) {
 }
 
 const char* launch_gemm(hipStream_t s, const GemmArgs& a) {
+    static const char* const tile_names[5] = {"q4_k_gemm_mfma_m256", "q5_k_gemm_mfma_m256", "iq4_xs_gemm_mfma_m256",
+                                              "q6_k_gemm_mfma_m256", "q8_0_gemm_mfma_m256"};
+    if (a.decoded_columns != 0) {
+        launch_gemm_decoded(s, a);   // the same tiles, bit for bit
+        return tile_names[cost_column(a.ggml_type)];
+    }
     if (a.rows_plan.rows != 0) {
         static const char* const names[2][5] = {
             {"q4_k_gemm_mfma_resident", "q5_k_gemm_mfma_resident", "q6_k_gemm_mfma_resident", "iq4_xs_gemm_mfma_resident",
@@ -1484,9 +1496,7 @@ const char* launch_gemm(hipStream_t s, const GemmArgs& a) {
             case kQ8_0: half ? launch_wide_nt<kQ8_0, 1>(s, a, plan, p32) : launch_wide_nt<kQ8_0, 2>(s, a, plan, p32); break;
             default: half ? launch_wide_nt<kQ6K, 1>(s, a, plan, p32) : launch_wide_nt<kQ6K, 2>(s, a, plan, p32); break;
         }
-        static const char* const names[5] = {"q4_k_gemm_mfma_m256", "q5_k_gemm_mfma_m256", "iq4_xs_gemm_mfma_m256",
-                                             "q6_k_gemm_mfma_m256", "q8_0_gemm_mfma_m256"};
-        return names[cost_column(a.ggml_type)];
+        return tile_names[cost_column(a.ggml_type)];
     }
     // 128 x 128 tiles, or 64 x 64 when those would leave most of the chip idle
     const uint64_t big_wgs = (uint64_t)((a.n + kBN - 1) / kBN) * ((a.m + kBM - 1) / kBM);

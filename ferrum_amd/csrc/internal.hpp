@@ -23,6 +23,8 @@ struct fh_tuning {
     int64_t gemm_wide_shape = 1;       // matrix instruction of the 128- and 256-row tiles: 0 = 16x16x32, 1 = whichever is estimated faster, 2 = 32x32x16
     int64_t gemm_wide32_tile = 0;      // 0 = by shape; 12, 14, 15 (128-row tile x 64, 128, 160 columns), 24, 25 (256-row tile)
     int64_t gemm_wide32_segments = 0;  // K segments of the 32x32x16 form: 0 = by shape (a forced tile or form: uncut), else at most that many (a forced tile: exactly)
+    int64_t gemm_decoded_min_rows = 1; // products that decode their weights into the scratch first: 0 never, 1 where estimated faster, else from that many rows on
+    int64_t gemm_decoded_tile = 0;     // their tile: 0 = by shape; 192, 256 or 320 columns
     int64_t gemm_wide_min_rows = 33;   // smallest M that takes the 256-row tile (it wins from there up)
     int64_t gemm_skinny_max_rows = 64; // with gemm_resident 0: largest M that takes the few-rows kernel (0 = never)
     int64_t expert_grouped_min_assignments = 32;  // fewest assignments grouped by expert (0 = never)
@@ -327,6 +329,9 @@ struct GemmArgs {
     int wide32_tile;     // 0 = chosen by shape; else 10 x (row tiles per wave) + column tiles of the 32x32x16 form
     int wide32_segments; // K segments of that form: 0 = by shape
     bool cut_tiles;      // its partial sums have room in the scratch (`partials`)
+    int decoded_min_rows;      // rows from which the weights may be decoded once, in panels (0 = never)
+    int decoded_tile;          // columns of the product's tile: 0 = by shape (gemm_takes_decoded sets it)
+    uint32_t decoded_columns;  // set by gemm_takes_decoded: columns of a panel, which lies in `partials`
     int skinny_max_rows; // largest M that takes the register-dequant kernel where the rows-resident one is switched off
     // routed-expert form of the register-dequant kernel: w is [experts, n, k],
     // x and y rows are assignments, m is their count; tokens of expert e are
@@ -364,7 +369,11 @@ const char* launch_gemm(hipStream_t s, const GemmArgs& a);
 // counters the caller then provides
 bool gemm_takes_rows(GemmArgs& a);
 
-// scratch for the partial sums of the kernel launch_gemm would run (0: its K is not cut)
+// whether the weights are decoded into the scratch first, a panel of a.decoded_columns at a time (gemm_decoded.hip)
+bool gemm_takes_decoded(GemmArgs& a);
+void launch_gemm_decoded(hipStream_t s, const GemmArgs& a);
+double gemm_fused_estimate(const GemmArgs& a);   // us of the kernel that decodes as it multiplies; 1e300: none is estimated
+// scratch for the partial sums (or the panel) of the kernel launch_gemm would run (0: its K is not cut)
 size_t gemm_partial_bytes(const GemmArgs& a);
 
 void launch_gemm_rows(hipStream_t s, const GemmArgs& a);   // gemm_rows.hip, by a.rows_plan

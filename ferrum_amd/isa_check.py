@@ -40,7 +40,7 @@ import re
 # `hipcc --version` of the toolchain every kernel here was validated with on gfx950
 VALIDATED_HIPCC = "7.2.26015"
 
-CHECKED_SOURCES = ("gemm.hip", "gemv_stream.hip", "gemm_skinny.hip", "probe.hip")
+CHECKED_SOURCES = ("gemm.hip", "gemm_decoded.hip", "gemv_stream.hip", "gemm_skinny.hip", "probe.hip")
 COUNTED_SOURCES = ("gemm_pairs.hip", "gemm_rows_q4_k.hip", "gemm_rows_q5_k.hip", "gemm_rows_q6_k.hip", "gemm_rows_iq4_xs.hip",
                    "gemm_rows_q8_0.hip")
 HAND_ISSUED_SOURCES = ("gemm_pairs.hip",)   # counted, and their LDS-direct loads are asm statements

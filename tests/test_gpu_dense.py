@@ -1418,3 +1418,65 @@ def test_f32_batches_with_infinities_and_nan(api, d, ggml):
     assert np.array_equal(np.isinf(got), inf) and np.array_equal(got[inf], want[inf]) and inf[2].any()
     fine = [r for r in range(m) if r not in (2, 5, 7, 9)]
     assert rel_l2(got[fine], want[fine]) <= 2.6e-7
+
+
+@pytest.mark.parametrize("ggml", [12, 13, 14, 23, 8], ids=["q4_k", "q5_k", "q6_k", "iq4_xs", "q8_0"])
+@pytest.mark.parametrize("m,n,k,dtype", [(257, 33, 256, "F16"), (300, 1000, 512, "BF16"), (513, 2571, 1280, "F16"), (700, 517, 2304, "BF16")])
+def test_weights_decoded_first_give_the_bits_of_the_fused_tiles(api, d, ggml, m, n, k, dtype):
+    # one to nine super-blocks, ragged rows and columns, every tile of the product; and the fused tiles against the oracle
+    packed = synth.matrix(ggml, n, k, seed=761)
+    w = qm(api, d, ggml, n, k, packed)
+    code = oracle.F16 if dtype == "F16" else oracle.BF16
+    x = oracle.round_storage(synth.activations(m, k, seed=762), code).reshape(m, k)
+    xt = api.Tensor.from_f32(d, (m, k), getattr(api.DType, dtype), x)
+    try:
+        d.set_tuning("gemm_wide32_tile", 25)
+        want = d.project_quantized(xt, w, out_dtype=api.DType.F32)
+        d.set_tuning("gemm_wide32_tile", 0)
+        d.set_tuning("gemm_decoded_min_rows", 2)
+        for tile in (192, 256, 320):
+            d.set_tuning("gemm_decoded_tile", tile)
+            got = d.project_quantized(xt, w, out_dtype=api.DType.F32)
+            assert got.operation == want.operation
+            assert np.array_equal(bits(got.tensor.to_f32()), bits(want.tensor.to_f32())), tile
+            stored = d.project_quantized(xt, w).tensor.to_f32()
+            assert np.array_equal(bits(stored), bits(oracle.round_storage(got.tensor.to_f32(), code).reshape(m, n)))
+    finally:
+        d.set_tuning("gemm_wide32_tile", 0)
+        d.set_tuning("gemm_decoded_min_rows", 1)
+        d.set_tuning("gemm_decoded_tile", 0)
+    rows = np.unique(np.concatenate([np.arange(0, 20), np.arange(n - 20, n)]))
+    assert_matmul_parity(want.tensor.to_f32()[:, rows], oracle_columns(ggml, packed, n, k, rows, x, weight_round=code, accumulate="f64"),
+                         "fused tiles")
+
+
+def test_decoded_panels_take_only_the_room_there_is(api):
+    # 1100 x 70000 x 2048 is two panels of at most 256 MiB.  A new device that records has no room for one and takes the
+    # fused tiles, which give the same bits; once a plain call has made room, a recording decodes too.
+    dev = api.Device.new()
+    m, n, k = 1100, 70000, 2048
+    tile = synth.matrix(Q6_K, 80, k, seed=771)
+    w = qm(api, dev, Q6_K, n, k, np.tile(tile, n // 80))
+    x = api.Tensor.from_f32(dev, (m, k), api.DType.F16, synth.activations(m, k, seed=772, f16=True))
+    recorded = api.Tensor.zeros(dev, (m, n), api.DType.F16)
+    dev.synchronize()
+    held = dev.get_tuning("held_scratch_bytes")
+    with dev.execution() as ex:
+        dev.project_quantized(x, w, out=recorded)
+    ex.graph.launch()
+    dev.synchronize()
+    assert dev.get_tuning("held_scratch_bytes") == held
+    first = recorded.raw()
+    direct = dev.project_quantized(x, w)
+    assert 100 << 20 < dev.get_tuning("held_scratch_bytes") <= 257 << 20
+    assert rel_l2(direct.tensor.to_f32(), recorded.to_f32()) <= 1e-4
+    again = api.Tensor.zeros(dev, (m, n), api.DType.F16)
+    with dev.execution() as decoded:
+        dev.project_quantized(x, w, out=again)
+    for _ in range(3):
+        decoded.graph.launch()
+        ex.graph.launch()
+        dev.synchronize()
+        assert np.array_equal(again.raw(), direct.tensor.raw()) and np.array_equal(recorded.raw(), first)
+    got = direct.tensor.to_f32()
+    assert np.array_equal(bits(got[:, :80]), bits(got[:, -80:])) and np.array_equal(bits(got[:, :80]), bits(got[:, 35200:35280]))
