@@ -1070,9 +1070,10 @@ fh_status project(fh_device* device, const fh_qmatrix* weight, const fh_view* x,
         a.cu_count = device->props.multiProcessorCount;
         a.x_mode = silu_mul ? kXSiluMul : kXPlain;
         a.x_rows = m;
-        // One activated row stays on the FMA kernel: the streamed one's operands are f16 pairs and the matrix core
-        // keeps few bits of a subnormal weight (rel-L2 to 64 bits 1e-6 for Q6_K and 2e-6 to 1.4e-5 for Q4_K on
-        // rows of mean weights, against 1.0e-7 to 2.0e-7).  In it every workgroup activates the whole row again;
+        // One activated row stays on the FMA kernel: the streamed Q4_K one's operands are f16 pairs and the matrix core
+        // keeps few bits of a subnormal weight (rel-L2 to 64 bits 2e-6 to 1.4e-5 on rows of mean weights, against 1.0e-7
+        // to 2.0e-7).  The streamed Q6_K kernel sums integers and is the closer one for f32 rows (1.0e-7 against 2.0e-7; 16-bit rows
+        // 0.95e-7 on either): they take it from 200,000 super-blocks on (5120 x 17408 27.7 us on the FMA kernel, 24.7).  In it every workgroup activates the whole row again;
         // for large matrices the row is written out first, as the separate expert_silu_mul would, with the same
         // bits.  us, in place against written first: 5120 x 17408 26.5 / 20.6 (Q6_K 36.2 / 28.2), 5120 x 5120
         // 10.8 / 10.0 (15.3 / 13.1), 2048 x 12800 12.3 / 11.8 (16.1 / 14.7); 4096 x 4096, where the second launch
@@ -1080,9 +1081,10 @@ fh_status project(fh_device* device, const fh_qmatrix* weight, const fh_view* x,
         if (silu_mul && m == 1 && (weight->ggml_type == kQ4K || weight->ggml_type == kQ6K) && n * (k / 256) >= 81920u) {
             GemvArgs plain = a;
             plain.x_mode = kXPlain;
-            plain.stream = 0;
-            const GemvScratch need = gemv_scratch(plain);
-            const size_t partial_bytes = align256((size_t)need.segments * n * sizeof(float));
+            if (weight->ggml_type != kQ6K || x->dtype != FH_F32 || n * (k / 256) < 200000u) plain.stream = 0;
+            auto partials_of = [&] { return align256((size_t)gemv_scratch(plain).segments * n * sizeof(float)); };
+            if (!scratch_available(device, partials_of() + (size_t)k * dtype_bytes(x->dtype))) plain.stream = 0;   // fewer segments
+            const size_t partial_bytes = partials_of();
             const size_t bytes = partial_bytes + (size_t)k * dtype_bytes(x->dtype);
             if (scratch_available(device, bytes)) {
                 st = ensure_scratch(device, bytes);

@@ -27,6 +27,11 @@
 //     own registers.
 //   * Per super-block a lane applies the two 6-bit scales and minimums of its chunk
 //     and the block's d and dmin once.
+// Q6_K quants are bytes and go to v_mfma_i32_16x16x64_i8 against four 8-bit digits of 30-bit fixed-point activations
+// (stage_block_q6k): four matrix instructions per super-block where f16 parts of nibbles and bit planes took sixteen, some
+// 100 vector instructions for 180, and sums of integers in place of sums over f16 subnormals: rel-L2 to 64 bits
+// 0.9 - 1.1e-7, as the FMA kernel's for 16-bit rows (1.6 - 2.3e-7 for f32 ones; the f16 form's was 1e-6).  Cold,
+// 151936 x 5120 145 -> 134 us, 128256 x 4096 103 -> 97, 34816 x 5120 40.2 -> 37.4.
 //
 // Activations.  A super-block of a tile is multiplied by exactly one wave, so that wave
 // also turns the block's activations into A operands: it requests them before the
@@ -45,16 +50,18 @@ namespace {
 constexpr uint32_t kQ4Bytes = 144;
 constexpr uint32_t kQ6Bytes = 210;
 constexpr uint32_t kSlotBytes = 1024u + 64u + 16u;   // A operands, {group sum, group sum, 1/s, -} per chunk, 16 zero bytes
-// Q6_K: A operands, {four group sums, four 1/s} per lane group, 16 zero bytes
-constexpr uint32_t kSlot6Bytes = 1024u + 128u + 16u;
+// Q6_K: A operands, -32 times the digit sums of every scale group, the groups' scales, 16 zero bytes
+constexpr uint32_t kAux6Bytes = 256u + 64u;
+constexpr uint32_t kSlot6Bytes = 1024u + kAux6Bytes + 16u;
 template <uint32_t TYPE> struct StreamFormat;
 template <> struct StreamFormat<kQ4K> { static constexpr uint32_t kBytes = kQ4Bytes, kSlot = kSlotBytes, kAux = 64u; };
-template <> struct StreamFormat<kQ6K> { static constexpr uint32_t kBytes = kQ6Bytes, kSlot = kSlot6Bytes, kAux = 128u; };
+template <> struct StreamFormat<kQ6K> { static constexpr uint32_t kBytes = kQ6Bytes, kSlot = kSlot6Bytes, kAux = kAux6Bytes; };
 
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef int i32x4 __attribute__((ext_vector_type(4)));
 
 struct StreamParams {
     const uint8_t* w;     // [n, nb] super-blocks
@@ -129,36 +136,52 @@ __device__ __forceinline__ void stage_block(float4 v, uint8_t* slot, uint32_t la
     aux[2] = __uint_as_float((e - 14u) << 23);
 }
 
-// The same for a Q6_K super-block (the layout src/metal/shaders/ops.metal:1397-1425 indexes).
+// A Q6_K super-block's activations (the layout src/metal/shaders/ops.metal:1397-1425 indexes) as integers.
 // Weight 128 h + 32 s + 16 e + j (half h, slice s, j < 16) has its low four bits in
 // nibble s / 2 of ql[64 h + 32 (s & 1) + 16 e + j] and its high two in bits 2 s of
 // qh[32 h + 16 e + j]; lane group g = 2 h + e of the B operand holds those three 16-byte pieces,
-// four scale groups of 16 weights.  Step u = 2 (s & 1) + j / 8 multiplies eight bytes of a ql
-// piece: rows 4 g + 0 / 1 of A carry the hi / lo parts of the activations under the low nibbles
-// (slice s & 1), rows 4 g + 2 / 3 those under the high nibbles (slice 2 + (s & 1)), and the same
-// operand serves the two bit planes of qh that belong to those slices.  Lane L holds activations
-// 4 L .. 4 L + 3, so L = 32 h + 8 s + 4 e + j / 4: a quad of lanes is one scale group, which gets
-// a power-of-two scale of its own.
+// four scale groups of 16 weights.  Lane L holds activations 4 L .. 4 L + 3, so L = 32 h + 8 s + 4 e + j / 4: a
+// quad of lanes is one scale group, which gets a power of two of its own: x 2^k = X, |X| < 2^30, and X = d0 + 256 d1 +
+// 65536 d2 + 2^24 d3 with digits of a signed byte.  Row 4 g + i of the A operand is digit i of lane group g's sixteen
+// activations, zero elsewhere, so one v_mfma_i32_16x16x64_i8 gives a lane the four exact digit sums of its scale group.
+// The quants go in as 0 .. 63: the accumulator starts from -32 times the digits' plain sums.
 __device__ __forceinline__ void stage_block_q6k(float4 v, uint8_t* slot, uint32_t lane) {
     uint32_t top = __float_as_uint(fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
+    // (fmaxf drops a NaN beside a number: the comparison below is made on the bits)
+    const uint32_t bits = max(max(__float_as_uint(v.x) << 1, __float_as_uint(v.y) << 1),
+                              max(__float_as_uint(v.z) << 1, __float_as_uint(v.w) << 1)) >> 1;
+    top = max(top, bits);
     top = dpp_umax<0xB1>(top);
     top = dpp_umax<0x4E>(top);
-    uint32_t ex = top >> 23;
-    ex = ex < 15u ? 15u : ex > 254u ? 254u : ex;
-    const float s = __uint_as_float((268u - ex) << 23);
-    const uint32_t h02 = hi_pair(v.x, v.z, s), h13 = hi_pair(v.y, v.w, s);
-    const uint32_t l02 = lo_pair(v.x, v.z, s, h02), l13 = lo_pair(v.y, v.w, s, h13);
-    const uint32_t h = lane >> 5, sl = (lane >> 3) & 3u, e = (lane >> 2) & 1u, up = (lane >> 1) & 1u;
-    const uint32_t g = 2u * h + e, u = 2u * (sl & 1u) + up, i = 2u * (sl >> 1);
-    uint8_t* const dst = slot + ((u * 4u + g) * 4u + i) * 16u + 8u * (lane & 1u);
-    *reinterpret_cast<uint2*>(dst) = make_uint2(h02, h13);
-    *reinterpret_cast<uint2*>(dst + 16) = make_uint2(l02, l13);
-    float sum = (v.x + v.y) + (v.z + v.w);
-    sum = dpp_add<0xB1>(sum);
-    sum = dpp_add<0x4E>(sum);   // the four lanes of a scale group now all hold its sum
-    float* const aux = reinterpret_cast<float*>(slot + 1024u) + 8u * g;
-    aux[sl] = sum;
-    aux[4u + sl] = __uint_as_float((ex - 14u) << 23);
+    const uint32_t ex = min(top >> 23, 254u);
+    const int shift = 156 - (int)ex;
+    const float e[4] = {v.x, v.y, v.z, v.w};
+    uint32_t z[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)   // (adding 128 to the lower three digits makes them unsigned bytes; the xor takes it back)
+        z[i] = ((uint32_t)(int)__builtin_ldexpf(e[i], shift) + 0x00808080u) ^ 0x00808080u;
+    const uint32_t h = lane >> 5, sl = (lane >> 3) & 3u, ee = (lane >> 2) & 1u, g = 2u * h + ee;
+    uint32_t* const dst = reinterpret_cast<uint32_t*>(slot + ((sl * 4u + g) * 4u) * 16u) + (lane & 3u);
+    // digit i of the four, side by side
+    const uint32_t a01 = __builtin_amdgcn_perm(z[1], z[0], 0x05010400u), a23 = __builtin_amdgcn_perm(z[3], z[2], 0x05010400u);
+    const uint32_t b01 = __builtin_amdgcn_perm(z[1], z[0], 0x07030602u), b23 = __builtin_amdgcn_perm(z[3], z[2], 0x07030602u);
+    const uint32_t digit[4] = {__builtin_amdgcn_perm(a23, a01, 0x05040100u), __builtin_amdgcn_perm(a23, a01, 0x07060302u),
+                               __builtin_amdgcn_perm(b23, b01, 0x05040100u), __builtin_amdgcn_perm(b23, b01, 0x07060302u)};
+    int sums[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        dst[4 * i] = digit[i];
+        int t = __builtin_amdgcn_sdot4((int)digit[i], (int)0xe0e0e0e0u, 0, false);   // -32 each
+        t += __builtin_amdgcn_update_dpp(0, t, 0xB1, 0xf, 0xf, false);
+        t += __builtin_amdgcn_update_dpp(0, t, 0x4E, 0xf, 0xf, false);
+        sums[i] = t;
+    }
+    // (every lane of the quad writes the same values)
+    *reinterpret_cast<int4*>(slot + 1024u + (g * 4u + sl) * 16u) = make_int4(sums[0], sums[1], sums[2], sums[3]);
+    // 2^(ex - 140): what undoes the shift, in units of 65536; a subnormal for the smallest.  NaN where the group has an
+    // infinity or a NaN
+    const uint32_t undo = top >= 0x7f800000u ? 0x7fc00000u : ex > 13u ? (ex - 13u) << 23 : 1u << (ex + 9u);
+    reinterpret_cast<uint32_t*>(slot + 1024u + 256u)[g * 4u + sl] = undo;
 }
 
 // 16 or 8 bytes of a tile in LDS that are only 2-byte aligned (Q6_K blocks are 210 bytes long)
@@ -171,6 +194,60 @@ __device__ __forceinline__ uint2 lds_u2_unaligned(const uint8_t* p) {
     uint2 v;
     __builtin_memcpy(&v, p, 8);
     return v;
+}
+
+// A lane's share of one super-block, chunk g of its row against the operands of stage_block, added to acc.
+__device__ __forceinline__ float multiply_q4k(const u32x4 (&xa)[4], float4 aux, uint4 hdr, uint4 qa, uint4 qb, uint32_t g, float acc) {
+    const uint32_t raw[8] = {qa.x, qa.y, qa.z, qa.w, qb.x, qb.y, qb.z, qb.w};
+    floatx4 dl = {0.f, 0.f, 0.f, 0.f}, dh = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const uint32_t q0 = raw[2 * u], q1 = raw[2 * u + 1];
+        const uint32_t s0 = q0 >> 8, s1 = q1 >> 8;
+        const u32x4 lo = {q0 & 0x000f000fu, s0 & 0x000f000fu, q1 & 0x000f000fu, s1 & 0x000f000fu};
+        const u32x4 hi = {q0 & 0x00f000f0u, s0 & 0x00f000f0u, q1 & 0x00f000f0u, s1 & 0x00f000f0u};
+        const half8 a = __builtin_bit_cast(half8, xa[u]);
+        dl = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, __builtin_bit_cast(half8, lo), dl, 0, 0, 0);
+        dh = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, __builtin_bit_cast(half8, hi), dh, 0, 0, 0);
+    }
+    float sc_lo, sc_hi, mn_lo, mn_hi;
+    q4k_chunk_scales(hdr.y, hdr.z, hdr.w, g, sc_lo, sc_hi, mn_lo, mn_hi);
+    const float d = f16_bits_to_f32(hdr.x & 0xffffu), dmin = f16_bits_to_f32(hdr.x >> 16);
+    // low nibbles were q * 2^-24, high nibbles 16 q * 2^-24
+    const float dots = fmaf(sc_lo * 16777216.f, dl[0] + dl[1], (sc_hi * 1048576.f) * (dh[2] + dh[3]));
+    const float mins = fmaf(mn_lo, aux.x, mn_hi * aux.y);
+    return fmaf(d * aux.z, dots, fmaf(-dmin, mins, acc));
+}
+
+// The same for Q6_K: the lane group's pieces qa, qb, qh, its half's eight scales and the block's scale; dots starts
+// from stage_block_q6k's sums.
+__device__ __forceinline__ float multiply_q6k(const u32x4 (&xa)[4], i32x4 (&dots)[4], float4 undo, uint4 qa, uint4 qb, uint4 qh, uint2 sc8,
+                                              uint16_t dbits, uint32_t e, float acc) {
+    const uint32_t ql[8] = {qa.x, qa.y, qa.z, qa.w, qb.x, qb.y, qb.z, qb.w};
+    const uint32_t ph[4] = {qh.x, qh.y, qh.z, qh.w};
+    i32x4 q[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        q[0][u] = (int)((ql[u] & 0x0f0f0f0fu) | ((ph[u] << 4) & 0x30303030u));
+        q[1][u] = (int)((ql[4 + u] & 0x0f0f0f0fu) | ((ph[u] << 2) & 0x30303030u));
+        q[2][u] = (int)(((ql[u] >> 4) & 0x0f0f0f0fu) | (ph[u] & 0x30303030u));
+        q[3][u] = (int)(((ql[4 + u] >> 4) & 0x0f0f0f0fu) | ((ph[u] >> 2) & 0x30303030u));
+    }
+    float r[4];
+    const float scale[4] = {undo.x, undo.y, undo.z, undo.w};
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+        dots[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(i32x4, xa[t]), q[t], dots[t], 0, 0, 0);
+        // a digit's sum is at most 2^16: two of them fit 32 bits and make one f32
+        const float upper = (float)((dots[t][3] << 8) + dots[t][2]), lower = (float)((dots[t][1] << 8) + dots[t][0]);
+        r[t] = fmaf(lower, 1.f / 65536.f, upper) * scale[t];
+    }
+    // the lane group's int8 scales: bytes e, e + 2, e + 4, e + 6 of its half's eight
+    const uint32_t lo = sc8.x >> (8u * e), hi = sc8.y >> (8u * e);
+    const float c0 = (float)(int)(int8_t)lo, c1 = (float)(int)(int8_t)(lo >> 16);
+    const float c2 = (float)(int)(int8_t)hi, c3 = (float)(int)(int8_t)(hi >> 16);
+    const float total = fmaf(c0, r[0], c1 * r[1]) + fmaf(c2, r[2], c3 * r[3]);
+    return fmaf(f16_bits_to_f32(dbits), total, acc);
 }
 
 // LDS map (bytes): [tile: tile_rows x row_stride][a slot per wave][row sums: waves x 16 f32]
@@ -331,28 +408,12 @@ __device__ __forceinline__ void gemv_stream_body(const StreamParams& p) {
                     asm volatile("s_waitcnt lgkmcnt(3)" ::: "memory");   // the five slot reads are the oldest
                     stage(xv[i + 1], slot, lane);
                 }
-                const uint32_t raw[8] = {qa.x, qa.y, qa.z, qa.w, qb.x, qb.y, qb.z, qb.w};
-                floatx4 dl = {0.f, 0.f, 0.f, 0.f}, dh = {0.f, 0.f, 0.f, 0.f};
-    #pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    const uint32_t q0 = raw[2 * u], q1 = raw[2 * u + 1];
-                    const uint32_t s0 = q0 >> 8, s1 = q1 >> 8;
-                    const u32x4 lo = {q0 & 0x000f000fu, s0 & 0x000f000fu, q1 & 0x000f000fu, s1 & 0x000f000fu};
-                    const u32x4 hi = {q0 & 0x00f000f0u, s0 & 0x00f000f0u, q1 & 0x00f000f0u, s1 & 0x00f000f0u};
-                    const half8 a = __builtin_bit_cast(half8, xa[u]);
-                    dl = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, __builtin_bit_cast(half8, lo), dl, 0, 0, 0);
-                    dh = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, __builtin_bit_cast(half8, hi), dh, 0, 0, 0);
-                }
-                float sc_lo, sc_hi, mn_lo, mn_hi;
-                q4k_chunk_scales(hdr.y, hdr.z, hdr.w, g, sc_lo, sc_hi, mn_lo, mn_hi);
-                const float d = f16_bits_to_f32(hdr.x & 0xffffu), dmin = f16_bits_to_f32(hdr.x >> 16);
-                // low nibbles were q * 2^-24, high nibbles 16 q * 2^-24
-                const float dots = fmaf(sc_lo * 16777216.f, dl[0] + dl[1], (sc_hi * 1048576.f) * (dh[2] + dh[3]));
-                const float mins = fmaf(mn_lo, aux.x, mn_hi * aux.y);
-                acc = fmaf(d * aux.z, dots, fmaf(-dmin, mins, acc));
+                acc = multiply_q4k(xa, aux, hdr, qa, qb, g, acc);
             } else {
-                const float4 sums = *reinterpret_cast<const float4*>(auxp);
-                const float4 inv = *reinterpret_cast<const float4*>(auxp + 4);
+                i32x4 dots[4];   // of the four scale groups, from -32 times the digits' sums
+#pragma unroll
+                for (int t = 0; t < 4; ++t) dots[t] = *reinterpret_cast<const i32x4*>(slot + 1024u + (g * 4u + t) * 16u);
+                const float4 undo = *reinterpret_cast<const float4*>(slot + 1024u + 256u + 16u * g);
                 asm volatile("" ::: "memory");   // the slot reads are issued before the tile reads
                 const uint8_t* const blk = wrow + b * kBlock;
                 const uint32_t h = g >> 1, e = g & 1u;
@@ -363,60 +424,11 @@ __device__ __forceinline__ void gemv_stream_body(const StreamParams& p) {
                 uint16_t dbits;
                 __builtin_memcpy(&dbits, blk + 208u, 2);
                 if (i + 1 < MAXB && b + kSWaves < nb) {
-                    // the six slot reads are the oldest; at least five instructions read the tile
+                    // the nine slot reads are the oldest; at least five instructions read the tile
                     asm volatile("s_waitcnt lgkmcnt(5)" ::: "memory");
                     stage(xv[i + 1], slot, lane);
                 }
-                const uint32_t ql[8] = {qa.x, qa.y, qa.z, qa.w, qb.x, qb.y, qb.z, qb.w};
-                const uint32_t ph[4] = {qh.x, qh.y, qh.z, qh.w};
-                // [piece][low nibbles, high nibbles, their bit planes]
-                floatx4 dn[2][4];
-#pragma unroll
-                for (int pc = 0; pc < 2; ++pc)
-#pragma unroll
-                    for (int t = 0; t < 4; ++t) dn[pc][t] = floatx4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int up = 0; up < 2; ++up) {
-                    const uint32_t p0 = ph[2 * up], p1 = ph[2 * up + 1];
-                    const uint32_t t0 = p0 >> 8, t1 = p1 >> 8;
-#pragma unroll
-                    for (int pc = 0; pc < 2; ++pc) {
-                        const uint32_t q0 = ql[4 * pc + 2 * up], q1 = ql[4 * pc + 2 * up + 1];
-                        const uint32_t s0 = q0 >> 8, s1 = q1 >> 8;
-                        // Bit planes 0 and 2 belong to the first ql piece, 1 and 3 to the second.  The matrix
-                        // core's sum keeps a fixed number of bits below the operands' exponent field, which is
-                        // the same for every subnormal, so what a dot product loses does not depend on where
-                        // in the field the bits sit, while the factor that undoes the position does: planes 0
-                        // and 1, whose values count sixteenfold, move to the top of the field (bits 8..9).
-                        const uint32_t mh = pc == 0 ? 0x00300030u : 0x00c000c0u;
-                        const u32x4 nl = {q0 & 0x000f000fu, s0 & 0x000f000fu, q1 & 0x000f000fu, s1 & 0x000f000fu};
-                        const u32x4 nh = {q0 & 0x00f000f0u, s0 & 0x00f000f0u, q1 & 0x00f000f0u, s1 & 0x00f000f0u};
-                        const u32x4 pl = pc == 0 ? u32x4{(p0 << 8) & 0x03000300u, p0 & 0x03000300u, (p1 << 8) & 0x03000300u,
-                                                         p1 & 0x03000300u}
-                                                 : u32x4{(p0 << 6) & 0x03000300u, (p0 >> 2) & 0x03000300u,
-                                                         (p1 << 6) & 0x03000300u, (p1 >> 2) & 0x03000300u};
-                        const u32x4 pw = {p0 & mh, t0 & mh, p1 & mh, t1 & mh};
-                        const half8 a = __builtin_bit_cast(half8, xa[2 * pc + up]);
-                        dn[pc][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, __builtin_bit_cast(half8, nl), dn[pc][0], 0, 0, 0);
-                        dn[pc][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, __builtin_bit_cast(half8, nh), dn[pc][1], 0, 0, 0);
-                        dn[pc][2] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, __builtin_bit_cast(half8, pl), dn[pc][2], 0, 0, 0);
-                        dn[pc][3] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, __builtin_bit_cast(half8, pw), dn[pc][3], 0, 0, 0);
-                    }
-                }
-                // The operands were (times 2^-24): low nibble q, high nibble 16 q, planes 0 and 1 256 v, plane 2
-                // 16 v, plane 3 64 v; a weight is q + 16 v - 32.  Slices 0 and 2 come from the first piece.
-                const float s0q = fmaf(16.f, dn[0][0][0] + dn[0][0][1], dn[0][2][0] + dn[0][2][1]) * 1048576.f;
-                const float s2q = fmaf(16.f, dn[0][3][2] + dn[0][3][3], dn[0][1][2] + dn[0][1][3]) * 1048576.f;
-                const float s1q = fmaf(16.f, dn[1][0][0] + dn[1][0][1], dn[1][2][0] + dn[1][2][1]) * 1048576.f;
-                const float s3q = fmaf(4.f, dn[1][3][2] + dn[1][3][3], dn[1][1][2] + dn[1][1][3]) * 1048576.f;
-                // the lane group's int8 scales: bytes e, e + 2, e + 4, e + 6 of its half's eight
-                const uint32_t lo = sc8.x >> (8u * e), hi = sc8.y >> (8u * e);
-                const float c0 = (float)(int)(int8_t)lo, c1 = (float)(int)(int8_t)(lo >> 16);
-                const float c2 = (float)(int)(int8_t)hi, c3 = (float)(int)(int8_t)(hi >> 16);
-                const float r0 = fmaf(s0q, inv.x, -32.f * sums.x), r1 = fmaf(s1q, inv.y, -32.f * sums.y);
-                const float r2 = fmaf(s2q, inv.z, -32.f * sums.z), r3 = fmaf(s3q, inv.w, -32.f * sums.w);
-                const float total = fmaf(c0, r0, c1 * r1) + fmaf(c2, r2, c3 * r3);
-                acc = fmaf(f16_bits_to_f32(dbits), total, acc);
+                acc = multiply_q6k(xa, dots, undo, qa, qb, qh, sc8, dbits, e, acc);
             }
         }
     }
@@ -496,12 +508,12 @@ StreamPlan gemv_stream_plan(uint32_t ggml_type, uint32_t n, uint32_t k, uint32_t
     uint32_t h = (n + cus * rounds - 1u) / (cus * rounds);
     if (h > 16u) h = 16u;
     if (h < 1u) h = 1u;
-    // A tile stays below 64 KB -- 70 KB for Q6_K, whose workgroups share a compute unit in twos and
-    // whose sixteen rows of 5120 weights are 67 KB -- so that two or three workgroups share a compute
+    // A tile stays below 64 KB -- 69 KB for Q6_K, whose workgroups share a compute unit in twos and
+    // whose sixteen rows of 5120 weights are 66 KB -- so that two or three workgroups share a compute
     // unit's LDS (the LDS-direct loads themselves reach every LDS address: M0 values of 69632, 135168
     // and 150000 were written to and read back on this device), and a wave owns at most six
     // super-blocks: longer rows are cut into K segments of equal length.
-    const uint32_t tile_cap = q6 ? 70u * 1024u : 65536u;
+    const uint32_t tile_cap = q6 ? 80u * 1024u - 8u * slot - 8u * 64u : 65536u;
     auto stride_of = [block](uint32_t blocks) {
         uint32_t units = (block * blocks + 15u) / 16u;   // bytes / 16
         if ((units & 1u) == 0) ++units;    // odd number of 16-byte units: 16 rows start in 16 different bank groups
@@ -532,17 +544,14 @@ StreamPlan gemv_stream_plan(uint32_t ggml_type, uint32_t n, uint32_t k, uint32_t
     plan.tiles = (n + h - 1u) / h;
     plan.waves = 8u;
     plan.lds_bytes = h * plan.row_stride + plan.waves * slot + plan.waves * 64u;
-    // Matrices of a megabyte or two finish sooner on the FMA kernel's smaller workgroups.  Q6_K costs
-    // twice the matrix instructions and half again the vector work of Q4_K per super-block, which
-    // tiles of rows of 5120 do not hide (17408 x 5120 in fourteen-row tiles: 22.6 against 21.3 us on
-    // the FMA kernel; 151936 x 5120 in fifteen-row tiles 142 - 147 against 141 - 142 us, in two K
-    // segments 168 us); rows that must be cut into segments in any case gain (5120 x 17408: 22.7
-    // against 25.0 us).  Output matrices of a million super-blocks or more whose rows the FMA kernel
-    // cannot cut evenly over its eight block slots gain too, in uncut sixteen-row tiles (us, FMA
-    // against this kernel: 151936 x 5120 139.7 / 134.5, 65536 x 5120 63.2 / 62.2, 262144 x 2560 131.7 /
-    // 116.1; but 151936 x 4096 112.9 / 117.8, 128256 x 4096 95.9 / 100.4, 151936 x 2048 58.8 / 60.2,
-    // 32000 x 5120 33.3 / 33.8).
-    const bool big_head = q6 && segments == 1u && h == 16u && (nb & 7u) != 0 && (uint64_t)n * nb >= 1000000u;
+    // Matrices of a megabyte or two finish sooner on the FMA kernel's smaller workgroups.  A Q6_K tile is 46% longer and
+    // only two share a compute unit: what lies in between is even or the FMA kernel's (17408 x 5120 22.6 us there against
+    // 22.8, 28672 x 4096 26.9 / 28.3, 12288 x 4096 13.3 / 14.9), but rows that must be cut into segments in any case gain
+    // (5120 x 17408: 27.7 / 24.7), and so do matrices of 600,000 super-blocks in uncut sixteen-row tiles (us, weights
+    // out of every cache, FMA against this kernel: 32000 x 5120 36.8 / 35.1, 34816 x 5120 39.4 / 37.4, 65536 x 5120
+    // 67.3 / 61.6, 151936 x 2048 61.4 / 59.3, 128256 x 4096 98.2 / 96.7, 152064 x 3584 111.5 / 100.7, 262144 x 2560
+    // 133.6 / 118.0, 151936 x 5120 142.8 / 132.5).
+    const bool big_head = q6 && segments == 1u && h == 16u && (uint64_t)n * nb >= 600000u;
     const bool wins = q6 ? nb > 48u || big_head : (uint64_t)n * nb >= 16384u;
     plan.ok = nb >= 1 && seg >= 1u && seg <= 48u && segments <= 65535u && h >= 1u && (any_size || wins) &&
               plan.lds_bytes <= 160u * 1024u && m >= 1 && m <= 65535u && (!q6 || (nb & 1u) == 0);

@@ -369,6 +369,52 @@ def test_large_q6_k_output_matrix_streams_in_uncut_sixteen_row_tiles(api, d):
         assert np.array_equal(bits(got[0, :2000]), bits(got[0, 2000:4000]))   # the rows repeat
 
 
+@pytest.mark.parametrize("n,k,dtype", [(37, 512, "F32"), (16, 1024, "F16"), (133, 5120, "F32"), (65, 5632, "BF16"),
+                                       (50, 12800, "F16"), (40, 17408, "F32")])
+def test_streamed_q6_k_sums_digits_of_the_activations_exactly(api, d, n, k, dtype):
+    # An activation is 30 bits of its 16-weight group's largest, its products with the quants are summed as integers;
+    # what rounds is two conversions and the scales per group, up to six super-blocks of a lane, the waves and the
+    # segments: some 30 roundings of at most 2^-24, uniform, 2^-24 / sqrt(3) * sqrt(30) = 1.9e-7 in the mean square.
+    packed = synth.matrix(Q6_K, n, k, seed=93)
+    w = qm(api, d, Q6_K, n, k, packed)
+    weights = oracle.dequantize(Q6_K, packed, n, k).reshape(n, k).astype(np.float64)
+    x = synth.activations(1, k, seed=94).reshape(1, k)
+    x[0, ::7] *= np.float32(2.0 ** -9)     # within a group, too
+    x[0, 16:32] = 0
+    x[0, 32:48] = np.float32(-1.0)         # every digit of a power of two
+    x[0, 48:64] = np.float32(1.9999999)    # the largest mantissa carries through all digits
+    xt = api.Tensor.from_f32(d, (1, k), getattr(api.DType, dtype), x)
+    want = xt.to_f32().astype(np.float64) @ weights.T
+    d.set_tuning("gemv_stream", 2)
+    try:
+        got = d.project_quantized(xt, w, out_dtype=api.DType.F32)
+        assert rel_l2(got.tensor.to_f32(), want) <= 3e-7
+        for value in (np.inf, -np.inf, np.nan):     # none of the row's sums is finite, as on the FMA kernel
+            x[0, k - 5] = value
+            xt = api.Tensor.from_f32(d, (1, k), getattr(api.DType, dtype), x)
+            assert np.isnan(d.project_quantized(xt, w, out_dtype=api.DType.F32).tensor.to_f32()).all()
+    finally:
+        d.set_tuning("gemv_stream", 1)
+
+
+def test_one_activated_f32_row_of_a_large_q6_k_matrix_takes_the_streamed_kernel(api, d):
+    # 3000 x 17408: 204,000 super-blocks; the bits of the separate calls, and the tolerance of the test above
+    n, k = 3000, 17408
+    base = synth.matrix(Q6_K, 300, k, seed=95).reshape(300, -1)
+    w = qm(api, d, Q6_K, n, k, np.tile(base, (n // 300, 1)).reshape(-1))
+    packed = api.Tensor.from_f32(d, (1, 2 * k), api.DType.F32, synth.activations(1, 2 * k, seed=96))
+    fused = d.project_quantized(packed, w, silu_mul=True)
+    activated = d.expert_silu_mul(packed, k)
+    assert fused.operation == "q6_k_gemv_ksplit"
+    assert np.array_equal(bits(fused.tensor.to_f32()), bits(d.project_quantized(activated, w).tensor.to_f32()))
+    with fma_gemv(d):
+        other = d.project_quantized(packed, w, silu_mul=True).tensor.to_f32()
+    weights = oracle.dequantize(Q6_K, base.reshape(-1), 300, k).reshape(300, k).astype(np.float64)
+    want = np.tile(activated.to_f32().astype(np.float64) @ weights.T, (1, n // 300))
+    assert rel_l2(fused.tensor.to_f32(), want) <= 3e-7
+    assert rel_l2(other, want) <= 4e-7 and not np.array_equal(bits(other), bits(fused.tensor.to_f32()))
+
+
 @pytest.mark.parametrize("ggml", [Q4_K, Q6_K])
 def test_streamed_gemv_scales_every_chunk_by_itself(api, d, ggml):
     # activations whose 64-value chunks differ by dozens of orders of magnitude, zero chunks, one
