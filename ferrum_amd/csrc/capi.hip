@@ -258,7 +258,11 @@ uint8_t* scratch_data(fh_device* d) {
 // Points a GEMV launch that cuts K into segments at the device scratch
 // (partial sums and one zeroed counter word per row tile and batch row).
 fh_status prepare_gemv(fh_device* d, GemvArgs& a) {
-    const GemvScratch plan = gemv_scratch(a);
+    GemvScratch plan = gemv_scratch(a);
+    if (a.ring != 0 && plan.segments > 1 && !scratch_available(d, (size_t)plan.segments * a.m * a.n * sizeof(float))) {
+        a.ring = 0;   // the ring may want more segments than the scratch of a recording has room for
+        plan = gemv_scratch(a);
+    }
     if (plan.segments > 1) {
         if ((uint64_t)plan.tiles * a.m > fh_device::kCounterWords)
             return fail(FH_ERR_SHAPE, "projection needs %llu row tiles, more than the K-split scratch holds",
@@ -360,6 +364,7 @@ constexpr struct {
     {"gemm_few_tiles_split", &fh_tuning::gemm_few_tiles_split},
     {"moe_fold_combine", &fh_tuning::moe_fold_combine},
     {"gemm_resident", &fh_tuning::gemm_resident},
+    {"gemv_ring", &fh_tuning::gemv_ring},
     {"gemv_stream_own_loads", &fh_tuning::gemv_stream_own_loads},
     {"expert_weight_ring", &fh_tuning::expert_weight_ring},
     {"gemv_stream", &fh_tuning::gemv_stream},
@@ -593,7 +598,7 @@ fh_status fh_set_tuning(fh_device* device, const char* key, int64_t value) {
         ok = value == 0 || value == 1;
     } else if (k == "gemv_stream_own_loads" || k == "expert_weight_ring") {
         ok = value == 0 || value == 1;
-    } else if (k == "gemv_stream" || k == "gemm_few_tiles_split") {
+    } else if (k == "gemv_stream" || k == "gemv_ring" || k == "gemm_few_tiles_split") {
         ok = value >= 0 && value <= 2;
     } else if (k == "gemm_wide_shape") {
         ok = value >= 0 && value <= 2;
@@ -1067,6 +1072,7 @@ fh_status project(fh_device* device, const fh_qmatrix* weight, const fh_view* x,
         a.ksplit = (int)device->tuning.k_quant_gemv_ksplit;
         a.stream = (int)device->tuning.gemv_stream;
         a.stream_own = device->tuning.gemv_stream_own_loads != 0;
+        a.ring = (int)device->tuning.gemv_ring;
         a.cu_count = device->props.multiProcessorCount;
         a.x_mode = silu_mul ? kXSiluMul : kXPlain;
         a.x_rows = m;
@@ -1151,10 +1157,15 @@ fh_status fh_project_quantized_no_alloc(fh_device* device, const fh_qmatrix* wei
     a.ksplit = (int)device->tuning.k_quant_gemv_ksplit;
     a.stream = (int)device->tuning.gemv_stream;
     a.stream_own = device->tuning.gemv_stream_own_loads != 0;
+    a.ring = (int)device->tuning.gemv_ring;
     a.cu_count = device->props.multiProcessorCount;
     a.x_mode = kXPlain;
     a.x_rows = m;
-    const GemvScratch plan = gemv_scratch(a);
+    GemvScratch plan = gemv_scratch(a);
+    if (a.ring != 0 && (uint64_t)plan.segments * m * n * sizeof(float) > kFixedScratchBytes - kFixedCounterWords * sizeof(uint32_t)) {
+        a.ring = 0;   // its segments may be more than the fixed scratch has room for
+        plan = gemv_scratch(a);
+    }
     if (plan.segments > 1) {
         const uint64_t counters = (uint64_t)plan.tiles * m;
         const uint64_t partial_bytes = (uint64_t)plan.segments * m * n * sizeof(float);

@@ -74,6 +74,7 @@ struct StreamParams {
     uint32_t x_dtype, y_dtype;
     // rows longer than a tile can hold: grid.y K segments of seg_blocks super-blocks each
     uint32_t segments, seg_blocks, m;
+    uint32_t depth;       // the ring's tiles in LDS
     float* partials;      // [segments][m][n]
     uint32_t* counters;   // one per (row tile, batch row), zero between launches
 };
@@ -493,12 +494,182 @@ __global__ __launch_bounds__(WAVES * kWave) void gemv_stream_q6k(const StreamPar
     gemv_stream_body<kQ6K, DT, WAVES, MAXB>(p);
 }
 
+// The Q4_K ring, for large matrices and one activation row: a workgroup of sixteen waves has a compute unit to itself and
+// multiplies tile after tile of sixteen rows, while the next depth - 1 tiles are on their way.  With a tile per
+// workgroup every sixteen rows read all activations again, turn them into operands again, and the compute
+// unit asks for nothing while they multiply; here the operands of a wave's super-blocks (wave and wave + 16 of the
+// segment) stay in registers for the whole launch and a hundred kilobytes of requests are always out.  Eight waves
+// with three blocks each left too little to cover a tile's LDS reads (34816 x 5120: 25.3 us, sixteen 23.2).  Cold, us,
+// a tile per workgroup against the ring: 34816 x 5120 24.7 / 23.2, 43008 x 5120 29.4 / 26.9, 128256 x 4096 57.8 / 54.3,
+// 57344 x 8192 61.1 / 48.3, 151936 x 5120 90.2 / 76.4 (5.7 TB/s).
+// LDS map: [depth tiles of 16 x row_stride][a slot per wave; after the operands are read: row sums of 16 waves x 16, then
+// the sums of all the workgroup's tiles].
+template <int DT, int MAXB>
+__device__ __forceinline__ void gemv_ring_body(const StreamParams& p) {
+    constexpr uint32_t kBlock = StreamFormat<kQ4K>::kBytes;
+    constexpr uint32_t kSlot = StreamFormat<kQ4K>::kSlot;
+    constexpr uint32_t kAux = StreamFormat<kQ4K>::kAux;
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    const uint32_t tid = threadIdx.x, lane = tid & 63u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t first = blockIdx.y * p.seg_blocks, nb = min(p.seg_blocks, p.nb - first);
+    const uint32_t row_bytes = nb * kBlock, full_row_bytes = p.nb * kBlock;
+    const uint32_t tiles = (p.n + 15u) / 16u;
+    const uint32_t count = (tiles - blockIdx.x + gridDim.x - 1u) / gridDim.x;   // tiles blockIdx.x + i gridDim.x
+    uint8_t* const slot = lds + p.depth * p.tile_bytes + wave * kSlot;
+    float* const rsum = reinterpret_cast<float*>(lds + p.depth * p.tile_bytes);
+    float* const sums = rsum + 256;
+
+    // 1. the activations, as in the kernel above
+    const size_t xrow = (size_t)first * 256u;
+    typename std::conditional<DT == FH_F32, u32x4, u32x2>::type xraw[MAXB];
+#pragma unroll
+    for (int i = 0; i < MAXB; ++i) {
+        const uint32_t b = min(wave + 16u * i, nb - 1u);
+        if constexpr (DT == FH_F32) {
+            const float* src = static_cast<const float*>(p.x) + xrow + b * 256u + lane * 4u;
+            asm volatile("global_load_dwordx4 %0, %1, off" : "=v"(xraw[i]) : "v"(src) : "memory");
+        } else {
+            const uint16_t* src = static_cast<const uint16_t*>(p.x) + xrow + b * 256u + lane * 4u;
+            asm volatile("global_load_dwordx2 %0, %1, off" : "=v"(xraw[i]) : "v"(src) : "memory");
+        }
+    }
+    // 2. a tile's requests: every wave asks for one row, a kilobyte per instruction; rows past the last repeat it, so that
+    // every tile is the same number of instructions
+    const uint32_t per_row = (row_bytes + 1023u) >> 10;
+    const uint32_t lds_base = (uint32_t)(uintptr_t)lds;
+    auto request = [&](uint32_t it, uint32_t buffer) {
+        const uint32_t row0 = (blockIdx.x + it * gridDim.x) * 16u;
+        const uint8_t* const base = p.w + (size_t)min(row0 + wave, p.n - 1u) * full_row_bytes + first * kBlock;
+        const uint32_t to = lds_base + buffer * p.tile_bytes + wave * p.row_stride;
+        for (uint32_t c = 0; c < per_row; ++c)
+            if (c * 1024u + lane * 16u < row_bytes) lds_load16_at(base, c * 1024u + lane * 16u, to + c * 1024u);
+    };
+    const uint32_t ahead = min(p.depth, count);
+    for (uint32_t it = 0; it < ahead; ++it) request(it, it);
+    if (lane < 4u) reinterpret_cast<uint32_t*>(slot + 1024u + kAux)[lane] = 0u;
+
+    // 3. operands into registers, through the wave's slot
+    const uint32_t n = lane & 15u, g = lane >> 4;
+    const bool active = (n >> 2) == g;
+    const uint8_t* const xlane = active ? slot + (g * 4u + (n & 3u)) * 16u : slot + 1024u + kAux;
+    const uint32_t xstep = active ? 256u : 0u;
+    wait_vmcnt(ahead * per_row);
+    u32x4 xa[MAXB][4];
+    float4 aux[MAXB];
+#pragma unroll
+    for (int i = 0; i < MAXB; ++i) {
+        asm volatile("" : "+v"(xraw[i])::"memory");
+        float4 v;
+        if constexpr (DT == FH_F32) {
+            v = make_float4(__uint_as_float(xraw[i].x), __uint_as_float(xraw[i].y), __uint_as_float(xraw[i].z),
+                            __uint_as_float(xraw[i].w));
+        } else if constexpr (DT == FH_F16) {
+            v = make_float4(f16_bits_to_f32(xraw[i].x & 0xffffu), f16_bits_to_f32(xraw[i].x >> 16),
+                            f16_bits_to_f32(xraw[i].y & 0xffffu), f16_bits_to_f32(xraw[i].y >> 16));
+        } else {
+            v = make_float4(bf16_bits_to_f32(xraw[i].x & 0xffffu), bf16_bits_to_f32(xraw[i].x >> 16),
+                            bf16_bits_to_f32(xraw[i].y & 0xffffu), bf16_bits_to_f32(xraw[i].y >> 16));
+        }
+        stage_block(v, slot, lane);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // written before other lanes read it
+#pragma unroll
+        for (int u = 0; u < 4; ++u) xa[i][u] = *reinterpret_cast<const u32x4*>(xlane + u * xstep);
+        aux[i] = *reinterpret_cast<const float4*>(slot + 1024u + 16u * g);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // read before the next block is written
+    }
+
+    // 4. the tiles in turn.  The barriers are bare: a __syncthreads would wait for the tiles on their way
+    uint32_t buffer = 0;
+    for (uint32_t it = 0; it < count; ++it) {
+        wait_vmcnt(min(p.depth - 1u, count - 1u - it) * per_row);   // this tile has landed, the later ones may be out
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        float acc = 0.f;
+#pragma unroll
+        for (int i = 0; i < MAXB; ++i) {
+            const uint32_t b = wave + 16u * i;
+            if (b < nb) {
+                const uint8_t* const blk = lds + buffer * p.tile_bytes + n * p.row_stride + b * kBlock;
+                const uint4 hdr = *reinterpret_cast<const uint4*>(blk);
+                const uint4 qa = *reinterpret_cast<const uint4*>(blk + 16u + 32u * g);
+                const uint4 qb = *reinterpret_cast<const uint4*>(blk + 32u + 32u * g);
+                acc = multiply_q4k(xa[i], aux[i], hdr, qa, qb, g, acc);
+            }
+        }
+        acc += __shfl_xor(acc, 16, 64);
+        acc += __shfl_xor(acc, 32, 64);
+        if (lane < 16u) rsum[wave * 16u + lane] = acc;
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");   // every wave has read its part of the tile
+        if (it + p.depth < count) request(it + p.depth, buffer);
+        buffer = buffer + 1u == p.depth ? 0u : buffer + 1u;
+        if (tid < 16u) {
+            float total = 0.f;
+#pragma unroll
+            for (int w = 0; w < 16; ++w) total += rsum[w * 16 + tid];
+            sums[it * 16u + tid] = total;
+        }
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (the last tile's wait was for all there are)
+    __syncthreads();
+
+    // 5. out, or to the scratch: the last of a row group's segments adds all of them, in segment order
+    auto row_of = [&](uint32_t i) { return (blockIdx.x + (i >> 4) * gridDim.x) * 16u + (i & 15u); };
+    if (p.segments == 1) {
+        for (uint32_t i = tid; i < count * 16u; i += 1024u)
+            if (row_of(i) < p.n) store_from_f32(p.y, row_of(i), p.y_dtype, sums[i]);
+        return;
+    }
+    for (uint32_t i = tid; i < count * 16u; i += 1024u)
+        if (row_of(i) < p.n)
+            __hip_atomic_store(&p.partials[(size_t)blockIdx.y * p.n + row_of(i)], sums[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): the stores above have completed
+    __syncthreads();
+    uint32_t* const flag = reinterpret_cast<uint32_t*>(rsum);
+    if (tid == 0) {
+        uint32_t* counter = p.counters + blockIdx.x;
+        const uint32_t ticket = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const uint32_t last = ticket == p.segments - 1 ? 1u : 0u;
+        if (last) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        *flag = last;
+    }
+    __syncthreads();
+    if (*flag == 0) return;
+    for (uint32_t i = tid; i < count * 16u; i += 1024u) {
+        if (row_of(i) >= p.n) continue;
+        float total = 0.f;
+        for (uint32_t sg = 0; sg < p.segments; ++sg)
+            total += __hip_atomic_load(&p.partials[(size_t)sg * p.n + row_of(i)], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        store_from_f32(p.y, row_of(i), p.y_dtype, total);
+    }
+}
+
+template <int DT, int MAXB>
+__global__ __launch_bounds__(1024) void gemv_ring_q4k(const StreamParams p) {
+    gemv_ring_body<DT, MAXB>(p);
+}
+
 }  // namespace
+
+// The ring's plan: sixteen-row tiles of as few K segments as leave a wave two super-blocks and LDS room for two tiles.
+static bool ring_plan(uint32_t n, uint32_t nb, uint32_t cus, StreamPlan* plan) {
+    const uint32_t tiles = (n + 15u) / 16u, wanted = (nb + 23u) / 24u;
+    const uint32_t seg = (nb + wanted - 1u) / wanted, segments = (nb + seg - 1u) / seg;
+    const uint32_t stride = ((kQ4Bytes * seg) / 16u | 1u) * 16u, tile = 16u * stride, slots = 16u * kSlotBytes;
+    const uint32_t per_row = (kQ4Bytes * seg + 1023u) / 1024u;
+    uint32_t depth = (160u * 1024u - slots) / tile;
+    if (depth > 4u) depth = 4u;
+    if (depth * per_row > 20u) depth = 20u / per_row;   // the waits count to twenty
+    const uint32_t most = cus / segments, groups = most < tiles ? most : tiles;
+    // (the sums of a workgroup's tiles take the slots' room)
+    if (depth < 2u || groups == 0 || ((tiles + groups - 1u) / groups) * 64u + 1024u > slots) return false;
+    *plan = StreamPlan{true, 16u, groups, 16u, stride, depth * tile + slots, segments, seg, depth};
+    return true;
+}
 
 // Tile height that spreads the rows evenly: the fewest 16-row rounds per compute unit, then the
 // smallest height that still fits them.
 StreamPlan gemv_stream_plan(uint32_t ggml_type, uint32_t n, uint32_t k, uint32_t m, int cu_count, bool any_size,
-                            int forced_segments) {
+                            int forced_segments, int ring) {
     StreamPlan plan{};
     const bool q6 = ggml_type == kQ6K;
     const uint32_t block = q6 ? kQ6Bytes : kQ4Bytes, slot = q6 ? kSlot6Bytes : kSlotBytes;
@@ -555,6 +726,16 @@ StreamPlan gemv_stream_plan(uint32_t ggml_type, uint32_t n, uint32_t k, uint32_t
     const bool wins = q6 ? nb > 48u || big_head : (uint64_t)n * nb >= 16384u;
     plan.ok = nb >= 1 && seg >= 1u && seg <= 48u && segments <= 65535u && h >= 1u && (any_size || wins) &&
               plan.lds_bytes <= 160u * 1024u && m >= 1 && m <= 65535u && (!q6 || (nb & 1u) == 0);
+    if (!q6 && m == 1 && forced_segments <= 1 && ring != 0 && (any_size || plan.ok)) {
+        // The ring pays its start, some 4 us without a tile finished, and the last round of tiles back on 100 MB of
+        // weights in rows of 5120 and more (us, cold, a tile per workgroup against the ring: 34816 x 5120 24.7 / 23.2, 52032
+        // x 6144 40.2 / 35.6, 39040 x 8192 43.6 / 37.2, 25984 x 12288 42.3 / 36.3, 18368 x 17408 42.4 / 38.6; but 22080 x 7168
+        // 22.6 / 23.4, 17408 x 5120 12.9 / 15.5).  Shorter rows leave some of the sixteen waves idle: 69440 x 4608
+        // 36.2 / 37.4, 89280 x 3584 37.8 / 37.7.
+        const bool ring_wins = nb >= 20u && (uint64_t)n * nb >= 680000u;
+        StreamPlan other{};
+        if ((ring == 2 || ring_wins) && ring_plan(n, nb, cus, &other)) return other;
+    }
     return plan;
 }
 
@@ -575,6 +756,7 @@ const char* launch_gemv_stream(hipStream_t s, const GemvArgs& a, const StreamPla
     p.m = a.m;
     p.partials = a.partials;
     p.counters = a.counters;
+    p.depth = plan.depth;
     typedef void (*Kernel)(const StreamParams);
     // [format][dtype][blocks per wave: 2, 3, 6]
     static const Kernel kernels[2][3][3] = {
@@ -593,6 +775,23 @@ const char* launch_gemv_stream(hipStream_t s, const GemvArgs& a, const StreamPla
                     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
                                               hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
     });
+    if (plan.depth != 0) {
+        // [dtype][super-blocks per wave: 1, 2]
+        static const Kernel rings[3][2] = {{gemv_ring_q4k<FH_F32, 1>, gemv_ring_q4k<FH_F32, 2>},
+                                           {gemv_ring_q4k<FH_F16, 1>, gemv_ring_q4k<FH_F16, 2>},
+                                           {gemv_ring_q4k<FH_BF16, 1>, gemv_ring_q4k<FH_BF16, 2>}};
+        static std::atomic<uint64_t> ring_raised{0};
+        once_per_device(ring_raised, [] {
+            for (const auto& row : rings)
+                for (Kernel kernel : row)
+                    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                              hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        });
+        p.tile_bytes = 16u * plan.row_stride;
+        hipLaunchKernelGGL(rings[a.x_dtype][plan.seg_blocks > 16u ? 1 : 0], dim3(plan.tiles, plan.segments), dim3(16u * kWave),
+                           plan.lds_bytes, s, p);
+        return plan.segments > 1 ? "q4_k_gemv_ksplit" : "q4_k_gemv_factored";
+    }
     const int shape = plan.seg_blocks <= 16u ? 0 : plan.seg_blocks <= 24u ? 1 : 2;
     const int format = a.ggml_type == kQ6K ? 1 : 0;
     // Q4_K tiles of up to 14 rows (two load instructions per super-block): every wave loads what it

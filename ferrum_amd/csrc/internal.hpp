@@ -32,6 +32,7 @@ struct fh_tuning {
     int64_t gemm_few_tiles_split = 1;  // few rows: a tile's super-blocks dealt over the waves, any K: 0 never (whole tiles per wave, the kernels for rows that fit LDS or not), 1 where it wins, 2 wherever it runs
     int64_t moe_fold_combine = 1;      // fh_moe_ffn with few tokens: down projection and weighted sum in one launch (0 = two)
     int64_t gemm_resident = 1;         // rows that fit LDS whole take the rows-resident kernel (0 = square tiles)
+    int64_t gemv_ring = 1;   // streamed GEMVs of one row keep a workgroup on every compute unit: 1 where that is faster, 0 never, 2 wherever it fits
     int64_t gemv_stream_own_loads = 1; // the streamed Q4_K GEMV's waves load the super-blocks they multiply (tiles of up to 14 rows); 0: the tile row by row
     int64_t expert_weight_ring = 1;    // grouped Q4_K / Q6_K expert projection with short rows: weights through LDS rings (0 = straight into registers)
     int64_t gemv_stream = 1;           // dense Q4_K / Q6_K GEMV on the streamed matrix-core kernel: 0 never, 1 where it wins, 2 wherever it runs
@@ -239,6 +240,7 @@ struct GemvArgs {
     void* shared_y;
     // the streamed matrix-core kernel may take the launch (dense Q4_K or Q6_K, plain rows, rows that fit LDS)
     int stream;           // 0 never, 1 where it is the faster kernel, 2 wherever it can run
+    int ring;             // fh_tuning::gemv_ring
     bool stream_own;      // the streamed Q4_K kernel's waves load their own super-blocks where tiles are <= 14 rows
     int cu_count;
     float* partials;      // scratch for K segments (gemv_plan says how much)
@@ -284,10 +286,12 @@ struct StreamPlan {
     // rows too long for one tile are cut into K segments (grid.y), met through the scratch
     // partials and counters exactly as the FMA kernel's segments are
     uint32_t segments, seg_blocks;
+    // the ring: a workgroup per compute unit, `tiles` of them per segment, with this many tiles in LDS (0: one tile per workgroup)
+    uint32_t depth;
 };
 // any_size: also matrices so small that the FMA kernel is the faster one
 StreamPlan gemv_stream_plan(uint32_t ggml_type, uint32_t n, uint32_t k, uint32_t m, int cu_count, bool any_size,
-                            int forced_segments);
+                            int forced_segments, int ring);
 const char* launch_gemv_stream(hipStream_t s, const GemvArgs& a, const StreamPlan& plan);
 // whether launch_gemv hands this launch to the streamed kernel, and its plan
 bool gemv_takes_stream(const GemvArgs& a, StreamPlan* plan);

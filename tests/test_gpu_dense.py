@@ -346,6 +346,51 @@ def test_streamed_gemv_matches_the_oracle(api, d, ggml, n, k, dtype):
     d.set_tuning("gemv_stream", 1)
 
 
+@pytest.mark.parametrize("n,k", [(5, 256), (37, 4096), (4113, 4352), (100, 6144), (8209, 2560), (77, 6400), (2100, 12544), (200, 34816)])
+@pytest.mark.parametrize("dtype", ["F32", "F16", "BF16"])
+def test_ring_gemv_matches_the_oracle(api, d, n, k, dtype):
+    # one tile and fewer, a workgroup's second and third tile, one and two super-blocks a wave, two to six K segments;
+    # the operands are those of the kernel that gives every tile a workgroup, only the waves' sums are cut otherwise:
+    # some 2 sqrt(nb) more roundings of 2^-24 / sqrt(3)
+    code = {"F32": oracle.F32, "F16": oracle.F16, "BF16": oracle.BF16}[dtype]
+    packed = synth.matrix(Q4_K, n, k, seed=n + k)
+    w = qm(api, d, Q4_K, n, k, packed)
+    x = oracle.round_storage(synth.activations(1, k, seed=7 * n + 1), code).reshape(1, k)
+    xt = api.Tensor.from_f32(d, (1, k), getattr(api.DType, dtype), x)
+    d.set_tuning("gemv_stream", 2)
+    try:
+        d.set_tuning("gemv_ring", 0)
+        tiles = d.project_quantized(xt, w, out_dtype=api.DType.F32).tensor.to_f32()
+        d.set_tuning("gemv_ring", 2)
+        out = d.project_quantized(xt, w, out_dtype=api.DType.F32)
+        again = d.project_quantized(xt, w, out_dtype=api.DType.F32).tensor.to_f32()
+    finally:
+        d.set_tuning("gemv_ring", 1)
+        d.set_tuning("gemv_stream", 1)
+    assert out.operation == ("q4_k_gemv_ksplit" if k > 6144 else "q4_k_gemv_factored")
+    got = out.tensor.to_f32()
+    assert np.array_equal(bits(got), bits(again))
+    assert_matmul_parity(got, oracle.project(Q4_K, packed, n, k, x, accumulate="f64"), f"ring {n}x{k} {dtype}")
+    assert rel_l2(got, tiles) <= 2 * np.sqrt(k / 256) * 2.0 ** -24 / np.sqrt(3) + 2.0 ** -24
+
+
+def test_large_q4_k_matrices_take_the_ring_by_themselves(api, d):
+    n, k = 34010, 5120      # 680,200 super-blocks
+    base = synth.matrix(Q4_K, 1790, k, seed=31).reshape(1790, -1)
+    w = qm(api, d, Q4_K, n, k, np.tile(base, (n // 1790, 1)).reshape(-1))
+    xt = api.Tensor.from_f32(d, (1, k), api.DType.F32, synth.activations(1, k, seed=32))
+    got = d.project_quantized(xt, w).tensor.to_f32()
+    d.set_tuning("gemv_ring", 2)
+    try:
+        forced = d.project_quantized(xt, w).tensor.to_f32()
+        d.set_tuning("gemv_ring", 0)
+        tiles = d.project_quantized(xt, w).tensor.to_f32()
+    finally:
+        d.set_tuning("gemv_ring", 1)
+    assert np.array_equal(bits(got), bits(forced)) and not np.array_equal(bits(got), bits(tiles))
+    assert rel_l2(got, tiles) <= 6e-7 and np.array_equal(bits(got[0, :1790]), bits(got[0, -1790:]))
+
+
 def test_large_q6_k_output_matrix_streams_in_uncut_sixteen_row_tiles(api, d):
     # a million super-blocks in rows the FMA kernel cannot cut evenly over its block slots (20 per row):
     # sixteen rows of 5120 Q6_K weights are a 67 KB tile
