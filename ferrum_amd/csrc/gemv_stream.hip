@@ -723,7 +723,15 @@ StreamPlan gemv_stream_plan(uint32_t ggml_type, uint32_t n, uint32_t k, uint32_t
     // 67.3 / 61.6, 151936 x 2048 61.4 / 59.3, 128256 x 4096 98.2 / 96.7, 152064 x 3584 111.5 / 100.7, 262144 x 2560
     // 133.6 / 118.0, 151936 x 5120 142.8 / 132.5).
     const bool big_head = q6 && segments == 1u && h == 16u && (uint64_t)n * nb >= 600000u;
-    const bool wins = q6 ? nb > 48u || big_head : (uint64_t)n * nb >= 16384u;
+    // One row of a Q4_K matrix of short rows is the FMA kernel's: a tile of sixteen is a few kilobytes of LDS for eight waves of
+    // which some own no super-block, and staging stands beside little arithmetic (us, cold, FMA against this kernel:
+    // 29952 x 256 3.7 / 8.3, 8448 x 512 3.5 / 4.2, 4224 x 1024 3.5 / 3.8, 99968 x 1024 14.1 / 23.6; rows of 5 - 8 super-blocks
+    // 4992 x 1536 4.4 / 4.2, 12480 x 2048 5.8 / 6.0, 24960 x 1536 8.4 / 9.1, 156224 x 2048 40.7 / 48.3; of 9 - 12
+    // 16640 x 3072 9.9 / 9.0, 40000 x 2560 16.0 / 16.0, 49984 x 2560 18.8 / 19.6, 104128 x 3072 34.6 / 38.8; of 14
+    // 89280 x 3584 39.8 / 37.8).
+    const uint64_t short_from = nb <= 4u ? 0u : nb <= 8u ? 100000u : nb <= 12u ? 450000u : ~0ull;
+    const bool short_rows = m == 1 && (uint64_t)n * nb >= short_from;
+    const bool wins = q6 ? nb > 48u || big_head : (uint64_t)n * nb >= 16384u && !short_rows;
     plan.ok = nb >= 1 && seg >= 1u && seg <= 48u && segments <= 65535u && h >= 1u && (any_size || wins) &&
               plan.lds_bytes <= 160u * 1024u && m >= 1 && m <= 65535u && (!q6 || (nb & 1u) == 0);
     if (!q6 && m == 1 && forced_segments <= 1 && ring != 0 && (any_size || plan.ok)) {

@@ -391,6 +391,26 @@ def test_large_q4_k_matrices_take_the_ring_by_themselves(api, d):
     assert rel_l2(got, tiles) <= 6e-7 and np.array_equal(bits(got[0, :1790]), bits(got[0, -1790:]))
 
 
+@pytest.mark.parametrize("n,k,fma", [(16400, 256, True), (4200, 1024, True), (3300, 1280, False), (20000, 1280, True), (12400, 2048, False),
+                                     (12512, 2048, True), (11200, 2304, False)])
+def test_short_q4_k_rows_take_the_fma_kernel(api, d, n, k, fma):
+    # every size above 16384 super-blocks in rows of up to four, from 100,000 on in rows of five to eight; batches as before
+    packed = synth.matrix(Q4_K, n, k, seed=33)
+    w = qm(api, d, Q4_K, n, k, packed)
+    for m in (1, 2):
+        x = synth.activations(m, k, seed=34).reshape(m, k)
+        xt = api.Tensor.from_f32(d, (m, k), api.DType.F32, x)
+        got = d.project_quantized(xt, w).tensor.to_f32()
+        d.set_tuning("gemv_stream", 0)
+        try:
+            other = d.project_quantized(xt, w).tensor.to_f32()
+        finally:
+            d.set_tuning("gemv_stream", 1)
+        assert np.array_equal(bits(got), bits(other)) == (fma and m == 1)
+        rows = np.unique(np.concatenate([np.arange(20), np.arange(n - 20, n)]))
+        assert_matmul_parity(got[:, rows], oracle_columns(Q4_K, packed, n, k, rows, x, accumulate="f64"), f"{n}x{k} m={m}")
+
+
 def test_large_q6_k_output_matrix_streams_in_uncut_sixteen_row_tiles(api, d):
     # a million super-blocks in rows the FMA kernel cannot cut evenly over its block slots (20 per row):
     # sixteen rows of 5120 Q6_K weights are a 67 KB tile
