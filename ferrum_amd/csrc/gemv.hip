@@ -745,7 +745,7 @@ bool gemv_takes_stream(const GemvArgs& a, StreamPlan* plan) {
     if (a.stream == 0 || (a.ggml_type != kQ4K && a.ggml_type != kQ6K) || a.metadata != nullptr || a.x_mode != kXPlain ||
         a.shared_w != nullptr)
         return false;
-    *plan = gemv_stream_plan(a.ggml_type, a.n, a.k, a.m, a.cu_count, a.stream == 2, a.ksplit, a.ring);
+    *plan = gemv_stream_plan(a.ggml_type, a.n, a.k, a.m, a.cu_count, a.stream == 2, a.ksplit, a.ring, a.x_dtype == FH_F32);
     return plan->ok;
 }
 

@@ -669,7 +669,7 @@ static bool ring_plan(uint32_t n, uint32_t nb, uint32_t cus, StreamPlan* plan) {
 // Tile height that spreads the rows evenly: the fewest 16-row rounds per compute unit, then the
 // smallest height that still fits them.
 StreamPlan gemv_stream_plan(uint32_t ggml_type, uint32_t n, uint32_t k, uint32_t m, int cu_count, bool any_size,
-                            int forced_segments, int ring) {
+                            int forced_segments, int ring, bool f32_rows) {
     StreamPlan plan{};
     const bool q6 = ggml_type == kQ6K;
     const uint32_t block = q6 ? kQ6Bytes : kQ4Bytes, slot = q6 ? kSlot6Bytes : kSlotBytes;
@@ -722,7 +722,10 @@ StreamPlan gemv_stream_plan(uint32_t ggml_type, uint32_t n, uint32_t k, uint32_t
     // out of every cache, FMA against this kernel: 32000 x 5120 36.8 / 35.1, 34816 x 5120 39.4 / 37.4, 65536 x 5120
     // 67.3 / 61.6, 151936 x 2048 61.4 / 59.3, 128256 x 4096 98.2 / 96.7, 152064 x 3584 111.5 / 100.7, 262144 x 2560
     // 133.6 / 118.0, 151936 x 5120 142.8 / 132.5).
-    const bool big_head = q6 && segments == 1u && h == 16u && (uint64_t)n * nb >= 600000u;
+    // Rows of 16 bits gain 1% there and are 0.9e-7 from 64 bits on the FMA kernel against 0.95e-7 here (f32 rows 1.9e-7 against
+    // 0.9e-7): they come from a million super-blocks on, where the FMA kernel cannot cut a row evenly over its eight block slots.
+    const bool big_head = q6 && segments == 1u && h == 16u &&
+                          (f32_rows ? (uint64_t)n * nb >= 600000u : (nb & 7u) != 0 && (uint64_t)n * nb >= 1000000u);
     // One row of a Q4_K matrix of short rows is the FMA kernel's: a tile of sixteen is a few kilobytes of LDS for eight waves of
     // which some own no super-block, and staging stands beside little arithmetic (us, cold, FMA against this kernel:
     // 29952 x 256 3.7 / 8.3, 8448 x 512 3.5 / 4.2, 4224 x 1024 3.5 / 3.8, 99968 x 1024 14.1 / 23.6; rows of 5 - 8 super-blocks

@@ -291,7 +291,7 @@ struct StreamPlan {
 };
 // any_size: also matrices so small that the FMA kernel is the faster one
 StreamPlan gemv_stream_plan(uint32_t ggml_type, uint32_t n, uint32_t k, uint32_t m, int cu_count, bool any_size,
-                            int forced_segments, int ring);
+                            int forced_segments, int ring, bool f32_rows);
 const char* launch_gemv_stream(hipStream_t s, const GemvArgs& a, const StreamPlan& plan);
 // whether launch_gemv hands this launch to the streamed kernel, and its plan
 bool gemv_takes_stream(const GemvArgs& a, StreamPlan* plan);

@@ -462,6 +462,19 @@ def test_streamed_q6_k_sums_digits_of_the_activations_exactly(api, d, n, k, dtyp
         d.set_tuning("gemv_stream", 1)
 
 
+def test_only_f32_rows_stream_q6_k_matrices_below_a_million_super_blocks(api, d):
+    n, k = 32000, 5120     # 640,000 super-blocks, sixteen-row tiles
+    base = synth.matrix(Q6_K, 2000, k, seed=35).reshape(2000, -1)
+    w = qm(api, d, Q6_K, n, k, np.tile(base, (n // 2000, 1)).reshape(-1))
+    for dtype, streamed in (("F32", True), ("F16", False), ("BF16", False)):
+        xt = api.Tensor.from_f32(d, (1, k), getattr(api.DType, dtype), synth.activations(1, k, seed=36))
+        got = d.project_quantized(xt, w, out_dtype=api.DType.F32).tensor.to_f32()
+        with fma_gemv(d):
+            other = d.project_quantized(xt, w, out_dtype=api.DType.F32).tensor.to_f32()
+        assert np.array_equal(bits(got), bits(other)) == (not streamed)
+        assert rel_l2(got, other) <= 7e-7
+
+
 def test_one_activated_f32_row_of_a_large_q6_k_matrix_takes_the_streamed_kernel(api, d):
     # 3000 x 17408: 204,000 super-blocks; the bits of the separate calls, and the tolerance of the test above
     n, k = 3000, 17408
