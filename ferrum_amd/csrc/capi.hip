@@ -256,9 +256,8 @@ uint8_t* scratch_data(fh_device* d) {
 }
 
 // Points a GEMV launch that cuts K into segments at the device scratch
-// (partial sums and one zeroed counter word per row tile and batch row).
-fh_status prepare_gemv(fh_device* d, GemvArgs& a) {
-    GemvScratch plan = gemv_scratch(a);
+// (partial sums and one zeroed counter word per row tile and batch row).  `plan` is gemv_scratch(a) and stays so.
+fh_status prepare_gemv(fh_device* d, GemvArgs& a, GemvScratch& plan) {
     if (a.ring != 0 && plan.segments > 1 && !scratch_available(d, (size_t)plan.segments * a.m * a.n * sizeof(float))) {
         a.ring = 0;   // the ring may want more segments than the scratch of a recording has room for
         plan = gemv_scratch(a);
@@ -279,15 +278,15 @@ fh_status prepare_gemv(fh_device* d, GemvArgs& a) {
 // extent and, where K is cut into segments, the counter words (one per row tile and batch
 // entry).  A launch that carries a shared expert is not cut.
 fh_status run_gemv(fh_device* d, GemvArgs a, const char** name) {
-    const GemvScratch plan = gemv_scratch(a);
+    GemvScratch plan = gemv_scratch(a);
     uint64_t most = 65535u;
     if (plan.segments > 1 && plan.tiles > 0) most = std::min<uint64_t>(most, fh_device::kCounterWords / plan.tiles);
     if (a.x_mode == kXDivide && a.x_div > 1) most -= most % a.x_div;   // the routes of a token stay together
     if (a.m <= most || a.shared_w != nullptr || most == 0) {
-        fh_status st = prepare_gemv(d, a);
+        fh_status st = prepare_gemv(d, a, plan);
         if (st != FH_OK) return st;
         if (a.m > 65535u) return fail(FH_ERR_SHAPE, "batch of %u entries exceeds the launch grid", a.m);
-        *name = launch_gemv(d->stream, a);
+        *name = launch_gemv(d->stream, a, plan);
         return FH_OK;
     }
     const uint32_t total = a.m;
@@ -307,9 +306,10 @@ fh_status run_gemv(fh_device* d, GemvArgs a, const char** name) {
             part.x = static_cast<const uint8_t*>(a.x) + (size_t)(first / div) * x_row;
             part.x_rows = part.m / div;
         }   // kXGather reads the token row named by each entry's metadata: x stays whole
-        fh_status st = prepare_gemv(d, part);
+        GemvScratch part_plan = gemv_scratch(part);
+        fh_status st = prepare_gemv(d, part, part_plan);
         if (st != FH_OK) return st;
-        *name = launch_gemv(d->stream, part);
+        *name = launch_gemv(d->stream, part, part_plan);
     }
     return FH_OK;
 }
@@ -1178,7 +1178,7 @@ fh_status fh_project_quantized_no_alloc(fh_device* device, const fh_qmatrix* wei
         a.counters = reinterpret_cast<uint32_t*>(base);
         a.partials = reinterpret_cast<float*>(base + kFixedCounterWords * sizeof(uint32_t));
     }
-    device->last_operation = launch_gemv(device->stream, a);
+    device->last_operation = launch_gemv(device->stream, a, plan);
     FH_HIP(hipGetLastError());
     return FH_OK;
 }

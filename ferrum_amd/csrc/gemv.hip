@@ -750,15 +750,21 @@ bool gemv_takes_stream(const GemvArgs& a, StreamPlan* plan) {
 }
 
 GemvScratch gemv_scratch(const GemvArgs& a) {
-    StreamPlan stream;
-    if (gemv_takes_stream(a, &stream)) return {stream.segments, stream.tiles};
+    GemvScratch need{};
+    if (gemv_takes_stream(a, &need.stream)) {
+        need.segments = need.stream.segments;
+        need.tiles = need.stream.tiles;
+        return need;
+    }
+    need.stream.ok = false;
     const GemvPlan plan = gemv_plan(a.n, a.k, a.m, a.ksplit);
-    return {plan.segments, plan.tiles};
+    need.segments = plan.segments;
+    need.tiles = plan.tiles;
+    return need;
 }
 
-const char* launch_gemv(hipStream_t s, const GemvArgs& a) {
-    StreamPlan stream;
-    if (gemv_takes_stream(a, &stream)) return launch_gemv_stream(s, a, stream);
+const char* launch_gemv(hipStream_t s, const GemvArgs& a, const GemvScratch& planned) {
+    if (planned.stream.ok) return launch_gemv_stream(s, a, planned.stream);
     const GemvPlan plan = gemv_plan(a.n, a.k, a.m, a.ksplit);
     Params p{};
     p.w = static_cast<const uint8_t*>(a.w);

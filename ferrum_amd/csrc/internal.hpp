@@ -255,7 +255,9 @@ struct GemvPlan {
     uint32_t segments, seg_len, rows_per_wg, tiles;
 };
 GemvPlan gemv_plan(uint32_t n, uint32_t k, uint32_t m, int forced_segments);
-const char* launch_gemv(hipStream_t s, const GemvArgs& a);
+struct GemvScratch;
+// planned: gemv_scratch(a)
+const char* launch_gemv(hipStream_t s, const GemvArgs& a, const GemvScratch& planned);
 // whether a launch with GemvArgs::route set exists for these rows and this router
 bool gemv_routes(uint32_t n, uint32_t k, uint32_t experts, uint32_t top_k);
 
@@ -295,9 +297,11 @@ StreamPlan gemv_stream_plan(uint32_t ggml_type, uint32_t n, uint32_t k, uint32_t
 const char* launch_gemv_stream(hipStream_t s, const GemvArgs& a, const StreamPlan& plan);
 // whether launch_gemv hands this launch to the streamed kernel, and its plan
 bool gemv_takes_stream(const GemvArgs& a, StreamPlan* plan);
-// K segments and row tiles of the kernel launch_gemv will run: what sizes the scratch
+// K segments and row tiles of the kernel launch_gemv will run: what sizes the scratch.  The plan is made once per call (the
+// smallest calls are bound by the host; here, for the scratch and for the launch it was made three times).
 struct GemvScratch {
     uint32_t segments, tiles;
+    StreamPlan stream;    // ok: the streamed kernel, with this plan
 };
 GemvScratch gemv_scratch(const GemvArgs& a);
 
