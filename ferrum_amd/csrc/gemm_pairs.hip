@@ -1,15 +1,20 @@
 // Projection of a batch of f32 rows, Y[M,N] = X[M,K] . W[N,K]^T for Q4_K / Q5_K / Q6_K / IQ4_XS weights, on the f16
-// matrix instruction without giving up a bit of f32: neither side is rounded to 16 bits.
+// matrix instruction, no farther from 64 bits than on the f32 one: neither side is rounded to 16 bits.
 //
 // * A weight of these formats is a block scale times an integer (less dmin times an integer).  sc * (q - 8) of Q4_K and
 //   sc * (q - 16) of Q5_K have at most ten bits and are exact f16 values; sc * (q - 32) of Q6_K and ls * codebook of
 //   IQ4_XS have up to thirteen and travel as their f16 rounding and the exact remainder.  The block scale d is applied
 //   to the f32 sums of a super-block.
 // * An activation is two f16 values: x * s = hi + lo, s a power of two per row and super-block that brings the largest
-//   to [2^14, 2^15).  hi and lo carry 23 significant bits and an error of at most 2^-24 of the element (or 2^-39 of the
-//   largest one), half a unit in the last place of f32.
+//   to [2^14, 2^15).  hi and lo carry 23 bits and the sign between them: five elements of six are exact, the others off by
+//   their last bit (2^-23 of the element at most, 0.6 2^-24 in the mean square; below 2^-15 of the largest one 2^-39 of that).
 // * What the centring by 8 or 16 leaves, sum over the eight groups of (centre * d * sc - dmin * m) * (sum of x), is
 //   four steps of the f32 matrix instruction per super-block, on group sums taken in f64.
+// * The sums of the super-blocks are added in f64 (and, where a weight has two parts, their pieces too), which pays for
+//   the operands' last bits.  rel-L2 to 64 bits in 1e-7, f32 instruction / f32 sums here / this, 24 x 5120 x 17408 Q6_K:
+//   normal rows 1.19 / 1.15 / 0.78, SiLU times up 1.18 / 1.25 / 0.92, a channel in 250 a thousand times the others
+//   1.17 / 1.36 / 1.08; Q4_K 1.19 / 1.07 / 0.85, 1.18 / 1.12 / 0.91, 1.18 / 1.21 / 1.01.  The projections of a layer of
+//   24 rows take 106.7 us, with f32 sums 106.4.
 //
 // The rows are split once per call by split_rows_kernel, into the order in which a wave reads matrix operands, so the
 // product itself has no conversion of activations.  The alternative, v_mfma_f32_16x16x4_f32 on exact f32 weights
@@ -17,8 +22,8 @@
 // every weight once per 16 rows.
 //
 // What bounds it: the waves' own instructions.  24 x 28672 x 4096 takes 37 us; with no weight or operand on its way in the
-// loop 30, also without decode 29, with half the multiplications 28: eight waves a compute unit (136 KB of operands, 170
-// registers) do not hide the vector instructions of one behind the matrix instructions of another as four would.
+// loop 30, also without decode 29, with half the multiplications 28: eight waves a compute unit (136 KB of operands, 217 -
+// 243 registers) do not hide the vector instructions of one behind the matrix instructions of another as four would.
 //
 // A workgroup is eight waves: two halves of K (every other super-block) x four tiles of 32 weight rows; all 32 rows of
 // the batch's group at once.  A super-block's operands are brought into LDS by LDS-direct loads one super-block ahead
@@ -403,9 +408,9 @@ __global__ __launch_bounds__(kThreads) void gemm_pairs_kernel(const PairsParams 
         }
     };
 
-    float16v acc;
+    double acc[16];
 #pragma unroll
-    for (int v = 0; v < 16; ++v) acc[v] = 0.f;
+    for (int v = 0; v < 16; ++v) acc[v] = 0.0;
 
     Raw raw[2];
     if (mine > 0) {
@@ -473,10 +478,13 @@ __global__ __launch_bounds__(kThreads) void gemm_pairs_kernel(const PairsParams 
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 const int v = 4 * v4 + j;
-                float sum = hi[0][v] + hi[1][v];
-                if constexpr (kChains == 4) sum += hi[2][v] + hi[3][v];
-                sum += lo[v];
-                acc[v] = fmaf(Raw::kOffset ? fmaf(d, sum, sums[v]) : d * sum, scale[j], acc[v]);
+                if constexpr (kChains == 4) {
+                    const double sum = ((double)hi[0][v] + (double)hi[1][v]) + ((double)hi[2][v] + (double)hi[3][v]) + (double)lo[v];
+                    acc[v] = fma(sum, (double)(d * scale[j]), acc[v]);
+                } else {
+                    const float sum = hi[0][v] + hi[1][v] + lo[v];
+                    acc[v] = fma((double)fmaf(d, sum, sums[v]), (double)scale[j], acc[v]);
+                }
             }
         }
     };
@@ -505,10 +513,10 @@ __global__ __launch_bounds__(kThreads) void gemm_pairs_kernel(const PairsParams 
     // the two halves of K meet in LDS
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    float4* const exchange = reinterpret_cast<float4*>(lds) + (size_t)tile_wave * 256 + lane;
+    double2* const exchange = reinterpret_cast<double2*>(lds) + (size_t)tile_wave * 512 + lane;
     if (half == 1) {
 #pragma unroll
-        for (int v = 0; v < 4; ++v) exchange[64 * v] = make_float4(acc[4 * v], acc[4 * v + 1], acc[4 * v + 2], acc[4 * v + 3]);
+        for (int v = 0; v < 8; ++v) exchange[64 * v] = make_double2(acc[2 * v], acc[2 * v + 1]);
     }
     __syncthreads();
     const uint32_t m0 = group * kGroupRows;
@@ -519,12 +527,12 @@ __global__ __launch_bounds__(kThreads) void gemm_pairs_kernel(const PairsParams 
     if (half == 0) {
 #pragma unroll
         for (int v4 = 0; v4 < 4; ++v4) {
-            const float4 other = exchange[64 * v4];
-            const float o[4] = {other.x, other.y, other.z, other.w};
+            const double2 first = exchange[128 * v4], second = exchange[128 * v4 + 64];
+            const double o[4] = {first.x, first.y, second.x, second.y};
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 const uint32_t token = m0 + 8 * v4 + 4 * kg + j;
-                const float sum = acc[4 * v4 + j] + o[j];
+                const float sum = (float)(acc[4 * v4 + j] + o[j]);
                 if (row < p.n && token < p.m) {
                     if (p.segments == 1)
                         store(token, sum);
@@ -549,9 +557,9 @@ __global__ __launch_bounds__(kThreads) void gemm_pairs_kernel(const PairsParams 
     if (last_flag == 0 || row >= p.n) return;
     // the last workgroup to arrive adds the segments in order; both halves of it, sixteen rows each, four segments of
     // eight outputs on their way at a time (one load after the other took longer than the product)
-    float total[8];
+    double total[8];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) total[j] = 0.f;
+    for (int j = 0; j < 8; ++j) total[j] = 0.0;
     const float* const from = p.partials + row;
     for (uint32_t s0 = 0; s0 < p.segments; s0 += 4) {
         float part[4][8];
@@ -567,13 +575,13 @@ __global__ __launch_bounds__(kThreads) void gemm_pairs_kernel(const PairsParams 
         for (uint32_t s = 0; s < 4; ++s)
             if (s0 + s < p.segments) {
 #pragma unroll
-                for (uint32_t j = 0; j < 8; ++j) total[j] += part[s][j];
+                for (uint32_t j = 0; j < 8; ++j) total[j] += (double)part[s][j];
             }
     }
 #pragma unroll
     for (uint32_t j = 0; j < 8; ++j) {
         const uint32_t token = m0 + 16 * half + 2 * j + kg;
-        if (token < p.m) store(token, total[j]);
+        if (token < p.m) store(token, (float)total[j]);
     }
 }
 

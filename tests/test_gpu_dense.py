@@ -1524,6 +1524,31 @@ def test_f32_batches_as_pairs_of_f16(api, d, ggml, m, n, k):
     assert np.array_equal(bits(half.to_f32()), bits(oracle.round_storage(got.tensor.to_f32(), oracle.F16).reshape(m, n)))
 
 
+@pytest.mark.parametrize("ggml", [12, 13, 14, 23], ids=["q4_k", "q5_k", "q6_k", "iq4_xs"])
+@pytest.mark.parametrize("rows", ["normal", "gated", "outliers"])
+def test_f32_batches_as_pairs_are_no_farther_from_64_bits_than_on_the_f32_instruction(api, d, ggml, rows):
+    # also where few elements carry a sum: what SiLU and a product make of normal values, and rows with a few channels
+    # a thousand times the others
+    m, n, k = 24, 2573, 17408
+    packed = synth.matrix(ggml, n, k, seed=745)
+    w = qm(api, d, ggml, n, k, packed)
+    g = synth.rng(746)
+    x = g.standard_normal((m, k))
+    if rows == "gated":
+        x = 3 * x / (1 + np.exp(-3 * x)) * g.standard_normal((m, k))
+    elif rows == "outliers":
+        x = x * np.where(g.random((1, k)) < 0.004, 1000.0, 1.0)
+    x = x.astype(np.float32)
+    xt = api.Tensor.from_f32(d, (m, k), api.DType.F32, x)
+    got = d.project_quantized(xt, w).tensor.to_f32()
+    assert d.get_tuning("last_rows_plan") // 1000 == 32
+    with few_rows(d, 2):
+        other = d.project_quantized(xt, w).tensor.to_f32()
+        assert d.get_tuning("last_rows_plan") // 1000 == 16
+    want = x.astype(np.float64) @ oracle.dequantize(ggml, packed, n, k).reshape(n, k).astype(np.float64).T
+    assert rel_l2(got, want) <= rel_l2(other, want)
+
+
 @pytest.mark.parametrize("ggml", [12, 14], ids=["q4_k", "q6_k"])
 def test_f32_batches_with_infinities_and_nan(api, d, ggml):
     # they reach the outputs that the products of the row as it is written give: the same ones as on the f32 instruction
