@@ -272,17 +272,21 @@ constexpr size_t kMostPanelBytes = 256u << 20;
 }  // namespace
 
 // Decode at the rate of its stores, then rounds of the product, the last one cheaper where it is not full; against the
-// fused tiles' estimate.  Both sides in turn, 40 calls each (us, fused tiles / this): Q4_K 1999 x 17408 x 5120 420 / 382,
-// 1999 x 12288 x 4096 230 / 206, 1024 rows 129 / 117; 1999 x 34816 x 5120 780 / 801 and 1999 x 5120 x 17408 343 / 403 stay
-// with the tiles; Q6_K 1999 x 34816 x 5120 946 / 802, 1999 x 17408 x 5120 506 / 391, 1024 x 12288 x 4096 156 / 119; Q8_0 1999
-// x 17408 x 5120 560 / 397, 1024 x 12288 x 4096 191 / 119; Q5_K 1999 x 34816 x 5120 817 / 752, 1500 x 9000 x 3072 133 / 99.
+// fused tiles' estimate.  All sides in turn, bf16, five formats x 20 shapes of 512 - 100000 columns and 512 - 17408 K x nine
+// row counts of 267 - 2048 (900 products, 885 with an estimate): 225 decode, the pick is 0.5% from the fastest of the four
+// in the mean and slower than the fused tiles by more than 3% for two (Q6_K 768 x 28672 x 4096 245 / 271, Q5_K 1500 x 19864
+// x 512 66 / 69).  us, fused tiles / 192 / 256 / 320 columns: Q4_K 1999 x 34816 x 5120 778 / 789 / 752 / 718, 1999 x 17408
+// x 5120 425 / 380 / 414 / 355, 1999 x 12288 x 4096 231 / 208 / 218 / 256, 1999 x 5120 x 17408 352 / 403 / 411 / 461; Q6_K
+// 1999 x 34816 x 5120 925 / 802 / 767 / 730, 1024 x 12288 x 4096 149 / 120 / 124 / 132; Q8_0 1999 x 17408 x 5120 553 / 400
+// / 423 / 367, 1500 x 8192 x 8192 336 / 319 / 221 / 234.
 bool gemm_takes_decoded(GemmArgs& a) {
     if (a.decoded_min_rows == 0 || a.wide32_tile != 0 || a.wide_shape != 1 || !a.resident_switch || a.m <= 256) return false;
     const uint32_t cus = a.cu_count > 0 ? (uint32_t)a.cu_count : 256u, tiles_m = (a.m + 255) / 256;
     const bool forced = a.decoded_min_rows > 1 && a.m >= (uint32_t)a.decoded_min_rows;
-    double best = forced ? 1e300 : gemm_fused_estimate(a) * 1.06;   // (low where the chip is full and hot)
+    const uint32_t asked = (uint32_t)a.decoded_tile;
+    double best = forced ? 1e300 : gemm_fused_estimate(a) * 1.1;   // (low where the chip is full and hot)
     for (const DecodedTile& t : kDecodedTiles) {
-        if (a.decoded_tile != 0 && (uint32_t)a.decoded_tile != t.columns) continue;
+        if (asked != 0 && asked != t.columns) continue;
         const uint64_t most = kMostPanelBytes / ((uint64_t)a.k * 2 * t.columns);
         if (most == 0) continue;
         // as many column tiles to a panel as make whole rounds
@@ -294,7 +298,7 @@ bool gemm_takes_decoded(GemmArgs& a) {
         for (uint32_t first = 0; first < tiles_n; first += tiles) {
             const double rounds = (double)std::min(tiles, tiles_n - first) * tiles_m / cus;
             const double whole = (double)(uint64_t)rounds, part = rounds - whole;
-            us += 5.0 + 14.0 * (whole + (part > 0)) + (whole + (part > 0 ? 0.6 + 0.4 * part : 0.0)) * t.round * a.k / 5120.0;
+            us += 11.0 + 17.0 * (whole + (part > 0)) + (whole + (part > 0 ? 0.6 + 0.4 * part : 0.0)) * t.round * a.k / 5120.0;
         }
         if (us < best) {
             best = us;

@@ -51,6 +51,7 @@ struct fh_device {
     hipDeviceProp_t props{};
     const char* last_operation = "";
     int64_t last_rows_plan = 0;   // of the last dense product: 0, or the few-rows kernel's rows, tiles and K segments
+    int64_t last_decoded_tile = 0;   // ... and 0, or the columns of its tile where its weights were decoded first
     std::atomic<bool> capturing{false};   // changes under pool_lock: what empties the pool waits on the stream
     fh_tuning tuning;
     // Blocks of freed buffers, by size, for the buffers to come (fh_buffer_alloc): hipMalloc and hipFree

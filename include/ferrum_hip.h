@@ -129,7 +129,8 @@ void* fh_device_stream(fh_device* device);
  *                       back what every device object on this GPU keeps
  *   held_scratch_bytes  the operators' common scratch
  *   last_rows_plan      how the last dense product ran on the few-rows kernel: 1000 x activation
- *                       rows (16 or 32) + 100 x weight tiles per wave + K segments; 0 on others */
+ *                       rows (16 or 32) + 100 x weight tiles per wave + K segments; 0 on others
+ *   last_decoded_tile   columns of its tile where it decoded its weights first; 0 on others */
 fh_status fh_set_tuning(fh_device* device, const char* key, int64_t value);
 fh_status fh_get_tuning(const fh_device* device, const char* key, int64_t* value);
 

@@ -1599,6 +1599,33 @@ def test_weights_decoded_first_give_the_bits_of_the_fused_tiles(api, d, ggml, m,
                          "fused tiles")
 
 
+@pytest.mark.parametrize("ggml,m,n,k,tile", [(14, 1024, 12288, 4096, 192), (8, 1999, 7147, 4352, 256), (14, 1500, 8192, 8192, 256),
+                                             (14, 1999, 17408, 5120, 320), (12, 1999, 17408, 5120, 320)])
+def test_the_fastest_of_the_decoded_tiles_is_taken(api, d, ggml, m, n, k, tile):
+    # shapes where one tile is the fastest of three by 5% to 30%, all of them faster than the fused tiles; also where the
+    # caller asks for panels and leaves the tile open
+    base = synth.matrix(ggml, 7, k, seed=781)
+    w = qm(api, d, ggml, n, k, np.resize(base, base.size // 7 * n))
+    xt = api.Tensor.from_f32(d, (m, k), api.DType.BF16, synth.activations(m, k, seed=782))
+    out = api.Tensor.zeros(d, (m, n), api.DType.BF16)
+    d.project_quantized(xt, w, out=out)
+    assert d.get_tuning("last_decoded_tile") == tile
+    first = out.raw()
+    try:
+        d.set_tuning("gemm_decoded_min_rows", m)
+        d.project_quantized(xt, w, out=out)
+        assert d.get_tuning("last_decoded_tile") == tile and np.array_equal(out.raw(), first)
+        d.set_tuning("gemm_decoded_tile", 192 if tile == 256 else 256)
+        d.project_quantized(xt, w, out=out)
+        assert d.get_tuning("last_decoded_tile") == (192 if tile == 256 else 256) and np.array_equal(out.raw(), first)
+        d.set_tuning("gemm_decoded_min_rows", 0)
+        d.project_quantized(xt, w, out=out)
+        assert d.get_tuning("last_decoded_tile") == 0
+    finally:
+        d.set_tuning("gemm_decoded_min_rows", 1)
+        d.set_tuning("gemm_decoded_tile", 0)
+
+
 def test_decoded_panels_take_only_the_room_there_is(api):
     # 1100 x 70000 x 2048 is two panels of at most 256 MiB.  A new device that records has no room for one and takes the
     # fused tiles, which give the same bits; once a plain call has made room, a recording decodes too.
