@@ -284,7 +284,10 @@ bool gemm_takes_decoded(GemmArgs& a) {
     const uint32_t cus = a.cu_count > 0 ? (uint32_t)a.cu_count : 256u, tiles_m = (a.m + 255) / 256;
     const bool forced = a.decoded_min_rows > 1 && a.m >= (uint32_t)a.decoded_min_rows;
     const uint32_t asked = (uint32_t)a.decoded_tile;
-    double best = forced ? 1e300 : gemm_fused_estimate(a) * 1.1;   // (low where the chip is full and hot)
+    // (the fused estimate is low where the chip is full and hot; a product that only the square tiles take, few columns and
+    // rows too long to be resident, has none: 300 x 512 x 4096 36 us there, 71 to 101 here)
+    double best = forced ? 1e300 : gemm_fused_estimate(a) * 1.1;
+    if (!forced && best >= 1e300) return false;
     for (const DecodedTile& t : kDecodedTiles) {
         if (asked != 0 && asked != t.columns) continue;
         const uint64_t most = kMostPanelBytes / ((uint64_t)a.k * 2 * t.columns);

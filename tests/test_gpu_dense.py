@@ -1626,6 +1626,19 @@ def test_the_fastest_of_the_decoded_tiles_is_taken(api, d, ggml, m, n, k, tile):
         d.set_tuning("gemm_decoded_tile", 0)
 
 
+@pytest.mark.parametrize("ggml", [12, 13, 14, 23, 8], ids=["q4_k", "q5_k", "q6_k", "iq4_xs", "q8_0"])
+@pytest.mark.parametrize("m,n,k", [(300, 512, 4096), (384, 512, 5120), (267, 580, 2816), (512, 256, 7168)])
+def test_products_with_few_columns_stay_on_the_square_tiles(api, d, ggml, m, n, k):
+    packed = synth.matrix(ggml, n, k, seed=783)
+    w = qm(api, d, ggml, n, k, packed)
+    x = oracle.round_storage(synth.activations(m, k, seed=784), oracle.F16).reshape(m, k)
+    out = d.project_quantized(api.Tensor.from_f32(d, (m, k), api.DType.F16, x), w, out_dtype=api.DType.F32)
+    assert out.operation.endswith("_gemm_mfma") and d.get_tuning("last_decoded_tile") == 0
+    rows = np.unique(np.concatenate([np.arange(0, 20), np.arange(n - 20, n)]))
+    assert_matmul_parity(out.tensor.to_f32()[:, rows], oracle_columns(ggml, packed, n, k, rows, x, weight_round=oracle.F16, accumulate="f64"),
+                         "square tiles")
+
+
 def test_decoded_panels_take_only_the_room_there_is(api):
     # 1100 x 70000 x 2048 is two panels of at most 256 MiB.  A new device that records has no room for one and takes the
     # fused tiles, which give the same bits; once a plain call has made room, a recording decodes too.
