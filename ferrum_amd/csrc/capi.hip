@@ -116,51 +116,116 @@ bool drain_pools(int ordinal) {
     return any;
 }
 
+// A block from the system; above the device's allocation_limit_bytes the request is one that no GPU has room for.
+hipError_t request(const fh_device* d, void** out, size_t bytes) {
+    const uint64_t limit = (uint64_t)d->tuning.allocation_limit_bytes;
+    return hipMalloc(out, limit != 0 && bytes > limit ? (size_t)1 << 60 : bytes);
+}
+
 // Memory from the system; what the pools on this GPU hold is given back when there is none.
 hipError_t allocate(fh_device* d, void** out, size_t bytes) {
-    hipError_t e = hipMalloc(out, bytes);
+    hipError_t e = request(d, out, bytes);
     if (e == hipErrorOutOfMemory) {
         (void)hipGetLastError();
-        if (drain_pools(d->ordinal)) e = hipMalloc(out, bytes);
+        if (drain_pools(d->ordinal)) e = request(d, out, bytes);
+        if (e == hipErrorOutOfMemory) (void)hipGetLastError();   // the caller's to report: a launch may follow instead
     }
     return e;
 }
 
-// Device scratch: kCounterWords zeroed counter words followed by a data area
-// of at least `data_bytes`.  Growing it waits for the stream first.  Recorded executions
-// carry the scratch address in their kernel arguments, so a block that is outgrown while
-// any of them is alive is kept (they replay on it unchanged) and freed with the last one.
-fh_status ensure_scratch(fh_device* d, size_t data_bytes) {
-    const size_t counter_bytes = fh_device::kCounterWords * sizeof(uint32_t);
-    if (d->scratch != nullptr && d->scratch_bytes >= counter_bytes + data_bytes) return FH_OK;
-    if (d->capturing)
-        return fail(FH_ERR_SYNCHRONIZATION, "device scratch must grow: run the operator once before recording it");
-    FH_HIP(hipStreamSynchronize(d->stream));
-    // at least twice the old data area, so the blocks kept for recordings add up to less than the live one
-    const size_t old_data = d->scratch_bytes > counter_bytes ? d->scratch_bytes - counter_bytes : 0;
-    if (data_bytes < 2 * old_data) data_bytes = 2 * old_data;
-    if (d->scratch) {
-        if (d->live_graphs > 0) {
-            d->retired_scratch.push_back(d->scratch);
-        } else {
-            (void)hipFree(d->scratch);
+constexpr size_t kScratchCounterBytes = fh_device::kCounterWords * sizeof(uint32_t);
+
+bool scratch_holds(const fh_device* d, size_t data_bytes) {
+    return d->scratch != nullptr && d->scratch_bytes >= kScratchCounterBytes + data_bytes;
+}
+
+// A new block for a scratch that holds less; the old one stays until the new one is there.  Recorded executions carry the
+// scratch address in their kernel arguments, so a block that is outgrown while any of them is alive is kept (they replay on
+// it unchanged) and freed with the last one.
+fh_status grow_scratch(fh_device* d, size_t data_bytes, bool optional) {
+    const size_t asked = std::max(data_bytes, fh_device::kScratchFloor);
+    // twice the old data area, so that the blocks kept for recordings add up to less than the live one and growth in small
+    // steps ends; but no more than the largest of the areas that only save time unless a request itself is larger
+    const size_t old_data = d->scratch != nullptr ? d->scratch_bytes - kScratchCounterBytes : 0;
+    size_t data = asked <= fh_device::kScratchOptional ? std::max(asked, std::min(2 * old_data, fh_device::kScratchOptional))
+                  : d->live_graphs > 0                 ? std::max(asked, 2 * old_data)
+                                                       : asked;
+    void* block = nullptr;
+    hipError_t e = allocate(d, &block, kScratchCounterBytes + data);
+    if (e == hipErrorOutOfMemory && data > asked) {
+        data = asked;
+        e = allocate(d, &block, kScratchCounterBytes + data);
+    }
+    if (e == hipErrorOutOfMemory && !optional && d->scratch != nullptr && d->live_graphs == 0) {
+        // the old block may be what is missing; if that is not it either, the device gets its smallest one back
+        FH_HIP(hipStreamSynchronize(d->stream));
+        (void)hipFree(d->scratch);
+        d->scratch = nullptr;
+        d->scratch_bytes = 0;
+        e = allocate(d, &block, kScratchCounterBytes + data);
+        if (e == hipErrorOutOfMemory && data > fh_device::kScratchFloor) {
+            const fh_status st = grow_scratch(d, 0, false);
+            if (st != FH_OK) return st;
         }
     }
-    d->scratch = nullptr;
-    d->scratch_bytes = 0;
-    size_t cap = counter_bytes + std::max(data_bytes, fh_device::kScratchFloor);
-    hipError_t e = allocate(d, &d->scratch, cap);
-    if (e != hipSuccess) return fail(FH_ERR_ALLOCATION, "hipMalloc(%zu): %s", cap, hipGetErrorString(e));
-    d->scratch_bytes = cap;
-    FH_HIP(hipMemsetAsync(d->scratch, 0, counter_bytes, d->stream));
+    if (e != hipSuccess)
+        return fail(FH_ERR_ALLOCATION, "hipMalloc(%zu): %s", kScratchCounterBytes + data, hipGetErrorString(e));
+    e = hipMemsetAsync(block, 0, kScratchCounterBytes, d->stream);
+    if (e == hipSuccess && d->scratch != nullptr && d->live_graphs == 0) e = hipStreamSynchronize(d->stream);
+    if (e != hipSuccess) {
+        (void)hipFree(block);
+        return hip_fail(e, "scratch");
+    }
+    if (d->scratch != nullptr) {
+        if (d->live_graphs > 0) d->retired_scratch.push_back(d->scratch);
+        else (void)hipFree(d->scratch);
+    }
+    d->scratch = block;
+    d->scratch_bytes = kScratchCounterBytes + data;
     return FH_OK;
+}
+
+// Device scratch: kCounterWords zeroed counter words followed by a data area of at least `data_bytes`.
+fh_status ensure_scratch(fh_device* d, size_t data_bytes) {
+    if (scratch_holds(d, data_bytes)) return FH_OK;
+    if (d->capturing)
+        return fail(FH_ERR_SYNCHRONIZATION, "device scratch must grow: run the operator once before recording it");
+    return grow_scratch(d, data_bytes, false);
 }
 
 // Whether the scratch can be brought to `data_bytes` now: it does not grow while an execution is being
 // recorded.  Kernels that only save time by using it leave such a call to those that need none.
-bool scratch_available(const fh_device* d, size_t data_bytes) {
-    return !d->capturing ||
-           (d->scratch != nullptr && d->scratch_bytes >= fh_device::kCounterWords * sizeof(uint32_t) + data_bytes);
+bool scratch_available(const fh_device* d, size_t data_bytes) { return !d->capturing || scratch_holds(d, data_bytes); }
+
+// The same for such a kernel's own needs: FH_ERR_ALLOCATION where there is no room.  A GPU that had none is asked again
+// only after some calls: each request that fails empties the pools, which waits for the stream.
+fh_status optional_scratch(fh_device* d, size_t data_bytes) {
+    constexpr uint32_t kCallsBetween = 256;
+    if (scratch_holds(d, data_bytes)) return FH_OK;
+    if (d->capturing) return FH_ERR_ALLOCATION;
+    if (d->scratch_refused != 0 && data_bytes >= d->scratch_refused && d->scratch_wait > 0) {
+        --d->scratch_wait;
+        return FH_ERR_ALLOCATION;
+    }
+    const fh_status st = grow_scratch(d, data_bytes, true);
+    if (st == FH_ERR_ALLOCATION) {
+        d->scratch_refused = data_bytes;
+        d->scratch_wait = kCallsBetween;
+    } else if (data_bytes >= d->scratch_refused) {
+        d->scratch_refused = 0;
+    }
+    return st;
+}
+
+// Brings the scratch back to its smallest size, unless recorded executions carry its address.
+fh_status shrink_scratch(fh_device* d) {
+    if (d->capturing) return fail(FH_ERR_SYNCHRONIZATION, "not available while an execution is being recorded");
+    if (d->live_graphs > 0 || d->scratch_bytes <= kScratchCounterBytes + fh_device::kScratchFloor) return FH_OK;
+    FH_HIP(hipStreamSynchronize(d->stream));
+    (void)hipFree(d->scratch);
+    d->scratch = nullptr;
+    d->scratch_bytes = 0;
+    return grow_scratch(d, 0, false);
 }
 
 // A block the library owns for its own temporaries (it holds no count on the device), grown like
@@ -370,6 +435,7 @@ constexpr struct {
     {"gemv_stream", &fh_tuning::gemv_stream},
     {"moe_routing_temporary_limit", &fh_tuning::moe_routing_temporary_limit},
     {"gemm_f32_min_rows", &fh_tuning::gemm_f32_min_rows},
+    {"allocation_limit_bytes", &fh_tuning::allocation_limit_bytes},
     {"probe_read_form", &fh_tuning::probe_read_form},
 };
 
@@ -585,6 +651,10 @@ fh_status fh_set_tuning(fh_device* device, const char* key, int64_t value) {
         drain_pools(device->ordinal);
         return FH_OK;
     }
+    if (std::strcmp(key, "held_scratch_bytes") == 0 && value == 0) {
+        FH_HIP(hipSetDevice(device->ordinal));
+        return shrink_scratch(device);
+    }
     int64_t* const setting = tuning_of(device, key);
     if (setting == nullptr) return fail(FH_ERR_PARAMETER, "unknown tuning key %s", key);
     std::string k(key);
@@ -608,7 +678,7 @@ fh_status fh_set_tuning(fh_device* device, const char* key, int64_t value) {
         ok = value >= 1;
     } else if (k == "gemm_skinny_max_rows") {
         ok = value >= 0 && value <= 64;
-    } else if (k == "expert_grouped_min_assignments") {
+    } else if (k == "expert_grouped_min_assignments" || k == "allocation_limit_bytes") {
         ok = value >= 0;
     } else if (k == "gemm_f32_min_rows") {
         ok = value == 0 || value >= 2;
@@ -629,6 +699,10 @@ fh_status fh_get_tuning(const fh_device* device, const char* key, int64_t* value
         return fail(FH_ERR_PARAMETER, "null argument");
     if (std::strcmp(key, "held_scratch_bytes") == 0) {
         *value = (int64_t)device->scratch_bytes;
+        return FH_OK;
+    }
+    if (std::strcmp(key, "retired_scratch_blocks") == 0) {
+        *value = (int64_t)device->retired_scratch.size();
         return FH_OK;
     }
     if (std::strcmp(key, "held_pool_bytes") == 0) {
@@ -931,11 +1005,9 @@ fh_status prepare_gemm(fh_device* device, GemmArgs& g, size_t used) {
     const size_t at = align256(used);
     fh_status st = FH_OK;
     for (;;) {
-        const size_t partial_bytes = gemm_partial_bytes(g), need = partial_bytes != 0 ? at + partial_bytes : used;
-        if (partial_bytes == 0 || scratch_available(device, need)) {
-            st = ensure_scratch(device, need);
-            if (st != FH_ERR_ALLOCATION || partial_bytes == 0) break;
-        }
+        const size_t partial_bytes = gemm_partial_bytes(g);
+        st = partial_bytes != 0 ? optional_scratch(device, at + partial_bytes) : ensure_scratch(device, used);
+        if (st != FH_ERR_ALLOCATION || partial_bytes == 0) break;
         if (g.decoded_columns != 0) {
             g.decoded_columns = 0;
         } else if (g.rows_plan.rows != 0) {

@@ -267,7 +267,7 @@ struct DecodedTile {
     double round;
 };
 constexpr DecodedTile kDecodedTiles[] = {{192, 104.0}, {256, 128.0}, {320, 160.0}};
-constexpr size_t kMostPanelBytes = 256u << 20;
+constexpr size_t kMostPanelBytes = fh_device::kScratchOptional;
 
 }  // namespace
 

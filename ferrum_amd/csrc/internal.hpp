@@ -38,6 +38,7 @@ struct fh_tuning {
     int64_t gemv_stream = 1;           // dense Q4_K / Q6_K GEMV on the streamed matrix-core kernel: 0 never, 1 where it wins, 2 wherever it runs
     int64_t moe_routing_temporary_limit = 128ll << 20;  // bytes of routing temporaries per SparseMoe chunk (src/metal/legacy.rs:95)
     int64_t gemm_f32_min_rows = 0;     // f32 activations take the f16 tile kernels from this many rows (0 = never)
+    int64_t allocation_limit_bytes = 0;  // requests for more fail as on a GPU without room (0 = none)
     int64_t probe_read_form = 0;       // fh_probe_read: 100 x threads per workgroup + loads per lane (+ 1000000: LDS-direct loads); 0 = 256 x 8
 };
 
@@ -71,6 +72,9 @@ struct fh_device {
     void* fixed_scratch = nullptr;
     static constexpr size_t kCounterWords = 1u << 16;
     static constexpr size_t kScratchFloor = 16u << 20;   // the data area is never smaller
+    static constexpr size_t kScratchOptional = 256u << 20;   // nor grown beyond this by kernels that only save time by it
+    size_t scratch_refused = 0;      // bytes such a kernel asked for in vain (0 = none)
+    uint32_t scratch_wait = 0;       // calls that take it for refused before the next request
     // Releases asked for while an execution is being recorded wait for its end:
     // freeing or synchronizing inside a stream capture would invalidate it.
     // scratch blocks that were outgrown while recorded executions (which carry their address)

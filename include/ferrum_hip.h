@@ -127,7 +127,9 @@ void* fh_device_stream(fh_device* device);
  * fh_get_tuning alone also answers for what the library does by itself:
  *   held_pool_bytes     freed buffers kept for the next ones (see below); fh_set_tuning with 0 gives
  *                       back what every device object on this GPU keeps
- *   held_scratch_bytes  the operators' common scratch
+ *   held_scratch_bytes  the operators' common scratch; fh_set_tuning with 0 brings it back to its smallest
+ *                       size where no recorded execution uses it
+ *   retired_scratch_blocks  scratch blocks that were outgrown and that recorded executions still use
  *   last_rows_plan      how the last dense product ran on the few-rows kernel: 1000 x activation
  *                       rows (16 or 32) + 100 x weight tiles per wave + K segments; 0 on others
  *   last_decoded_tile   columns of its tile where it decoded its weights first; 0 on others */

@@ -860,6 +860,74 @@ def test_partial_sums_of_tiles_take_only_the_room_there_is(api):
         assert np.array_equal(bits(again.to_f32()), bits(direct))
 
 
+@pytest.mark.parametrize("live_graph", [False, True])
+@pytest.mark.parametrize("ggml,m,n,k,wanted", [(Q4_K, 512, 5120, 17408, 42), (Q6_K, 1500, 8192, 4096, 67)])
+def test_products_run_without_the_scratch_they_would_like(api, live_graph, ggml, m, n, k, wanted):
+    # planes of partial sums and a panel of decoded weights, on a GPU that has no room for them: a limit on single
+    # allocations makes the request a real one that fails.  No error, no block changes hands, and the GPU is not asked again
+    # on every call; once there is room, the scratch grows to what is asked for.
+    dev = api.Device.new()
+    base = synth.matrix(ggml, 64, k, seed=185)
+    w = qm(api, dev, ggml, n, k, np.resize(base, base.size // 64 * n))
+    x = api.Tensor.from_f32(dev, (m, k), api.DType.F16, synth.activations(m, k, seed=186, f16=True))
+    y, held = api.Tensor.zeros(dev, (m, n), api.DType.F32), dev.get_tuning("held_scratch_bytes")
+    graph = None
+    if live_graph:
+        with dev.execution() as ex:
+            dev.project_quantized(x, w, out=y)
+        graph = ex.graph
+    dev.set_tuning("allocation_limit_bytes", 20 << 20)
+    dev.project_quantized(x, w, out=y)
+    first = y.to_f32()
+    for _ in range(3):
+        dev.project_quantized(x, w, out=y)
+        assert dev.get_tuning("held_scratch_bytes") == held and dev.get_tuning("retired_scratch_blocks") == 0
+    assert np.array_equal(bits(y.to_f32()), bits(first))
+    dev.set_tuning("allocation_limit_bytes", 0)
+    dev.project_quantized(x, w, out=y)
+    assert dev.get_tuning("held_scratch_bytes") == held      # one that failed just now is not asked for again
+    for _ in range(600):      # ... before 256 calls have done without (a product may try two sizes)
+        dev.project_quantized(x, w, out=y)
+    dev.synchronize()
+    grown = dev.get_tuning("held_scratch_bytes")
+    assert wanted * 10 ** 6 <= grown <= (wanted + 1) * 10 ** 6 + (1 << 20)
+    assert dev.get_tuning("retired_scratch_blocks") == (1 if live_graph else 0)
+    assert rel_l2(y.to_f32(), first) <= 1e-5
+    dev.set_tuning("held_scratch_bytes", 0)
+    assert dev.get_tuning("held_scratch_bytes") == (grown if live_graph else held)
+    if live_graph:
+        graph.launch()
+        dev.synchronize()
+        assert np.array_equal(bits(y.to_f32()), bits(first))
+        ex.graph = graph = None
+        assert dev.get_tuning("retired_scratch_blocks") == 0
+        dev.set_tuning("held_scratch_bytes", 0)
+        assert dev.get_tuning("held_scratch_bytes") == held
+    dev.project_quantized(x, w, out=y)
+    assert rel_l2(y.to_f32(), first) <= 1e-5
+
+
+def test_a_required_scratch_that_cannot_grow_is_an_error_and_nothing_is_lost(api):
+    dev = api.Device.new()
+    n, k, m = 96, 8192, 3000        # f32 rows rounded into the scratch: 49 MB
+    packed = synth.matrix(Q4_K, n, k, seed=187)
+    w = qm(api, dev, Q4_K, n, k, packed)
+    x = api.Tensor.from_f32(dev, (m, k), api.DType.F32, synth.activations(m, k, seed=188))
+    few = api.Tensor.from_f32(dev, (8, k), api.DType.F32, synth.activations(8, k, seed=189))
+    dev.set_tuning("gemm_f32_min_rows", 5)
+    before = dev.project_quantized(few, w).tensor.to_f32()
+    dev.set_tuning("allocation_limit_bytes", 20 << 20)
+    for _ in range(2):
+        with pytest.raises(Exception, match="hipMalloc"):
+            dev.project_quantized(x, w)
+        assert np.array_equal(bits(dev.project_quantized(few, w).tensor.to_f32()), bits(before))
+    dev.set_tuning("allocation_limit_bytes", 0)
+    out = dev.project_quantized(x, w).tensor.to_f32()
+    rows = np.arange(n)
+    rounded = oracle.round_storage(x.to_f32()[:8], oracle.F16).reshape(8, k)
+    assert_matmul_parity(out[:8], oracle_columns(Q4_K, packed, n, k, rows, rounded, weight_round=oracle.F16, accumulate="f64"), "grown")
+
+
 @pytest.mark.parametrize("m", [80, 128, 200, 330, 512])
 def test_the_tile_picked_by_row_count_gives_the_bits_of_the_largest(api, d, m):
     # 17000 columns at every row count that changes the tile (128 x 68 of the 96-column tile up to
