@@ -1010,6 +1010,9 @@ fh_status prepare_gemm(fh_device* device, GemmArgs& g, size_t used) {
         if (st != FH_ERR_ALLOCATION || partial_bytes == 0) break;
         if (g.decoded_columns != 0) {
             g.decoded_columns = 0;
+        } else if (g.rows_plan.pairs) {
+            g.rows_plan = g.rows_else;
+            if (g.rows_plan.rows == 0) return ensure_scratch(device, used);
         } else if (g.rows_plan.rows != 0) {
             g.rows_plan = RowsPlan{};
             if (g.x_dtype == FH_F32) return ensure_scratch(device, used);   // no tile takes exact f32 rows
@@ -1114,8 +1117,10 @@ fh_status project(fh_device* device, const fh_qmatrix* weight, const fh_view* x,
             (!g.few_rows_always && !gemv_streams(device, weight->ggml_type, n, k, m) &&
              !f32_rows_pay(g.rows_plan, g.ggml_type, g.n, g.k, m, g.cu_count)))
             g.rows_plan = RowsPlan{};
-        if (!g.few_rows_always && pairs_pay(g.ggml_type, g.n, g.k, m) && ((uintptr_t)xr.begin & 15u) == 0)
+        if (!g.few_rows_always && pairs_pay(g.ggml_type, g.n, g.k, m) && ((uintptr_t)xr.begin & 15u) == 0) {
+            g.rows_else = g.rows_plan;
             g.rows_plan = gemm_pairs_plan(g.n, g.k, g.m, g.cu_count);
+        }
     }
     if (tile && !gemm_takes_rows(g)) gemm_takes_decoded(g);
     if (tile || g.rows_plan.rows != 0) {

@@ -373,6 +373,7 @@ struct GemmArgs {
     bool few_rows;        // the few-rows kernel may take the product (gemm_takes_rows)
     bool few_rows_always; // ... and does, whatever the estimates say
     RowsPlan rows_plan;   // set by gemm_takes_rows; its K segments and the tiles' meet in these:
+    RowsPlan rows_else;   // where rows_plan is of pairs and has no room: the f32 instruction's, or none
     float* partials;
     uint32_t* counters;
     bool weight_ring;     // routed form, rows resident: Q4_K and Q6_K weights through LDS rings where they fit beside the rows

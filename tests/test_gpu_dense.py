@@ -1617,6 +1617,30 @@ def test_f32_batches_as_pairs_are_no_farther_from_64_bits_than_on_the_f32_instru
     assert rel_l2(got, want) <= rel_l2(other, want)
 
 
+def test_f32_batches_without_room_for_pairs_take_the_f32_instruction(api):
+    # 43000 x 4352: the operands of 32 rows and their sums of three K segments are 17.1 MB, more than the scratch of a
+    # new device holds while it records
+    dev = api.Device.new()
+    m, n, k = 32, 43000, 4352
+    base = synth.matrix(Q4_K, 100, k, seed=747)
+    w = qm(api, dev, Q4_K, n, k, np.resize(base, base.size // 100 * n))
+    x = synth.activations(m, k, seed=748).reshape(m, k)
+    xt = api.Tensor.from_f32(dev, (m, k), api.DType.F32, x)
+    recorded = api.Tensor.zeros(dev, (m, n), api.DType.F32)
+    with dev.execution() as ex:
+        dev.project_quantized(xt, w, out=recorded)
+    assert dev.get_tuning("last_rows_plan") // 1000 == 16
+    with few_rows(dev, 2):
+        other = dev.project_quantized(xt, w).tensor.to_f32()
+    got = dev.project_quantized(xt, w).tensor.to_f32()
+    assert dev.get_tuning("last_rows_plan") // 1000 == 32
+    for _ in range(2):
+        ex.graph.launch()
+        dev.synchronize()
+        assert np.array_equal(bits(recorded.to_f32()), bits(other))
+    assert rel_l2(got, other) <= 2.6e-7 and np.array_equal(bits(got[:, :100]), bits(got[:, 42900:]))
+
+
 @pytest.mark.parametrize("ggml", [12, 14], ids=["q4_k", "q6_k"])
 def test_f32_batches_with_infinities_and_nan(api, d, ggml):
     # they reach the outputs that the products of the row as it is written give: the same ones as on the f32 instruction
