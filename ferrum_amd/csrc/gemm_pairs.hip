@@ -22,8 +22,8 @@
 // every weight once per 16 rows.
 //
 // What bounds it: the waves' own instructions.  24 x 28672 x 4096 takes 37 us; with no weight or operand on its way in the
-// loop 30, also without decode 29, with half the multiplications 28: eight waves a compute unit (136 KB of operands, 217 -
-// 243 registers) do not hide the vector instructions of one behind the matrix instructions of another as four would.
+// loop 30, also without decode 29, with half the multiplications 28: eight waves a compute unit (136 KB of operands, 222 -
+// 247 registers) do not hide the vector instructions of one behind the matrix instructions of another as four would.
 //
 // A workgroup is eight waves: two halves of K (every other super-block) x four tiles of 32 weight rows; all 32 rows of
 // the batch's group at once.  A super-block's operands are brought into LDS by LDS-direct loads one super-block ahead
@@ -83,9 +83,10 @@ __global__ __launch_bounds__(256) void split_rows_kernel(const float* __restrict
         uint32_t most = 0;
 #pragma unroll
         for (int j = 0; j < 4; ++j) most = max(most, __float_as_uint(e[j]) & 0x7fffffffu);
+        const bool has_nan = __ballot(most > 0x7f800000u) != 0;
         most = __float_as_uint(wave_max(__uint_as_float(min(most, 0x7f800000u))));   // (NaN counts as an infinity)
-        // (a super-block with an infinity or a NaN has no such scale: it counts as zeros and a NaN inverse, and whoever
-        // meets a NaN sum takes the plain products)
+        // (a super-block with an infinity or a NaN has no such scale: it counts as zeros and an infinite or NaN inverse,
+        // either of which makes the sum NaN: resolve_nan)
         const bool finite = most < 0x7f800000u;
         const uint32_t exponent = min(max(268u - (most >> 23), 1u), 253u);
         const float s = __uint_as_float(exponent << 23), inverse = __uint_as_float((254u - exponent) << 23);
@@ -108,7 +109,8 @@ __global__ __launch_bounds__(256) void split_rows_kernel(const float* __restrict
         if ((lane & 7u) == 0)
             *reinterpret_cast<float*>(base + kSumsAt + (g & 3u) * 256 + (row + 32 * (g >> 2)) * 4) = (float)sum;
         if (lane == 0)
-            *reinterpret_cast<float*>(base + kInverseAt + 4 * row) = finite ? inverse : __uint_as_float(0x7fc00000u);
+            *reinterpret_cast<float*>(base + kInverseAt + 4 * row) =
+                finite ? inverse : __uint_as_float(has_nan ? 0x7fc00000u : 0x7f800000u);
     }
 }
 
@@ -351,13 +353,71 @@ __device__ __forceinline__ float weight_of(const uint8_t* w, uint32_t row, uint3
     else return iq4xs_weight(w, row, column, nb);
 }
 
-// The product of one row and one weight row as it is written: for rows with infinities or NaN, whose sums the split
-// cannot give (an output that overflows on the way, or of a NaN scale, comes here too and stays what it is).
+// A wave's sums that are NaN, for a row of the batch with infinities but no NaN (x, and its inverse scales, which say
+// which super-blocks have them): the products of the infinities and the lane's weight row are what decides.  `sum` is 0, or NaN where the
+// weights themselves have a scale that is not finite.  Over as soon as every lane has met a NaN (infinities of both
+// signs, or one times a weight of zero).
 template <uint32_t TYPE>
-__device__ __attribute__((noinline)) float plain_product(const uint8_t* w, const float* x, uint32_t row, uint32_t nb) {
-    float sum = 0.f;
-    for (uint32_t k = 0; k < nb * 256; ++k) sum = fmaf(weight_of<TYPE>(w, row, k, nb), x[k], sum);
+__device__ __attribute__((noinline)) float infinite_products(const uint8_t* w, const float* x, const uint8_t* inverse, uint32_t row,
+                                                             uint32_t nb, float sum) {
+    const uint32_t lane = threadIdx.x & 63u;
+    for (uint32_t b0 = 0; b0 < nb; b0 += 64) {
+        const float f = *reinterpret_cast<const float*>(inverse + (size_t)min(b0 + lane, nb - 1) * kOperandBytes);
+        uint64_t blocks = __ballot(b0 + lane < nb && __builtin_isinf(f));
+        for (; blocks != 0; blocks &= blocks - 1) {
+            const uint32_t b = b0 + (uint32_t)__builtin_ctzll(blocks);
+            const float4 v = *reinterpret_cast<const float4*>(x + (size_t)b * 256 + 4 * lane);
+            const float e[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+            for (uint32_t j = 0; j < 4; ++j) {
+                uint64_t lanes = __ballot(__builtin_isinf(e[j]));
+                for (; lanes != 0; lanes &= lanes - 1) {
+                    const uint32_t from = (uint32_t)__builtin_ctzll(lanes);
+                    sum = fmaf(weight_of<TYPE>(w, row, b * 256 + 4 * from + j, nb), __shfl(e[j], (int)from, 64), sum);
+                    if (__ballot(sum == sum) == 0) return sum;
+                }
+            }
+        }
+    }
     return sum;
+}
+
+// The sums of a wave, COUNT a lane, where one is NaN: v[i] of lane half kg belongs to row first(i) + kg * step of the
+// group.  Rows with a NaN keep it; rows with infinities get their products' sum; any other NaN (a scale of the weights, an overflow
+// in both directions) stays.  24 x 5120 x 17408 Q6_K, us: finite rows 52, NaN rows 57, one infinity 95, one in every row 132,
+// all of every row 180.  (Multiplying a row out again, value by value, took 4 ms, for all rows 65.)
+template <uint32_t TYPE, int COUNT, class First>
+__device__ __forceinline__ void resolve_nan(const PairsParams& p, float (&v)[COUNT], uint32_t group, uint32_t row, First&& first,
+                                            uint32_t step) {
+    uint64_t any = 0;
+#pragma unroll
+    for (int i = 0; i < COUNT; ++i) any |= __ballot(v[i] != v[i]);
+    if (any == 0) return;
+    const uint32_t lane = threadIdx.x & 63u, kg = lane >> 5;
+    const uint8_t* const inverse = p.operands + (size_t)group * p.nb * kOperandBytes + kInverseAt;
+    bool nan = false, infinite = false;   // of row lane % 32, every other super-block
+    for (uint32_t b = kg; b < p.nb; b += 2) {
+        const float f = *reinterpret_cast<const float*>(inverse + (size_t)b * kOperandBytes + 4 * (lane & 31u));
+        nan = nan || f != f;
+        infinite = infinite || __builtin_isinf(f);
+    }
+    const uint64_t nans = __ballot(nan), infinities = __ballot(infinite);
+    const uint32_t rows = ((uint32_t)infinities | (uint32_t)(infinities >> 32)) & ~((uint32_t)nans | (uint32_t)(nans >> 32));
+    if (rows == 0) return;
+    const uint32_t weight_row = min(row, p.n - 1);
+    float zero = 0.f;
+    for (uint32_t b = 0; b < p.nb; ++b) zero = fmaf(weight_of<TYPE>(p.w, weight_row, b * 256, p.nb), 0.f, zero);
+#pragma unroll
+    for (int i = 0; i < COUNT; ++i) {
+#pragma unroll
+        for (uint32_t h = 0; h < 2; ++h) {
+            const uint32_t t = first(i) + h * step;
+            if ((rows >> t & 1u) == 0) continue;
+            const float sum = infinite_products<TYPE>(p.w, p.x + (size_t)(group * kGroupRows + t) * p.nb * 256, inverse + 4 * t, weight_row,
+                                                      p.nb, zero);
+            if (kg == h) v[i] = sum;
+        }
+    }
 }
 
 template <uint32_t TYPE>
@@ -520,26 +580,24 @@ __global__ __launch_bounds__(kThreads) void gemm_pairs_kernel(const PairsParams 
     }
     __syncthreads();
     const uint32_t m0 = group * kGroupRows;
-    auto store = [&](uint32_t token, float v) {
-        if (v != v) v = plain_product<TYPE>(p.w, p.x + (size_t)token * p.nb * 256, row, p.nb);
-        store_from_f32(p.y, (size_t)token * p.n + row, p.y_dtype, v);
-    };
     if (half == 0) {
+        float sum[16];
 #pragma unroll
-        for (int v4 = 0; v4 < 4; ++v4) {
-            const double2 first = exchange[128 * v4], second = exchange[128 * v4 + 64];
-            const double o[4] = {first.x, first.y, second.x, second.y};
+        for (int v = 0; v < 8; ++v) {
+            const double2 other = exchange[64 * v];
+            sum[2 * v] = (float)(acc[2 * v] + other.x);
+            sum[2 * v + 1] = (float)(acc[2 * v + 1] + other.y);
+        }
+        if (p.segments == 1) resolve_nan<TYPE>(p, sum, group, row, [](int v) { return (uint32_t)(8 * (v / 4) + v % 4); }, 4);
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const uint32_t token = m0 + 8 * v4 + 4 * kg + j;
-                const float sum = (float)(acc[4 * v4 + j] + o[j]);
-                if (row < p.n && token < p.m) {
-                    if (p.segments == 1)
-                        store(token, sum);
-                    else   // device scope: coherent across the chip's L2 slices without cache-wide flushes
-                        __hip_atomic_store(p.partials + ((size_t)segment * p.m + token) * p.n + row, sum, __ATOMIC_RELAXED,
-                                           __HIP_MEMORY_SCOPE_AGENT);
-                }
+        for (int v = 0; v < 16; ++v) {
+            const uint32_t token = m0 + 8 * (v / 4) + 4 * kg + v % 4;
+            if (row < p.n && token < p.m) {
+                if (p.segments == 1)
+                    store_from_f32(p.y, (size_t)token * p.n + row, p.y_dtype, sum[v]);
+                else   // device scope: coherent across the chip's L2 slices without cache-wide flushes
+                    __hip_atomic_store(p.partials + ((size_t)segment * p.m + token) * p.n + row, sum[v], __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_AGENT);
             }
         }
     }
@@ -554,13 +612,13 @@ __global__ __launch_bounds__(kThreads) void gemm_pairs_kernel(const PairsParams 
         last_flag = last;
     }
     __syncthreads();
-    if (last_flag == 0 || row >= p.n) return;
+    if (last_flag == 0) return;
     // the last workgroup to arrive adds the segments in order; both halves of it, sixteen rows each, four segments of
     // eight outputs on their way at a time (one load after the other took longer than the product)
     double total[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) total[j] = 0.0;
-    const float* const from = p.partials + row;
+    const float* const from = p.partials + min(row, p.n - 1);
     for (uint32_t s0 = 0; s0 < p.segments; s0 += 4) {
         float part[4][8];
 #pragma unroll
@@ -578,10 +636,14 @@ __global__ __launch_bounds__(kThreads) void gemm_pairs_kernel(const PairsParams 
                 for (uint32_t j = 0; j < 8; ++j) total[j] += (double)part[s][j];
             }
     }
+    float sum[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) sum[j] = (float)total[j];
+    resolve_nan<TYPE>(p, sum, group, row, [half](int j) { return 16 * half + 2 * (uint32_t)j; }, 1);
 #pragma unroll
     for (uint32_t j = 0; j < 8; ++j) {
         const uint32_t token = m0 + 16 * half + 2 * j + kg;
-        if (token < p.m) store(token, (float)total[j]);
+        if (row < p.n && token < p.m) store_from_f32(p.y, (size_t)token * p.n + row, p.y_dtype, sum[j]);
     }
 }
 

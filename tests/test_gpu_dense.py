@@ -1661,6 +1661,56 @@ def test_f32_batches_with_infinities_and_nan(api, d, ggml):
     assert rel_l2(got[fine], want[fine]) <= 2.6e-7
 
 
+@pytest.mark.parametrize("ggml", [12, 13, 14, 23], ids=["q4_k", "q5_k", "q6_k", "iq4_xs"])
+@pytest.mark.parametrize("m,n,k", [(20, 33000, 512), (60, 2573, 17408)])
+def test_infinities_in_f32_batches_are_the_products_of_the_infinite_values(api, d, ggml, m, n, k):
+    # one and several K segments; infinities of one sign and of both, in one super-block and in many, in many rows at once,
+    # beside a NaN
+    packed = synth.matrix(ggml, n, k, seed=755)
+    w = qm(api, d, ggml, n, k, packed)
+    x = np.asarray(synth.activations(m, k, seed=756), dtype=np.float32).reshape(m, k)
+    x[0, k - 1] = np.inf
+    x[1, 3], x[1, 4] = np.inf, -np.inf
+    x[2, ::97] = -np.inf
+    x[3] = np.inf
+    x[4], x[4, 5] = np.inf, np.nan
+    x[5, 255], x[5, 256] = -np.inf, -np.inf
+    x[6] = np.nan
+    x[m - 1, k // 2 + 1] = np.nan
+    x[m - 9:m - 2, 40] = np.inf
+    xt = api.Tensor.from_f32(d, x.shape, api.DType.F32, x)
+    got = d.project_quantized(xt, w).tensor.to_f32()
+    assert d.get_tuning("last_rows_plan") // 1000 == 32
+    rows = np.unique(np.concatenate([np.arange(0, 130), np.arange(n - 130, n)]))
+    row_bytes = packed.size // n
+    weights = oracle.dequantize(ggml, np.ascontiguousarray(packed.reshape(n, row_bytes)[rows]).reshape(-1), len(rows), k)
+    with np.errstate(invalid="ignore"):
+        want = x.astype(np.float64) @ weights.reshape(len(rows), k).astype(np.float64).T
+    out = got[:, rows]
+    assert np.array_equal(np.isnan(out), np.isnan(want)) and np.isnan(got[[4, 6, m - 1]]).all()
+    inf = np.isinf(want)
+    assert np.array_equal(np.isinf(out), inf) and np.array_equal(out[inf], want[inf]) and inf[0].any() and inf[m - 5].any()
+    fine = [r for r in range(7, m - 9)]
+    assert rel_l2(out[fine], want[fine]) <= 1.6e-7
+
+
+@pytest.mark.parametrize("value", [np.nan, np.inf])
+def test_values_that_are_not_finite_do_not_multiply_the_time_of_a_batch(api, d, value):
+    # some 40 us with finite rows; 60 ms when every output was multiplied out again
+    m, n, k = 24, 2573, 17408
+    w = qm(api, d, Q6_K, n, k, synth.matrix(Q6_K, n, k, seed=757))
+    x = np.asarray(synth.activations(m, k, seed=758), dtype=np.float32).reshape(m, k)
+    x[:, 77] = value
+    xt, y = api.Tensor.from_f32(d, (m, k), api.DType.F32, x), api.Tensor.zeros(d, (m, n), api.DType.F32)
+    d.project_quantized(xt, w, out=y)
+    start, end = api.Event(d), api.Event(d)
+    start.record()
+    d.project_quantized(xt, w, out=y)
+    end.record()
+    d.synchronize()
+    assert start.elapsed_ms(end) < 3.0
+
+
 @pytest.mark.parametrize("ggml", [12, 13, 14, 23, 8], ids=["q4_k", "q5_k", "q6_k", "iq4_xs", "q8_0"])
 @pytest.mark.parametrize("m,n,k,dtype", [(257, 33, 256, "F16"), (300, 1000, 512, "BF16"), (513, 2571, 1280, "F16"), (700, 517, 2304, "BF16")])
 def test_weights_decoded_first_give_the_bits_of_the_fused_tiles(api, d, ggml, m, n, k, dtype):
