@@ -862,13 +862,14 @@ __device__ __forceinline__ void lds_direct16(const void* g, uint32_t lds_addr) {
 }
 
 // Where the tiles alone would leave part of the chip idle, K is cut into segments of `seg_blocks`
-// super-blocks each: segment s writes its f32 sums to plane s of y, which is then the scratch, and
-// add_segments_kernel adds the planes.
+// super-blocks each, the first `longer` of them one more: segment s writes its f32 sums to plane s of y, which is then the
+// scratch, and add_segments_kernel adds the planes.
 template <uint32_t TYPE, int DT, int NT, int RT>
 __global__ __launch_bounds__(512) void gemm_wide32_kernel(const uint8_t* __restrict__ w,
                                                           const uint16_t* __restrict__ x,
                                                           void* __restrict__ y, uint32_t m, uint32_t n,
-                                                          uint32_t row_blocks, uint32_t seg_blocks, uint32_t y_dtype,
+                                                          uint32_t row_blocks, uint32_t seg_blocks, uint32_t longer,
+                                                          uint32_t y_dtype,
                                                           uint32_t cols, uint32_t tiles_m, uint32_t tiles_n,
                                                           uint32_t segments) {
     extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
@@ -896,7 +897,8 @@ __global__ __launch_bounds__(512) void gemm_wide32_kernel(const uint8_t* __restr
     const uint32_t n0 = tile_n * cols, m0 = tile_m * Geo::kTileRows;
     const uint32_t ncols = n - n0 < cols ? n - n0 : cols;
     const uint32_t k = row_blocks << 8;
-    const uint32_t first = segment * seg_blocks, nb = min(seg_blocks, row_blocks - first);   // this segment's super-blocks
+    // this segment's super-blocks
+    const uint32_t first = segment * seg_blocks + min(segment, longer), nb = seg_blocks + (segment < longer ? 1u : 0u);
     w += (size_t)first * kBlockBytes;
     x += (size_t)first * 256;
     if (segments > 1) y = static_cast<float*>(y) + (size_t)segment * m * n;
@@ -1214,12 +1216,13 @@ double wide32_estimate(const Wide32Tile& t, uint32_t ggml_type, uint32_t seg_blo
 constexpr size_t kMostSegmentBytes = 48u << 20;   // scratch for partial sums: one round of the largest tile is 42 MB
 size_t segment_bytes(uint32_t m, uint32_t n, uint32_t segments) { return (size_t)segments * m * n * sizeof(float); }
 
-// Cuts K into exactly `segments` runs of super-blocks, none shorter than four (sixteen slabs); false: it does not go.
+// Cuts K into `segments` runs of super-blocks that differ by one at most, none shorter than four (sixteen slabs); false:
+// it does not go.  seg_blocks is the longest.
 bool wide32_cut(WidePlan& p, uint32_t k, uint32_t segments) {
     const uint32_t nb = k / 256;
     p.segments = segments;
     p.seg_blocks = (nb + segments - 1) / segments;
-    return (nb + p.seg_blocks - 1) / p.seg_blocks == segments && (segments == 1 || nb / segments >= 4);
+    return segments == 1 || nb / segments >= 4;
 }
 
 // The launch that adds the segments and what writing and reading their sums takes.
@@ -1305,7 +1308,8 @@ void launch_wide32(hipStream_t s, const GemmArgs& a, const WidePlan& plan) {
     const bool cut = plan.segments > 1;
     hipLaunchKernelGGL((gemm_wide32_kernel<TYPE, DT, NT, RT>), grid, dim3(512), lds, s,
                        static_cast<const uint8_t*>(a.w), static_cast<const uint16_t*>(a.x), cut ? a.partials : a.y, a.m, a.n,
-                       a.k / 256, plan.seg_blocks, cut ? (uint32_t)FH_F32 : a.y_dtype, plan.cols, plan.tiles_m, plan.tiles_n,
+                       a.k / 256, a.k / 256 / plan.segments, a.k / 256 % plan.segments,
+                       cut ? (uint32_t)FH_F32 : a.y_dtype, plan.cols, plan.tiles_m, plan.tiles_n,
                        plan.segments);
     if (!cut) return;
     const uint32_t count = a.m * a.n;

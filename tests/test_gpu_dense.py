@@ -828,6 +828,36 @@ def test_tiles_whose_k_is_cut_into_segments(api, d, ggml, m, n, k, segments, dty
         d.set_tuning("gemm_wide32_tile", 0)
 
 
+@pytest.mark.parametrize("m,n,blocks,segments,last", [(40, 131, 21, 5, 17), (65, 70, 36, 8, 32), (129, 96, 32, 7, 28), (33, 64, 17, 4, 13)])
+def test_segments_of_tiles_differ_by_one_super_block_at_most(api, d, m, n, blocks, segments, last):
+    # 21 super-blocks in five segments are 5 4 4 4 4 and not 5 5 5 5 1.  Where the last segment begins shows in what
+    # cancels: big values of opposite sign in the super-blocks before and at its first one meet after the segments' own sums,
+    # so a small value behind the second of them is lost there, and kept if both lie in one segment.
+    k = blocks * 256
+    packed = synth.matrix(Q4_K, n, k, seed=183)
+    w = qm(api, d, Q4_K, n, k, packed)
+    x = oracle.round_storage(synth.activations(m, k, seed=184), oracle.F16).reshape(m, k)
+    weights = oracle.round_storage(oracle.dequantize(Q4_K, packed, n, k), oracle.F16).reshape(n, k)
+    split = np.zeros((m, k), dtype=np.float32)
+    split[0, (last + 1) * 256 - 1] = 2.0 ** -14
+    kept = split[0] @ weights.T
+    at = (last - 1) * 256 + 255, last * 256      # neighbours on either side of the boundary
+    split[0, at[0]], split[0, at[1]] = -16384.0, 16384.0
+    try:
+        d.set_tuning("gemm_wide32_segments", segments)
+        for tile in (12, 15, 24):
+            d.set_tuning("gemm_wide32_tile", tile)
+            got = d.project_quantized(api.Tensor.from_f32(d, (m, k), api.DType.F16, x), w, out_dtype=api.DType.F32).tensor.to_f32()
+            assert_matmul_parity(got, x.astype(np.float64) @ weights.T.astype(np.float64), f"tile {tile}")
+            got = d.project_quantized(api.Tensor.from_f32(d, (m, k), api.DType.F16, split), w, out_dtype=api.DType.F32).tensor.to_f32()
+            # plane `segments - 1` is fl(16384 w + small), the one before it -16384 w' exactly
+            want = (np.float32(-16384.0) * weights[:, at[0]]) + (np.float32(16384.0) * weights[:, at[1]] + kept).astype(np.float32)
+            assert np.array_equal(got[0], want.astype(np.float32)), tile
+    finally:
+        d.set_tuning("gemm_wide32_segments", 0)
+        d.set_tuning("gemm_wide32_tile", 0)
+
+
 def test_partial_sums_of_tiles_take_only_the_room_there_is(api):
     # 512 x 5120 x 17408 in four segments: 42 MB of sums, which the scratch of a new device does not hold.  While it
     # records the device takes another kernel; a plain call grows the scratch, and the recording stays what it was.
