@@ -674,6 +674,12 @@ fh_status fh_set_tuning(fh_device* device, const char* key, int64_t value) {
         ok = value >= 0 && value <= 2;
     } else if (k == "gemm_wide32_tile") {
         ok = value == 0 || value == 12 || value == 13 || value == 14 || value == 15 || value == 24 || value == 25;
+    } else if (k == "gemm_wide32_segments") {
+        ok = value >= 0 && value <= 8;
+    } else if (k == "gemm_decoded_min_rows") {
+        ok = value >= 0 && value <= INT32_MAX;
+    } else if (k == "gemm_decoded_tile") {
+        ok = value == 0 || value == 192 || value == 256 || value == 320;
     } else if (k == "gemm_wide_min_rows") {
         ok = value >= 1;
     } else if (k == "gemm_skinny_max_rows") {

@@ -282,7 +282,8 @@ constexpr size_t kMostPanelBytes = fh_device::kScratchOptional;
 bool gemm_takes_decoded(GemmArgs& a) {
     if (a.decoded_min_rows == 0 || a.wide32_tile != 0 || a.wide_shape != 1 || !a.resident_switch || a.m <= 256) return false;
     const uint32_t cus = a.cu_count > 0 ? (uint32_t)a.cu_count : 256u, tiles_m = (a.m + 255) / 256;
-    const bool forced = a.decoded_min_rows > 1 && a.m >= (uint32_t)a.decoded_min_rows;
+    const bool forced = a.decoded_min_rows > 1;   // from that many rows on, whatever the estimates say
+    if (forced && a.m < (uint32_t)a.decoded_min_rows) return false;
     const uint32_t asked = (uint32_t)a.decoded_tile;
     // (the fused estimate is low where the chip is full and hot; a product that only the square tiles take, few columns and
     // rows too long to be resident, has none: 300 x 512 x 4096 36 us there, 71 to 101 here)

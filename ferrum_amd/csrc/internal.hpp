@@ -22,8 +22,8 @@ struct fh_tuning {
     int64_t gemm_min_rows = 2;         // smallest M that takes the MFMA tile path
     int64_t gemm_wide_shape = 1;       // matrix instruction of the 128- and 256-row tiles: 0 = 16x16x32, 1 = whichever is estimated faster, 2 = 32x32x16
     int64_t gemm_wide32_tile = 0;      // 0 = by shape; 12, 14, 15 (128-row tile x 64, 128, 160 columns), 24, 25 (256-row tile)
-    int64_t gemm_wide32_segments = 0;  // K segments of the 32x32x16 form: 0 = by shape (a forced tile or form: uncut), else at most that many (a forced tile: exactly)
-    int64_t gemm_decoded_min_rows = 1; // products that decode their weights into the scratch first: 0 never, 1 where estimated faster, else from that many rows on
+    int64_t gemm_wide32_segments = 0;  // K segments of the 32x32x16 form: 0 = by shape (a forced tile or form: uncut), else at most that many, up to 8 (a forced tile: exactly)
+    int64_t gemm_decoded_min_rows = 1; // products that decode their weights into the scratch first: 0 never, 1 where estimated faster, else from that many rows on (and 257), fewer never
     int64_t gemm_decoded_tile = 0;     // their tile: 0 = by shape; 192, 256 or 320 columns
     int64_t gemm_wide_min_rows = 33;   // smallest M that takes the 256-row tile (it wins from there up)
     int64_t gemm_skinny_max_rows = 64; // with gemm_resident 0: largest M that takes the few-rows kernel (0 = never)

@@ -1811,6 +1811,38 @@ def test_products_with_few_columns_stay_on_the_square_tiles(api, d, ggml, m, n, 
                          "square tiles")
 
 
+def test_the_switches_of_segments_and_panels_take_only_what_they_mean(api, d):
+    for key, good, bad in (("gemm_wide32_segments", (0, 1, 8), (-1, 9, 1 << 32)),
+                           ("gemm_decoded_min_rows", (0, 1, 2, 300, 2 ** 31 - 1), (-1, 2 ** 31, 1 << 32)),
+                           ("gemm_decoded_tile", (0, 192, 256, 320), (-192, 100, 128, (1 << 32) + 192))):
+        before = d.get_tuning(key)
+        try:
+            for value in good:
+                d.set_tuning(key, value)
+                assert d.get_tuning(key) == value
+            for value in bad:
+                with pytest.raises(Exception, match="out of range"):
+                    d.set_tuning(key, value)
+                assert d.get_tuning(key) == good[-1]
+        finally:
+            d.set_tuning(key, before)
+    # a row count asked for is the line, also where the estimate would decode below it
+    m, n, k = 1024, 12288, 4096
+    base = synth.matrix(Q6_K, 3, k, seed=785)
+    w = qm(api, d, Q6_K, n, k, np.resize(base, base.size // 3 * n))
+    xt = api.Tensor.from_f32(d, (m, k), api.DType.F16, synth.activations(m, k, seed=786))
+    out = api.Tensor.zeros(d, (m, n), api.DType.F16)
+    taken = []
+    try:
+        for rows in (1, 1025, 1024):
+            d.set_tuning("gemm_decoded_min_rows", rows)
+            d.project_quantized(xt, w, out=out)
+            taken.append(d.get_tuning("last_decoded_tile"))
+    finally:
+        d.set_tuning("gemm_decoded_min_rows", 1)
+    assert taken == [192, 0, 192]
+
+
 def test_decoded_panels_take_only_the_room_there_is(api):
     # 1100 x 70000 x 2048 is two panels of at most 256 MiB.  A new device that records has no room for one and takes the
     # fused tiles, which give the same bits; once a plain call has made room, a recording decodes too.
