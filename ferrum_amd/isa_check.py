@@ -1,7 +1,7 @@
 """Build-time check of the hand-scheduled loads in this library's own kernels.
 
-Three sources issue memory instructions through ``asm volatile`` that the compiler
-cannot see the timing of:
+Six sources (``CHECKED_SOURCES`` and ``HAND_ISSUED_SOURCES``) issue memory instructions through
+``asm volatile`` that the compiler cannot see the timing of:
 
 * LDS-direct loads (``s_mov_b32 m0, <lds address>`` followed by
   ``global_load_lds_dwordx4``): the statement writes M0, which an asm statement cannot
@@ -19,17 +19,17 @@ cannot see the timing of:
   a hand-issued load and the hand-placed wait that covers it; there must be none, except
   stores behind LDS-direct loads, which can only lengthen the wait.
 
-A second kind of kernel (``COUNTED_SOURCES``) leaves its LDS-direct loads and its register
-loads to the compiler, which orders and counts both, and only says when the former have
-landed: ``s_waitcnt vmcnt(n)``, n being the register loads the source issues behind them.
+A second kind of kernel (``COUNTED_SOURCES``) leaves its register loads to the compiler, which orders and counts them,
+and but for ``HAND_ISSUED_SOURCES`` its LDS-direct loads too, and only says when the latter have landed: ``s_waitcnt
+vmcnt(n)``, n being the register loads the source issues behind them.
 The invariant is that the generated code has at least n of them there
 (``counted_violations``): with fewer, n outstanding loads could include one that the wait
-is for.
+is for.  Of the hand-issued ones M0 and scratch are checked as above (``m0_violations``).
 
 The check reads the assembly hipcc writes with ``-S`` for this library's own sources
 (text, before it becomes a code object) and returns every violation it finds.  It is a
 linear scan in program-text order, which is the order these straight-line stretches are
-laid out in.  ``ferrum_amd.build.build`` runs it and refuses to produce a library when
+laid out in, and for counted loads also follows branches back over them.  ``ferrum_amd.build.build`` runs it and refuses to produce a library when
 it fails; the hipcc release the kernels were validated with is recorded in
 ``VALIDATED_HIPCC`` and any other release is reported.
 """
@@ -133,44 +133,52 @@ def violations(asm: str, source: str = "", counted: bool = False) -> list[str]:
 
 
 def counted_violations(asm: str, source: str = "") -> list[str]:
-    """Kernels that wait for LDS-direct loads by counting the register loads behind them: behind every run of the
-    former there must be at least as many of the latter as the next hand-placed ``s_waitcnt vmcnt(n)`` leaves
-    outstanding, along the text and along every branch back over the run."""
+    """Kernels that wait for LDS-direct loads by counting the register loads behind them.  Behind every run of the former,
+    up to the next hand-placed wait, the next run or the function's end, there must be at least as many of the latter as the
+    hand-placed ``s_waitcnt vmcnt(n)`` leave outstanding: the largest n of the kernel where the compiler issues the runs; in
+    ``HAND_ISSUED_SOURCES``, whose last rounds request nothing behind a run and wait for all, the n of the next wait, and one
+    must follow.  Likewise along every branch back over a run, up to the first wait behind its target."""
     found: list[str] = []
     where = (source + ":") if source else ""
+    next_wait_counts = source in HAND_ISSUED_SOURCES
     for name, body in _functions(asm, labels=True):
         at_label = {text[:-1]: at for at, (_, text, _) in enumerate(body) if text.endswith(":")}
         waits = {at: int(m.group(1)) for at, (_, text, in_asm) in enumerate(body)
                  if in_asm and (m := re.match(r"s_waitcnt vmcnt\((\d+)\)", text))}
-
-        def allowed_from(at):
-            return next((waits[w] for w in sorted(waits) if w >= at), None)
-
         lds = [at for at, (_, text, _) in enumerate(body) if text.startswith("global_load_lds_")]
+        if lds and not waits:
+            found.append(f"{where}{body[lds[0]][0]}: {name}: LDS-direct loads without a hand-placed wait")
+            continue
         for at in lds:
             number = body[at][0]
-            if not waits:
-                found.append(f"{where}{number}: {name}: LDS-direct loads without a hand-placed wait")
-                break
-            behind, needs, skip = 0, [], False
+            behind, needs, end = 0, [], "the function's end"
             for here in range(at + 1, len(body)):
-                _, text, in_asm = body[here]
+                _, text, _ = body[here]
                 if text.startswith("global_load_lds_"):
-                    skip = behind == 0        # the run goes on: its last load counts
-                    if skip:
+                    if behind == 0:
+                        end = "more of the run"
                         break
-                if here in waits:
-                    needs.append((waits[here], behind))
+                    if not next_wait_counts:
+                        end = "the next run"
+                        break
+                elif here in waits:
+                    end = "a wait"
                     break
-                if text.startswith("global_load_") and not text.startswith("global_load_lds_"):
+                elif text.startswith("global_load_"):
                     behind += 1
                 target = text.split()[-1] if text.startswith(("s_cbranch", "s_branch")) else None
                 if target in at_label and at_label[target] < at:
-                    needs.append((allowed_from(at_label[target]), behind))
-            if skip:
+                    needs.append((next((waits[w] for w in sorted(waits) if w >= at_label[target]), None), behind))
+            if end == "more of the run":    # its last load counts
                 continue
+            if not next_wait_counts:
+                needs.append((max(waits.values()), behind))
+            else:
+                needs.append((waits[here] if end == "a wait" else None, behind))
             for allowed, behind in needs:
-                if allowed is not None and behind < allowed:
+                if allowed is None:
+                    found.append(f"{where}{number}: {name}: no hand-placed wait follows this LDS-direct load")
+                elif behind < allowed:
                     found.append(f"{where}{number}: {name}: {behind} register loads follow this LDS-direct load, "
                                  f"the wait for it allows {allowed} outstanding")
     return found

@@ -116,6 +116,73 @@ def test_the_compilers_loads_behind_a_counted_lds_load_are_counted():
     assert any("without a hand-placed wait" in v for v in isa_check.counted_violations(unwaited, "x.hip"))
 
 
+LOOP = """
+_Z4loopv:
+	s_mov_b32 s0, 0
+.LBB0_1:
+	;;#ASMSTART
+	s_waitcnt vmcnt(2)
+	;;#ASMEND
+	ds_read_b128 v[20:23], v1
+	;;#ASMSTART
+	s_mov_b32 m0, s3
+	global_load_lds_dwordx4 v2, s[8:9]
+	;;#ASMEND
+	;;#ASMSTART
+	s_mov_b32 m0, s4
+	global_load_lds_dwordx4 v3, s[8:9]
+	;;#ASMEND
+	global_load_dwordx4 v[8:11], v[6:7], off
+	global_load_dwordx4 v[12:15], v[6:7], off offset:16
+	s_cbranch_scc1 .LBB0_1
+	;;#ASMSTART
+	s_waitcnt vmcnt(0)
+	;;#ASMEND
+	s_endpgm
+.Lfunc_end0:
+	.amdhsa_kernel _Z4loopv
+		.amdhsa_private_segment_fixed_size 0
+	.end_amdhsa_kernel
+"""
+HAND = isa_check.HAND_ISSUED_SOURCES[0]
+
+
+@pytest.mark.parametrize("source", ["x.hip", HAND])
+def test_counted_loads_are_counted_along_a_branch_back_over_them(source):
+    assert isa_check.counted_violations(LOOP, source) == []
+    # one register load less on the way round; on the way out nothing is left outstanding
+    load = "\tglobal_load_dwordx4 v[12:15], v[6:7], off offset:16\n"
+    found = isa_check.counted_violations(LOOP.replace(load, "", 1), source)
+    assert any("1 register loads follow" in v and "allows 2" in v for v in found), found
+    # the same load behind the branch is not on the way round either
+    found = isa_check.counted_violations(LOOP.replace(load, "", 1).replace("s_cbranch_scc1 .LBB0_1\n", "s_cbranch_scc1 .LBB0_1\n" + load, 1),
+                                         source)
+    assert any("1 register loads follow" in v and "allows 2" in v for v in found), found
+
+
+def test_hand_issued_counted_loads_need_a_wait_behind_them():
+    end = LOOP[LOOP.index("\tglobal_load_dwordx4 v[8:11]"):LOOP.index("\ts_endpgm")]
+    straight = LOOP.replace(end, "", 1)     # a run with nothing behind it but the function's end
+    found = isa_check.counted_violations(straight, HAND)
+    assert any("no hand-placed wait follows" in v for v in found), found
+    # where the compiler issues the runs, such a one is held to the strictest wait of the kernel, and so is one whose next wait is laxer
+    assert any("0 register loads follow" in v for v in isa_check.counted_violations(straight, "x.hip"))
+    last = LOOP.replace("\ts_cbranch_scc1 .LBB0_1\n", "", 1)
+    last = last.replace("\tglobal_load_dwordx4 v[12:15], v[6:7], off offset:16\n", "", 1)    # 1 behind, then vmcnt(0)
+    assert isa_check.counted_violations(last, HAND) == []
+    assert any("1 register loads follow" in v for v in isa_check.counted_violations(last, "x.hip"))
+
+
+def test_hand_issued_counted_loads_keep_m0_and_have_no_scratch():
+    assert isa_check.m0_violations(LOOP, HAND) == []
+    broken = LOOP.replace("s_mov_b32 s0, 0", "s_mov_b32 m0, s0", 1)
+    assert any("M0 is used outside" in v for v in isa_check.m0_violations(broken, HAND))
+    broken = LOOP.replace("fixed_size 0", "fixed_size 16", 1)
+    assert any("bytes of scratch" in v for v in isa_check.m0_violations(broken, HAND))
+    # what else is in flight is not this check's business
+    assert isa_check.violations(LOOP, HAND) != []
+
+
 def test_the_release_is_read_from_hipcc_version_text():
     assert isa_check.hipcc_release("HIP version: 7.2.26015-fc0010cf6a\nAMD clang version 22") == "7.2.26015"
     assert isa_check.hipcc_release("nothing") == ""
@@ -137,3 +204,5 @@ def test_the_built_library_came_through_the_check():
             asm = f.read()
         assert isa_check.counted_violations(asm, source) == []
         assert "global_load_lds_dwordx4" in asm
+        if source in isa_check.HAND_ISSUED_SOURCES:
+            assert isa_check.m0_violations(asm, source) == []
