@@ -1025,6 +1025,7 @@ fh_status prepare_gemm(fh_device* device, GemmArgs& g, size_t used) {
             if (!g.cut_tiles) g.few_rows = false;
         } else {
             g.cut_tiles = false;
+            g.tile = TileChoice{};
             gemm_takes_rows(g);
         }
     }
@@ -1034,7 +1035,7 @@ fh_status prepare_gemm(fh_device* device, GemmArgs& g, size_t used) {
     return FH_OK;
 }
 
-const char* run_gemm(fh_device* device, const GemmArgs& g) {
+const char* run_gemm(fh_device* device, GemmArgs& g) {
     const RowsPlan& plan = g.rows_plan;
     device->last_rows_plan = plan.rows * 1000 + plan.tiles * 100 + plan.segments;
     device->last_decoded_tile = g.decoded_columns != 0 ? g.decoded_tile : 0;

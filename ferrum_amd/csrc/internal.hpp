@@ -329,6 +329,20 @@ RowsPlan gemm_rows_plan(uint32_t ggml_type, uint32_t n, uint32_t k, uint32_t m, 
 bool f32_rows_pay(const RowsPlan& plan, uint32_t ggml_type, uint32_t n, uint32_t k, uint32_t m, int cu_count);
 
 // gemm.hip
+struct WidePlan {
+    int nt;
+    uint32_t cols, tiles_m, tiles_n;
+    int rt;   // 32x32x16 form: row tiles of 32 per multiplying wave (2: 256-row tile, 1: 128-row tile)
+    uint32_t segments, seg_blocks;   // 32x32x16 form: K segments
+};
+// Which of the tile forms would take a product of at least wide_min_rows rows, and the estimates.
+struct TileChoice {
+    bool made;
+    bool wide_pays;      // the 16x16x32 form's workgroups cover at least half the chip
+    WidePlan p32;        // the 32x32x16 form's tile, nt = 0 when it does not compete
+    double us32, us16;
+};
+
 struct GemmArgs {
     uint32_t ggml_type;
     const void* w;
@@ -342,6 +356,7 @@ struct GemmArgs {
     int wide32_tile;     // 0 = chosen by shape; else 10 x (row tiles per wave) + column tiles of the 32x32x16 form
     int wide32_segments; // K segments of that form: 0 = by shape
     bool cut_tiles;      // its partial sums have room in the scratch (`partials`)
+    TileChoice tile;     // made when first asked for; to be made again when cut_tiles changes
     int decoded_min_rows;      // rows from which the weights may be decoded once, in panels (0 = never)
     int decoded_tile;          // columns of the product's tile: 0 = by shape (gemm_takes_decoded sets it)
     uint32_t decoded_columns;  // set by gemm_takes_decoded: columns of a panel, which lies in `partials`
@@ -378,7 +393,7 @@ struct GemmArgs {
     uint32_t* counters;
     bool weight_ring;     // routed form, rows resident: Q4_K and Q6_K weights through LDS rings where they fit beside the rows
 };
-const char* launch_gemm(hipStream_t s, const GemmArgs& a);
+const char* launch_gemm(hipStream_t s, GemmArgs& a);
 // whether launch_gemm hands this product to the few-rows kernel: fills a.rows_plan, whose partial sums and
 // counters the caller then provides
 bool gemm_takes_rows(GemmArgs& a);
@@ -386,9 +401,9 @@ bool gemm_takes_rows(GemmArgs& a);
 // whether the weights are decoded into the scratch first, a panel of a.decoded_columns at a time (gemm_decoded.hip)
 bool gemm_takes_decoded(GemmArgs& a);
 void launch_gemm_decoded(hipStream_t s, const GemmArgs& a);
-double gemm_fused_estimate(const GemmArgs& a);   // us of the kernel that decodes as it multiplies; 1e300: none is estimated
+double gemm_fused_estimate(GemmArgs& a);   // us of the kernel that decodes as it multiplies; 1e300: none is estimated
 // scratch for the partial sums (or the panel) of the kernel launch_gemm would run (0: its K is not cut)
-size_t gemm_partial_bytes(const GemmArgs& a);
+size_t gemm_partial_bytes(GemmArgs& a);
 
 void launch_gemm_rows(hipStream_t s, const GemmArgs& a);   // gemm_rows.hip, by a.rows_plan
 
