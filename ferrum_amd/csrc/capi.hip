@@ -1168,8 +1168,11 @@ fh_status project(fh_device* device, const fh_qmatrix* weight, const fh_view* x,
         // One activated row stays on the FMA kernel: the streamed Q4_K one's operands are f16 pairs and the matrix core
         // keeps few bits of a subnormal weight (rel-L2 to 64 bits 2e-6 to 1.4e-5 on rows of mean weights, against 1.0e-7
         // to 2.0e-7).  The streamed Q6_K kernel sums integers and is the closer one for f32 rows (1.0e-7 against
-        // 2.0e-7; 16-bit rows 0.95e-7 on either): they take it from 200,000 super-blocks on (5120 x 17408 27.7 us on
-        // the FMA kernel, 24.7).  Activating in place, every workgroup activates the whole row again;
+        // 2.0e-7; 16-bit rows 0.95e-7 on either): they take it from 200,000 super-blocks on.  us with the activation, weights
+        // out of every cache, FMA / streamed: 2048 x 28672 22.3 / 21.9, 4096 x 12800 22.7 / 20.5, 4096 x 14336 23.3 / 20.7, 5120 x
+        // 17408 29.2 / 26.7, 4096 x 28672 36.0 / 34.0, 8192 x 14336 37.8 / 31.6; below, the longest rows gain nothing
+        // (1024 x 28672 16.6 / 16.8, 1250 x 17408 13.9 / 13.9), shorter ones up to a seventh (3000 x 12800 19.6 / 16.7).
+        // Activating in place, every workgroup activates the whole row again;
         // for large matrices the row is written out first, as the separate expert_silu_mul would, with the same
         // bits.  us, in place against written first: 5120 x 17408 26.5 / 20.6 (Q6_K 36.2 / 28.2), 5120 x 5120
         // 10.8 / 10.0 (15.3 / 13.1), 2048 x 12800 12.3 / 11.8 (16.1 / 14.7); 4096 x 4096, where the second launch
