@@ -1150,9 +1150,9 @@ WidePlan wide_plan(uint32_t m, uint32_t n, int cus) {
 // What a launch of one 32x32x16 tile takes, in us: a start (launch, first loads, stores) and, per super-block of its K
 // segment, a time that depends on the format's decode and a little on how much of the chip is busy (`full`, times the
 // share of the compute units that have a workgroup); alone on their compute units, or two on some of them where LDS
-// and registers hold two.  Fitted to 4700 measurements: the five formats, twelve shapes from 1024 x 4096 to
-// 34816 x 5120, 40 - 1999 rows, one to eight segments; within 5% in the mean square, and the pick by it is on
-// average 0.4% and at most 10% slower than the fastest one.
+// and registers hold two.  Fitted to profiles/tile_k_segments_us.txt: the five formats, fourteen shapes from 1024 x 4096 to
+// 34816 x 5120, 40 - 1999 rows, one to eight segments; within 5.3% in the mean square, and the pick by it is on
+// average 0.5% and at most 10% slower than the fastest one.
 struct Wide32Cost {
     double start, block[5], full;   // Q4_K, Q5_K, IQ4_XS, Q6_K, Q8_0
 };

@@ -272,7 +272,7 @@ constexpr size_t kMostPanelBytes = fh_device::kScratchOptional;
 }  // namespace
 
 // Decode at the rate of its stores, then rounds of the product, the last one cheaper where it is not full; against the
-// fused tiles' estimate.  All sides in turn, bf16, five formats x 20 shapes of 512 - 100000 columns and 512 - 17408 K x nine
+// fused tiles' estimate.  All sides in turn (profiles/decoded_panels_us.txt), bf16, five formats x 20 shapes of 512 - 100000 columns and 512 - 17408 K x nine
 // row counts of 267 - 2048 (900 products, 885 with an estimate): 225 decode, the pick is 0.5% from the fastest of the four
 // in the mean and slower than the fused tiles by more than 3% for two (Q6_K 768 x 28672 x 4096 245 / 271, Q5_K 1500 x 19864
 // x 512 66 / 69).  us, fused tiles / 192 / 256 / 320 columns: Q4_K 1999 x 34816 x 5120 778 / 789 / 752 / 718, 1999 x 17408

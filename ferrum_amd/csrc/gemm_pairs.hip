@@ -661,7 +661,7 @@ void launch_one(hipStream_t s, const PairsParams& p) {
 
 }  // namespace
 
-// Against the f32 matrix instruction (us, that / this; 24 rows Q4_K 28672 x 4096 117 / 37, 5120 x 17408 86 / 35, 34816 x 5120
+// Against the f32 matrix instruction (profiles/f32_batches_pairs_us.txt; us, that / this; 24 rows Q4_K 28672 x 4096 117 / 37, 5120 x 17408 86 / 35, 34816 x 5120
 // 148 / 69, 4096 x 4096 21.4 / 19.4; Q6_K 4096 x 14336 65 / 41).  A launch of this kernel and the one that splits the rows
 // take 16 us however small the matrix, and up to 16 rows half of the 32 it multiplies are empty, so those go by format:
 // 16 rows Q4_K 17408 x 5120 48 / 38, 5120 x 5120 20.1 / 20.5, 4096 x 4096 12 / 19, Q6_K 34816 x 5120 97 / 125.  33 to 48

@@ -83,8 +83,8 @@ RowsPlan gemm_rows_plan(uint32_t ggml_type, uint32_t n, uint32_t k, uint32_t m, 
     plan.estimate_us = counted * (kStartUs + per_wave * plan.tiles * unit_us(ggml_type, x_dtype, plan.rows)) +
                        (plan.segments > 1 ? kExchangeUs : 0.0);
     if (plan.rows == 32 && m > 32) {
-        // several groups share the weights in an L2 and the longest and shortest waves a SIMD: fitted to 440
-        // measurements of 40 - 128 rows on eleven shapes and five formats, 8% in the mean square (Q6_K's decode of four
+        // several groups share the weights in an L2 and the longest and shortest waves a SIMD: fitted to the 385 plans of
+        // 40 - 128 rows in profiles/few_rows_against_tiles_us.txt (eleven shapes, five formats), 8% in the mean square (Q6_K's decode of four
         // and five tiles is above the fit)
         const double tile = ggml_type == kQ4K     ? 1.39
                             : ggml_type == kQ5K   ? 1.88
