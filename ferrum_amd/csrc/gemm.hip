@@ -1461,7 +1461,7 @@ const char* launch_gemm(hipStream_t s, GemmArgs& a) {
     static const char* const tile_names[5] = {"q4_k_gemm_mfma_m256", "q5_k_gemm_mfma_m256", "iq4_xs_gemm_mfma_m256",
                                               "q6_k_gemm_mfma_m256", "q8_0_gemm_mfma_m256"};
     if (a.decoded_columns != 0) {
-        launch_gemm_decoded(s, a);   // the same tiles, bit for bit
+        launch_gemm_decoded(s, a);   // (the bits of the 32x32x16 tiles, uncut)
         return tile_names[cost_column(a.ggml_type)];
     }
     if (a.rows_plan.rows != 0) {

@@ -922,7 +922,10 @@ def test_products_run_without_the_scratch_they_would_like(api, live_graph, ggml,
     grown = dev.get_tuning("held_scratch_bytes")
     assert wanted * 10 ** 6 <= grown <= (wanted + 1) * 10 ** 6 + (1 << 20)
     assert dev.get_tuning("retired_scratch_blocks") == (1 if live_graph else 0)
-    assert rel_l2(y.to_f32(), first) <= 1e-5
+    if ggml == Q6_K:      # panels, and in their place the uncut tiles of the 32x32x16 form: the same sums
+        assert dev.get_tuning("last_decoded_tile") != 0 and np.array_equal(bits(y.to_f32()), bits(first))
+    else:
+        assert rel_l2(y.to_f32(), first) <= 1e-5
     dev.set_tuning("held_scratch_bytes", 0)
     assert dev.get_tuning("held_scratch_bytes") == (grown if live_graph else held)
     if live_graph:
@@ -983,6 +986,26 @@ def test_the_tile_picked_by_row_count_gives_the_bits_of_the_largest(api, d, m):
         d.set_tuning("gemm_wide_shape", shape)
     assert picked.operation == largest.operation == "q4_k_gemm_mfma_m256"
     assert np.array_equal(picked.tensor.raw(), largest.tensor.raw())
+
+
+@pytest.mark.parametrize("n,k", [(5120, 17408), (17000, 2816), (2560, 8192)])
+def test_rows_of_the_default_kernels_agree_at_every_row_count(api, d, n, k):
+    # Which kernel, tile and K segments take a product follows from its row count, and with them the order of a row's sums, not
+    # its bits.  An instruction brings at least the eight products of a lane group into an f32 accumulator, so at most k / 8
+    # sums follow each other there, each off by 2^-24 at most, uniform: 2^-24 / sqrt(3) * sqrt(k / 16) in the mean square
+    # from 64 bits on the rounded weights, on either side of a comparison.
+    w = qm(api, d, Q4_K, n, k, synth.matrix(Q4_K, n, k, seed=175))
+    x = synth.activations(512, k, seed=176, f16=True).reshape(512, k)
+    bound = 2.0 ** -24 / np.sqrt(3) * np.sqrt(k / 16)
+    cols = np.unique(np.concatenate([np.arange(0, 60), np.arange(n - 60, n)]))
+    want = oracle_columns(Q4_K, synth.matrix(Q4_K, n, k, seed=175), n, k, cols, x[:33], weight_round=oracle.F16, accumulate="f64")
+    last = None
+    for m in (33, 64, 80, 128, 200, 256, 330, 512):
+        got = d.project_quantized(api.Tensor.from_f32(d, (m, k), api.DType.F16, x[:m]), w, out_dtype=api.DType.F32).tensor.to_f32()
+        assert rel_l2(got[:33][:, cols], want) <= bound, m
+        if last is not None:
+            assert rel_l2(got[: len(last)], last) <= np.sqrt(2) * bound, m
+        last = got
 
 
 @pytest.mark.parametrize("ggml", [12, 13, 14, 23, 8], ids=["q4_k", "q5_k", "q6_k", "iq4_xs", "q8_0"])
@@ -1845,7 +1868,7 @@ def test_the_switches_of_segments_and_panels_take_only_what_they_mean(api, d):
 
 def test_decoded_panels_take_only_the_room_there_is(api):
     # 1100 x 70000 x 2048 is two panels of at most 256 MiB.  A new device that records has no room for one and takes the
-    # fused tiles, which give the same bits; once a plain call has made room, a recording decodes too.
+    # fused tiles (f16 outputs of sums that may be of another order); once a plain call has made room, a recording decodes too.
     dev = api.Device.new()
     m, n, k = 1100, 70000, 2048
     tile = synth.matrix(Q6_K, 80, k, seed=771)
