@@ -723,9 +723,11 @@ StreamPlan gemv_stream_plan(uint32_t ggml_type, uint32_t n, uint32_t k, uint32_t
     // 67.3 / 61.6, 151936 x 2048 61.4 / 59.3, 128256 x 4096 98.2 / 96.7, 152064 x 3584 111.5 / 100.7, 262144 x 2560
     // 133.6 / 118.0, 151936 x 5120 142.8 / 132.5).
     // Rows of 16 bits gain 1% there and are 0.9e-7 from 64 bits on the FMA kernel against 0.95e-7 here (f32 rows 1.9e-7 against
-    // 0.9e-7): they come from a million super-blocks on, where the FMA kernel cannot cut a row evenly over its eight block slots.
+    // 0.9e-7), and two or three f32 rows share their weights through the caches on the FMA kernel (2 x 34816 x 5120 58.3 us there
+    // against 64.6, 2 x 100000 x 2048 67.6 / 74.5): they come from a million super-blocks on, where the FMA kernel
+    // cannot cut a row evenly over its eight block slots.
     const bool big_head = q6 && segments == 1u && h == 16u &&
-                          (f32_rows ? (uint64_t)n * nb >= 600000u : (nb & 7u) != 0 && (uint64_t)n * nb >= 1000000u);
+                          (f32_rows && m == 1 ? (uint64_t)n * nb >= 600000u : (nb & 7u) != 0 && (uint64_t)n * nb >= 1000000u);
     // One row of a Q4_K matrix of short rows is the FMA kernel's: a tile of sixteen is a few kilobytes of LDS for eight waves of
     // which some own no super-block, and staging stands beside little arithmetic (us, cold, FMA against this kernel:
     // 29952 x 256 3.7 / 8.3, 8448 x 512 3.5 / 4.2, 4224 x 1024 3.5 / 3.8, 99968 x 1024 14.1 / 23.6; rows of 5 - 8 super-blocks

@@ -475,6 +475,19 @@ def test_only_f32_rows_stream_q6_k_matrices_below_a_million_super_blocks(api, d)
         assert rel_l2(got, other) <= 7e-7
 
 
+@pytest.mark.parametrize("m", [2, 3])
+def test_two_or_three_f32_rows_of_such_a_matrix_stay_on_the_fma_kernel(api, d, m):
+    n, k = 32000, 5120
+    base = synth.matrix(Q6_K, 2000, k, seed=35).reshape(2000, -1)
+    w = qm(api, d, Q6_K, n, k, np.tile(base, (n // 2000, 1)).reshape(-1))
+    xt = api.Tensor.from_f32(d, (m, k), api.DType.F32, synth.activations(m, k, seed=37))
+    got = d.project_quantized(xt, w).tensor.to_f32()
+    with fma_gemv(d):
+        assert np.array_equal(bits(got), bits(d.project_quantized(xt, w).tensor.to_f32()))
+    want = xt.to_f32().reshape(m, k).astype(np.float64) @ oracle.dequantize(Q6_K, base.reshape(-1), 2000, k).reshape(2000, k).astype(np.float64).T
+    assert rel_l2(got[:, :2000], want) <= 4e-7
+
+
 def test_one_activated_f32_row_of_a_large_q6_k_matrix_takes_the_streamed_kernel(api, d):
     # 3000 x 17408: 204,000 super-blocks; the bits of the separate calls, and the tolerance of the test above
     n, k = 3000, 17408
