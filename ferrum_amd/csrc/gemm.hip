@@ -1257,11 +1257,13 @@ WidePlan wide32_plan(uint32_t ggml_type, uint32_t m, uint32_t n, uint32_t k, int
 }
 
 // The 16x16x32 form keeps two workgroups on a compute unit, one storing while the other
-// multiplies, so its rounds need not be whole: 2048 x 17408 x 5120 takes 442 us in 4.25 rounds.
+// multiplies, so its rounds need not be whole: 2048 x 17408 x 5120 takes 442 us in 4.25 rounds.  An estimate from below:
+// where it is within 8% of the 32x32x16 form's, that form is the faster one (Q8_0 512 x 17408 x 5120 139 us here and 133
+// there, 512 x 34816 x 5120 294 / 282, 768 x 17408 x 5120 240 / 204, Q4_K 196 / 172).
 double wide16_estimate(uint32_t m, uint32_t n, uint32_t k, int cus) {
     const uint64_t wgs = (uint64_t)((m + kWM - 1) / kWM) * ((n + 127) / 128);
     const double rounds = (double)wgs / (double)cus;
-    return (rounds < 1.0 ? 1.0 : rounds) * 105.0 * wide_row_length_factor(k);
+    return (rounds < 1.0 ? 1.0 : rounds) * 113.0 * wide_row_length_factor(k);
 }
 
 // The rows-resident kernel: a start (the rows' gather, then the first weights), the stream of the matrix, and a decode of every weight per group

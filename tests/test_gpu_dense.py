@@ -1001,6 +1001,26 @@ def test_the_tile_picked_by_row_count_gives_the_bits_of_the_largest(api, d, m):
     assert np.array_equal(picked.tensor.raw(), largest.tensor.raw())
 
 
+@pytest.mark.parametrize("ggml,m,n,k", [(8, 512, 17408, 5120), (8, 400, 34816, 4096)])
+def test_the_32x32x16_form_is_taken_where_the_forms_are_close(api, d, ggml, m, n, k):
+    base = synth.matrix(ggml, 11, k, seed=191)
+    w = qm(api, d, ggml, n, k, np.resize(base, base.size // 11 * n))
+    xt = api.Tensor.from_f32(d, (m, k), api.DType.F16, synth.activations(m, k, seed=192, f16=True))
+    out, results = api.Tensor.zeros(d, (m, n), api.DType.F32), {}
+    try:
+        for name, key, value in (("default", "gemm_wide_shape", 1), ("32", "gemm_wide32_tile", 25), ("16", "gemm_wide_shape", 0)):
+            d.set_tuning(key, value)
+            d.project_quantized(xt, w, out=out)
+            assert d.get_tuning("last_decoded_tile") == 0
+            results[name] = out.raw()
+            d.set_tuning("gemm_wide_shape", 1)
+            d.set_tuning("gemm_wide32_tile", 0)
+    finally:
+        d.set_tuning("gemm_wide_shape", 1)
+        d.set_tuning("gemm_wide32_tile", 0)
+    assert np.array_equal(results["default"], results["32"]) and not np.array_equal(results["default"], results["16"])
+
+
 @pytest.mark.parametrize("n,k", [(5120, 17408), (17000, 2816), (2560, 8192)])
 def test_rows_of_the_default_kernels_agree_at_every_row_count(api, d, n, k):
     # Which kernel, tile and K segments take a product follows from its row count, and with them the order of a row's sums, not
