@@ -1703,6 +1703,17 @@ def test_f32_batches_as_pairs_are_no_farther_from_64_bits_than_on_the_f32_instru
     assert rel_l2(got, want) <= rel_l2(other, want)
 
 
+@pytest.mark.parametrize("ggml,n,k,pairs", [(12, 7147, 4352, True), (13, 7147, 4352, False), (13, 6144, 6144, True), (12, 7000, 4352, False)])
+def test_up_to_sixteen_f32_rows_take_pairs_by_format_and_size(api, d, ggml, n, k, pairs):
+    base = synth.matrix(ggml, 7, k, seed=759)
+    w = qm(api, d, ggml, n, k, np.resize(base, base.size // 7 * n))
+    x = api.Tensor.from_f32(d, (16, k), api.DType.F32, synth.activations(16, k, seed=760))
+    got = d.project_quantized(x, w).tensor.to_f32()
+    assert d.get_tuning("last_rows_plan") // 1000 == (32 if pairs else 16)
+    want = x.to_f32().reshape(16, k).astype(np.float64) @ oracle.dequantize(ggml, base, 7, k).reshape(7, k).astype(np.float64).T
+    assert rel_l2(got[:, :7], want) <= 1.8e-7    # (1.6e-7 over many outputs, as above; here 112)
+
+
 def test_f32_batches_without_room_for_pairs_take_the_f32_instruction(api):
     # 43000 x 4352: the operands of 32 rows and their sums of three K segments are 17.1 MB, more than the scratch of a
     # new device holds while it records
