@@ -273,9 +273,9 @@ constexpr size_t kMostPanelBytes = fh_device::kScratchOptional;
 
 // Decode at the rate of its stores, then rounds of the product, the last one cheaper where it is not full; against the
 // fused tiles' estimate.  All sides in turn (profiles/decoded_panels_us.txt), bf16, five formats x 20 shapes of 512 - 100000 columns and 512 - 17408 K x nine
-// row counts of 267 - 2048 (900 products, 885 with an estimate): 225 decode, the pick is 0.5% from the fastest of the four
-// in the mean and slower than the fused tiles by more than 3% for two (Q6_K 768 x 28672 x 4096 245 / 271, Q5_K 1500 x 19864
-// x 512 66 / 69).  us, fused tiles / 192 / 256 / 320 columns: Q4_K 1999 x 34816 x 5120 778 / 789 / 752 / 718, 1999 x 17408
+// row counts of 267 - 2048 (900 products, 885 with an estimate): 222 decode, the pick is 0.5% from the fastest of the four
+// in the mean and slower than the fused tiles by more than 3% for one (Q5_K 1500 x 19864 x 512 66 / 69; with one margin for all
+// also Q6_K 768 x 28672 x 4096 245 / 271).  us, fused tiles / 192 / 256 / 320 columns: Q4_K 1999 x 34816 x 5120 778 / 789 / 752 / 718, 1999 x 17408
 // x 5120 425 / 380 / 414 / 355, 1999 x 12288 x 4096 231 / 208 / 218 / 256, 1999 x 5120 x 17408 352 / 403 / 411 / 461; Q6_K
 // 1999 x 34816 x 5120 925 / 802 / 767 / 730, 1024 x 12288 x 4096 149 / 120 / 124 / 132; Q8_0 1999 x 17408 x 5120 553 / 400
 // / 423 / 367, 1500 x 8192 x 8192 336 / 319 / 221 / 234.
@@ -285,9 +285,9 @@ bool gemm_takes_decoded(GemmArgs& a) {
     const bool forced = a.decoded_min_rows > 1;   // from that many rows on, whatever the estimates say
     if (forced && a.m < (uint32_t)a.decoded_min_rows) return false;
     const uint32_t asked = (uint32_t)a.decoded_tile;
-    // (the fused estimate is low where the chip is full and hot; a product that only the square tiles take, few columns and
+    // (the fused estimate is 4 - 6% low where the chip is full and hot, Q6_K's 1%; a product that only the square tiles take, few columns and
     // rows too long to be resident, has none: 300 x 512 x 4096 36 us there, 71 to 101 here)
-    double best = forced ? 1e300 : gemm_fused_estimate(a) * 1.1;
+    double best = forced ? 1e300 : gemm_fused_estimate(a) * (a.ggml_type == kQ6K ? 1.05 : 1.1);
     if (!forced && best >= 1e300) return false;
     for (const DecodedTile& t : kDecodedTiles) {
         if (asked != 0 && asked != t.columns) continue;

@@ -1865,6 +1865,16 @@ def test_the_fastest_of_the_decoded_tiles_is_taken(api, d, ggml, m, n, k, tile):
         d.set_tuning("gemm_decoded_tile", 0)
 
 
+@pytest.mark.parametrize("ggml,m,n,k", [(14, 768, 28672, 4096), (12, 1999, 5120, 17408), (8, 512, 17408, 5120)])
+def test_products_that_the_fused_tiles_run_faster_are_not_decoded(api, d, ggml, m, n, k):
+    # us, fused / the best panel: 245 / 271, 352 / 403, 141 / 170
+    base = synth.matrix(ggml, 3, k, seed=787)
+    w = qm(api, d, ggml, n, k, np.resize(base, base.size // 3 * n))
+    xt = api.Tensor.from_f32(d, (m, k), api.DType.BF16, synth.activations(m, k, seed=788))
+    d.project_quantized(xt, w, out=api.Tensor.zeros(d, (m, n), api.DType.BF16))
+    assert d.get_tuning("last_decoded_tile") == 0
+
+
 @pytest.mark.parametrize("ggml", [12, 13, 14, 23, 8], ids=["q4_k", "q5_k", "q6_k", "iq4_xs", "q8_0"])
 @pytest.mark.parametrize("m,n,k", [(300, 512, 4096), (384, 512, 5120), (267, 580, 2816), (512, 256, 7168)])
 def test_products_with_few_columns_stay_on_the_square_tiles(api, d, ggml, m, n, k):
