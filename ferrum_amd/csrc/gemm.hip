@@ -1391,36 +1391,6 @@ const TileChoice& tile_choice(GemmArgs& a) {
     return c;
 }
 
-}  // namespace
-
-// Up to 128 rows the few-rows kernel competes: the smallest estimate among it, the kernel that keeps
-// rows in LDS (where they fit) and the tiles takes the call.  It wins wherever a round or two of its
-// workgroups cover the matrix (Q4_K, f16, us, against the kernel that had these rows: 16 / 32 / 64 x
-// 17408 x 5120 17.7 / 21.2 / 37.8 against 19.7 / 31.9 / 45.9, 16 x 4096 x 2048 4.4 / 5.4), and for rows
-// too long for LDS there is nothing else (8 / 64 / 128 x 5120 x 17408 20.9 / 40.7 / 77 against 43.6 /
-// 106 / 189 on a slab and a square-tile kernel).  Over many rounds its starts add up and the resident
-// kernel's waves, which stream from tile to tile, are ahead (16 x 151936 x 5120 133 against 116).
-bool gemm_takes_rows(GemmArgs& a) {
-    if (!a.few_rows || a.m < 2 || a.m > 128) return false;
-    if (a.wide32_tile != 0 && a.wide_shape != 0 && a.m >= (uint32_t)a.wide_min_rows) return false;   // a tile is asked for
-    const RowsPlan plan = gemm_rows_plan(a.ggml_type, a.n, a.k, a.m, a.x_dtype, a.cu_count);
-    if (plan.counters > fh_device::kCounterWords) return false;
-    if (!a.few_rows_always && a.resident_switch) {
-        const TileChoice& c = tile_choice(a);
-        // (a cut tile has to gain a sixth on a plan that needs no partial sums: 80 x 17408 x 5120 stays here, 55 us
-        // against 49)
-        double other = std::min(c.p32.segments > 1 && plan.segments == 1 ? c.us32 * 1.18 : c.us32, c.us16);
-        if (a.rows_resident) other = std::min(other, resident_estimate(a.ggml_type, a.m, a.n, a.k));
-        if (plan.estimate_us >= other) return false;
-    } else if (!a.few_rows_always && a.m > (uint32_t)a.skinny_max_rows) {
-        return false;
-    }
-    a.rows_plan = plan;
-    return true;
-}
-
-namespace {
-
 // Rows that fit LDS for their whole length take the kernel that keeps them there and streams
 // the weights past them through registers: against the square tiles 1.4 - 2.2 times
 // (512 x 1024 x 2048: 11.5 against 22.8 us).
@@ -1445,6 +1415,35 @@ bool takes_resident(const GemmArgs& a, const TileChoice& c) {
 }
 
 }  // namespace
+
+// Up to 128 rows the few-rows kernel competes: the smallest estimate among it, the kernel that keeps
+// rows in LDS (where they fit) and the tiles takes the call.  It wins wherever a round or two of its
+// workgroups cover the matrix (Q4_K, f16, us, against the kernel that had these rows: 16 / 32 / 64 x
+// 17408 x 5120 17.7 / 21.2 / 37.8 against 19.7 / 31.9 / 45.9, 16 x 4096 x 2048 4.4 / 5.4), and for rows
+// too long for LDS there is nothing else (8 / 64 / 128 x 5120 x 17408 20.9 / 40.7 / 77 against 43.6 /
+// 106 / 189 on a slab and a square-tile kernel).  Over many rounds its starts add up and the resident
+// kernel's waves, which stream from tile to tile, are ahead (16 x 151936 x 5120 133 against 116).
+bool gemm_takes_rows(GemmArgs& a) {
+    if (!a.few_rows || a.m < 2 || a.m > 128) return false;
+    if (a.wide32_tile != 0 && a.wide_shape != 0 && a.m >= (uint32_t)a.wide_min_rows) return false;   // a tile is asked for
+    const RowsPlan plan = gemm_rows_plan(a.ggml_type, a.n, a.k, a.m, a.x_dtype, a.cu_count);
+    if (plan.counters > fh_device::kCounterWords) return false;
+    if (!a.few_rows_always && a.resident_switch) {
+        const TileChoice& c = tile_choice(a);
+        // (a cut tile has to gain a sixth on a plan that needs no partial sums: 80 x 17408 x 5120 stays here, 55 us
+        // against 49)
+        double other = std::min(c.p32.segments > 1 && plan.segments == 1 ? c.us32 * 1.18 : c.us32, c.us16);
+        // (short rows stay on the resident kernel whatever a tile promises: that one is the rival then.  Q6_K, 43 x 27495 x 256
+        // 13.3 us here and 20.6 there, 59617 x 256 20.3 / 24.5)
+        if (takes_resident(a, c)) other = resident_estimate(a.ggml_type, a.m, a.n, a.k);
+        else if (a.rows_resident) other = std::min(other, resident_estimate(a.ggml_type, a.m, a.n, a.k));
+        if (plan.estimate_us >= other) return false;
+    } else if (!a.few_rows_always && a.m > (uint32_t)a.skinny_max_rows) {
+        return false;
+    }
+    a.rows_plan = plan;
+    return true;
+}
 
 double gemm_fused_estimate(GemmArgs& a) {
     const TileChoice& c = tile_choice(a);

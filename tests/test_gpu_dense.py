@@ -1163,6 +1163,21 @@ def test_16_bit_rows_take_the_faster_of_two_kernels(api, d, ggml, m, n, k, few):
     assert np.array_equal(bits(got), bits(np.tile(got[:, :64], n // 64)))
 
 
+def taken_by(api, d, ggml, m, n, k):
+    """Which kernel takes m f16 rows: "rows" (few-rows), "resident" or "m256" (the tiles)."""
+    base = synth.matrix(ggml, 251, k, seed=760).reshape(251, -1)
+    w = qm(api, d, ggml, n, k, np.resize(base, (n, base.shape[1])).reshape(-1))
+    xt = api.Tensor.from_f32(d, (m, k), api.DType.F16, synth.activations(m, k, seed=761))
+    got = d.project_quantized(xt, w)
+    return "rows" if d.get_tuning("last_rows_plan") else got.operation.split("_")[-1]
+
+
+@pytest.mark.parametrize("m,n", [(43, 27495), (42, 59617), (70, 41115)])
+def test_a_tile_that_is_not_taken_keeps_no_call_from_the_few_rows_kernel(api, d, m, n):
+    # rows of 256 are the resident kernel's where the few-rows kernel does not take them, whatever a tile would cost
+    assert taken_by(api, d, Q6_K, m, n, 256) == "rows"
+
+
 @pytest.mark.parametrize("ggml", [12, 13, 14, 23, 8], ids=["q4_k", "q5_k", "q6_k", "iq4_xs", "q8_0"])
 @pytest.mark.parametrize("m,n,k", [(16, 256, 256), (48, 100, 512), (8, 1024, 1024), (6, 4096, 4096), (40, 4100, 1024)])
 def test_small_f32_batches_stay_on_the_gemv(api, d, ggml, m, n, k):
