@@ -665,13 +665,15 @@ void launch_one(hipStream_t s, const PairsParams& p) {
 // 148 / 69, 4096 x 4096 21.4 / 19.4; Q6_K 4096 x 14336 65 / 41).  A launch of this kernel and the one that splits the rows
 // take 16 us however small the matrix, and up to 16 rows half of the 32 it multiplies are empty, so those go by format:
 // 16 rows Q4_K 17408 x 5120 48 / 38, 5120 x 5120 20.1 / 20.5, 4096 x 4096 12 / 19, Q5_K 6144 x 6144 25.2 / 24.4, 7147 x 4352
-// 20.6 / 22.3, Q6_K 34816 x 5120 97 / 125.  33 to 48
+// 20.6 / 22.3, Q6_K 34816 x 5120 97 / 125.  Rows of one or two super-blocks leave one K half of a workgroup idle or both with a
+// single round: 8 x 126084 x 256 Q4_K 18.3 / 22.5, 14 x 76728 x 512 Q5_K 24.1 / 28.5 and even at 300,000 super-blocks; of three
+// 10 x 50643 x 768 Q4_K 31.6 / 21.4.  33 to 48
 // rows are two groups here and three there: 48 rows Q4_K 5120 x 5120 36 / 30, 4096 x 4096 30 / 31, Q6_K 5120 x 5120 44 / 47,
 // 6144 x 6144 73 / 55.
 bool pairs_pay(uint32_t ggml_type, uint32_t n, uint32_t k, uint32_t m) {
     const uint64_t blocks = (uint64_t)n * (k / 256);
     if (ggml_type == kQ8_0 || m < 7 || n < 2560) return false;
-    if (m <= 16) return (ggml_type == kQ4K && blocks >= 120000u) || (ggml_type == kQ5K && blocks >= 140000u);
+    if (m <= 16) return k > 512 && ((ggml_type == kQ4K && blocks >= 120000u) || (ggml_type == kQ5K && blocks >= 140000u));
     if (m > 32 && m <= 48) return blocks >= (ggml_type == kQ6K ? 131072u : 100000u);
     return blocks >= 65536u;
 }

@@ -1718,7 +1718,8 @@ def test_f32_batches_as_pairs_are_no_farther_from_64_bits_than_on_the_f32_instru
     assert rel_l2(got, want) <= rel_l2(other, want)
 
 
-@pytest.mark.parametrize("ggml,n,k,pairs", [(12, 7147, 4352, True), (13, 7147, 4352, False), (13, 6144, 6144, True), (12, 7000, 4352, False)])
+@pytest.mark.parametrize("ggml,n,k,pairs", [(12, 7147, 4352, True), (13, 7147, 4352, False), (13, 6144, 6144, True), (12, 7000, 4352, False),
+                                             (12, 126084, 256, False), (13, 76728, 512, False), (12, 50643, 768, True)])
 def test_up_to_sixteen_f32_rows_take_pairs_by_format_and_size(api, d, ggml, n, k, pairs):
     base = synth.matrix(ggml, 7, k, seed=759)
     w = qm(api, d, ggml, n, k, np.resize(base, base.size // 7 * n))
