@@ -1153,6 +1153,9 @@ WidePlan wide_plan(uint32_t m, uint32_t n, int cus) {
 // and registers hold two.  Fitted to profiles/tile_k_segments_us.txt: the five formats, fourteen shapes from 1024 x 4096 to
 // 34816 x 5120, 40 - 1999 rows, one to eight segments; within 5.3% in the mean square, and the pick by it is on
 // average 0.5% and at most 10% slower than the fastest one.
+// The 128 x 96 tile's are from rows of 256 - 17408 (profiles/routes_us.txt): those of the long rows alone gave it 20% too much
+// at short ones (Q6_K 45 x 22548 x 1280 23.6 us on it, 27.1 on the resident kernel that was taken; 198 x 8811 x 1024 19.6, 21.9 with
+// 64 columns).
 struct Wide32Cost {
     double start, block[5], full;   // Q4_K, Q5_K, IQ4_XS, Q6_K, Q8_0
 };
@@ -1162,7 +1165,7 @@ struct Wide32Tile {
 };
 constexpr Wide32Tile kWide32Tiles[] = {
     {1, 2, {5.9, {1.73, 1.96, 1.81, 2.24, 2.45}, 0.42}, {8.0, {2.59, 3.14, 2.99, 3.51, 3.57}, 0.18}},
-    {1, 3, {10.2, {2.27, 2.56, 2.36, 3.04, 3.44}, 0.0}, {}},
+    {1, 3, {7.6, {2.34, 2.56, 2.54, 3.14, 3.15}, 0.0}, {}},
     {1, 4, {10.2, {2.09, 2.46, 2.22, 2.99, 3.38}, 0.37}, {8.4, {3.98, 4.55, 4.31, 5.20, 5.78}, 0.35}},
     {1, 5, {11.7, {2.65, 2.97, 2.75, 4.77, 5.03}, 0.40}, {}},
     {2, 4, {13.1, {2.79, 3.06, 2.86, 3.51, 4.02}, 0.90}, {}},

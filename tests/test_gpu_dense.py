@@ -1178,6 +1178,11 @@ def test_a_tile_that_is_not_taken_keeps_no_call_from_the_few_rows_kernel(api, d,
     assert taken_by(api, d, Q6_K, m, n, 256) == "rows"
 
 
+@pytest.mark.parametrize("ggml,m,n,k", [(14, 45, 22548, 1280), (8, 73, 23033, 1792)])
+def test_the_96_column_tile_takes_rows_of_a_few_super_blocks(api, d, ggml, m, n, k):
+    assert taken_by(api, d, ggml, m, n, k) == "m256"
+
+
 @pytest.mark.parametrize("ggml", [12, 13, 14, 23, 8], ids=["q4_k", "q5_k", "q6_k", "iq4_xs", "q8_0"])
 @pytest.mark.parametrize("m,n,k", [(16, 256, 256), (48, 100, 512), (8, 1024, 1024), (6, 4096, 4096), (40, 4100, 1024)])
 def test_small_f32_batches_stay_on_the_gemv(api, d, ggml, m, n, k):
