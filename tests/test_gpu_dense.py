@@ -1178,6 +1178,12 @@ def test_a_tile_that_is_not_taken_keeps_no_call_from_the_few_rows_kernel(api, d,
     assert taken_by(api, d, Q6_K, m, n, 256) == "rows"
 
 
+@pytest.mark.parametrize("ggml,m,n,k,kernel", [(23, 67, 13035, 3328, "m256"), (8, 102, 2271, 2816, "resident"),
+                                               (8, 92, 8535, 2304, "resident")])
+def test_uneven_shares_of_a_row_count_against_the_few_rows_kernel(api, d, ggml, m, n, k, kernel):
+    assert taken_by(api, d, ggml, m, n, k) == kernel
+
+
 @pytest.mark.parametrize("ggml,m,n,k", [(14, 45, 22548, 1280), (8, 73, 23033, 1792)])
 def test_the_96_column_tile_takes_rows_of_a_few_super_blocks(api, d, ggml, m, n, k):
     assert taken_by(api, d, ggml, m, n, k) == "m256"
