@@ -287,8 +287,10 @@ bool gemm_takes_decoded(GemmArgs& a) {
     const uint32_t asked = (uint32_t)a.decoded_tile;
     // (the fused estimate is 4 - 6% low where the chip is full and hot, Q6_K's 1%; a product that only the square tiles take, few columns and
     // rows too long to be resident, has none: 300 x 512 x 4096 36 us there, 71 to 101 here)
+    // Rows of one super-block are all starts and stores, which the fused estimate puts too high: 786 x 144422 x 256 Q5_K 178 us
+    // there, 228 here, nine of eleven such products slower (profiles/routes_us.txt); from two super-blocks on they gain.
     double best = forced ? 1e300 : gemm_fused_estimate(a) * (a.ggml_type == kQ6K ? 1.05 : 1.1);
-    if (!forced && best >= 1e300) return false;
+    if (!forced && (best >= 1e300 || a.k < 512)) return false;
     for (const DecodedTile& t : kDecodedTiles) {
         if (asked != 0 && asked != t.columns) continue;
         const uint64_t most = kMostPanelBytes / ((uint64_t)a.k * 2 * t.columns);

@@ -1892,9 +1892,10 @@ def test_the_fastest_of_the_decoded_tiles_is_taken(api, d, ggml, m, n, k, tile):
         d.set_tuning("gemm_decoded_tile", 0)
 
 
-@pytest.mark.parametrize("ggml,m,n,k", [(14, 768, 28672, 4096), (12, 1999, 5120, 17408), (8, 512, 17408, 5120)])
+@pytest.mark.parametrize("ggml,m,n,k", [(14, 768, 28672, 4096), (12, 1999, 5120, 17408), (8, 512, 17408, 5120),
+                                         (13, 786, 144422, 256)])
 def test_products_that_the_fused_tiles_run_faster_are_not_decoded(api, d, ggml, m, n, k):
-    # us, fused / the best panel: 245 / 271, 352 / 403, 141 / 170
+    # us, fused / the best panel: 245 / 271, 352 / 403, 141 / 170, 178 / 222
     base = synth.matrix(ggml, 3, k, seed=787)
     w = qm(api, d, ggml, n, k, np.resize(base, base.size // 3 * n))
     xt = api.Tensor.from_f32(d, (m, k), api.DType.BF16, synth.activations(m, k, seed=788))
