@@ -1184,6 +1184,10 @@ def test_uneven_shares_of_a_row_count_against_the_few_rows_kernel(api, d, ggml, 
     assert taken_by(api, d, ggml, m, n, k) == kernel
 
 
+def test_a_last_round_behind_one_of_pairs_counts_against_the_tiles(api, d):
+    assert taken_by(api, d, Q4_K, 41, 96877, 1536) == "resident"
+
+
 @pytest.mark.parametrize("ggml,m,n,k", [(14, 45, 22548, 1280), (8, 73, 23033, 1792)])
 def test_the_96_column_tile_takes_rows_of_a_few_super_blocks(api, d, ggml, m, n, k):
     assert taken_by(api, d, ggml, m, n, k) == "m256"
