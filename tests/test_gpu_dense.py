@@ -462,6 +462,35 @@ def test_streamed_q6_k_sums_digits_of_the_activations_exactly(api, d, n, k, dtyp
         d.set_tuning("gemv_stream", 1)
 
 
+@pytest.mark.parametrize("rows", ["normal", "gated", "outliers", "spread"])
+@pytest.mark.parametrize("n,k", [(1000, 5120), (700, 17408)])
+def test_streamed_q6_k_rows_are_no_farther_from_64_bits_than_on_the_fma_kernel(api, d, n, k, rows):
+    # also where a group's largest activation leaves the others few of its 30 bits: a channel in 250 a thousand times the
+    # others, magnitudes spread over 2^20
+    packed = synth.matrix(Q6_K, n, k, seed=95)
+    w = qm(api, d, Q6_K, n, k, packed)
+    g = synth.rng(96)
+    x = g.standard_normal((1, k))
+    if rows == "gated":
+        x = 3 * x / (1 + np.exp(-3 * x)) * g.standard_normal((1, k))
+    elif rows == "outliers":
+        x = x * np.where(g.random((1, k)) < 0.004, 1000.0, 1.0)
+    elif rows == "spread":
+        x = x * 2.0 ** g.uniform(-20, 0, (1, k))
+    x = x.astype(np.float32)
+    xt = api.Tensor.from_f32(d, (1, k), api.DType.F32, x)
+    d.set_tuning("gemv_stream", 2)
+    try:
+        got = d.project_quantized(xt, w).tensor.to_f32()
+    finally:
+        d.set_tuning("gemv_stream", 1)
+    with fma_gemv(d):
+        other = d.project_quantized(xt, w).tensor.to_f32()
+    assert not np.array_equal(bits(got), bits(other))
+    want = x.astype(np.float64) @ oracle.dequantize(Q6_K, packed, n, k).reshape(n, k).astype(np.float64).T
+    assert rel_l2(got, want) <= rel_l2(other, want)
+
+
 def test_only_f32_rows_stream_q6_k_matrices_below_a_million_super_blocks(api, d):
     n, k = 32000, 5120     # 640,000 super-blocks, sixteen-row tiles
     base = synth.matrix(Q6_K, 2000, k, seed=35).reshape(2000, -1)
