@@ -260,22 +260,23 @@ void launch_tile(hipStream_t s, const DecodedParams& p, uint32_t columns) {
     else launch_product<DT, 4, 2, 4>(s, p);
 }
 
-// What a round of 256 workgroups of a tile takes per 5120 of K, in us (rows of real data, where the chip lowers its clock;
-// of zeros a round of 256 x 256 takes 105 instead of 128).
+// What a round of 256 workgroups of a tile takes, in us: a start (first loads, stores) and a time per 5120 of K (rows of real
+// data, where the chip lowers its clock; of zeros a round of 256 x 256 takes a sixth less).
 struct DecodedTile {
     uint32_t columns;
-    double round;
+    double start, round;
 };
-constexpr DecodedTile kDecodedTiles[] = {{192, 104.0}, {256, 128.0}, {320, 160.0}};
+constexpr DecodedTile kDecodedTiles[] = {{192, 11.7, 89.8}, {256, 16.2, 104.3}, {320, 18.8, 127.3}};
 constexpr size_t kMostPanelBytes = fh_device::kScratchOptional;
 
 }  // namespace
 
-// Decode at the rate of its stores, then rounds of the product, the last one cheaper where it is not full; against the
-// fused tiles' estimate.  All sides in turn (profiles/decoded_panels_us.txt), bf16, five formats x 20 shapes of 512 - 100000 columns and 512 - 17408 K x nine
-// row counts of 267 - 2048 (900 products, 885 with an estimate): 222 decode, the pick is 0.5% from the fastest of the four
-// in the mean and slower than the fused tiles by more than 3% for one (Q5_K 1500 x 19864 x 512 66 / 69; with one margin for all
-// also Q6_K 768 x 28672 x 4096 245 / 271).  us, fused tiles / 192 / 256 / 320 columns: Q4_K 1999 x 34816 x 5120 778 / 789 / 752 / 718, 1999 x 17408
+// The decode by its bytes, then rounds of the product, the last one cheaper where it is not full; against the fused tiles'
+// estimate.  Fitted to the 2463 panels timed in profiles/routes_us.txt (rows of 256 - 17408), 6.4% in the mean square; constants from long
+// rows with one start for all tiles were 19% too high in the mean, most for 192 columns and short rows, and margins on the other side did
+// not make up for it (us, taken by those / now: Q6_K 1791 x 5002 x 1536 57 / 51, 741 x 19548 x 1024 67 / 61, Q5_K 1030 x 14387 x 2048
+// 108 / 100).  Over the 821 products there the pick is 0.3% from the fastest of the four in the mean, and so it is over
+// the 885 of profiles/decoded_panels_us.txt, where 245 decode and five are slower than the fused tiles by more than 3%.  us, fused tiles / 192 / 256 / 320 columns: Q4_K 1999 x 34816 x 5120 778 / 789 / 752 / 718, 1999 x 17408
 // x 5120 425 / 380 / 414 / 355, 1999 x 12288 x 4096 231 / 208 / 218 / 256, 1999 x 5120 x 17408 352 / 403 / 411 / 461; Q6_K
 // 1999 x 34816 x 5120 925 / 802 / 767 / 730, 1024 x 12288 x 4096 149 / 120 / 124 / 132; Q8_0 1999 x 17408 x 5120 553 / 400
 // / 423 / 367, 1500 x 8192 x 8192 336 / 319 / 221 / 234.
@@ -285,12 +286,13 @@ bool gemm_takes_decoded(GemmArgs& a) {
     const bool forced = a.decoded_min_rows > 1;   // from that many rows on, whatever the estimates say
     if (forced && a.m < (uint32_t)a.decoded_min_rows) return false;
     const uint32_t asked = (uint32_t)a.decoded_tile;
-    // (the fused estimate is 4 - 6% low where the chip is full and hot, Q6_K's 1%; a product that only the square tiles take, few columns and
-    // rows too long to be resident, has none: 300 x 512 x 4096 36 us there, 71 to 101 here)
+    // (Q6_K's fused estimate is 2 - 4% high from 512 rows on: 768 x 28672 x 4096 245 us there, 271 here; a product that only the square
+    // tiles take, few columns and rows too long to be resident, has none: 300 x 512 x 4096 36 us there, 71 to 101 here)
     // Rows of one super-block are all starts and stores, which the fused estimate puts too high: 786 x 144422 x 256 Q5_K 178 us
     // there, 228 here, nine of eleven such products slower (profiles/routes_us.txt); from two super-blocks on they gain.
-    double best = forced ? 1e300 : gemm_fused_estimate(a) * (a.ggml_type == kQ6K ? 1.05 : 1.1);
-    if (!forced && (best >= 1e300 || a.k < 512)) return false;
+    const double fused = forced ? 1e300 : gemm_fused_estimate(a);
+    if (!forced && (fused >= 1e300 || a.k < 512)) return false;
+    double best = a.ggml_type == kQ6K ? 0.96 * fused : fused;
     for (const DecodedTile& t : kDecodedTiles) {
         if (asked != 0 && asked != t.columns) continue;
         const uint64_t most = kMostPanelBytes / ((uint64_t)a.k * 2 * t.columns);
@@ -300,11 +302,11 @@ bool gemm_takes_decoded(GemmArgs& a) {
         uint32_t tiles = (uint32_t)std::min<uint64_t>(most, tiles_n);
         if (tiles < tiles_n && (uint64_t)tiles * tiles_m > cus)
             tiles = std::max(1u, (uint32_t)((uint64_t)tiles * tiles_m / cus * cus / tiles_m));
-        double us = 3.0 + (double)a.n * a.k * (2.0 + block_bytes(a.ggml_type) / 256.0) / 5.6e6;
+        double us = (double)a.n * a.k * (2.0 + block_bytes(a.ggml_type) / 256.0) / 4.28e6;
         for (uint32_t first = 0; first < tiles_n; first += tiles) {
             const double rounds = (double)std::min(tiles, tiles_n - first) * tiles_m / cus;
             const double whole = (double)(uint64_t)rounds, part = rounds - whole;
-            us += 11.0 + 17.0 * (whole + (part > 0)) + (whole + (part > 0 ? 0.6 + 0.4 * part : 0.0)) * t.round * a.k / 5120.0;
+            us += 5.2 + t.start * (whole + (part > 0)) + (whole + (part > 0 ? 0.68 + 0.32 * part : 0.0)) * t.round * a.k / 5120.0;
         }
         if (us < best) {
             best = us;

@@ -1899,7 +1899,8 @@ def test_weights_decoded_first_give_the_bits_of_the_fused_tiles(api, d, ggml, m,
 
 
 @pytest.mark.parametrize("ggml,m,n,k,tile", [(14, 1024, 12288, 4096, 192), (8, 1999, 7147, 4352, 256), (14, 1500, 8192, 8192, 256),
-                                             (14, 1999, 17408, 5120, 320), (12, 1999, 17408, 5120, 320)])
+                                             (14, 1999, 17408, 5120, 320), (12, 1999, 17408, 5120, 320),
+                                             (14, 741, 19548, 1024, 256), (13, 1030, 14387, 2048, 320)])
 def test_the_fastest_of_the_decoded_tiles_is_taken(api, d, ggml, m, n, k, tile):
     # shapes where one tile is the fastest of three by 5% to 30%, all of them faster than the fused tiles; also where the
     # caller asks for panels and leaves the tile open
