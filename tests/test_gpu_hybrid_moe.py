@@ -329,3 +329,32 @@ def test_hybrid_entry_points_reject_bad_geometry(api, d):
     with pytest.raises(api.DTypeError):
         d.hybrid_moe_combine(down, api.Tensor.zeros(d, (8,), f32), None, api.Tensor.zeros(d, (4, 64), f32),
                              api.Tensor.zeros(d, (4,), f32), 2)
+
+
+@pytest.mark.parametrize("used,hidden", [(1, 4), (7, 1028), (8, 6), (9, 2048), (17, 36)])
+@pytest.mark.parametrize("sorted_rows", [False, True])
+def test_combine_takes_its_routes_eight_at_a_time(api, d, used, hidden, sorted_rows):
+    # one, a group less and more one, two groups and one more; rows of whole float4s and of single floats.  A chain of
+    # used + 1 fused products, each off by 2^-24 of a sum that stays below that of the magnitudes, on either side
+    tokens, rng, f32 = 5, synth.rng(461 + used), api.DType.F32
+    down = rng.standard_normal((tokens * used, hidden)).astype(np.float32)
+    weights = rng.random((tokens, used)).astype(np.float32)
+    shared = rng.standard_normal((tokens, hidden)).astype(np.float32)
+    gate = rng.random(tokens).astype(np.float32)
+    position = rng.permutation(tokens * used).astype(np.uint32)
+    place = carrier(api, d, position) if sorted_rows else None
+    got = d.hybrid_moe_combine(api.Tensor.from_f32(d, down.shape, f32, down), api.Tensor.from_f32(d, weights.shape, f32, weights),
+                               place, api.Tensor.from_f32(d, shared.shape, f32, shared),
+                               api.Tensor.from_f32(d, gate.shape, f32, gate), used).to_f32()
+    rows = (down[position] if sorted_rows else down).reshape(tokens, used, hidden).astype(np.float64)
+    terms = np.concatenate([rows * weights[:, :, None], (gate[:, None] * shared.astype(np.float64))[:, None]], axis=1)
+    assert np.all(np.abs(got - terms.sum(axis=1)) <= (used + 1) * 2.0 ** -24 * np.abs(terms).sum(axis=1))
+
+
+@pytest.mark.parametrize("hidden,dtype", [(3, "F16"), (1, "F32"), (4096, "F32"), (4100, "F32"), (8192, "BF16"), (1030, "BF16"), (20480, "F16")])
+def test_gather_copies_rows_of_any_number_of_pieces(api, d, hidden, dtype):
+    tokens, used = 7, 3
+    x = api.Tensor.from_f32(d, (tokens, hidden), api.DType[dtype], synth.activations(tokens, hidden, seed=471))
+    order = synth.rng(472).permutation(tokens * used).astype(np.uint32)
+    got = d.hybrid_moe_gather(x, carrier(api, d, order), used)
+    assert np.array_equal(bits(got.to_f32()), bits(x.to_f32()[order // used]))

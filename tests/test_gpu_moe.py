@@ -163,6 +163,21 @@ def test_silu_mul_and_combine_keep_the_storage_rounding_points(api, d):
         assert np.array_equal(bits(got), bits(want))
 
 
+@pytest.mark.parametrize("rows,inter", [(1, 8), (3, 520), (257, 2056)])
+@pytest.mark.parametrize("source", ["F32", "F16", "BF16"])
+@pytest.mark.parametrize("target", ["F32", "F16", "BF16"])
+def test_silu_mul_between_all_pairs_of_types(api, d, rows, inter, source, target):
+    # eight columns at a time, for every pair of types; rows of one group, of a ragged number, and more than a block of them
+    x = synth.activations(rows, 2 * inter, seed=25)
+    t = api.Tensor.from_f32(d, (rows, 2 * inter), api.DType[source], x)
+    out = d.expert_silu_mul(t, inter, out=api.Tensor.zeros(d, (rows, inter), api.DType[target])).to_f32()
+    want = oracle.expert_silu_mul(t.to_f32(), inter, getattr(oracle, target))
+    # f32: an exponential of up to two units in the last place, a sum, a division and a product, on either side: six.  16
+    # bits: SiLU and the product are rounded to storage, each by a step at most where those differ
+    step = {"F32": 6 * 2.0 ** -23, "F16": 2.0 ** -9, "BF16": 2.0 ** -6}[target]
+    assert np.all(np.abs(out - want) <= step * np.maximum(np.abs(want), 1e-3))
+
+
 @pytest.mark.parametrize("tokens", [1, 48])
 def test_routed_ffn_pipeline_matches_the_oracle(api, d, tokens):
     # hidden 2048, intermediate 512, top-8; 16 experts keep the CPU side quick
