@@ -422,6 +422,7 @@ constexpr struct {
     {"gemm_wide32_segments", &fh_tuning::gemm_wide32_segments},
     {"gemm_decoded_min_rows", &fh_tuning::gemm_decoded_min_rows},
     {"gemm_decoded_tile", &fh_tuning::gemm_decoded_tile},
+    {"gemm_decoded_segments", &fh_tuning::gemm_decoded_segments},
     {"gemm_wide_min_rows", &fh_tuning::gemm_wide_min_rows},
     {"gemm_skinny_max_rows", &fh_tuning::gemm_skinny_max_rows},
     {"expert_grouped_min_assignments", &fh_tuning::expert_grouped_min_assignments},
@@ -668,7 +669,8 @@ fh_status fh_set_tuning(fh_device* device, const char* key, int64_t value) {
         ok = value == 0 || value == 1;
     } else if (k == "gemv_stream_own_loads" || k == "expert_weight_ring") {
         ok = value == 0 || value == 1;
-    } else if (k == "gemv_stream" || k == "gemv_ring" || k == "gemm_few_tiles_split") {
+    } else if (k == "gemv_stream" || k == "gemv_ring" || k == "gemm_few_tiles_split" ||
+               k == "gemm_decoded_segments") {
         ok = value >= 0 && value <= 2;
     } else if (k == "gemm_wide_shape") {
         ok = value >= 0 && value <= 2;
@@ -722,6 +724,10 @@ fh_status fh_get_tuning(const fh_device* device, const char* key, int64_t* value
     }
     if (std::strcmp(key, "last_decoded_tile") == 0) {
         *value = device->last_decoded_tile;
+        return FH_OK;
+    }
+    if (std::strcmp(key, "last_decoded_cut") == 0) {
+        *value = device->last_decoded_cut;
         return FH_OK;
     }
     const int64_t* const setting = tuning_of(device, key);
@@ -995,6 +1001,7 @@ GemmArgs gemm_args(const fh_device* device, uint32_t ggml_type, uint64_t n, uint
     g.wide32_segments = (int)device->tuning.gemm_wide32_segments;
     g.decoded_min_rows = (int)device->tuning.gemm_decoded_min_rows;
     g.decoded_tile = (int)device->tuning.gemm_decoded_tile;
+    g.decoded_segments = (int)device->tuning.gemm_decoded_segments;
     g.cut_tiles = true;
     g.skinny_max_rows = (int)device->tuning.gemm_skinny_max_rows;
     g.resident_switch = device->tuning.gemm_resident != 0;
@@ -1014,8 +1021,8 @@ fh_status prepare_gemm(fh_device* device, GemmArgs& g, size_t used) {
         const size_t partial_bytes = gemm_partial_bytes(g);
         st = partial_bytes != 0 ? optional_scratch(device, at + partial_bytes) : ensure_scratch(device, used);
         if (st != FH_ERR_ALLOCATION || partial_bytes == 0) break;
-        if (g.decoded_columns != 0) {
-            g.decoded_columns = 0;
+        if (g.decoded.runs != 0) {
+            g.decoded.runs = 0;
         } else if (g.rows_plan.pairs) {
             g.rows_plan = g.rows_else;
             if (g.rows_plan.rows == 0) return ensure_scratch(device, used);
@@ -1038,7 +1045,9 @@ fh_status prepare_gemm(fh_device* device, GemmArgs& g, size_t used) {
 const char* run_gemm(fh_device* device, GemmArgs& g) {
     const RowsPlan& plan = g.rows_plan;
     device->last_rows_plan = plan.rows * 1000 + plan.tiles * 100 + plan.segments;
-    device->last_decoded_tile = g.decoded_columns != 0 ? g.decoded_tile : 0;
+    const int64_t decoded_tile = g.decoded.runs != 0 ? g.decoded.run[0].tile : 0;
+    device->last_decoded_tile = g.decoded.segments == 1 ? decoded_tile : 0;
+    device->last_decoded_cut = g.decoded.segments == 2 ? decoded_tile : 0;
     return launch_gemm(device->stream, g);
 }
 
@@ -1115,7 +1124,7 @@ fh_status project(fh_device* device, const fh_qmatrix* weight, const fh_view* x,
     const bool f32_batch = !tile && !silu_mul && x->dtype == FH_F32 && m >= (weight->ggml_type == kQ4K ? 5u : 4u) &&
                            m >= (uint32_t)device->tuning.gemm_min_rows && device->tuning.gemv_stream == 1 &&
                            device->tuning.k_quant_gemv_ksplit == 0;
-    device->last_rows_plan = device->last_decoded_tile = 0;
+    device->last_rows_plan = device->last_decoded_tile = device->last_decoded_cut = 0;
     GemmArgs g{};
     if (tile || f32_batch) g = gemm_args(device, weight->ggml_type, n, k, m, f32_tile ? FH_F16 : x->dtype, y->dtype);
     if (f32_batch && g.few_rows) {

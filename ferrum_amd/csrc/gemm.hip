@@ -1459,7 +1459,7 @@ double gemm_fused_estimate(GemmArgs& a) {
 }
 
 size_t gemm_partial_bytes(GemmArgs& a) {
-    if (a.decoded_columns != 0) return (size_t)(std::min(a.decoded_columns, a.n) + 31) / 32 * 32 * a.k * 2;
+    if (a.decoded.runs != 0) return a.decoded.panel_bytes + a.decoded.sum_bytes;
     if (a.rows_plan.rows != 0) return a.rows_plan.partial_bytes;
     const TileChoice& c = tile_choice(a);
     if (c.p32.nt == 0 || c.p32.segments == 1 || c.us16 < c.us32 || takes_resident(a, c)) return 0;
@@ -1469,8 +1469,8 @@ size_t gemm_partial_bytes(GemmArgs& a) {
 const char* launch_gemm(hipStream_t s, GemmArgs& a) {
     static const char* const tile_names[5] = {"q4_k_gemm_mfma_m256", "q5_k_gemm_mfma_m256", "iq4_xs_gemm_mfma_m256",
                                               "q6_k_gemm_mfma_m256", "q8_0_gemm_mfma_m256"};
-    if (a.decoded_columns != 0) {
-        launch_gemm_decoded(s, a);   // (the bits of the 32x32x16 tiles, uncut)
+    if (a.decoded.runs != 0) {
+        launch_gemm_decoded(s, a);   // (the bits of the 32x32x16 tiles where both are uncut)
         return tile_names[cost_column(a.ggml_type)];
     }
     if (a.rows_plan.rows != 0) {

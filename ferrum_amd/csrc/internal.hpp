@@ -25,6 +25,7 @@ struct fh_tuning {
     int64_t gemm_wide32_segments = 0;  // K segments of the 32x32x16 form: 0 = by shape (a forced tile or form: uncut), else at most that many, up to 8 (a forced tile: exactly)
     int64_t gemm_decoded_min_rows = 1; // products that decode their weights into the scratch first: 0 never, 1 where estimated faster, else from that many rows on (and 257), fewer never
     int64_t gemm_decoded_tile = 0;     // their tile: 0 = by shape; 192, 256 or 320 columns
+    int64_t gemm_decoded_segments = 0; // and their K segments: 0 = by shape, 1 = uncut, 2 = two
     int64_t gemm_wide_min_rows = 33;   // smallest M that takes the 256-row tile (it wins from there up)
     int64_t gemm_skinny_max_rows = 64; // with gemm_resident 0: largest M that takes the few-rows kernel (0 = never)
     int64_t expert_grouped_min_assignments = 32;  // fewest assignments grouped by expert (0 = never)
@@ -52,7 +53,8 @@ struct fh_device {
     hipDeviceProp_t props{};
     const char* last_operation = "";
     int64_t last_rows_plan = 0;   // of the last dense product: 0, or the few-rows kernel's rows, tiles and K segments
-    int64_t last_decoded_tile = 0;   // ... and 0, or the columns of its tile where its weights were decoded first
+    int64_t last_decoded_tile = 0;   // ... and 0, or the columns of its (first) tile where its weights were decoded first
+    int64_t last_decoded_cut = 0;    // ... where its K was cut in two besides: this one and not the one before
     std::atomic<bool> capturing{false};   // changes under pool_lock: what empties the pool waits on the stream
     fh_tuning tuning;
     // Blocks of freed buffers, by size, for the buffers to come (fh_buffer_alloc): hipMalloc and hipFree
@@ -343,6 +345,17 @@ struct TileChoice {
     double us32, us16;
 };
 
+// How a product multiplies weights that were decoded first: its columns in up to three runs of tiles, a panel of each run at a time.
+struct DecodedPlan {
+    struct Run {
+        uint32_t columns, tile, panel;   // of the matrix; of a tile; decoded at a time, a multiple of `tile`
+    } run[3];
+    int runs;              // 0: the weights are not decoded first
+    uint32_t segments;     // K segments: 1, or 2 (one run then)
+    size_t panel_bytes, sum_bytes;   // scratch: the largest panel, then the sums of one segment's tiles
+    double estimate_us;
+};
+
 struct GemmArgs {
     uint32_t ggml_type;
     const void* w;
@@ -358,8 +371,9 @@ struct GemmArgs {
     bool cut_tiles;      // its partial sums have room in the scratch (`partials`)
     TileChoice tile;     // made when first asked for; to be made again when cut_tiles changes
     int decoded_min_rows;      // rows from which the weights may be decoded once, in panels (0 = never)
-    int decoded_tile;          // columns of the product's tile: 0 = by shape (gemm_takes_decoded sets it)
-    uint32_t decoded_columns;  // set by gemm_takes_decoded: columns of a panel, which lies in `partials`
+    int decoded_tile;          // columns of the product's tile: 0 = by shape
+    int decoded_segments;      // K segments of the product: 0 = by shape, else 1 or 2
+    DecodedPlan decoded;       // set by gemm_takes_decoded; its panel and sums lie in `partials`
     int skinny_max_rows; // largest M that takes the register-dequant kernel where the rows-resident one is switched off
     // routed-expert form of the register-dequant kernel: w is [experts, n, k],
     // x and y rows are assignments, m is their count; tokens of expert e are
@@ -398,7 +412,7 @@ const char* launch_gemm(hipStream_t s, GemmArgs& a);
 // counters the caller then provides
 bool gemm_takes_rows(GemmArgs& a);
 
-// whether the weights are decoded into the scratch first, a panel of a.decoded_columns at a time (gemm_decoded.hip)
+// whether the weights are decoded into the scratch first (gemm_decoded.hip): fills a.decoded
 bool gemm_takes_decoded(GemmArgs& a);
 void launch_gemm_decoded(hipStream_t s, const GemmArgs& a);
 double gemm_fused_estimate(GemmArgs& a);   // us of the kernel that decodes as it multiplies; 1e300: none is estimated

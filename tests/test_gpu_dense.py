@@ -1898,6 +1898,66 @@ def test_weights_decoded_first_give_the_bits_of_the_fused_tiles(api, d, ggml, m,
                          "fused tiles")
 
 
+@pytest.mark.parametrize("ggml,m,n,k,dtype", [(12, 257, 33, 512, "F16"), (14, 300, 1000, 768, "BF16"), (8, 513, 2572, 1280, "F16"),
+                                              (23, 700, 517, 2304, "BF16"), (13, 1025, 644, 4352, "F16"), (12, 2048, 1280, 2048, "BF16")])
+def test_decoded_products_with_k_cut_in_two(api, d, ggml, m, n, k, dtype):
+    # two super-blocks to seventeen, even and odd, ragged rows and columns, rows that are whole fours and rows that are not, one
+    # tile and several rows of them.  At most k / 8 sums follow each other on either side, each off by 2^-24 at most, uniform.
+    packed = synth.matrix(ggml, n, k, seed=771)
+    w = qm(api, d, ggml, n, k, packed)
+    code = oracle.F16 if dtype == "F16" else oracle.BF16
+    x = oracle.round_storage(synth.activations(m, k, seed=772), code).reshape(m, k)
+    xt = api.Tensor.from_f32(d, (m, k), getattr(api.DType, dtype), x)
+    rows = np.unique(np.concatenate([np.arange(0, 20), np.arange(n - 20, n)]))
+    want = oracle_columns(ggml, packed, n, k, rows, x, weight_round=code, accumulate="f64")
+    bound = 2.0 ** -24 / np.sqrt(3) * np.sqrt(k / 16)
+    try:
+        d.set_tuning("gemm_decoded_min_rows", 2)
+        for tile in (192, 256, 320):
+            d.set_tuning("gemm_decoded_tile", tile)
+            d.set_tuning("gemm_decoded_segments", 1)
+            whole = d.project_quantized(xt, w, out_dtype=api.DType.F32).tensor.to_f32()
+            assert (d.get_tuning("last_decoded_tile"), d.get_tuning("last_decoded_cut")) == (tile, 0)
+            d.set_tuning("gemm_decoded_segments", 2)
+            got = d.project_quantized(xt, w, out_dtype=api.DType.F32).tensor.to_f32()
+            assert (d.get_tuning("last_decoded_tile"), d.get_tuning("last_decoded_cut")) == (0, tile)
+            assert rel_l2(got[:, rows], want) <= bound and rel_l2(got, whole) <= np.sqrt(2) * bound
+            stored = api.Tensor.zeros(d, (m, n), getattr(api.DType, dtype))
+            with d.execution() as recording:       # whichever segment ends first, the same bits; also replayed
+                d.project_quantized(xt, w, out=stored)
+            for _ in range(3):
+                recording.graph.launch()
+                d.synchronize()
+                assert np.array_equal(bits(stored.to_f32()), bits(oracle.round_storage(got, code).reshape(m, n)))
+                assert np.array_equal(bits(d.project_quantized(xt, w, out_dtype=api.DType.F32).tensor.to_f32()), bits(got))
+    finally:
+        d.set_tuning("gemm_decoded_min_rows", 1)
+        d.set_tuning("gemm_decoded_tile", 0)
+        d.set_tuning("gemm_decoded_segments", 0)
+
+
+@pytest.mark.parametrize("m,n", [(300, 57344), (300, 57001), (520, 34816), (600, 24000), (1300, 14336)])
+def test_runs_of_several_decoded_tiles_give_the_bits_of_one(api, d, m, n):
+    # columns of more than a round of the chip, in runs of up to three tiles: every column comes from one of them
+    k = 512
+    base = synth.matrix(Q4_K, 251, k, seed=775).reshape(251, -1)
+    w = qm(api, d, Q4_K, n, k, np.resize(base, (n, base.shape[1])).reshape(-1))
+    xt = api.Tensor.from_f32(d, (m, k), api.DType.F16, synth.activations(m, k, seed=776))
+    out = api.Tensor.zeros(d, (m, n), api.DType.F16)
+    try:
+        d.set_tuning("gemm_decoded_min_rows", 2)
+        d.project_quantized(xt, w, out=out)
+        runs = out.raw()
+        assert d.get_tuning("last_decoded_tile") != 0
+        for tile in (192, 256, 320):
+            d.set_tuning("gemm_decoded_tile", tile)
+            d.project_quantized(xt, w, out=out)
+            assert np.array_equal(out.raw(), runs), tile
+    finally:
+        d.set_tuning("gemm_decoded_min_rows", 1)
+        d.set_tuning("gemm_decoded_tile", 0)
+
+
 @pytest.mark.parametrize("ggml,m,n,k,tile", [(14, 1024, 12288, 4096, 192), (8, 1999, 7147, 4352, 256), (14, 1500, 8192, 8192, 256),
                                              (14, 1999, 17408, 5120, 320), (12, 1999, 17408, 5120, 320),
                                              (14, 741, 19548, 1024, 256), (13, 1030, 14387, 2048, 320)])
