@@ -77,11 +77,13 @@ bool fits_u32(uint64_t v) { return v <= 0xffffffffull; }
 // Gives back what the pool holds; whether that was anything.  The caller has pool_lock.  A device that is
 // recording keeps its blocks: neither a wait on its stream nor a free may fall into a recording.
 bool drain_locked(fh_device* d) {
-    if (d->pool.empty() || d->capturing) return false;
+    if ((d->pool.empty() && d->leaving.empty()) || d->capturing) return false;
     (void)hipStreamSynchronize(d->stream);
     for (auto& block : d->pool) (void)hipFree(block.second);
+    for (auto& block : d->leaving) (void)hipFree(block.second);
     d->pool.clear();
-    d->pool_bytes = 0;
+    d->leaving.clear();
+    d->pool_bytes = d->leaving_bytes = 0;
     return true;
 }
 
@@ -452,6 +454,7 @@ auto tuning_of(Device* d, const char* key) -> decltype(&(d->tuning.gemm_min_rows
 
 constexpr size_t kPoolBytes = 256u << 20;       // most memory kept
 constexpr size_t kPoolBlockBytes = 64u << 20;   // largest block kept
+constexpr size_t kLeavingBytes = 64u << 20, kLeavingBlocks = 512;   // blocks that wait for the GPU together
 
 // Blocks come in sizes a quarter of a power of two apart (4 KiB at least), so that a batch a little larger
 // or smaller finds them.
@@ -476,12 +479,43 @@ hipError_t take_block(fh_device* d, size_t capacity, void** out) {
     return allocate(d, out, capacity);
 }
 
+// Blocks whose address the caller has been given: one goes back to the system, and hipFree waits for all work on the GPU, on
+// whatever stream, that was asked for before; none of the others is in use any more then.  The caller has pool_lock.
+void settle_leaving(fh_device* d) {
+    (void)hipFree(d->leaving.back().second);
+    d->leaving.pop_back();
+    for (auto& block : d->leaving) {
+        bool kept = false;
+        if (d->pool_bytes + block.first <= kPoolBytes) {
+            try {
+                d->pool.emplace(block.first, block.second);
+                d->pool_bytes += block.first;
+                kept = true;
+            } catch (...) {   // no memory for the entry
+            }
+        }
+        if (!kept) (void)hipFree(block.second);
+    }
+    d->leaving.clear();
+    d->leaving_bytes = 0;
+}
+
 // Takes a freed buffer's block into the pool; false: the caller frees it.  Nothing waits: whatever the
 // library still has to do with the block comes before the next buffer's work on the stream.  A block whose
-// address the caller has been given may be in use elsewhere and goes back to the system.
+// address the caller has been given may be in use elsewhere and waits, with others, until it cannot be.
 bool keep_block(fh_device* d, const fh_buffer& buffer) {
     std::lock_guard<std::mutex> hold(d->pool_lock);
-    if (d->closed || d->capturing || buffer.exposed || buffer.capacity > kPoolBlockBytes) return false;
+    if (d->closed || d->capturing || buffer.capacity > kPoolBlockBytes) return false;
+    if (buffer.exposed) {
+        try {
+            d->leaving.emplace_back(buffer.capacity, buffer.ptr);
+        } catch (...) {
+            return false;
+        }
+        d->leaving_bytes += buffer.capacity;
+        if (d->leaving_bytes >= kLeavingBytes || d->leaving.size() >= kLeavingBlocks) settle_leaving(d);
+        return true;
+    }
     if (d->pool_bytes + buffer.capacity > kPoolBytes) drain_locked(d);   // it holds sizes that are no longer asked for
     try {
         d->pool.emplace(buffer.capacity, buffer.ptr);

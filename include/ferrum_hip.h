@@ -145,7 +145,9 @@ fh_status fh_get_tuning(const fh_device* device, const char* key, int64_t* value
  * 64 MiB each) for the next ones and returns them to the system when it is
  * destroyed or an allocation of any device object on that GPU finds no memory;
  * freeing does not wait for the stream then.
- * Buffers whose address fh_buffer_device_ptr has given out are not kept. */
+ * Buffers whose address fh_buffer_device_ptr has given out wait until nothing on the GPU, on whatever stream, can still use
+ * them: up to 64 MiB or 512 of them gather, then one hipFree, which waits for the GPU, serves all, and the others are kept.
+ * held_pool_bytes does not count those that wait; setting it to 0 gives them back too. */
 fh_status fh_buffer_alloc(fh_device* device, size_t bytes, fh_buffer** out);
 fh_status fh_buffer_alloc_uninitialized(fh_device* device, size_t bytes, fh_buffer** out);
 void fh_buffer_free(fh_buffer* buffer);

@@ -7,6 +7,7 @@ with its closed-form inputs and its tolerances; the second half applies the
 benchmark's bars (dequant bit-exact; max relative error 1e-3 and relative L2
 1e-5 with f32 accumulation) at the benchmark shapes on seeded synthetic blocks.
 """
+import ctypes
 import functools
 
 import numpy as np
@@ -1355,6 +1356,44 @@ def test_a_full_pool_makes_room_and_an_exposed_address_is_not_handed_on(api):
     assert not x.raw().any()
     with pytest.raises(api.Error):
         dev.set_tuning("held_pool_bytes", 1)
+
+
+def test_blocks_whose_address_has_left_wait_for_all_work_on_the_gpu(api):
+    dev, size, steps = api.Device.new(), 4 << 20, 40     # more than wait together
+    kept = lambda: dev.get_tuning("held_pool_bytes")
+    hip, other = api._lib, ctypes.c_void_p()             # (the runtime the library is linked with)
+    assert hip.hipStreamCreateWithFlags(ctypes.byref(other), 1) == 0
+    copy = lambda to, source, count: hip.hipMemcpyAsync(ctypes.c_void_p(to), ctypes.c_void_p(source), ctypes.c_size_t(count), 3, other)
+    busy, copies, reused = api.Buffer(dev, 512 << 20), api.Buffer(dev, steps * size), False
+    dev.synchronize()
+    for step in range(steps):
+        b = api.Buffer(dev, size)
+        b.upload(0, np.full(size // 4, step + 1, np.uint32))
+        # its last use, on a stream of the caller's, is far from done when the buffer is dropped
+        for _ in range(2):
+            assert copy(busy.device_ptr(), busy.device_ptr() + (256 << 20), 256 << 20) == 0
+        assert copy(copies.device_ptr() + step * size, b.device_ptr(), size) == 0
+        before = kept()
+        del b
+        assert kept() <= 64 << 20
+        reused = reused or kept() > before
+        fresh = api.Buffer(dev, size)                    # may get its block, and clears it at once
+        del fresh
+    assert hip.hipStreamSynchronize(other) == 0 and hip.hipStreamDestroy(other) == 0
+    for step in range(steps):
+        assert np.all(copies.download(step * size, size).view(np.uint32) == step + 1), step
+    assert reused
+    b = api.Buffer(dev, 1 << 20)
+    assert b.device_ptr()
+    del b
+    dev.set_tuning("held_pool_bytes", 0)
+    assert kept() == 0
+    small = [api.Buffer(dev, 4096) for _ in range(600)]     # and no more blocks than that, however small
+    assert all(x.device_ptr() for x in small)
+    small.clear()
+    assert 0 < kept() <= 600 * 4096
+    dev.set_tuning("held_pool_bytes", 0)
+    assert kept() == 0
 
 
 def test_one_device_object_gives_back_what_another_on_the_gpu_keeps(api):
