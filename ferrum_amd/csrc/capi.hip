@@ -1163,7 +1163,7 @@ fh_status project(fh_device* device, const fh_qmatrix* weight, const fh_view* x,
     if (tile || f32_batch) g = gemm_args(device, weight->ggml_type, n, k, m, f32_tile ? FH_F16 : x->dtype, y->dtype);
     if (f32_batch && g.few_rows) {
         g.rows_plan = gemm_rows_plan(g.ggml_type, g.n, g.k, g.m, g.x_dtype, g.cu_count);
-        if (g.rows_plan.counters > fh_device::kCounterWords ||
+        if (g.rows_plan.counters > fh_device::kCounterWords || !rows_batch_fits(g.rows_plan, g.k, g.x_dtype) ||
             (!g.few_rows_always && !gemv_streams(device, weight->ggml_type, n, k, m) &&
              !f32_rows_pay(g.rows_plan, g.ggml_type, g.n, g.k, m, g.cu_count)))
             g.rows_plan = RowsPlan{};

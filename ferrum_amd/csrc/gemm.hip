@@ -1435,7 +1435,7 @@ bool gemm_takes_rows(GemmArgs& a) {
     if (!a.few_rows || a.m < 2 || a.m > 128) return false;
     if (a.wide32_tile != 0 && a.wide_shape != 0 && a.m >= (uint32_t)a.wide_min_rows) return false;   // a tile is asked for
     const RowsPlan plan = gemm_rows_plan(a.ggml_type, a.n, a.k, a.m, a.x_dtype, a.cu_count);
-    if (plan.counters > fh_device::kCounterWords) return false;
+    if (plan.counters > fh_device::kCounterWords || !rows_batch_fits(plan, a.k, a.x_dtype)) return false;
     if (!a.few_rows_always && a.resident_switch) {
         const TileChoice& c = tile_choice(a);
         // (a cut tile has to gain a sixth on a plan that needs no partial sums: 80 x 17408 x 5120 stays here, 55 us

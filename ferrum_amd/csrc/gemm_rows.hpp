@@ -12,7 +12,7 @@
 // last workgroup to arrive.
 //
 // Activations travel as whole cache lines straight into a piece of LDS that belongs to the wave
-// (global_load_lds, 16 bytes a lane) and from there into operand order; loading operands from
+// (buffer_load .. lds, 16 bytes a lane) and from there into operand order; loading operands from
 // memory as they are used would touch one line per lane.  They are requested one super-block ahead,
 // like the weights: loads return in order, so a nearer request would wait for the farther ones.
 #pragma once
@@ -22,6 +22,7 @@
 
 #include "device_utils.hpp"
 #include "internal.hpp"
+#include "lds_direct.hpp"
 #include "quarter.hpp"
 #include "tile_decode.hpp"
 
@@ -122,40 +123,42 @@ __global__ __launch_bounds__(kRowsThreads) void gemm_rows_kernel(const RowsParam
         for (int i = 0; i < TT; ++i) acc[t][i] = float4v{0.f, 0.f, 0.f, 0.f};
 
     if (b0 < end) {
-        // rows past the matrix re-read its last one; what they produce is never stored
+        // weight rows past the matrix re-read its last one; what they produce is never stored
         const uint8_t* wrow[T];
 #pragma unroll
         for (int t = 0; t < T; ++t) wrow[t] = p.w + (size_t)min((tile0 + t) * 16 + r, p.n - 1) * p.nb * kBB;
         // request j of a block brings rows kTokensPerLoad * j ..; the 16-byte piece c of row t lands at
-        // piece c ^ (t & 15), so that the sixteen rows an operand read touches fall on different banks
+        // piece c ^ (t & 15), so that the sixteen rows an operand read touches fall on different banks.  (Rows past the
+        // batch lie past the buffer, without traffic: the columns they would feed are never stored.  The descriptor and the rows'
+        // offsets are made behind the first loads and only for waves with more than one super-block: 57 x 665 x 1024 takes
+        // 4.5 us, and 4.8 where they stand ahead of the first requests.)
         uint8_t* const slab = lds + wave * kWaveLds<DT, ROWS>;
-        const size_t x_row = (size_t)p.nb * kRowBytes;
+        const uint32_t x_row = p.nb * kRowBytes;
         const uint32_t sub = DT == 0 ? 0u : lane >> 5, piece = DT == 0 ? lane : lane & 31u;
-        auto request_rows = [&](uint32_t b) {
-#pragma unroll
-            for (int j = 0; j < kLoads; ++j) {
-                const uint32_t tok = (uint32_t)j * kTokensPerLoad + sub;
-                const uint8_t* src = p.x + (size_t)(m0 + min(tok, mt - 1)) * x_row + (size_t)b * kRowBytes +
-                                     16u * (piece ^ (tok & 15u));
-                __builtin_amdgcn_global_load_lds(
-                    (const __attribute__((address_space(1))) void*)src,
-                    (__attribute__((address_space(3))) void*)(slab + 1024 * j), 16, 0, 0);
-            }
-        };
         Quarter<TYPE> raw[T];
-        request_rows(b0);
+        // the first ones, ahead of every load that the compiler counts (and of every M0 that it writes), by hand
+        const uint8_t* const first_rows = p.x + (size_t)m0 * x_row + (size_t)b0 * kRowBytes;
+        const uint32_t slab_at = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)slab;
+#pragma unroll
+        for (int j = 0; j < kLoads; ++j) {
+            const uint32_t tok = (uint32_t)j * kTokensPerLoad + sub;
+            lds_load16_uniform(first_rows, min(tok, mt - 1) * x_row + 16u * (piece ^ (tok & 15u)), slab_at + 1024u * j);
+        }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int t = 0; t < T; ++t) {
             raw[t].load(wrow[t] + (size_t)b0 * kBB, g);
             __builtin_amdgcn_sched_barrier(0);
         }
-        auto block = [&](uint32_t b, auto more) {
+        auto block = [&](uint32_t b, auto more, auto&& request_rows) {
             constexpr bool kMore = decltype(more)::value;
             // This block's rows have landed once no more than the T tiles' weight requests behind them are
             // outstanding (loads retire in order).  The compiler counts its own waits with these requests in
             // sight but puts none of its own before the reads of what they write; the build counts the loads
-            // between the two in the generated code (ferrum_amd/isa_check.py).
+            // between the two in the generated code (ferrum_amd/isa_check.py).  (Requested by the builtin for global
+            // loads, which is a flat access to the compiler, they made it wait for everything outstanding before the first
+            // tile of every super-block.  us then / now: 16 x 28672 x 4096 27.8 / 25.3, 64 x 5120 x 17408 43.0 / 40.5,
+            // Q6_K 32 x 5120 x 17408 37.2 / 34.0, f32 8 x 17408 x 5120 47.2 / 44.3.)
             asm volatile("s_waitcnt vmcnt(%0)" ::"n"(T * Quarter<TYPE>::kLoads) : "memory");
             u32x4 frag[TT][kFrags];
 #pragma unroll
@@ -193,8 +196,25 @@ __global__ __launch_bounds__(kRowsThreads) void gemm_rows_kernel(const RowsParam
             }
         };
         uint32_t b = b0;
-        for (; b + p.k_waves < end; b += p.k_waves) block(b, std::true_type{});
-        block(b, std::false_type{});
+        if (b + p.k_waves < end) {
+            const __amdgpu_buffer_rsrc_t rows = __builtin_amdgcn_make_buffer_rsrc(
+                reinterpret_cast<void*>(uniform_address(p.x + (size_t)m0 * x_row)), 0, mt * x_row, 0x00027000);
+            uint32_t row_at[kLoads];
+#pragma unroll
+            for (int j = 0; j < kLoads; ++j) {
+                const uint32_t tok = (uint32_t)j * kTokensPerLoad + sub;
+                row_at[j] = tok < mt ? tok * x_row + 16u * (piece ^ (tok & 15u)) : kRowsBatchBytes;
+            }
+            auto request_rows = [&](uint32_t of) {
+#pragma unroll
+                for (int j = 0; j < kLoads; ++j) lds_load16_counted(rows, slab + 1024 * j, row_at[j], of * kRowBytes);
+            };
+            do {
+                block(b, std::true_type{}, request_rows);
+                b += p.k_waves;
+            } while (b + p.k_waves < end);
+        }
+        block(b, std::false_type{}, [](uint32_t) {});
     }
 
     // the waves' partial sums, in the place of the activations

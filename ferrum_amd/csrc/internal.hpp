@@ -316,7 +316,9 @@ struct GemvScratch {
 };
 GemvScratch gemv_scratch(const GemvArgs& a);
 
-// gemm_rows.hip: a few rows, f16 / bf16 on weights rounded to their type or f32 on exact f32 weights
+// gemm_rows.hip: a few rows, f16 / bf16 on weights rounded to their type or f32 on exact f32 weights.  A workgroup's rows
+// are a buffer of less than this (rows of more than sixty million elements go to the other kernels).
+constexpr uint32_t kRowsBatchBytes = 0xf0000000u;
 struct RowsPlan {
     uint32_t rows;            // rows a workgroup multiplies: 16 or 32
     uint32_t run_rows;        // rows of one launch; a larger batch is several, one after the other
@@ -330,6 +332,9 @@ struct RowsPlan {
     bool pairs;               // f32 rows as pairs of f16 operands: gemm_pairs.hip
     size_t operand_bytes;     // ... which come first in the scratch
 };
+inline bool rows_batch_fits(const RowsPlan& plan, uint32_t k, uint32_t x_dtype) {
+    return (uint64_t)plan.rows * k * dtype_bytes(x_dtype) <= kRowsBatchBytes;
+}
 RowsPlan gemm_rows_plan(uint32_t ggml_type, uint32_t n, uint32_t k, uint32_t m, uint32_t x_dtype, int cu_count);
 // whether that plan's kernel, and not the FMA GEMV once per row, takes m exact f32 rows
 bool f32_rows_pay(const RowsPlan& plan, uint32_t ggml_type, uint32_t n, uint32_t k, uint32_t m, int cu_count);

@@ -35,6 +35,20 @@ __device__ __forceinline__ void lds_load16_at(const void* base, uint32_t offset,
     asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(offset), "s"(sb), "s"(a) : "memory");
 }
 
+// The same where the compiler knows that address and base are the whole wave's.
+__device__ __forceinline__ void lds_load16_uniform(const void* base, uint32_t offset, uint32_t lds_addr) {
+    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(offset), "s"(base), "s"(lds_addr) : "memory");
+}
+
+// The same as a buffer load that the compiler issues and counts: 16 bytes a lane from `offset` + `base` in `rows` to `to` + 16 * lane.
+// (A global load into LDS by builtin is a flat access to the compiler: before it uses the result of any load it then waits
+// for everything outstanding.)
+__device__ __forceinline__ void lds_load16_counted(__amdgpu_buffer_rsrc_t rows, void* to, uint32_t offset, uint32_t base) {
+#ifdef __HIP_DEVICE_COMPILE__
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rows, (__attribute__((address_space(3))) void*)to, 16, offset, base, 0, 0);
+#endif
+}
+
 // s_waitcnt vmcnt(n), n a wave-uniform run-time value up to 20 (0 beyond)
 __device__ __forceinline__ void wait_vmcnt(uint32_t n) {
 #define FH_VM(N) case N: asm volatile("s_waitcnt vmcnt(" #N ")" ::: "memory"); break;

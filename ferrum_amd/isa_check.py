@@ -24,7 +24,7 @@ and but for ``HAND_ISSUED_SOURCES`` its LDS-direct loads too, and only says when
 vmcnt(n)``, n being the register loads the source issues behind them.
 The invariant is that the generated code has at least n of them there
 (``counted_violations``): with fewer, n outstanding loads could include one that the wait
-is for.  Of the hand-issued ones M0 and scratch are checked as above (``m0_violations``).
+is for.  Where such a kernel issues some LDS-direct loads itself, each of the compiler's has to find an M0 that the compiler wrote.  Of the hand-issued ones M0 and scratch are checked as above (``m0_violations``).
 
 The check reads the assembly hipcc writes with ``-S`` for this library's own sources
 (text, before it becomes a code object) and returns every violation it finds.  It is a
@@ -50,6 +50,7 @@ _VREG_RANGE = re.compile(r"\bv\[(\d+):(\d+)\]")
 _VREG_ONE = re.compile(r"\bv(\d+)\b")
 _REG_LOAD = re.compile(r"^global_load_dwordx[234]\s+(v\[\d+:\d+\]|v\d+)\s*,")
 _VMEM = re.compile(r"^(global_|buffer_|flat_|scratch_)(load|store|atomic)")
+_LDS_LOAD = re.compile(r"^(global_load_lds_|buffer_load_\w+ .*\blds$)")
 _STORE = re.compile(r"^(global_|buffer_|flat_)store")
 
 
@@ -145,7 +146,13 @@ def counted_violations(asm: str, source: str = "") -> list[str]:
         at_label = {text[:-1]: at for at, (_, text, _) in enumerate(body) if text.endswith(":")}
         waits = {at: int(m.group(1)) for at, (_, text, in_asm) in enumerate(body)
                  if in_asm and (m := re.match(r"s_waitcnt vmcnt\((\d+)\)", text))}
-        lds = [at for at, (_, text, _) in enumerate(body) if text.startswith("global_load_lds_")]
+        lds = [at for at, (_, text, _) in enumerate(body) if _LDS_LOAD.match(text)]
+        theirs = True    # M0 is as the compiler last wrote it
+        for number, text, in_asm in body:
+            if re.match(r"s_\w+ m0,", text):
+                theirs = not in_asm
+            elif _LDS_LOAD.match(text) and not in_asm and not theirs:
+                found.append(f"{where}{number}: {name}: the compiler's LDS-direct load finds M0 as an asm statement left it")
         if lds and not waits:
             found.append(f"{where}{body[lds[0]][0]}: {name}: LDS-direct loads without a hand-placed wait")
             continue
@@ -154,7 +161,7 @@ def counted_violations(asm: str, source: str = "") -> list[str]:
             behind, needs, end = 0, [], "the function's end"
             for here in range(at + 1, len(body)):
                 _, text, _ = body[here]
-                if text.startswith("global_load_lds_"):
+                if _LDS_LOAD.match(text):
                     if behind == 0:
                         end = "more of the run"
                         break
@@ -164,7 +171,7 @@ def counted_violations(asm: str, source: str = "") -> list[str]:
                 elif here in waits:
                     end = "a wait"
                     break
-                elif text.startswith("global_load_"):
+                elif text.startswith(("global_load_", "buffer_load_")):
                     behind += 1
                 target = text.split()[-1] if text.startswith(("s_cbranch", "s_branch")) else None
                 if target in at_label and at_label[target] < at:

@@ -160,6 +160,14 @@ def test_counted_loads_are_counted_along_a_branch_back_over_them(source):
     assert any("1 register loads follow" in v and "allows 2" in v for v in found), found
 
 
+def test_the_compilers_lds_loads_find_their_own_m0():
+    mixed = COUNTED.replace("_Z4rowsv:\n", "_Z4rowsv:\n\t;;#ASMSTART\n\ts_mov_b32 m0, s4\n\t;;#ASMEND\n"
+                            "\ts_mov_b32 m0, s5\n\tbuffer_load_dwordx4 v1, s[0:3], 0 offen lds\n")
+    assert isa_check.counted_violations(mixed) == []
+    found = isa_check.counted_violations(mixed.replace("\ts_mov_b32 m0, s5\n", ""), "x.hip")
+    assert found and "finds M0 as an asm statement left it" in found[0], found
+
+
 def test_hand_issued_counted_loads_need_a_wait_behind_them():
     end = LOOP[LOOP.index("\tglobal_load_dwordx4 v[8:11]"):LOOP.index("\ts_endpgm")]
     straight = LOOP.replace(end, "", 1)     # a run with nothing behind it but the function's end
