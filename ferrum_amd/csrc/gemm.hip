@@ -146,12 +146,12 @@ struct RawW<kIQ4XS> {
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
             const uint32_t l = iq4_lookup4(q[t]), u = iq4_lookup4(q[t] >> 4);
-            const uint32_t l01 = bytes01_as_halves(l), l23 = bytes23_as_halves(l);
-            const uint32_t u01 = bytes01_as_halves(u), u23 = bytes23_as_halves(u);
-            out_lo[2 * t] = fma_pair<DT>(lo_half(l01), hi_half(l01), scale, offset);
-            out_lo[2 * t + 1] = fma_pair<DT>(lo_half(l23), hi_half(l23), scale, offset);
-            out_hi[2 * t] = fma_pair<DT>(lo_half(u01), hi_half(u01), scale, offset);
-            out_hi[2 * t + 1] = fma_pair<DT>(lo_half(u23), hi_half(u23), scale, offset);
+            const uint32_t l02 = bytes02_as_halves(l), l13 = bytes13_as_halves(l);
+            const uint32_t u02 = bytes02_as_halves(u), u13 = bytes13_as_halves(u);
+            out_lo[2 * t] = fma_pair<DT>(lo_half(l02), lo_half(l13), scale, offset);
+            out_lo[2 * t + 1] = fma_pair<DT>(hi_half(l02), hi_half(l13), scale, offset);
+            out_hi[2 * t] = fma_pair<DT>(lo_half(u02), lo_half(u13), scale, offset);
+            out_hi[2 * t + 1] = fma_pair<DT>(hi_half(u02), hi_half(u13), scale, offset);
         }
     }
 };
@@ -177,10 +177,10 @@ struct RawW<kQ8_0> {
 #pragma unroll
         for (int t = 0; t < 8; ++t) {
             const uint32_t u = q[t] ^ 0x80808080u;
-            const uint32_t u01 = bytes01_as_halves(u), u23 = bytes23_as_halves(u);
+            const uint32_t u02 = bytes02_as_halves(u), u13 = bytes13_as_halves(u);
             uint32_t* out = t < 4 ? out_lo : out_hi;
-            out[2 * (t & 3)] = fma_pair<DT>(lo_half(u01), hi_half(u01), scale, offset);
-            out[2 * (t & 3) + 1] = fma_pair<DT>(lo_half(u23), hi_half(u23), scale, offset);
+            out[2 * (t & 3)] = fma_pair<DT>(lo_half(u02), lo_half(u13), scale, offset);
+            out[2 * (t & 3) + 1] = fma_pair<DT>(hi_half(u02), hi_half(u13), scale, offset);
         }
     }
 };
@@ -483,12 +483,12 @@ struct BlockW<kIQ4XS> {
     __device__ __forceinline__ void decode(int c, uint32_t, int t, const Scales& s, uint32_t (&out)[4]) const {
         const uint32_t v = pick4(q[c], t);
         const uint32_t l = iq4_lookup4(v), u = iq4_lookup4(v >> 4);
-        const uint32_t l01 = bytes01_as_halves(l), l23 = bytes23_as_halves(l);
-        const uint32_t u01 = bytes01_as_halves(u), u23 = bytes23_as_halves(u);
-        out[0] = fma_pair<DT>(lo_half(l01), hi_half(l01), s.a_lo, s.b_lo);
-        out[1] = fma_pair<DT>(lo_half(l23), hi_half(l23), s.a_lo, s.b_lo);
-        out[2] = fma_pair<DT>(lo_half(u01), hi_half(u01), s.a_hi, s.b_hi);
-        out[3] = fma_pair<DT>(lo_half(u23), hi_half(u23), s.a_hi, s.b_hi);
+        const uint32_t l02 = bytes02_as_halves(l), l13 = bytes13_as_halves(l);
+        const uint32_t u02 = bytes02_as_halves(u), u13 = bytes13_as_halves(u);
+        out[0] = fma_pair<DT>(lo_half(l02), lo_half(l13), s.a_lo, s.b_lo);
+        out[1] = fma_pair<DT>(hi_half(l02), hi_half(l13), s.a_lo, s.b_lo);
+        out[2] = fma_pair<DT>(lo_half(u02), lo_half(u13), s.a_hi, s.b_hi);
+        out[3] = fma_pair<DT>(hi_half(u02), hi_half(u13), s.a_hi, s.b_hi);
     }
 };
 
@@ -518,9 +518,9 @@ struct BlockW<kQ8_0> {
     __device__ __forceinline__ void decode(int c, uint32_t, int t, const Scales& s, uint32_t (&out)[4]) const {
         const uint32_t v[8] = {q[c][0].x, q[c][0].y, q[c][0].z, q[c][0].w, q[c][1].x, q[c][1].y, q[c][1].z, q[c][1].w};
         const uint32_t u = v[t] ^ 0x80808080u;
-        const uint32_t u01 = bytes01_as_halves(u), u23 = bytes23_as_halves(u);
-        out[0] = fma_pair<DT>(lo_half(u01), hi_half(u01), s.scale, s.offset);
-        out[1] = fma_pair<DT>(lo_half(u23), hi_half(u23), s.scale, s.offset);
+        const uint32_t u02 = bytes02_as_halves(u), u13 = bytes13_as_halves(u);
+        out[0] = fma_pair<DT>(lo_half(u02), lo_half(u13), s.scale, s.offset);
+        out[1] = fma_pair<DT>(hi_half(u02), hi_half(u13), s.scale, s.offset);
         out[2] = 0;
         out[3] = 0;
     }

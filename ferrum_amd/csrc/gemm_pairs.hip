@@ -319,7 +319,7 @@ struct Half<kIQ4XS> {
             const u32x4& from = q[slice];
             const uint32_t w = ((u & 1) ? (j ? from.w : from.z) : (j ? from.y : from.x)) >> (u >= 2 ? 4 : 0);
             const uint32_t bytes = iq4_lookup4(w);
-            const uint32_t q02 = __builtin_amdgcn_perm(0u, bytes, 0x0c020c00u), q13 = __builtin_amdgcn_perm(0u, bytes, 0x0c030c01u);
+            const uint32_t q02 = bytes02_as_halves(bytes), q13 = bytes13_as_halves(bytes);
             scaled_parts(as_half2(q02) + centre, a[slice], o[2 * j], r[2 * j]);
             scaled_parts(as_half2(q13) + centre, a[slice], o[2 * j + 1], r[2 * j + 1]);
         }

@@ -177,18 +177,18 @@ struct Frag<kIQ4XS> {
             const int sub = t >> 2, u = 8 * sub + (t & 3);      // float4 of the low nibbles; the high ones sit 4 on
             const float4 xl = xc[u * 4], xh = xc[(u + 4) * 4];
             const uint32_t lo = iq4_lookup4(q[t]), hi = iq4_lookup4(q[t] >> 4);
-            const uint32_t l01 = bytes01_as_halves(lo), l23 = bytes23_as_halves(lo);
-            const uint32_t h01 = bytes01_as_halves(hi), h23 = bytes23_as_halves(hi);
+            const uint32_t l02 = bytes02_as_halves(lo), l13 = bytes13_as_halves(lo);
+            const uint32_t h02 = bytes02_as_halves(hi), h13 = bytes13_as_halves(hi);
             float& a = acc[sub][0];
             float& b = acc[sub][1];
-            a = fmaf(lo_half(l01), xl.x, a);
-            b = fmaf(hi_half(l01), xl.y, b);
-            a = fmaf(lo_half(l23), xl.z, a);
-            b = fmaf(hi_half(l23), xl.w, b);
-            a = fmaf(lo_half(h01), xh.x, a);
-            b = fmaf(hi_half(h01), xh.y, b);
-            a = fmaf(lo_half(h23), xh.z, a);
-            b = fmaf(hi_half(h23), xh.w, b);
+            a = fmaf(lo_half(l02), xl.x, a);
+            b = fmaf(lo_half(l13), xl.y, b);
+            a = fmaf(hi_half(l02), xl.z, a);
+            b = fmaf(hi_half(l13), xl.w, b);
+            a = fmaf(lo_half(h02), xh.x, a);
+            b = fmaf(lo_half(h13), xh.y, b);
+            a = fmaf(hi_half(h02), xh.z, a);
+            b = fmaf(hi_half(h13), xh.w, b);
         }
         // bytes were (value + 128) * 2^-24
         const float r0 = fmaf(acc[0][0] + acc[0][1], 16777216.f, -128.f * (s.x + s.y));
@@ -211,11 +211,11 @@ struct Frag<kQ8_0> {
             for (int j = 0; j < 8; ++j) {
                 const float4 x = xc[(8 * blk + j) * 4];
                 const uint32_t u = p.biased(blk, j);
-                const uint32_t u01 = bytes01_as_halves(u), u23 = bytes23_as_halves(u);
-                acc[blk][0] = fmaf(lo_half(u01), x.x, acc[blk][0]);
-                acc[blk][1] = fmaf(hi_half(u01), x.y, acc[blk][1]);
-                acc[blk][0] = fmaf(lo_half(u23), x.z, acc[blk][0]);
-                acc[blk][1] = fmaf(hi_half(u23), x.w, acc[blk][1]);
+                const uint32_t u02 = bytes02_as_halves(u), u13 = bytes13_as_halves(u);
+                acc[blk][0] = fmaf(lo_half(u02), x.x, acc[blk][0]);
+                acc[blk][1] = fmaf(lo_half(u13), x.y, acc[blk][1]);
+                acc[blk][0] = fmaf(hi_half(u02), x.z, acc[blk][0]);
+                acc[blk][1] = fmaf(hi_half(u13), x.w, acc[blk][1]);
             }
         }
         const float r0 = fmaf(acc[0][0] + acc[0][1], 16777216.f, -128.f * (s.x + s.y));

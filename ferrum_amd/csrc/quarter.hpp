@@ -138,13 +138,13 @@ struct Quarter<kIQ4XS> {
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
                 const uint32_t l = iq4_lookup4(v[4 * sub + t]), h = iq4_lookup4(v[4 * sub + t] >> 4);
-                const uint32_t l01 = bytes01_as_halves(l), l23 = bytes23_as_halves(l);
-                const uint32_t h01 = bytes01_as_halves(h), h23 = bytes23_as_halves(h);
+                const uint32_t l02 = bytes02_as_halves(l), l13 = bytes13_as_halves(l);
+                const uint32_t h02 = bytes02_as_halves(h), h13 = bytes13_as_halves(h);
                 // weights 0..15 of the sub-block are its low nibbles, 16..31 its high ones
-                out.pair(16 * sub + 2 * t, lo_half(l01), hi_half(l01), scale, offset);
-                out.pair(16 * sub + 2 * t + 1, lo_half(l23), hi_half(l23), scale, offset);
-                out.pair(16 * sub + 8 + 2 * t, lo_half(h01), hi_half(h01), scale, offset);
-                out.pair(16 * sub + 8 + 2 * t + 1, lo_half(h23), hi_half(h23), scale, offset);
+                out.pair(16 * sub + 2 * t, lo_half(l02), lo_half(l13), scale, offset);
+                out.pair(16 * sub + 2 * t + 1, hi_half(l02), hi_half(l13), scale, offset);
+                out.pair(16 * sub + 8 + 2 * t, lo_half(h02), lo_half(h13), scale, offset);
+                out.pair(16 * sub + 8 + 2 * t + 1, hi_half(h02), hi_half(h13), scale, offset);
             }
         }
     }
@@ -168,13 +168,13 @@ struct Quarter<kQ8_0> {
 #pragma unroll
             for (int s = 0; s < 4; ++s) {
                 const uint32_t u0 = p.biased(blk, 2 * s), u1 = p.biased(blk, 2 * s + 1);
-                const uint32_t a01 = bytes01_as_halves(u0), a23 = bytes23_as_halves(u0);
-                const uint32_t b01 = bytes01_as_halves(u1), b23 = bytes23_as_halves(u1);
+                const uint32_t a02 = bytes02_as_halves(u0), a13 = bytes13_as_halves(u0);
+                const uint32_t b02 = bytes02_as_halves(u1), b13 = bytes13_as_halves(u1);
                 const int word = 16 * blk + 4 * s;
-                out.pair(word, lo_half(a01), hi_half(a01), scale, offset);
-                out.pair(word + 1, lo_half(a23), hi_half(a23), scale, offset);
-                out.pair(word + 2, lo_half(b01), hi_half(b01), scale, offset);
-                out.pair(word + 3, lo_half(b23), hi_half(b23), scale, offset);
+                out.pair(word, lo_half(a02), lo_half(a13), scale, offset);
+                out.pair(word + 1, hi_half(a02), hi_half(a13), scale, offset);
+                out.pair(word + 2, lo_half(b02), lo_half(b13), scale, offset);
+                out.pair(word + 3, hi_half(b02), hi_half(b13), scale, offset);
             }
         }
     }
