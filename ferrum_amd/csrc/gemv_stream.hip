@@ -197,6 +197,19 @@ __device__ __forceinline__ uint2 lds_u2_unaligned(const uint8_t* p) {
     return v;
 }
 
+// 16 bytes at a dword, and 16 that begin two bytes behind one
+__device__ __forceinline__ uint4 lds_u4_dword(const uint8_t* p) {
+    typedef uint32_t dwords __attribute__((ext_vector_type(4), aligned(4)));
+    const dwords v = *reinterpret_cast<const dwords*>(p);
+    return make_uint4(v.x, v.y, v.z, v.w);
+}
+__device__ __forceinline__ uint4 lds_u4_behind_2(const uint8_t* p) {
+    const uint4 v = lds_u4_dword(p - 2);
+    const uint32_t end = *reinterpret_cast<const uint32_t*>(p + 14);
+    return make_uint4(__builtin_amdgcn_alignbyte(v.y, v.x, 2), __builtin_amdgcn_alignbyte(v.z, v.y, 2),
+                      __builtin_amdgcn_alignbyte(v.w, v.z, 2), __builtin_amdgcn_alignbyte(end, v.w, 2));
+}
+
 // A lane's share of one super-block, chunk g of its row against the operands of stage_block, added to acc.
 __device__ __forceinline__ float multiply_q4k(const u32x4 (&xa)[4], float4 aux, uint4 hdr, uint4 qa, uint4 qb, uint32_t g, float acc) {
     const uint32_t raw[8] = {qa.x, qa.y, qa.z, qa.w, qb.x, qb.y, qb.z, qb.w};
@@ -418,11 +431,26 @@ __device__ __forceinline__ void gemv_stream_body(const StreamParams& p) {
                 asm volatile("" ::: "memory");   // the slot reads are issued before the tile reads
                 const uint8_t* const blk = wrow + b * kBlock;
                 const uint32_t h = g >> 1, e = g & 1u;
-                const uint4 qa = lds_u4_unaligned(blk + 64u * h + 16u * e);
-                const uint4 qb = lds_u4_unaligned(blk + 64u * h + 32u + 16u * e);
-                const uint4 qh = lds_u4_unaligned(blk + 128u + 32u * h + 16u * e);
-                const uint2 sc8 = lds_u2_unaligned(blk + 192u + 8u * h);
+                uint4 qa, qb, qh;
+                uint2 sc8;
                 uint16_t dbits;
+                // A read of 16 bytes that begins between two dwords takes LDS longer than the two aligned ones that cover it
+                // (us: 151936 x 5120 141 / 133, 34816 x 5120 39.4 / 36.5, 5120 x 17408 23.7 / 22.8).  With rows of 16 bits and two
+                // blocks a wave their registers would leave two workgroups a compute unit instead of three (8192 x 28672 54 / 59).
+                constexpr bool kByDwords = DT == FH_F32 || MAXB != 2;
+                if (kByDwords && (b & 1u)) {   // two bytes behind a dword
+                    qa = lds_u4_behind_2(blk + 64u * h + 16u * e);
+                    qb = lds_u4_behind_2(blk + 64u * h + 32u + 16u * e);
+                    qh = lds_u4_behind_2(blk + 128u + 32u * h + 16u * e);
+                    const uint4 last = lds_u4_dword(blk + 190u + 8u * h);   // (of the second half its third dword ends the block)
+                    sc8 = make_uint2(__builtin_amdgcn_alignbyte(last.y, last.x, 2), __builtin_amdgcn_alignbyte(last.z, last.y, 2));
+                } else {
+                    auto read = [](const uint8_t* p) { return kByDwords ? lds_u4_dword(p) : lds_u4_unaligned(p); };
+                    qa = read(blk + 64u * h + 16u * e);
+                    qb = read(blk + 64u * h + 32u + 16u * e);
+                    qh = read(blk + 128u + 32u * h + 16u * e);
+                    sc8 = lds_u2_unaligned(blk + 192u + 8u * h);
+                }
                 __builtin_memcpy(&dbits, blk + 208u, 2);
                 if (i + 1 < MAXB && b + kSWaves < nb) {
                     // the nine slot reads are the oldest; at least five instructions read the tile
@@ -716,18 +744,19 @@ StreamPlan gemv_stream_plan(uint32_t ggml_type, uint32_t n, uint32_t k, uint32_t
     plan.waves = 8u;
     plan.lds_bytes = h * plan.row_stride + plan.waves * slot + plan.waves * 64u;
     // Matrices of a megabyte or two finish sooner on the FMA kernel's smaller workgroups.  A Q6_K tile is 46% longer and
-    // only two share a compute unit: what lies in between is even or the FMA kernel's (17408 x 5120 22.6 us there against
-    // 22.8, 28672 x 4096 26.9 / 28.3, 12288 x 4096 13.3 / 14.9), but rows that must be cut into segments in any case gain
-    // (5120 x 17408: 27.7 / 24.7), and so do matrices of 600,000 super-blocks in uncut sixteen-row tiles (us, weights
-    // out of every cache, FMA against this kernel: 32000 x 5120 36.8 / 35.1, 34816 x 5120 39.4 / 37.4, 65536 x 5120
-    // 67.3 / 61.6, 151936 x 2048 61.4 / 59.3, 128256 x 4096 98.2 / 96.7, 152064 x 3584 111.5 / 100.7, 262144 x 2560
-    // 133.6 / 118.0, 151936 x 5120 142.8 / 132.5).
+    // only two share a compute unit: rows that must be cut into segments in any case gain (5120 x 17408: 27.7 / 22.8), and so do large
+    // matrices (us, weights out of every cache, FMA against this kernel: 34816 x 5120 39.4 / 36.5, 128256 x 4096 104 / 95, 152064 x 3584
+    // 111.5 / 100, 151936 x 5120 142.8 / 133).
     // Rows of 16 bits gain 1% there and are 0.9e-7 from 64 bits on the FMA kernel against 0.95e-7 here (f32 rows 1.9e-7 against
     // 0.9e-7), and two or three f32 rows share their weights through the caches on the FMA kernel (2 x 34816 x 5120 58.3 us there
     // against 64.6, 2 x 100000 x 2048 67.6 / 74.5): they come from a million super-blocks on, where the FMA kernel
     // cannot cut a row evenly over its eight block slots.
-    const bool big_head = q6 && segments == 1u && h == 16u &&
-                          (f32_rows && m == 1 ? (uint64_t)n * nb >= 600000u : (nb & 7u) != 0 && (uint64_t)n * nb >= 1000000u);
+    // One f32 row of eight super-blocks and more gains from a quarter of a million of them on, whole or cut (22000 x 3072 17.4 / 15.1,
+    // 17408 x 5120 22.6 / 21.3, 60000 x 2048 27.8 / 26.2, 36000 x 3584 31.7 / 28.2, 12000 x 10240 36.3 / 29.3; but 9000 x 6144 15.4 / 16.1,
+    // 5120 x 8192 12.3 / 13.6, 7000 x 4096 8.4 / 8.7, and of shorter rows 40000 x 1536 17.3 / 17.2, 100000 x 1024 21.2 / 31.2).
+    const uint64_t blocks = (uint64_t)n * nb;
+    const bool big_head = q6 && (f32_rows && m == 1 ? (nb >= 8u && blocks >= 250000u) || (segments == 1u && h == 16u && blocks >= 600000u)
+                                                    : segments == 1u && h == 16u && (nb & 7u) != 0 && blocks >= 1000000u);
     // One row of a Q4_K matrix of short rows is the FMA kernel's: a tile of sixteen is a few kilobytes of LDS for eight waves of
     // which some own no super-block, and staging stands beside little arithmetic (us, cold, FMA against this kernel:
     // 29952 x 256 3.7 / 8.3, 8448 x 512 3.5 / 4.2, 4224 x 1024 3.5 / 3.8, 99968 x 1024 14.1 / 23.6; rows of 5 - 8 super-blocks

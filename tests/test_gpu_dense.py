@@ -392,6 +392,27 @@ def test_large_q4_k_matrices_take_the_ring_by_themselves(api, d):
     assert rel_l2(got, tiles) <= 6e-7 and np.array_equal(bits(got[0, :1790]), bits(got[0, -1790:]))
 
 
+@pytest.mark.parametrize("n,k,streamed", [(22000, 3072, True), (31250, 2048, True), (6300, 10240, True), (31200, 2048, False),
+                                          (9000, 6144, False), (50000, 1536, False)])
+def test_large_q6_k_matrices_of_long_rows_are_streamed(api, d, n, k, streamed):
+    # from 250,000 super-blocks in rows of eight on, whole rows and cut ones, an f32 row alone takes the streamed kernel
+    base = synth.matrix(Q6_K, 50, k, seed=k).reshape(50, -1)
+    w = qm(api, d, Q6_K, n, k, np.resize(base, (n, base.shape[1])).reshape(-1))
+    x = synth.activations(1, k, seed=k + 1).reshape(1, k)
+    xt = api.Tensor.from_f32(d, (1, k), api.DType.F32, x)
+    got = d.project_quantized(xt, w).tensor.to_f32()
+    other = {}
+    for mode in (0, 2):
+        d.set_tuning("gemv_stream", mode)
+        try:
+            other[mode] = d.project_quantized(xt, w).tensor.to_f32()
+        finally:
+            d.set_tuning("gemv_stream", 1)
+    assert np.array_equal(bits(got), bits(other[2 if streamed else 0])) and not np.array_equal(bits(other[0]), bits(other[2]))
+    assert_matmul_parity(got[:, :50], oracle.project(Q6_K, base.reshape(-1), 50, k, x, accumulate="f64"), f"{n} x {k}")
+    assert np.array_equal(bits(got), bits(got[:, np.arange(n) % 50]))
+
+
 @pytest.mark.parametrize("n,k,fma", [(16400, 256, True), (4200, 1024, True), (3300, 1280, False), (20000, 1280, True), (12400, 2048, False),
                                      (12512, 2048, True), (11200, 2304, False)])
 def test_short_q4_k_rows_take_the_fma_kernel(api, d, n, k, fma):
