@@ -302,6 +302,19 @@ struct Q8Pair {
     }
 };
 
+// 16 bytes of LDS at a dword, and 16 that begin two bytes behind one
+__device__ __forceinline__ uint4 lds_u4_dword(const uint8_t* p) {
+    typedef uint32_t dwords __attribute__((ext_vector_type(4), aligned(4)));
+    const dwords v = *reinterpret_cast<const dwords*>(p);
+    return make_uint4(v.x, v.y, v.z, v.w);
+}
+__device__ __forceinline__ uint4 lds_u4_behind_2(const uint8_t* p) {
+    const uint4 v = lds_u4_dword(p - 2);
+    const uint32_t end = *reinterpret_cast<const uint32_t*>(p + 14);
+    return make_uint4(__builtin_amdgcn_alignbyte(v.y, v.x, 2), __builtin_amdgcn_alignbyte(v.z, v.y, 2),
+                      __builtin_amdgcn_alignbyte(v.w, v.z, 2), __builtin_amdgcn_alignbyte(end, v.w, 2));
+}
+
 // ---- wave reductions -----------------------------------------------------------
 
 template <int CTRL>

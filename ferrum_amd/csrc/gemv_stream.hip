@@ -197,19 +197,6 @@ __device__ __forceinline__ uint2 lds_u2_unaligned(const uint8_t* p) {
     return v;
 }
 
-// 16 bytes at a dword, and 16 that begin two bytes behind one
-__device__ __forceinline__ uint4 lds_u4_dword(const uint8_t* p) {
-    typedef uint32_t dwords __attribute__((ext_vector_type(4), aligned(4)));
-    const dwords v = *reinterpret_cast<const dwords*>(p);
-    return make_uint4(v.x, v.y, v.z, v.w);
-}
-__device__ __forceinline__ uint4 lds_u4_behind_2(const uint8_t* p) {
-    const uint4 v = lds_u4_dword(p - 2);
-    const uint32_t end = *reinterpret_cast<const uint32_t*>(p + 14);
-    return make_uint4(__builtin_amdgcn_alignbyte(v.y, v.x, 2), __builtin_amdgcn_alignbyte(v.z, v.y, 2),
-                      __builtin_amdgcn_alignbyte(v.w, v.z, 2), __builtin_amdgcn_alignbyte(end, v.w, 2));
-}
-
 // A lane's share of one super-block, chunk g of its row against the operands of stage_block, added to acc.
 __device__ __forceinline__ float multiply_q4k(const u32x4 (&xa)[4], float4 aux, uint4 hdr, uint4 qa, uint4 qb, uint32_t g, float acc) {
     const uint32_t raw[8] = {qa.x, qa.y, qa.z, qa.w, qb.x, qb.y, qb.z, qb.w};

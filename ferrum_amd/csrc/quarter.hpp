@@ -195,6 +195,16 @@ struct Quarter<kQ6K> {
         sc = load_u4_unaligned(block + 192);
         d = load_u16_unaligned(block + 208);
     }
+    // out of LDS, `behind`: the block begins two bytes behind a dword, else at one
+    __device__ __forceinline__ void load_by_dwords(const uint8_t* block, uint32_t g, bool behind) {
+        const uint32_t h = g >> 1, j0 = (g & 1u) * 16;
+        auto read = [behind](const uint8_t* p) { return behind ? lds_u4_behind_2(p) : lds_u4_dword(p); };
+        la = read(block + 64 * h + j0);
+        lb = read(block + 64 * h + 32 + j0);
+        ph = read(block + 128 + 32 * h + j0);
+        sc = read(block + 192);
+        d = load_u16_unaligned(block + 208);
+    }
     // operand s: slice s / 2 (32 weights each), positions j0 + 8 (s & 1) ..
     static __device__ __forceinline__ uint32_t klocal(uint32_t g, int s) {
         return 128 * (g >> 1) + 32 * (s >> 1) + 16 * (g & 1u) + 8 * (s & 1);
