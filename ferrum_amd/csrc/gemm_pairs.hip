@@ -503,41 +503,23 @@ __global__ __launch_bounds__(kThreads) void gemm_pairs_kernel(const PairsParams 
 #pragma unroll
             for (int c = 0; c < kChains; ++c) hi[c][v] = 0.f;
         }
-        // A step's operands are read and its weights decoded while the step before multiplies.  Left to itself the compiler read
-        // most operands right ahead of their product, a round trip to LDS for every two (us: Q4_K 64 x 17408 x 5120 72.2 / 69.2, 24 x 28672 x 4096 38.0 - 39.7 / 37.3,
-        // Q5_K 46.0 / 44.9, IQ4_XS 52.7 / 51.5).  Q6_K, four products a step on two reads, hides them anyhow and has no registers
-        // for a second set: 61.1 as it is, 62.2 a step ahead.
-        constexpr bool kAhead = TYPE != kQ6K;
-        struct Step {
-            uint4 xh, xl, first, rest;
-        };
-        auto make = [&](Step& of, auto at) {
-            constexpr int s = decltype(at)::value;
-            of.xh = *reinterpret_cast<const uint4*>(slot + 1024 * s + 16 * lane);
-            of.xl = *reinterpret_cast<const uint4*>(slot + kLoAt + 1024 * s + 16 * lane);
-            here.template step<s>(of.first, of.rest);
-        };
-        auto steps = [&](auto self, auto at, Step& now, Step& next) {
+        auto steps = [&](auto self, auto at) {
             constexpr int s = decltype(at)::value;
             if constexpr (s < 16) {
-                if constexpr (!kAhead) make(now, at);
-                else if constexpr (s < 15) make(next, std::integral_constant<int, s + 1>{});
-                hi[s * kChains / 16] = mfma_f16(now.xh, now.first, hi[s * kChains / 16]);
-                lo = mfma_f16(now.xl, now.first, lo);
+                uint4 first, rest;
+                here.template step<s>(first, rest);
+                const uint4 xh = *reinterpret_cast<const uint4*>(slot + 1024 * s + 16 * lane);
+                const uint4 xl = *reinterpret_cast<const uint4*>(slot + kLoAt + 1024 * s + 16 * lane);
+                hi[s * kChains / 16] = mfma_f16(xh, first, hi[s * kChains / 16]);
+                lo = mfma_f16(xl, first, lo);
                 if constexpr (Raw::kParts == 2) {
-                    lo = mfma_f16(now.xh, now.rest, lo);
-                    lo = mfma_f16(now.xl, now.rest, lo);
+                    lo = mfma_f16(xh, rest, lo);
+                    lo = mfma_f16(xl, rest, lo);
                 }
-                if constexpr (kAhead) {
-                    asm volatile("" : "+v"(lo));   // (else the compiler puts all of these products last, their operands in scratch)
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-                self(self, std::integral_constant<int, s + 1>{}, next, now);
+                self(self, std::integral_constant<int, s + 1>{});
             }
         };
-        Step even, odd_step;
-        if constexpr (kAhead) make(even, std::integral_constant<int, 0>{});
-        steps(steps, std::integral_constant<int, 0>{}, even, odd_step);
+        steps(steps, std::integral_constant<int, 0>{});
         if constexpr (Raw::kOffset) {
 #pragma unroll
             for (int s = 0; s < 4; ++s) {
