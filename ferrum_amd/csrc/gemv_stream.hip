@@ -741,8 +741,10 @@ StreamPlan gemv_stream_plan(uint32_t ggml_type, uint32_t n, uint32_t k, uint32_t
     // One f32 row of eight super-blocks and more gains from a quarter of a million of them on, whole or cut (22000 x 3072 17.4 / 15.1,
     // 17408 x 5120 22.6 / 21.3, 60000 x 2048 27.8 / 26.2, 36000 x 3584 31.7 / 28.2, 12000 x 10240 36.3 / 29.3; but 9000 x 6144 15.4 / 16.1,
     // 5120 x 8192 12.3 / 13.6, 7000 x 4096 8.4 / 8.7, and of shorter rows 40000 x 1536 17.3 / 17.2, 100000 x 1024 21.2 / 31.2).
+    // Cut rows only while their partial sums fit any scratch, the fixed one of calls that must not allocate among them: the FMA kernel
+    // would need none.
     const uint64_t blocks = (uint64_t)n * nb;
-    const bool big_head = q6 && (f32_rows && m == 1 ? (nb >= 8u && blocks >= 250000u) || (segments == 1u && h == 16u && blocks >= 600000u)
+    const bool big_head = q6 && (f32_rows && m == 1 ? (nb >= 8u && blocks >= 250000u && (segments == 1u || (uint64_t)segments * n <= 100000u)) || (segments == 1u && h == 16u && blocks >= 600000u)
                                                     : segments == 1u && h == 16u && (nb & 7u) != 0 && blocks >= 1000000u);
     // One row of a Q4_K matrix of short rows is the FMA kernel's: a tile of sixteen is a few kilobytes of LDS for eight waves of
     // which some own no super-block, and staging stands beside little arithmetic (us, cold, FMA against this kernel:
