@@ -24,7 +24,6 @@ double unit_us(uint32_t ggml_type, uint32_t x_dtype, uint32_t rows) {
 
 constexpr double kStartUs = 4.0;      // launch, first loads, exchange of the waves' sums
 constexpr double kExchangeUs = 4.0;   // partial sums of K segments through device memory
-constexpr double kSecondSetUs = 1.0;  // of a super-block, where two sets of tiles bring its rows in
 
 constexpr uint32_t kMostWorkgroups = 1u << 22;   // of a launch, and half of what a grid of 512 threads each may have
 
@@ -34,37 +33,30 @@ RowsPlan gemm_rows_plan(uint32_t ggml_type, uint32_t n, uint32_t k, uint32_t m, 
     RowsPlan plan{};
     const uint32_t nb = k / 256, tiles = (n + 15) / 16, cus = cu_count > 0 ? (uint32_t)cu_count : 256u;
     plan.rows = x_dtype != FH_F32 && m > 16 ? 32 : 16;
-    const uint32_t most_waves = nb >= 8 ? 8 : nb >= 4 ? 4 : nb >= 2 ? 2 : 1;
+    plan.k_waves = nb >= 8 ? 8 : nb >= 4 ? 4 : nb >= 2 ? 2 : 1;
+    const uint32_t tile_waves = 8 / plan.k_waves;
     const double unit = unit_us(ggml_type, x_dtype, 16);
-    // Tiles per wave, waves along K and K segments, from the matrix alone: the sums of a row then do not depend on how
+    // Tiles per wave and K segments, from the matrix alone: the sums of a row then do not depend on how
     // many rows come with it.  Rounds of one workgroup per compute unit, each as long as the
     // super-blocks of its longest wave.  8 x 17408 x 5120: 17.2 us with five tiles in one round of 218
     // workgroups, 21 - 26 with fewer tiles in more rounds, 25 - 31 with K cut in two; 8 x 5120 x 17408:
     // 20.8 with four tiles and three segments, 22 - 41 without segments.
-    // Up to 16 rows of 16 bits: four waves along K, each with five of twenty super-blocks, and two sets of five tiles are one
-    // round of 34816 x 5120 (8 / 16 rows 29.4 / 32.3 us; eight waves, with two or three super-blocks each, are two rounds,
-    // 34.8 / 36.0, the rows-resident kernel 35.3 / 35.7; two waves 36.5 / 38.9).  The two sets bring the rows in twice.
-    const bool halves = plan.rows == 16 && x_dtype != FH_F32 && most_waves == 8 && nb % 8 != 0;
     double best = 1e300;
-    for (uint32_t waves = most_waves; waves >= (halves ? 4u : most_waves); waves /= 2) {
-        const uint32_t tile_waves = 8 / waves;
-        for (uint32_t segments = 1; segments <= (waves < most_waves ? 1u : 8u); ++segments) {
-            const uint32_t seg_blocks = (nb + segments - 1) / segments;
-            if ((nb + seg_blocks - 1) / seg_blocks != segments || (segments > 1 && seg_blocks < waves)) continue;
-            const uint32_t per_wave = (seg_blocks + waves - 1) / waves;
-            for (uint32_t t = 1; t <= 5; ++t) {
-                const uint32_t tile_groups = (tiles + t * tile_waves - 1) / (t * tile_waves);
-                const uint64_t wgs = (uint64_t)tile_groups * segments;
-                const double us = (double)((wgs + cus - 1) / cus) * (kStartUs + per_wave * (t * unit + (waves < most_waves ? kSecondSetUs : 0.0))) +
-                                  (segments > 1 ? kExchangeUs : 0.0);
-                if (us < best) {
-                    best = us;
-                    plan.k_waves = waves;
-                    plan.tiles = t;
-                    plan.segments = segments;
-                    plan.seg_blocks = seg_blocks;
-                    plan.tile_groups = tile_groups;
-                }
+    for (uint32_t segments = 1; segments <= 8; ++segments) {
+        const uint32_t seg_blocks = (nb + segments - 1) / segments;
+        if ((nb + seg_blocks - 1) / seg_blocks != segments || (segments > 1 && seg_blocks < plan.k_waves)) continue;
+        const uint32_t per_wave = (seg_blocks + plan.k_waves - 1) / plan.k_waves;
+        for (uint32_t t = 1; t <= 5; ++t) {
+            const uint32_t tile_groups = (tiles + t * tile_waves - 1) / (t * tile_waves);
+            const uint64_t wgs = (uint64_t)tile_groups * segments;
+            const double us = (double)((wgs + cus - 1) / cus) * (kStartUs + per_wave * t * unit) +
+                              (segments > 1 ? kExchangeUs : 0.0);
+            if (us < best) {
+                best = us;
+                plan.tiles = t;
+                plan.segments = segments;
+                plan.seg_blocks = seg_blocks;
+                plan.tile_groups = tile_groups;
             }
         }
     }

@@ -1198,23 +1198,26 @@ def test_few_rows_with_four_tiles_and_three_segments(api, d, ggml):
         assert np.array_equal(bits(got), bits(np.tile(got[:, :80], n // 80)))
 
 
-# Two sets of tiles of four waves each, where eight waves would share a row's super-blocks unevenly: 9 and 20 of them, three to
-# five tiles a set, a ragged last tile, a second set without tiles, every batch size at which the rows' buffer ends differently.
+# A row's sums do not depend on how many rows come with it, on either side of the line between row groups of 16 and 32 either: rows
+# of a number of super-blocks that eight waves share unevenly (9, 20, 12) and evenly, several tiles a wave, a ragged last tile.
 @pytest.mark.parametrize("ggml", [12, 13, 14, 23, 8], ids=["q4_k", "q5_k", "q6_k", "iq4_xs", "q8_0"])
-@pytest.mark.parametrize("n,k", [(28001, 2304), (34816, 5120), (24131, 3072)])
-def test_few_rows_with_two_sets_of_tiles(api, d, ggml, n, k):
+@pytest.mark.parametrize("n,k", [(28001, 2304), (34816, 5120), (24131, 3072), (16750, 2048)])
+def test_few_rows_sums_do_not_depend_on_the_rows_beside_them(api, d, ggml, n, k):
     block = synth.matrix(ggml, 61, k, seed=301).reshape(61, -1)      # over and over: neighbouring tiles are different
     w = qm(api, d, ggml, n, k, np.resize(block, (n, block.shape[1])).reshape(-1))
-    for m, dtype in ((2, "F16"), (9, "BF16"), (16, "F16")):
-        code = oracle.F16 if dtype == "F16" else oracle.BF16
-        x = oracle.round_storage(synth.activations(m, k, seed=302 + m), code).reshape(m, k)
-        with few_rows(d, 2):
-            got = d.project_quantized(api.Tensor.from_f32(d, (m, k), getattr(api.DType, dtype), x), w,
-                                      out_dtype=api.DType.F32).tensor.to_f32()
-        assert d.get_tuning("last_rows_plan") in (16301, 16401, 16501)
+    for dtype, code in (("F16", oracle.F16), ("BF16", oracle.BF16)):
+        x = oracle.round_storage(synth.activations(33, k, seed=302), code).reshape(33, k)
         want = oracle.project(ggml, block.reshape(-1), 61, k, x, accumulate="f64", weight_round=code, threads=8)
-        assert_matmul_parity(got[:, :61], want, f"{m} {dtype} rows")
-        assert np.array_equal(bits(got), bits(got[:, np.arange(n) % 61]))
+        first = None
+        for m in (2, 9, 16, 17, 33):
+            with few_rows(d, 2):
+                got = d.project_quantized(api.Tensor.from_f32(d, (m, k), getattr(api.DType, dtype), x[:m]), w,
+                                          out_dtype=api.DType.F32).tensor.to_f32()
+            assert d.get_tuning("last_rows_plan") // 1000 == (32 if m > 16 else 16)
+            assert_matmul_parity(got[:, :61], want[:m], f"{m} {dtype} rows")
+            assert np.array_equal(bits(got), bits(got[:, np.arange(n) % 61]))
+            first = got[:2] if first is None else first
+            assert np.array_equal(bits(got[:2]), bits(first)), (m, dtype)
 
 
 @pytest.mark.parametrize("ggml,m,n,k,few", [(13, 8, 151936, 2048, False), (12, 8, 28672, 4096, False), (13, 16, 28672, 4096, False),
