@@ -135,5 +135,18 @@ def build_gguf_probe(sanitize: bool = False) -> str:
     return out
 
 
+def build_freed_blocks_test(sanitize: bool = False) -> str:
+    """Compiles tests/cpp/freed_blocks_test.cpp (the rule for freed buffers; host code only, nothing to link).  `sanitize` builds a
+    second binary under ThreadSanitizer."""
+    root = os.path.dirname(HERE)
+    out = os.path.join(root, "tests", "cpp", "freed_blocks_test_san" if sanitize else "freed_blocks_test")
+    flags = ["-O1", "-g", "-fsanitize=thread"] if sanitize else ["-O2"]
+    cmd = ["g++", "-std=c++17", *flags, "-Wall", "-Werror", "-pthread", os.path.join(root, "tests", "cpp", "freed_blocks_test.cpp"), "-o", out]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"g++ failed for the test of freed blocks:\n{proc.stdout}\n{proc.stderr}")
+    return out
+
+
 if __name__ == "__main__":
     print(build(sys.argv[1:]))

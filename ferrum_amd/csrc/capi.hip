@@ -74,17 +74,22 @@ fh_status resolve(const fh_device* device, const fh_view* view, uint64_t element
 
 bool fits_u32(uint64_t v) { return v <= 0xffffffffull; }
 
-// Gives back what the pool holds; whether that was anything.  The caller has pool_lock.  A device that is
+// A block back to the system; hipFree waits for all work on the block's GPU when it succeeds.
+bool give_back(const fh_device* d, void* block) {
+    int current = d->ordinal;
+    (void)hipGetDevice(&current);
+    if (current != d->ordinal) (void)hipSetDevice(d->ordinal);
+    const hipError_t e = hipFree(block);
+    if (e != hipSuccess) (void)hipGetLastError();
+    if (current != d->ordinal) (void)hipSetDevice(current);
+    return e == hipSuccess;
+}
+
+// Gives back what the device keeps for buffers to come; whether that was anything.  A device that is
 // recording keeps its blocks: neither a wait on its stream nor a free may fall into a recording.
-bool drain_locked(fh_device* d) {
-    if ((d->pool.empty() && d->leaving.empty()) || d->capturing) return false;
-    (void)hipStreamSynchronize(d->stream);
-    for (auto& block : d->pool) (void)hipFree(block.second);
-    for (auto& block : d->leaving) (void)hipFree(block.second);
-    d->pool.clear();
-    d->leaving.clear();
-    d->pool_bytes = d->leaving_bytes = 0;
-    return true;
+bool drain(fh_device* d) {
+    return d->freed.drain([d] { return !d->capturing; }, [d] { (void)hipStreamSynchronize(d->stream); },
+                          [d](void* block) { return give_back(d, block); });
 }
 
 // Every device object between fh_device_create and fh_device_destroy.
@@ -112,8 +117,7 @@ bool drain_pools(int ordinal) {
     std::lock_guard<std::mutex> hold(g_live_lock);
     for (fh_device* d = g_live; d != nullptr; d = d->next_live) {
         if (d->ordinal != ordinal) continue;
-        std::lock_guard<std::mutex> hold_pool(d->pool_lock);
-        any = drain_locked(d) || any;
+        any = drain(d) || any;
     }
     return any;
 }
@@ -452,78 +456,33 @@ auto tuning_of(Device* d, const char* key) -> decltype(&(d->tuning.gemm_min_rows
 
 // ---- freed blocks kept for the next buffers ----------------------------------------------
 
-constexpr size_t kPoolBytes = 256u << 20;       // most memory kept
-constexpr size_t kPoolBlockBytes = 64u << 20;   // largest block kept
-constexpr size_t kLeavingBytes = 64u << 20, kLeavingBlocks = 512;   // blocks that wait for the GPU together
-
 // Blocks come in sizes a quarter of a power of two apart (4 KiB at least), so that a batch a little larger
 // or smaller finds them.
 size_t block_capacity(size_t bytes) {
-    if (bytes > kPoolBlockBytes) return bytes;
+    if (bytes > FreedBlocks::kPoolBlockBytes) return bytes;
     size_t step = 4096;
     while (step * 8 < bytes) step *= 2;
     return (bytes + step - 1) / step * step;
 }
 
 hipError_t take_block(fh_device* d, size_t capacity, void** out) {
-    {
-        std::lock_guard<std::mutex> hold(d->pool_lock);
-        const auto found = d->pool.find(capacity);
-        if (found != d->pool.end()) {
-            *out = found->second;
-            d->pool_bytes -= capacity;
-            d->pool.erase(found);
-            return hipSuccess;
-        }
-    }
-    return allocate(d, out, capacity);
+    return d->freed.take(capacity, out) ? hipSuccess : allocate(d, out, capacity);
 }
 
-// Blocks whose address the caller has been given: one goes back to the system, and hipFree waits for all work on the GPU, on
-// whatever stream, that was asked for before; none of the others is in use any more then.  The caller has pool_lock.
-void settle_leaving(fh_device* d) {
-    (void)hipFree(d->leaving.back().second);
-    d->leaving.pop_back();
-    for (auto& block : d->leaving) {
-        bool kept = false;
-        if (d->pool_bytes + block.first <= kPoolBytes) {
-            try {
-                d->pool.emplace(block.first, block.second);
-                d->pool_bytes += block.first;
-                kept = true;
-            } catch (...) {   // no memory for the entry
-            }
-        }
-        if (!kept) (void)hipFree(block.second);
-    }
-    d->leaving.clear();
-    d->leaving_bytes = 0;
-}
-
-// Takes a freed buffer's block into the pool; false: the caller frees it.  Nothing waits: whatever the
+// Keeps a freed buffer's block; false: the caller frees it.  Nothing waits: whatever the
 // library still has to do with the block comes before the next buffer's work on the stream.  A block whose
 // address the caller has been given may be in use elsewhere and waits, with others, until it cannot be.
 bool keep_block(fh_device* d, const fh_buffer& buffer) {
-    std::lock_guard<std::mutex> hold(d->pool_lock);
-    if (d->closed || d->capturing || buffer.capacity > kPoolBlockBytes) return false;
+    const auto may = [d] { return !d->closed && !d->capturing; };
+    if (buffer.capacity > FreedBlocks::kPoolBlockBytes) return false;
     if (buffer.exposed) {
-        try {
-            d->leaving.emplace_back(buffer.capacity, buffer.ptr);
-        } catch (...) {
-            return false;
-        }
-        d->leaving_bytes += buffer.capacity;
-        if (d->leaving_bytes >= kLeavingBytes || d->leaving.size() >= kLeavingBlocks) settle_leaving(d);
+        bool full = false;
+        if (!d->freed.gather(buffer.capacity, buffer.ptr, may, &full)) return false;
+        if (full) d->freed.settle(may, [d](void* block) { return give_back(d, block); });
         return true;
     }
-    if (d->pool_bytes + buffer.capacity > kPoolBytes) drain_locked(d);   // it holds sizes that are no longer asked for
-    try {
-        d->pool.emplace(buffer.capacity, buffer.ptr);
-        d->pool_bytes += buffer.capacity;
-    } catch (...) {   // no memory for the entry
-        return false;
-    }
-    return true;
+    if (!d->freed.fits(buffer.capacity)) drain(d);   // it holds sizes that are no longer asked for
+    return d->freed.keep(buffer.capacity, buffer.ptr, may);
 }
 
 }  // namespace
@@ -619,10 +578,11 @@ void fh_device_destroy(fh_device* device) {
     drain_deferred(device);
     leave_live(device);
     {
-        std::lock_guard<std::mutex> hold(device->pool_lock);
-        drain_locked(device);
+        std::lock_guard<std::mutex> alone(device->freed.settling);
+        std::lock_guard<std::mutex> hold(device->freed.lock);
         device->closed = true;   // buffers freed from here on are not kept
     }
+    drain(device);
     if (device->stream) {
         (void)hipStreamSynchronize(device->stream);
         (void)hipStreamDestroy(device->stream);
@@ -748,8 +708,11 @@ fh_status fh_get_tuning(const fh_device* device, const char* key, int64_t* value
         return FH_OK;
     }
     if (std::strcmp(key, "held_pool_bytes") == 0) {
-        std::lock_guard<std::mutex> hold(device->pool_lock);
-        *value = (int64_t)device->pool_bytes;
+        *value = (int64_t)device->freed.held_bytes();
+        return FH_OK;
+    }
+    if (std::strcmp(key, "waiting_pool_bytes") == 0) {
+        *value = (int64_t)device->freed.waiting_bytes();
         return FH_OK;
     }
     if (std::strcmp(key, "last_rows_plan") == 0) {
@@ -2475,7 +2438,8 @@ fh_status fh_moe_ffn(fh_device* device, const fh_view* hidden, const fh_view* ro
 fh_status fh_execution_begin(fh_device* device) {
     if (device == nullptr) return fail(FH_ERR_PARAMETER, "null device");
     if (device->capturing) return fail(FH_ERR_DISPATCH, "nested executions are not supported");
-    std::lock_guard<std::mutex> hold(device->pool_lock);   // no thread is waiting on the stream to empty the pool
+    std::lock_guard<std::mutex> alone(device->freed.settling);   // no thread is waiting for the GPU to empty the pool
+    std::lock_guard<std::mutex> hold(device->freed.lock);
     FH_HIP(hipStreamBeginCapture(device->stream, hipStreamCaptureModeThreadLocal));
     device->capturing = true;
     return FH_OK;

@@ -7,14 +7,13 @@
 #include <atomic>
 #include <cstdint>
 #include <cstdio>
-#include <map>
-#include <mutex>
 #include <utility>
 #include <vector>
 #include <string>
 
 #include "../../include/ferrum_hip.h"
 #include "../../include/ferrum_hip_probe.h"
+#include "freed_blocks.hpp"
 
 // Kernel-selection switches, set by name through fh_set_tuning (kTuningKeys in capi.hip).
 struct fh_tuning {
@@ -55,21 +54,17 @@ struct fh_device {
     int64_t last_rows_plan = 0;   // of the last dense product: 0, or the few-rows kernel's rows, tiles and K segments
     int64_t last_decoded_tile = 0;   // ... and 0, or the columns of its (first) tile where its weights were decoded first
     int64_t last_decoded_cut = 0;    // ... where its K was cut in two besides: this one and not the one before
-    std::atomic<bool> capturing{false};   // changes under pool_lock: what empties the pool waits on the stream
+    std::atomic<bool> capturing{false};   // set under freed.settling: what empties the pool waits on the stream
     fh_tuning tuning;
     // Blocks of freed buffers, by size, for the buffers to come (fh_buffer_alloc): hipMalloc and hipFree
     // take 10 - 20 us each and the latter waits for the GPU (a routed FFN of 200 f32 tokens whose operators
     // return new tensors: 453 us without the pool, 286 with it).  All work of the library on a buffer is on
     // `stream`, so a block can be handed on at once.  What has been done elsewhere with a buffer whose address has left the
-    // library only a wait for the whole GPU covers: such blocks gather in `leaving`, and one wait serves all of them (the same FFN, three
+    // library only a wait for the whole GPU covers: such blocks gather, and one wait serves all of them (the same FFN, three
     // of its outputs seen by torch: a wait for each, 110 us of host time, kept the host from running ahead: 248 us, now 205).
     // Python may drop a buffer on any thread, and another device object on the same GPU that finds no memory
     // empties this one's pool: the pool has a lock.
-    mutable std::mutex pool_lock;
-    std::multimap<size_t, void*> pool;
-    size_t pool_bytes = 0;
-    std::vector<std::pair<size_t, void*>> leaving;   // freed blocks whose address has left the library, by size
-    size_t leaving_bytes = 0;
+    fh::FreedBlocks freed;
     fh_device* next_live = nullptr;   // device objects that have not been destroyed (g_live in capi.hip)
     // scratch owned by the device: [counter words | floats / ids]
     void* scratch = nullptr;

@@ -127,6 +127,7 @@ void* fh_device_stream(fh_device* device);
  * fh_get_tuning alone also answers for what the library does by itself:
  *   held_pool_bytes     freed buffers kept for the next ones (see below); fh_set_tuning with 0 gives
  *                       back what every device object on this GPU keeps
+ *   waiting_pool_bytes  freed buffers that wait until nothing can still use them (see below)
  *   held_scratch_bytes  the operators' common scratch; fh_set_tuning with 0 brings it back to its smallest
  *                       size where no recorded execution uses it
  *   retired_scratch_blocks  scratch blocks that were outgrown and that recorded executions still use
@@ -147,7 +148,8 @@ fh_status fh_get_tuning(const fh_device* device, const char* key, int64_t* value
  * freeing does not wait for the stream then.
  * Buffers whose address fh_buffer_device_ptr has given out wait until nothing on the GPU, on whatever stream, can still use
  * them: up to 64 MiB or 512 of them gather, then one hipFree, which waits for the GPU, serves all, and the others are kept.
- * held_pool_bytes does not count those that wait; setting it to 0 gives them back too. */
+ * While such a free is refused (a stream of this process is being captured) none of them is used again.
+ * held_pool_bytes does not count those that wait (waiting_pool_bytes does); setting it to 0 gives them back too. */
 fh_status fh_buffer_alloc(fh_device* device, size_t bytes, fh_buffer** out);
 fh_status fh_buffer_alloc_uninitialized(fh_device* device, size_t bytes, fh_buffer** out);
 void fh_buffer_free(fh_buffer* buffer);

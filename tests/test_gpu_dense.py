@@ -1403,7 +1403,7 @@ def test_a_full_pool_makes_room_and_an_exposed_address_is_not_handed_on(api):
 
 def test_blocks_whose_address_has_left_wait_for_all_work_on_the_gpu(api):
     dev, size, steps = api.Device.new(), 4 << 20, 40     # more than wait together
-    kept = lambda: dev.get_tuning("held_pool_bytes")
+    kept, waiting = lambda: dev.get_tuning("held_pool_bytes"), lambda: dev.get_tuning("waiting_pool_bytes")
     hip, other = api._lib, ctypes.c_void_p()             # (the runtime the library is linked with)
     assert hip.hipStreamCreateWithFlags(ctypes.byref(other), 1) == 0
     copy = lambda to, source, count: hip.hipMemcpyAsync(ctypes.c_void_p(to), ctypes.c_void_p(source), ctypes.c_size_t(count), 3, other)
@@ -1418,7 +1418,7 @@ def test_blocks_whose_address_has_left_wait_for_all_work_on_the_gpu(api):
         assert copy(copies.device_ptr() + step * size, b.device_ptr(), size) == 0
         before = kept()
         del b
-        assert kept() <= 64 << 20
+        assert kept() <= 64 << 20 and waiting() < 64 << 20
         reused = reused or kept() > before
         fresh = api.Buffer(dev, size)                    # may get its block, and clears it at once
         del fresh
@@ -1428,15 +1428,17 @@ def test_blocks_whose_address_has_left_wait_for_all_work_on_the_gpu(api):
     assert reused
     b = api.Buffer(dev, 1 << 20)
     assert b.device_ptr()
+    before = waiting()
     del b
+    assert waiting() == before + (1 << 20)
     dev.set_tuning("held_pool_bytes", 0)
-    assert kept() == 0
+    assert kept() == waiting() == 0
     small = [api.Buffer(dev, 4096) for _ in range(600)]     # and no more blocks than that, however small
     assert all(x.device_ptr() for x in small)
     small.clear()
-    assert 0 < kept() <= 600 * 4096
+    assert kept() == 511 * 4096 and waiting() == 88 * 4096     # 512 of them, of which one has gone back
     dev.set_tuning("held_pool_bytes", 0)
-    assert kept() == 0
+    assert kept() == waiting() == 0
 
 
 def test_one_device_object_gives_back_what_another_on_the_gpu_keeps(api):
