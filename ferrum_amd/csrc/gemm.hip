@@ -854,11 +854,12 @@ struct Wide32 {
 // sound while the compiler keeps nothing of its own in M0 in this kernel, which has no other
 // client of it.  The load returns no register and is covered only by the hand-placed
 // `s_waitcnt vmcnt(0)` statements of the main loop; those wait for everything, so loads of the
-// compiler's own in between cannot make them wrong.  The build checks the generated text for
-// the M0 rule and for scratch (ferrum_amd/isa_check.py).
+// compiler's own in between cannot make them wrong.  (s_nop: the wait state that a load into LDS needs behind the
+// instruction that writes its M0.)  The build checks the generated text for
+// the M0 rules and for scratch (ferrum_amd/isa_check.py).
 __device__ __forceinline__ void lds_direct16(const void* g, uint32_t lds_addr) {
     const uint32_t a = __builtin_amdgcn_readfirstlane(lds_addr);
-    asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(a) : "memory");
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(a) : "memory");
 }
 
 // Where the tiles alone would leave part of the chip idle, K is cut into segments of `seg_blocks`

@@ -24,20 +24,22 @@ __device__ __forceinline__ uint64_t uniform_address(const void* pointer) {
 // M0 in a clobber list.  It is sound as long as the compiler keeps no value of its own in M0 across
 // the statement, which holds for code that uses none of M0's other clients (s_movrel, GWS and
 // sendmsg operands, ds_*_addtid, lane-indexed v_readlane through M0): these kernels have none.
+// A load into LDS may not be the next instruction behind the scalar one that writes its M0 (one wait state, which the compiler
+// inserts for its own loads and cannot for these): hence the s_nop.
 // The load is counted in vmcnt like any vector-memory load and returns no register; the only wait
 // that covers it is the author's wait_vmcnt / s_waitcnt vmcnt below, so between such a load and
 // the wait that counts it there must be no vector-memory instruction of the compiler's.  The
-// build compiles this file to assembly text as well and checks all three facts there
+// build compiles this file to assembly text as well and checks these facts there
 // (ferrum_amd/isa_check.py); it refuses to link a library that breaks one.
 __device__ __forceinline__ void lds_load16_at(const void* base, uint32_t offset, uint32_t lds_addr) {
     const uint32_t a = __builtin_amdgcn_readfirstlane(lds_addr);
     const uint64_t sb = uniform_address(base);
-    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(offset), "s"(sb), "s"(a) : "memory");
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(offset), "s"(sb), "s"(a) : "memory");
 }
 
 // The same where the compiler knows that address and base are the whole wave's.
 __device__ __forceinline__ void lds_load16_uniform(const void* base, uint32_t offset, uint32_t lds_addr) {
-    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(offset), "s"(base), "s"(lds_addr) : "memory");
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(offset), "s"(base), "s"(lds_addr) : "memory");
 }
 
 // The same as a buffer load that the compiler issues and counts: 16 bytes a lane from `offset` + `base` in `rows` to `to` + 16 * lane.

@@ -3,11 +3,12 @@
 Six sources (``CHECKED_SOURCES`` and ``HAND_ISSUED_SOURCES``) issue memory instructions through
 ``asm volatile`` that the compiler cannot see the timing of:
 
-* LDS-direct loads (``s_mov_b32 m0, <lds address>`` followed by
+* LDS-direct loads (``s_mov_b32 m0, <lds address>``, ``s_nop 0``,
   ``global_load_lds_dwordx4``): the statement writes M0, which an asm statement cannot
   name as a clobber on this target.  The invariant is that the compiler keeps nothing of
   its own in M0 inside these kernels: every mention of M0 in a kernel's code must be one
-  of these statements.
+  of these statements.  A load into LDS may not be the next instruction behind the one that writes its M0: the
+  compiler puts a wait state between the two, and so must the statement.
 * register loads (``global_load_dwordx2/x4 vDST, vADDR, off`` in gemv_stream.hip): the
   destination registers hold the data only after the hand-placed ``s_waitcnt vmcnt(n)``
   that follows.  The invariant is that nothing between the load and that wait reads or
@@ -52,6 +53,10 @@ _REG_LOAD = re.compile(r"^global_load_dwordx[234]\s+(v\[\d+:\d+\]|v\d+)\s*,")
 _VMEM = re.compile(r"^(global_|buffer_|flat_|scratch_)(load|store|atomic)")
 _LDS_LOAD = re.compile(r"^(global_load_lds_|buffer_load_\w+ .*\blds$)")
 _STORE = re.compile(r"^(global_|buffer_|flat_)store")
+
+
+def _no_wait_state(where: str, number: int, name: str) -> str:
+    return f"{where}{number}: {name}: no wait state between M0 and the LDS-direct load that uses it"
 
 
 def _vregs(text: str) -> set[int]:
@@ -120,6 +125,8 @@ def violations(asm: str, source: str = "", counted: bool = False) -> list[str]:
                     nxt.startswith("global_load_lds_") or (nxt.startswith("s_nop") and nxt2.startswith("global_load_lds_")))
                 if not ours:
                     found.append(f"{where}{number}: {name}: M0 is used outside an LDS-direct load statement: {text}")
+                elif not nxt.startswith("s_nop"):
+                    found.append(_no_wait_state(where, number, name))
             if in_asm and text.startswith("global_load_lds_"):
                 hand_loads = True
                 if not counted:
@@ -148,9 +155,11 @@ def counted_violations(asm: str, source: str = "") -> list[str]:
                  if in_asm and (m := re.match(r"s_waitcnt vmcnt\((\d+)\)", text))}
         lds = [at for at, (_, text, _) in enumerate(body) if _LDS_LOAD.match(text)]
         theirs = True    # M0 is as the compiler last wrote it
-        for number, text, in_asm in body:
+        for at, (number, text, in_asm) in enumerate(body):
             if re.match(r"s_\w+ m0,", text):
                 theirs = not in_asm
+                if at + 1 < len(body) and _LDS_LOAD.match(body[at + 1][1]):
+                    found.append(_no_wait_state(where, number, name))
             elif _LDS_LOAD.match(text) and not in_asm and not theirs:
                 found.append(f"{where}{number}: {name}: the compiler's LDS-direct load finds M0 as an asm statement left it")
         if lds and not waits:

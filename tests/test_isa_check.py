@@ -16,6 +16,7 @@ _Z6kernelv:
 	v_add_u32_e32 v9, v8, v7
 	;;#ASMSTART
 	s_mov_b32 m0, s3
+	s_nop 0
 	global_load_lds_dwordx4 v[2:3], off
 	;;#ASMEND
 	s_add_u32 s2, s2, 1
@@ -44,6 +45,8 @@ def test_a_clean_kernel_passes():
     # the compiler keeps something of its own in M0
     ("s_add_u32 s2, s2, 1", "s_mov_b32 m0, s9", "M0 is used outside"),
     ("s_add_u32 s2, s2, 1", "ds_gws_init v0 gds", None),
+    # the load right behind its M0, without the wait state between the two
+    ("s_mov_b32 m0, s3\n\ts_nop 0\n", "s_mov_b32 m0, s3\n", "no wait state"),
     # spill space in a kernel with such loads
     (".amdhsa_private_segment_fixed_size 0", ".amdhsa_private_segment_fixed_size 64", "bytes of scratch"),
     # a register load that no hand-placed wait follows
@@ -126,10 +129,12 @@ _Z4loopv:
 	ds_read_b128 v[20:23], v1
 	;;#ASMSTART
 	s_mov_b32 m0, s3
+	s_nop 0
 	global_load_lds_dwordx4 v2, s[8:9]
 	;;#ASMEND
 	;;#ASMSTART
 	s_mov_b32 m0, s4
+	s_nop 0
 	global_load_lds_dwordx4 v3, s[8:9]
 	;;#ASMEND
 	global_load_dwordx4 v[8:11], v[6:7], off
@@ -162,10 +167,12 @@ def test_counted_loads_are_counted_along_a_branch_back_over_them(source):
 
 def test_the_compilers_lds_loads_find_their_own_m0():
     mixed = COUNTED.replace("_Z4rowsv:\n", "_Z4rowsv:\n\t;;#ASMSTART\n\ts_mov_b32 m0, s4\n\t;;#ASMEND\n"
-                            "\ts_mov_b32 m0, s5\n\tbuffer_load_dwordx4 v1, s[0:3], 0 offen lds\n")
+                            "\ts_mov_b32 m0, s5\n\ts_nop 0\n\tbuffer_load_dwordx4 v1, s[0:3], 0 offen lds\n")
     assert isa_check.counted_violations(mixed) == []
     found = isa_check.counted_violations(mixed.replace("\ts_mov_b32 m0, s5\n", ""), "x.hip")
     assert found and "finds M0 as an asm statement left it" in found[0], found
+    found = isa_check.counted_violations(mixed.replace("\ts_nop 0\n", ""), "x.hip")
+    assert len(found) == 1 and "no wait state" in found[0], found
 
 
 def test_hand_issued_counted_loads_need_a_wait_behind_them():
