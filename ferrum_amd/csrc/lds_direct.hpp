@@ -28,7 +28,8 @@ __device__ __forceinline__ uint64_t uniform_address(const void* pointer) {
 // inserts for its own loads and cannot for these): hence the s_nop.
 // The load is counted in vmcnt like any vector-memory load and returns no register; the only wait
 // that covers it is the author's wait_vmcnt / s_waitcnt vmcnt below, so between such a load and
-// the wait that counts it there must be no vector-memory instruction of the compiler's.  The
+// the wait that counts it there must be no vector-memory instruction of the compiler's, or, where the wait counts the
+// compiler's own loads behind it, no fewer of them than it allows.  The
 // build compiles this file to assembly text as well and checks these facts there
 // (ferrum_amd/isa_check.py); it refuses to link a library that breaks one.
 __device__ __forceinline__ void lds_load16_at(const void* base, uint32_t offset, uint32_t lds_addr) {

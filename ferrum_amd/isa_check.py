@@ -1,6 +1,6 @@
 """Build-time check of the hand-scheduled loads in this library's own kernels.
 
-Six sources (``CHECKED_SOURCES`` and ``HAND_ISSUED_SOURCES``) issue memory instructions through
+The sources in ``CHECKED_SOURCES`` and ``COUNTED_SOURCES`` issue memory instructions through
 ``asm volatile`` that the compiler cannot see the timing of:
 
 * LDS-direct loads (``s_mov_b32 m0, <lds address>``, ``s_nop 0``,
@@ -21,11 +21,13 @@ Six sources (``CHECKED_SOURCES`` and ``HAND_ISSUED_SOURCES``) issue memory instr
   stores behind LDS-direct loads, which can only lengthen the wait.
 
 A second kind of kernel (``COUNTED_SOURCES``) leaves its register loads to the compiler, which orders and counts them,
-and but for ``HAND_ISSUED_SOURCES`` its LDS-direct loads too, and only says when the latter have landed: ``s_waitcnt
-vmcnt(n)``, n being the register loads the source issues behind them.
+and only says when its LDS-direct loads have landed: ``s_waitcnt vmcnt(n)``, n being the register loads the source issues behind them.
 The invariant is that the generated code has at least n of them there
 (``counted_violations``): with fewer, n outstanding loads could include one that the wait
-is for.  Where such a kernel issues some LDS-direct loads itself, each of the compiler's has to find an M0 that the compiler wrote.  Of the hand-issued ones M0 and scratch are checked as above (``m0_violations``).
+is for.  In ``HAND_ISSUED_SOURCES`` all LDS-direct loads are asm statements: M0 and scratch are checked as above (``m0_violations``).
+In the others the first ones are and the compiler issues the rest: M0 then belongs to the statements and to the compiler's own
+LDS-direct loads, each of which finds the M0 that the compiler wrote for it.  Scratch may be there: no register is
+loaded by a statement, and a spill between a load and its wait only lengthens the wait.
 
 The check reads the assembly hipcc writes with ``-S`` for this library's own sources
 (text, before it becomes a code object) and returns every violation it finds.  It is a
@@ -44,7 +46,7 @@ VALIDATED_HIPCC = "7.2.26015"
 CHECKED_SOURCES = ("gemm.hip", "gemm_decoded.hip", "gemv_stream.hip", "gemm_skinny.hip", "probe.hip")
 COUNTED_SOURCES = ("gemm_pairs.hip", "gemm_rows_q4_k.hip", "gemm_rows_q5_k.hip", "gemm_rows_q6_k.hip", "gemm_rows_iq4_xs.hip",
                    "gemm_rows_q8_0.hip")
-HAND_ISSUED_SOURCES = ("gemm_pairs.hip",)   # counted, and their LDS-direct loads are asm statements
+HAND_ISSUED_SOURCES = ("gemm_pairs.hip",)   # counted, and all their LDS-direct loads are asm statements
 
 _KERNEL_LABEL = re.compile(r"^(_Z\w+|\w+):\s*(;.*)?$")
 _VREG_RANGE = re.compile(r"\bv\[(\d+):(\d+)\]")
@@ -145,7 +147,8 @@ def counted_violations(asm: str, source: str = "") -> list[str]:
     up to the next hand-placed wait, the next run or the function's end, there must be at least as many of the latter as the
     hand-placed ``s_waitcnt vmcnt(n)`` leave outstanding: the largest n of the kernel where the compiler issues the runs; in
     ``HAND_ISSUED_SOURCES``, whose last rounds request nothing behind a run and wait for all, the n of the next wait, and one
-    must follow.  Likewise along every branch back over a run, up to the first wait behind its target."""
+    must follow.  Likewise along every branch back over a run, up to the first wait behind its target.  The compiler uses M0 for
+    LDS-direct loads of its own alone and writes it for each run of them."""
     found: list[str] = []
     where = (source + ":") if source else ""
     next_wait_counts = source in HAND_ISSUED_SOURCES
@@ -160,6 +163,11 @@ def counted_violations(asm: str, source: str = "") -> list[str]:
                 theirs = not in_asm
                 if at + 1 < len(body) and _LDS_LOAD.match(body[at + 1][1]):
                     found.append(_no_wait_state(where, number, name))
+                own = next((asm for _, t, asm in body[at + 1:] if _LDS_LOAD.match(t)), None) is False
+                if not in_asm and (not own or "m0" in text.split(",", 1)[1]):
+                    found.append(f"{where}{number}: {name}: M0 is used outside an LDS-direct load: {text}")
+            elif re.search(r"\bm0\b", text):
+                found.append(f"{where}{number}: {name}: M0 is used outside an LDS-direct load: {text}")
             elif _LDS_LOAD.match(text) and not in_asm and not theirs:
                 found.append(f"{where}{number}: {name}: the compiler's LDS-direct load finds M0 as an asm statement left it")
         if lds and not waits:

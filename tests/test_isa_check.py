@@ -173,6 +173,12 @@ def test_the_compilers_lds_loads_find_their_own_m0():
     assert found and "finds M0 as an asm statement left it" in found[0], found
     found = isa_check.counted_violations(mixed.replace("\ts_nop 0\n", ""), "x.hip")
     assert len(found) == 1 and "no wait state" in found[0], found
+    # M0 is read, or written for something that is no load into LDS of the compiler's
+    for line in ("\ts_mov_b32 s9, m0\n", "\ts_add_u32 m0, m0, s9\n", "\tv_movrels_b32_e32 v1, m0\n"):
+        found = isa_check.counted_violations(mixed.replace("\ts_mov_b32 m0, s5\n", line + "\ts_mov_b32 m0, s5\n"), "x.hip")
+        assert len(found) == 1 and "M0 is used outside" in found[0], found
+    found = isa_check.counted_violations(mixed.replace("\tds_read_b128", "\ts_mov_b32 m0, s6\n\tds_read_b128"), "x.hip")
+    assert len(found) == 1 and "M0 is used outside" in found[0], found
 
 
 def test_hand_issued_counted_loads_need_a_wait_behind_them():
