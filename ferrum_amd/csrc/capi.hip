@@ -727,6 +727,10 @@ fh_status fh_get_tuning(const fh_device* device, const char* key, int64_t* value
         *value = device->last_decoded_cut;
         return FH_OK;
     }
+    if (std::strcmp(key, "last_decoded_runs") == 0) {
+        *value = device->last_decoded_runs;
+        return FH_OK;
+    }
     const int64_t* const setting = tuning_of(device, key);
     if (setting == nullptr) return fail(FH_ERR_PARAMETER, "unknown tuning key %s", key);
     *value = *setting;
@@ -1045,6 +1049,7 @@ const char* run_gemm(fh_device* device, GemmArgs& g) {
     const int64_t decoded_tile = g.decoded.runs != 0 ? g.decoded.run[0].tile : 0;
     device->last_decoded_tile = g.decoded.segments == 1 ? decoded_tile : 0;
     device->last_decoded_cut = g.decoded.segments == 2 ? decoded_tile : 0;
+    device->last_decoded_runs = g.decoded.runs;
     return launch_gemm(device->stream, g);
 }
 
@@ -1121,7 +1126,7 @@ fh_status project(fh_device* device, const fh_qmatrix* weight, const fh_view* x,
     const bool f32_batch = !tile && !silu_mul && x->dtype == FH_F32 && m >= (weight->ggml_type == kQ4K ? 5u : 4u) &&
                            m >= (uint32_t)device->tuning.gemm_min_rows && device->tuning.gemv_stream == 1 &&
                            device->tuning.k_quant_gemv_ksplit == 0;
-    device->last_rows_plan = device->last_decoded_tile = device->last_decoded_cut = 0;
+    device->last_rows_plan = device->last_decoded_tile = device->last_decoded_cut = device->last_decoded_runs = 0;
     GemmArgs g{};
     if (tile || f32_batch) g = gemm_args(device, weight->ggml_type, n, k, m, f32_tile ? FH_F16 : x->dtype, y->dtype);
     if (f32_batch && g.few_rows) {

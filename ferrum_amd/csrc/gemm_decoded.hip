@@ -349,7 +349,7 @@ void launch_tile(hipStream_t s, const DecodedParams& p, uint32_t columns) {
 }
 
 // Four outputs of a row in a store of a lane take 694 us where single ones of neighbouring columns take 706 (1999 x 34816 x 5120, 320
-// columns; 8192 x 4096, 1500 rows, 256 columns: 115 / 119), but only where every row starts on a four.
+// columns; 8192 x 4096, 1500 rows, 256 columns asked for: 115 / 119), but only where every row starts on a four.
 template <int DT>
 void launch_tile_of(hipStream_t s, const DecodedParams& p, uint32_t columns, bool cut) {
     if (p.n % 4 == 0) cut ? launch_tile<DT, true, true>(s, p, columns) : launch_tile<DT, false, true>(s, p, columns);
@@ -392,20 +392,21 @@ double run_us(const DecodedTile& t, uint32_t columns, uint32_t tiles_m, uint32_t
 }  // namespace
 
 // The decode by its bytes, then rounds of the product, the last one cheaper where it is not full; against the fused tiles'
-// estimate.  Fitted to the 2400 plans timed for 400 products of 400 - 2048 rows and K of 512 - 17408, 5.8% in the mean square.  Of the 500
-// other products in profiles/decoded_runs_us.txt 236 decode, three of them slower than the fused tiles by more than 2%; the pick is
-// 1.7% from the fastest in the mean.  (With a margin of a twentieth on the panels' side eight are slower and nothing is gained.)
+// estimate.  Of the 500 products of 400 - 2048 rows and K of 512 - 17408 in profiles/decoded_runs_us.txt, none of which the constants
+// were fitted to, 236 decode, three of them slower than the fused tiles by more than 2%, and the dispatched time is 1.9% from the fastest
+// in the mean.  264 stay fused; 50 of those lose more than 5% by it and 24 more than 10%, where the fused estimate is too
+// low (Q6_K 411 x 21004 x 6144 272 against 217 us).
 //
 // Runs of tiles.  A round of a tile takes what it takes however few workgroups it has, so columns that do not make whole rounds of
-// one tile are better cut into whole rounds of two and the rest on a third: 1999 x 34816 x 5120 is 3.4 rounds of 320 columns, 694 us, or
-// two of those, one of 256 columns and one of 192, 674.  All tiles sum in the same order.
+// one tile are better cut into whole rounds of one and the rest on another: 1999 x 34816 x 5120 is 3.4 rounds of 320 columns, 717 us, or
+// one of those and three of 256 columns, 687 (three of 30,000 random products would gain by a third tile).  All tiles sum in the same order.
 //
 // Two segments of K.  5120 columns and 1999 rows are 128 tiles of 320 x 256: half of the chip, or 216 of 192 columns.  Cut in two, the
 // former are one round.  Q6_K 1999 x 5120 x 17408 uncut 401 (192 columns), 456 (320), cut 349 us (320), fused tiles 421; Q4_K 392 / 450
 // / 343 / 353; 1999 x 5120 x 5120 stays uncut, 114 / 125 / 122 / 118.
 //
-// us, fused tiles / 192 / 256 / 320 columns: Q4_K 1999 x 34816 x 5120 771 / 766 / 728 / 694; 1500 x 8192 x 4096 133 / 167 / 116 / 123;
-// Q8_0 2048 x 4096 x 4096 100 / 83 / 85 / 98.
+// us, fused tiles / 192 / 256 / 320 columns: Q4_K 1999 x 34816 x 5120 775 / 777 / 745 / 717; 1500 x 8192 x 4096 127 / 162 / 111 / 116 (it
+// stays fused, whose estimate is lower); Q8_0 2048 x 4096 x 4096 100 / 83 / 85 / 98.
 bool gemm_takes_decoded(GemmArgs& a) {
     if (a.decoded_min_rows == 0 || a.wide32_tile != 0 || a.wide_shape != 1 || !a.resident_switch || a.m <= 256) return false;
     const uint32_t cus = a.cu_count > 0 ? (uint32_t)a.cu_count : 256u, tiles_m = (a.m + 255) / 256;
@@ -421,15 +422,13 @@ bool gemm_takes_decoded(GemmArgs& a) {
     DecodedPlan& plan = a.decoded;
     const double decode = (double)a.n * a.k * (2.0 + block_bytes(a.ggml_type) / 256.0) / 4.69e6;
     const bool any_tile = a.decoded_tile == 0;
-    // whole rounds of one tile, whole rounds of a second, and the rest on a third: a round takes what its tile does, however
-    // few of its workgroups there are
+    // whole rounds of one tile and the rest on another: a round takes what its tile does, however few of its workgroups there are
     for (const DecodedTile& last : kDecodedTiles) {
         if (!any_tile && (uint32_t)a.decoded_tile != last.columns) continue;
         for (const DecodedTile& one : kDecodedTiles) {
             const uint32_t one_round = cus / tiles_m * one.columns, one_most = any_tile && &one != &last ? (a.n - 1) / std::max(one_round, 1u) : 0u;
             for (uint32_t i = 0; i <= (one_round ? one_most : 0u); ++i) {
                 if (i == 0 && &one != kDecodedTiles) continue;   // (the same plan from every tile)
-                const uint32_t behind = a.n - i * one_round;
                 DecodedPlan p{};
                 double us = decode;
                 auto add = [&](const DecodedTile& t, uint32_t columns) {
@@ -440,22 +439,11 @@ bool gemm_takes_decoded(GemmArgs& a) {
                     us += here == 0.0 ? 1e300 : here + (p.runs > 1 ? kRunUs : 0.0);
                 };
                 if (i > 0) add(one, i * one_round);
-                const DecodedPlan head = p;
-                const double head_us = us;
-                for (const DecodedTile& two : kDecodedTiles) {
-                    const uint32_t two_round = cus / tiles_m * two.columns;
-                    for (uint32_t j = 0; j <= (i > 0 && &two != &one && &two != &last ? 1u : 0u); ++j) {
-                        if (j == 0 ? &two != kDecodedTiles : behind <= two_round) continue;
-                        p = head;
-                        us = head_us;
-                        if (j > 0) add(two, two_round);
-                        add(last, behind - j * two_round);
-                        if (us < best) {
-                            best = us;
-                            plan = p;
-                            plan.segments = 1;
-                        }
-                    }
+                add(last, a.n - i * one_round);
+                if (us < best) {
+                    best = us;
+                    plan = p;
+                    plan.segments = 1;
                 }
             }
         }

@@ -54,6 +54,7 @@ struct fh_device {
     int64_t last_rows_plan = 0;   // of the last dense product: 0, or the few-rows kernel's rows, tiles and K segments
     int64_t last_decoded_tile = 0;   // ... and 0, or the columns of its (first) tile where its weights were decoded first
     int64_t last_decoded_cut = 0;    // ... where its K was cut in two besides: this one and not the one before
+    int64_t last_decoded_runs = 0;   // ... and its runs of tiles
     std::atomic<bool> capturing{false};   // set under freed.settling: what empties the pool waits on the stream
     fh_tuning tuning;
     // Blocks of freed buffers, by size, for the buffers to come (fh_buffer_alloc): hipMalloc and hipFree
@@ -349,15 +350,14 @@ struct TileChoice {
     double us32, us16;
 };
 
-// How a product multiplies weights that were decoded first: its columns in up to three runs of tiles, a panel of each run at a time.
+// How a product multiplies weights that were decoded first: its columns in one or two runs of tiles, a panel of each run at a time.
 struct DecodedPlan {
     struct Run {
         uint32_t columns, tile, panel;   // of the matrix; of a tile; decoded at a time, a multiple of `tile`
-    } run[3];
+    } run[2];
     int runs;              // 0: the weights are not decoded first
     uint32_t segments;     // K segments: 1, or 2 (one run then)
     size_t panel_bytes, sum_bytes;   // scratch: the largest panel, then the sums of one segment's tiles
-    double estimate_us;
 };
 
 struct GemmArgs {

@@ -134,7 +134,8 @@ void* fh_device_stream(fh_device* device);
  *   last_rows_plan      how the last dense product ran on the few-rows kernel: 1000 x activation
  *                       rows (16 or 32) + 100 x weight tiles per wave + K segments; 0 on others
  *   last_decoded_tile   columns of its (first) tile where it decoded its weights first; 0 on others
- *   last_decoded_cut    ... where it cut K in two besides: then this one is not 0 and the one before is */
+ *   last_decoded_cut    ... where it cut K in two besides: then this one is not 0 and the one before is
+ *   last_decoded_runs   runs of tiles such a product's columns came in, 1 or 2; 0 on others */
 fh_status fh_set_tuning(fh_device* device, const char* key, int64_t value);
 fh_status fh_get_tuning(const fh_device* device, const char* key, int64_t* value);
 

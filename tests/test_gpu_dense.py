@@ -2020,9 +2020,11 @@ def test_decoded_products_with_k_cut_in_two(api, d, ggml, m, n, k, dtype):
         d.set_tuning("gemm_decoded_segments", 0)
 
 
-@pytest.mark.parametrize("m,n", [(300, 57344), (300, 57001), (520, 34816), (600, 24000), (1300, 14336)])
-def test_runs_of_several_decoded_tiles_give_the_bits_of_one(api, d, m, n):
-    # columns of more than a round of the chip, in runs of up to three tiles: every column comes from one of them
+@pytest.mark.parametrize("m,n,count", [(300, 57344, 1), (300, 57001, 1), (520, 34816, 1), (600, 24000, 1), (1300, 14336, 1),
+                                       (1025, 52844, 2), (1025, 54838, 2), (1300, 43871, 2), (2047, 32904, 2), (2047, 52845, 2)])
+def test_runs_of_several_decoded_tiles_give_the_bits_of_one(api, d, m, n, count):
+    # columns of more than a round of the chip, in one run of tiles or whole rounds of one tile and the rest on another (320 first and
+    # 256 first, the second run ragged, rows that are whole fours and rows that are not): every column comes from one of them
     k = 512
     base = synth.matrix(Q4_K, 251, k, seed=775).reshape(251, -1)
     w = qm(api, d, Q4_K, n, k, np.resize(base, (n, base.shape[1])).reshape(-1))
@@ -2032,10 +2034,11 @@ def test_runs_of_several_decoded_tiles_give_the_bits_of_one(api, d, m, n):
         d.set_tuning("gemm_decoded_min_rows", 2)
         d.project_quantized(xt, w, out=out)
         runs = out.raw()
-        assert d.get_tuning("last_decoded_tile") != 0
+        assert d.get_tuning("last_decoded_tile") != 0 and d.get_tuning("last_decoded_runs") == count
         for tile in (192, 256, 320):
             d.set_tuning("gemm_decoded_tile", tile)
             d.project_quantized(xt, w, out=out)
+            assert (d.get_tuning("last_decoded_tile"), d.get_tuning("last_decoded_runs")) == (tile, 1)
             assert np.array_equal(out.raw(), runs), tile
     finally:
         d.set_tuning("gemm_decoded_min_rows", 1)
@@ -2097,7 +2100,8 @@ def test_products_with_few_columns_stay_on_the_square_tiles(api, d, ggml, m, n, 
 def test_the_switches_of_segments_and_panels_take_only_what_they_mean(api, d):
     for key, good, bad in (("gemm_wide32_segments", (0, 1, 8), (-1, 9, 1 << 32)),
                            ("gemm_decoded_min_rows", (0, 1, 2, 300, 2 ** 31 - 1), (-1, 2 ** 31, 1 << 32)),
-                           ("gemm_decoded_tile", (0, 192, 256, 320), (-192, 100, 128, (1 << 32) + 192))):
+                           ("gemm_decoded_tile", (0, 192, 256, 320), (-192, 100, 128, (1 << 32) + 192)),
+                           ("gemm_decoded_segments", (0, 1, 2), (-1, 3, 1 << 32))):
         before = d.get_tuning(key)
         try:
             for value in good:
