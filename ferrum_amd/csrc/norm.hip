@@ -27,19 +27,11 @@ constexpr int kNormThreads = 256;
 constexpr int kNormMaxCache = 16;  // most groups of 4 a thread keeps between the passes
 
 // sum over the workgroup, returned in every thread
-template <int THREADS>
 __device__ __forceinline__ float block_sum(float v, float* partial) {
     v = wave_sum(v);
     if ((threadIdx.x & 63u) == 0) partial[threadIdx.x >> 6] = v;
     __syncthreads();
-    float sums[THREADS / 64];
-#pragma unroll
-    for (int i = 0; i < THREADS / 64; ++i) sums[i] = partial[i];
-#pragma unroll
-    for (int step = THREADS / 128; step > 0; step /= 2)
-#pragma unroll
-        for (int i = 0; i < step; ++i) sums[i] = sums[2 * i] + sums[2 * i + 1];
-    return sums[0];
+    return (partial[0] + partial[1]) + (partial[2] + partial[3]);
 }
 
 template <int DT, class Raw>
@@ -74,24 +66,24 @@ __device__ __forceinline__ float4 rounded_sum(float4 x, float4 y) {
                        round_storage(x.z + y.z, DT), round_storage(x.w + y.w, DT));
 }
 
-// width % 4 == 0 and width <= 4 * THREADS * kNormCache
+// width % 4 == 0 and width <= 4 * kNormThreads * kNormCache
 //
 // A row or a few of them are one chain: launch, loads, sum, store.  All loads are requested before the first is waited for
 // (groups past the row read its last one again and count for nothing); waited for group by group, from a graph, us: 1 x 5120 f32
 // 3.0, now 2.4, 8 x 5120 f16 3.2 / 2.5, 24 x 4096 f32 3.0 / 2.4, 128 x 5120 bf16 3.5 / 2.8, 100 x 8192 f32 5.0 / 3.8, 512 x
 // 5120 f16 4.9 / 4.5, 1999 x 5120 bf16 13.2 / 13.0 (6.3 TB/s).  512 threads a row take the same, 1024 a tenth more.
-template <int DT, int THREADS, int kNormCache>
-__global__ __launch_bounds__(THREADS) void add_rmsnorm_rows_kernel(
+template <int DT, int kNormCache>
+__global__ __launch_bounds__(kNormThreads) void add_rmsnorm_rows_kernel(
     const void* __restrict__ a, const void* __restrict__ b, const void* __restrict__ weight,
     void* __restrict__ residual, void* __restrict__ normed, uint32_t width, float eps) {
     typedef typename std::conditional<DT == 0, float4, uint2>::type Raw;
-    __shared__ float partial[THREADS / 64];
+    __shared__ float partial[kNormThreads / 64];
     const uint32_t tid = threadIdx.x, groups = width >> 2;
     const size_t base = (size_t)blockIdx.x * groups;
     Raw ra[kNormCache], rb[kNormCache], rw[kNormCache];
 #pragma unroll
     for (int s = 0; s < kNormCache; ++s) {
-        const uint32_t g = min(tid + s * THREADS, groups - 1);
+        const uint32_t g = min(tid + s * kNormThreads, groups - 1);
         ra[s] = static_cast<const Raw*>(a)[base + g];
         rb[s] = static_cast<const Raw*>(b)[base + g];
         rw[s] = static_cast<const Raw*>(weight)[g];
@@ -100,7 +92,7 @@ __global__ __launch_bounds__(THREADS) void add_rmsnorm_rows_kernel(
     float sum = 0.f;
 #pragma unroll
     for (int s = 0; s < kNormCache; ++s) {
-        const uint32_t g = tid + s * THREADS;
+        const uint32_t g = tid + s * kNormThreads;
         x[s] = rounded_sum<DT>(widened<DT>(ra[s]), widened<DT>(rb[s]));
         if (g < groups) {
             store4<DT>(residual, base + g, x[s]);
@@ -111,11 +103,11 @@ __global__ __launch_bounds__(THREADS) void add_rmsnorm_rows_kernel(
             sum += x[s].w * x[s].w;
         }
     }
-    sum = block_sum<THREADS>(sum, partial);
+    sum = block_sum(sum, partial);
     const float inv = rsqrtf(sum / (float)width + eps);
 #pragma unroll
     for (int s = 0; s < kNormCache; ++s) {
-        const uint32_t g = tid + s * THREADS;
+        const uint32_t g = tid + s * kNormThreads;
         const float4 w = widened<DT>(rw[s]);
         if (g < groups)
             store4<DT>(normed, base + g, make_float4(x[s].x * inv * w.x, x[s].y * inv * w.y, x[s].z * inv * w.z, x[s].w * inv * w.w));
@@ -136,7 +128,7 @@ __global__ __launch_bounds__(kNormThreads) void add_rmsnorm_any_kernel(
         store_from_f32(residual, base + j, dtype, x);
         sum += x * x;
     }
-    sum = block_sum<kNormThreads>(sum, partial);
+    sum = block_sum(sum, partial);
     const float inv = rsqrtf(sum / (float)width + eps);
     for (uint32_t j = tid; j < width; j += kNormThreads) {
         const float x = round_storage(load_as_f32(a, base + j, dtype) + load_as_f32(b, base + j, dtype), dtype);
@@ -149,18 +141,18 @@ void launch_dtype(hipStream_t s, const void* a, const void* b, const void* weigh
                   uint32_t rows, uint32_t width, float eps) {
     const dim3 grid(rows), block(kNormThreads);
     const uint32_t per_thread = (width / 4 + kNormThreads - 1) / kNormThreads;
-#define FH_NORM(T, C)                                                                                                        \
-    hipLaunchKernelGGL((add_rmsnorm_rows_kernel<DT, T, C>), grid, dim3(T), 0, s, a, b, weight, residual, normed, width, eps)
+#define FH_NORM(C) \
+    hipLaunchKernelGGL((add_rmsnorm_rows_kernel<DT, C>), grid, block, 0, s, a, b, weight, residual, normed, width, eps)
     if (width % 4 != 0 || per_thread > (uint32_t)kNormMaxCache) {
         hipLaunchKernelGGL(add_rmsnorm_any_kernel<DT>, grid, block, 0, s, a, b, weight, residual, normed, width, eps);
     } else if (per_thread <= 2) {
-        FH_NORM(256, 2);
+        FH_NORM(2);
     } else if (per_thread <= 5) {
-        FH_NORM(256, 5);
+        FH_NORM(5);
     } else if (per_thread <= 8) {
-        FH_NORM(256, 8);
+        FH_NORM(8);
     } else {
-        FH_NORM(256, kNormMaxCache);
+        FH_NORM(kNormMaxCache);
     }
 #undef FH_NORM
 }
