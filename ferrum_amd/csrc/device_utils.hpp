@@ -210,8 +210,9 @@ constexpr uint32_t kIq4Table3 = 0xf1d9c5b5u;  //    53   69   89  113
 // zeros or ones in the other: their exclusive or is the entry, where the halves hold what the other's ones would flip,
 // flipped.  (A third v_perm_b32 that picks by the top bit, and its selector, took 10.9 ns of a SIMD for four nibbles, this takes 7.5, and
 // the widening below a mask for one of two v_perm_b32: a quarter of a super-block is 260 vector instructions instead of 292.  us,
-// before / now: 16 f16 rows of 8192 x 4096 10.2 / 9.3, 512 of 17408 x 5120 121.3 / 118.4, one f32 row of 151936 x 2048 55.6 / 50.6,
-// the routed FFN of 200 f32 tokens, 256 experts, 194 / 187.)
+// before / now: 16 f16 rows of 8192 x 4096 9.6 / 8.7, 106 bf16 rows of 21557 x 512 18.3 / 17.5, one f32 row of 151936 x 2048 48.1 / 46.3,
+// the routed FFN of 512 f16 tokens, 256 experts, 192 / 181; the 256-row tiles, 512 of 17408 x 5120, even:
+// profiles/waits_loads_lookups_us.txt.)
 constexpr uint32_t kIq4Lower0 = 0x3f2d18feu, kIq4Lower1 = 0x8995a24fu, kIq4Upper0 = 0x59668d81u, kIq4Upper1 = 0x0e263ab5u;
 constexpr uint32_t iq4_selected(uint64_t table, uint32_t selector) {   // one byte of v_perm_b32
     return (uint32_t)(selector < 8    ? table >> (8 * selector) & 0xff

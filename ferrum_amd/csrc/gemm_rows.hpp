@@ -157,8 +157,9 @@ __global__ __launch_bounds__(kRowsThreads) void gemm_rows_kernel(const RowsParam
             // sight but puts none of its own before the reads of what they write; the build counts the loads
             // between the two in the generated code (ferrum_amd/isa_check.py).  (Requested by the builtin for global
             // loads, which is a flat access to the compiler, they made it wait for everything outstanding before the first
-            // tile of every super-block.  us then / now: 16 x 28672 x 4096 27.8 / 25.3, 64 x 5120 x 17408 43.0 / 40.5,
-            // Q6_K 32 x 5120 x 17408 37.2 / 34.0, f32 8 x 17408 x 5120 47.2 / 44.3.)
+            // tile of every super-block.  us then / now: 64 x 5120 x 17408 44.1 / 42.7, Q6_K
+            // 32 x 5120 x 17408 38.1 / 34.9, Q4_K 16 x 28672 x 4096 27.8 / 24.9 where it is asked to take it; 36 drawn products
+            // 1.04 x in the mean: profiles/waits_loads_lookups_us.txt.)
             asm volatile("s_waitcnt vmcnt(%0)" ::"n"(T * Quarter<TYPE>::kLoads) : "memory");
             u32x4 frag[TT][kFrags];
 #pragma unroll

@@ -592,7 +592,7 @@ __global__ __launch_bounds__(kResThreads) void expert_ring_kernel(const uint8_t*
             for (int b = 0; b < NB; ++b) {
                 // Rows of an even number of 210-byte blocks begin at a dword, every other block between two, where LDS takes longer
                 // for 16 bytes than for the two aligned reads that cover them (us, routed FFN of 256 experts, Q4_K with Q6_K 2048 x 512
-                // down, 200 / 512 / 1024 tokens: 222 / 200 / 343, so 205 / 190 / 322).  (Where rows are of an odd number the lanes
+                // down, 200 / 512 / 1024 tokens: 224 / 195 / 343, so 208 / 184 / 320).  (Where rows are of an odd number the lanes
                 // differ.)
                 if constexpr (TYPE == kQ6K && NB % 2 == 0) q[b].load_by_dwords(slot + b * kBB, g, (b & 1) != 0);
                 else q[b].load(slot + b * kBB, g);

@@ -422,7 +422,7 @@ __device__ __forceinline__ void gemv_stream_body(const StreamParams& p) {
                 uint2 sc8;
                 uint16_t dbits;
                 // A read of 16 bytes that begins between two dwords takes LDS longer than the two aligned ones that cover it
-                // (us: 151936 x 5120 141 / 133, 34816 x 5120 39.4 / 36.5, 5120 x 17408 23.7 / 22.8).  With rows of 16 bits and two
+                // (us: 151936 x 5120 126 / 117, 34816 x 5120 34.8 / 32.7, 5120 x 17408 22.5 / 21.5; profiles/waits_loads_lookups_us.txt).  With rows of 16 bits and two
                 // blocks a wave their registers would leave two workgroups a compute unit instead of three (8192 x 28672 54 / 59).
                 constexpr bool kByDwords = DT == FH_F32 || MAXB != 2;
                 if (kByDwords && (b & 1u)) {   // two bytes behind a dword
@@ -731,16 +731,16 @@ StreamPlan gemv_stream_plan(uint32_t ggml_type, uint32_t n, uint32_t k, uint32_t
     plan.waves = 8u;
     plan.lds_bytes = h * plan.row_stride + plan.waves * slot + plan.waves * 64u;
     // Matrices of a megabyte or two finish sooner on the FMA kernel's smaller workgroups.  A Q6_K tile is 46% longer and
-    // only two share a compute unit: rows that must be cut into segments in any case gain (5120 x 17408: 27.7 / 22.8), and so do large
-    // matrices (us, weights out of every cache, FMA against this kernel: 34816 x 5120 39.4 / 36.5, 128256 x 4096 104 / 95, 152064 x 3584
-    // 111.5 / 100, 151936 x 5120 142.8 / 133).
+    // only two share a compute unit: rows that must be cut into segments in any case gain (5120 x 17408: 25.2 / 21.5), and so do large
+    // matrices (us, weights out of every cache, FMA against this kernel: 34816 x 5120 36.5 / 32.7, 128256 x 4096 92 / 84, 152064 x 3584
+    // 105 / 90, 151936 x 5120 137 / 117; profiles/waits_loads_lookups_us.txt).
     // Rows of 16 bits gain 1% there and are 0.9e-7 from 64 bits on the FMA kernel against 0.95e-7 here (f32 rows 1.9e-7 against
     // 0.9e-7), and two or three f32 rows share their weights through the caches on the FMA kernel (2 x 34816 x 5120 58.3 us there
     // against 64.6, 2 x 100000 x 2048 67.6 / 74.5): they come from a million super-blocks on, where the FMA kernel
     // cannot cut a row evenly over its eight block slots.
-    // One f32 row of eight super-blocks and more gains from a quarter of a million of them on, whole or cut (22000 x 3072 17.4 / 15.1,
-    // 17408 x 5120 22.6 / 21.3, 60000 x 2048 27.8 / 26.2, 36000 x 3584 31.7 / 28.2, 12000 x 10240 36.3 / 29.3; but 9000 x 6144 15.4 / 16.1,
-    // 5120 x 8192 12.3 / 13.6, 7000 x 4096 8.4 / 8.7, and of shorter rows 40000 x 1536 17.3 / 17.2, 100000 x 1024 21.2 / 31.2).
+    // One f32 row of eight super-blocks and more gains from a quarter of a million of them on, whole or cut (22000 x 3072 16.3 / 15.0,
+    // 17408 x 5120 21.9 / 20.1, 60000 x 2048 27.2 / 24.8, 36000 x 3584 29.8 / 26.5, 12000 x 10240 33.6 / 27.7; but 9000 x 6144 14.8 / 15.4,
+    // 5120 x 8192 11.6 / 12.9, 7000 x 4096 7.8 / 8.3, and of shorter rows 40000 x 1536 16.8 / 16.1, 100000 x 1024 22.0 / 28.6).
     // Cut rows only while their partial sums fit any scratch, the fixed one of calls that must not allocate among them: the FMA kernel
     // would need none.
     const uint64_t blocks = (uint64_t)n * nb;

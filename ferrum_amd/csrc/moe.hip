@@ -119,8 +119,8 @@ __device__ __forceinline__ void store8(void* p, size_t i, uint32_t dtype, const 
 }
 
 // The types are template parameters, and the row of an element group is a 32-bit division (element counts fit 32 bits): with
-// switches on the types and a 64-bit division per group, us from a graph: 1 x 17408 f32 2.8, now 2.2, 8 x 17408 f16 3.3 / 2.1, 128 x 17408
-// bf16 5.1 / 4.3, 512 x 17408 f16 14.2 / 12.8, 1999 x 17408 bf16 39.4 / 37.4 (5.6 TB/s).
+// switches on the types and a 64-bit division per group, us from a graph: 1 x 17408 f32 2.6, now 1.9, 8 x 17408 f16 3.1 / 2.0, 128 x 17408
+// bf16 4.9 / 4.1, 512 x 17408 f16 12.9 / 11.9, 1999 x 17408 bf16 35.0 / 33.7 (6.2 TB/s; profiles/waits_loads_lookups_us.txt).
 template <uint32_t in_dtype, uint32_t out_dtype>
 __device__ __forceinline__ void silu_mul8(const void* in, void* out, size_t row, uint32_t column, uint32_t intermediate, size_t to) {
     float gate[8], up[8], result[8];

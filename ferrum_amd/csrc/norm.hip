@@ -70,8 +70,9 @@ __device__ __forceinline__ float4 rounded_sum(float4 x, float4 y) {
 //
 // A row or a few of them are one chain: launch, loads, sum, store.  All loads are requested before the first is waited for
 // (groups past the row read its last one again and count for nothing); waited for group by group, from a graph, us: 1 x 5120 f32
-// 3.0, now 2.4, 8 x 5120 f16 3.2 / 2.5, 24 x 4096 f32 3.0 / 2.4, 128 x 5120 bf16 3.5 / 2.8, 100 x 8192 f32 5.0 / 3.8, 512 x
-// 5120 f16 4.9 / 4.5, 1999 x 5120 bf16 13.2 / 13.0 (6.3 TB/s).  512 threads a row take the same, 1024 a tenth more.
+// 2.8, now 2.2, 8 x 5120 f16 3.0 / 2.4, 24 x 4096 f32 2.8 / 2.3, 128 x 5120 bf16 3.3 / 2.6, 100 x 8192 f32 4.8 / 3.6, 512 x
+// 5120 f16 4.6 / 4.3, 1999 x 5120 bf16 13.0 / 12.5 (6.5 TB/s; profiles/waits_loads_lookups_us.txt).  512 threads a row take the same, 1024 a
+// tenth more.
 template <int DT, int kNormCache>
 __global__ __launch_bounds__(kNormThreads) void add_rmsnorm_rows_kernel(
     const void* __restrict__ a, const void* __restrict__ b, const void* __restrict__ weight,
